@@ -5,10 +5,11 @@
 Compiles the translation units below with hipcc, in parallel, and links them into
 chromo_amd/libchromo_hip.so:
 
-* chromo_hip.hip: one-wavefront kernels, RNG, density, tape, host entry points;
+* chromo_hip.hip: RNG, density, tape, checkpoints, host entry points;
 * chromo_energy.hip: energies and their adjoint;
-* chromo_spec.hip, once per W in SPEC_WAVES (2): the speculative kernel with W
-  wavefronts per replica.
+* chromo_step.hip: one proposal per launch, and the kernel for replicas of any kind;
+* chromo_run.hip and chromo_spec.hip, once per binder count (1..4): the one-wavefront
+  and the speculative persistent kernels.
 
 -ffp-contract=off keeps every multiply and add separately rounded, as in the
 reference's x86-64 build; packed FP32 instructions are disabled.
@@ -28,12 +29,13 @@ ROOT = HERE.parent
 CSRC = HERE / "csrc"
 OUT = HERE / "libchromo_hip.so"
 ARCH = os.environ.get("CHROMO_OFFLOAD_ARCH", "gfx950")
-SPEC_WAVES = (2,)
+BINDERS = (1, 2, 3, 4)
 
-# (source, extra flags, object name)
-UNITS = [(CSRC / "chromo_hip.hip", [], "chromo_hip.o"),
-         (CSRC / "chromo_energy.hip", [], "chromo_energy.o")] + \
-        [(CSRC / "chromo_spec.hip", [f"-DCHROMO_SPEC_W={w}"], f"chromo_spec_w{w}.o") for w in SPEC_WAVES]
+# (source, extra flags, object name), the longest to compile first
+UNITS = [(CSRC / "chromo_step.hip", [], "chromo_step.o")] + \
+        [(CSRC / f"chromo_{k}.hip", [f"-DCHROMO_NB={b}"], f"chromo_{k}_{b}.o")
+         for b in reversed(BINDERS) for k in ("spec", "run")] + \
+        [(CSRC / "chromo_energy.hip", [], "chromo_energy.o"), (CSRC / "chromo_hip.hip", [], "chromo_hip.o")]
 
 FLAGS = [
     f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-ffp-contract=off",

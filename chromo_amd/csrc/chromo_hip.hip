@@ -1,7 +1,7 @@
-// chromo_hip.hip -- MI355X (gfx950) kernels and C ABI for chromo's Monte Carlo inner loop:
-// the one-wavefront persistent and one-move-per-launch kernels, RNG seeding,
-// density initialisation, the field-dE tape and the host entry points.  The
-// speculative multi-wavefront kernel is in chromo_spec.hip.
+// chromo_hip.hip -- C ABI of chromo's Monte Carlo inner loop on MI355X (gfx950): RNG
+// seeding, density initialisation, the field-dE tape, checkpoints and the host entry
+// points.  The Monte Carlo kernels are in chromo_run.hip (one wavefront per replica),
+// chromo_spec.hip (speculative) and chromo_step.hip (one proposal per launch).
 #include <hip/hip_runtime.h>
 
 #include <math.h>
@@ -18,164 +18,22 @@
 using namespace chromo;
 
 namespace chromo {
-hipError_t spec_launch_w2(const chromo_replica *, int, int64_t, int, hipStream_t);
+// chromo_run.hip and chromo_spec.hip, one translation unit per binder count
+hipError_t run_launch_1(const chromo_replica *, int, int64_t, bool, hipStream_t);
+hipError_t run_launch_2(const chromo_replica *, int, int64_t, bool, hipStream_t);
+hipError_t run_launch_3(const chromo_replica *, int, int64_t, bool, hipStream_t);
+hipError_t run_launch_4(const chromo_replica *, int, int64_t, bool, hipStream_t);
+hipError_t spec_launch_1(const chromo_replica *, int, int64_t, hipStream_t);
+hipError_t spec_launch_2(const chromo_replica *, int, int64_t, hipStream_t);
+hipError_t spec_launch_3(const chromo_replica *, int, int64_t, hipStream_t);
+hipError_t spec_launch_4(const chromo_replica *, int, int64_t, hipStream_t);
+// chromo_step.hip
+hipError_t step_setup(int lds_limit);
+hipError_t step_launch(const chromo_replica *, int rep, int ctrl, hipStream_t);
+hipError_t run_any_launch(const chromo_replica *, int, int64_t, hipStream_t);
 }  // namespace chromo
 
 namespace {
-
-// Persistent mc_sim: one workgroup (one wave) per replica.
-__global__ void __launch_bounds__(64) k_mc_run(const chromo_replica *__restrict__ reps, int n_reps, int64_t steps,
-                                               int max_bp1)
-{
-    const int r = blockIdx.x;
-    if (r >= n_reps) return;
-    __shared__ chromo_replica Rs;
-    load_record(&Rs, &reps[r]);
-    wave_sync();
-    const chromo_replica *R = &Rs;
-    if (R->counters[CHROMO_CNT_ERROR] != 0) return;
-    if (R->B < 1 || R->B + 1 > max_bp1) {
-        counters_error(R, ERR_NBINDERS);
-        return;
-    }
-    const int Bp1 = R->B + 1;
-    const SegLds G = seg_lds(lds_dyn, Bp1);
-    seg_clear(G);
-    uint32_t *mt_lds = (uint32_t *)(lds_dyn + wide_lds_bytes(Bp1));
-    const bool need_mt = any_binding(R);
-    WaveRng rng;
-    rng_load(R, rng, mt_lds, need_mt);
-    Counters K;
-    counters_load(R, K);
-    const int nc = R->n_ctrl < MAX_CTRL ? R->n_ctrl : MAX_CTRL;
-    __shared__ chromo_ctrl sctrl[MAX_CTRL];
-    if (lane_id() == 0)
-        for (int i = 0; i < nc; ++i) sctrl[i] = R->ctrl[i];
-    __syncthreads();
-    int err = 0;
-    if (R->twist) {
-        switch (R->B) {
-        case 1: run_steps<1, true>(R, rng, K, sctrl, nc, steps, err, G, lds_dyn); break;
-        case 2: run_steps<2, true>(R, rng, K, sctrl, nc, steps, err, G, lds_dyn); break;
-        case 3: run_steps<3, true>(R, rng, K, sctrl, nc, steps, err, G, lds_dyn); break;
-        case 4: run_steps<4, true>(R, rng, K, sctrl, nc, steps, err, G, lds_dyn); break;
-        default: err = ERR_NBINDERS; break;
-        }
-    } else {
-        switch (R->B) {
-        case 1: run_steps<1>(R, rng, K, sctrl, nc, steps, err, G, lds_dyn); break;
-        case 2: run_steps<2>(R, rng, K, sctrl, nc, steps, err, G, lds_dyn); break;
-        case 3: run_steps<3>(R, rng, K, sctrl, nc, steps, err, G, lds_dyn); break;
-        case 4: run_steps<4>(R, rng, K, sctrl, nc, steps, err, G, lds_dyn); break;
-        default: err = ERR_NBINDERS; break;
-        }
-    }
-    rng_store(R, rng, need_mt);
-    if (lane_id() == 0)
-        for (int i = 0; i < nc; ++i) R->ctrl[i] = sctrl[i];
-    counters_store(R, K, err);
-}
-
-// k_mc_run for the replicas with NB binder types and twist flag TW only; the others
-// are left to the launch of their own kind.  One instantiation per kernel, so
-// that its registers are allocated for that one alone (the all-kinds kernel above
-// spills for the largest of its eight).
-template <int NB, bool TW>
-__global__ void __launch_bounds__(64) k_mc_run_nb(const chromo_replica *__restrict__ reps, int n_reps,
-                                                  int64_t steps)
-{
-    const int r = blockIdx.x;
-    if (r >= n_reps) return;
-    __shared__ chromo_replica Rs;
-    load_record(&Rs, &reps[r]);
-    wave_sync();
-    const chromo_replica *R = &Rs;
-    if (R->B != NB || (R->twist != 0) != TW) return;
-    if (R->counters[CHROMO_CNT_ERROR] != 0) return;
-    constexpr int Bp1 = NB + 1;
-    const SegLds G = seg_lds(lds_dyn, Bp1);
-    seg_clear(G);
-    uint32_t *mt_lds = (uint32_t *)(lds_dyn + wide_lds_bytes(Bp1));
-    const bool need_mt = any_binding(R);
-    WaveRng rng;
-    rng_load(R, rng, mt_lds, need_mt);
-    Counters K;
-    counters_load(R, K);
-    const int nc = R->n_ctrl < MAX_CTRL ? R->n_ctrl : MAX_CTRL;
-    __shared__ chromo_ctrl sctrl[MAX_CTRL];
-    if (lane_id() == 0)
-        for (int i = 0; i < nc; ++i) sctrl[i] = R->ctrl[i];
-    __syncthreads();
-    int err = 0;
-    run_steps<NB, TW>(R, rng, K, sctrl, nc, steps, err, G, lds_dyn);
-    rng_store(R, rng, need_mt);
-    if (lane_id() == 0)
-        for (int i = 0; i < nc; ++i) R->ctrl[i] = sctrl[i];
-    counters_store(R, K, err);
-}
-
-template <int NB, bool TW>
-hipError_t launch_run_nb(const chromo_replica *d_reps, int n_reps, int64_t steps, hipStream_t st)
-{
-    // the attribute is set once per process: setting it costs far more than a launch
-    static bool attr_set = false;
-    const size_t bytes = mc_lds_bytes(NB + 1);
-    if (!attr_set) {
-        hipError_t e = hipFuncSetAttribute((const void *)k_mc_run_nb<NB, TW>,
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
-        if (e != hipSuccess) return e;
-        attr_set = true;
-    }
-    hipLaunchKernelGGL((k_mc_run_nb<NB, TW>), dim3(n_reps), dim3(WAVE), bytes, st, d_reps, n_reps, steps);
-    return hipGetLastError();
-}
-
-// One mc_step per launch (the plain path / mc_step API).
-__global__ void __launch_bounds__(64) k_mc_step(const chromo_replica *__restrict__ reps, int rep, int ci,
-                                                int max_bp1)
-{
-    __shared__ chromo_replica Rs;
-    load_record(&Rs, &reps[rep]);
-    wave_sync();
-    const chromo_replica *R = &Rs;
-    if (R->counters[CHROMO_CNT_ERROR] != 0) return;
-    if (R->B < 1 || R->B + 1 > max_bp1) {
-        counters_error(R, ERR_NBINDERS);
-        return;
-    }
-    const int Bp1 = R->B + 1;
-    const SegLds G = seg_lds(lds_dyn, Bp1);
-    seg_clear(G);
-    uint32_t *mt_lds = (uint32_t *)(lds_dyn + wide_lds_bytes(Bp1));
-    chromo_ctrl C = R->ctrl[ci];
-    const bool need_mt = (C.move == CHROMO_CHANGE_BINDING_STATE);
-    WaveRng rng;
-    rng_load(R, rng, mt_lds, need_mt);
-    Counters K;
-    counters_load(R, K);
-    MoveOut o;
-    if (R->twist) {
-        switch (R->B) {
-        case 1: mc_step_dev<1, true>(R, rng, C, o, G, lds_dyn, 1); break;
-        case 2: mc_step_dev<2, true>(R, rng, C, o, G, lds_dyn, 1); break;
-        case 3: mc_step_dev<3, true>(R, rng, C, o, G, lds_dyn, 1); break;
-        case 4: mc_step_dev<4, true>(R, rng, C, o, G, lds_dyn, 1); break;
-        default: o.err = ERR_NBINDERS; o.n = 0; break;
-        }
-    } else {
-        switch (R->B) {
-        case 1: mc_step_dev<1>(R, rng, C, o, G, lds_dyn, 1); break;
-        case 2: mc_step_dev<2>(R, rng, C, o, G, lds_dyn, 1); break;
-        case 3: mc_step_dev<3>(R, rng, C, o, G, lds_dyn, 1); break;
-        case 4: mc_step_dev<4>(R, rng, C, o, G, lds_dyn, 1); break;
-        default: o.err = ERR_NBINDERS; o.n = 0; break;
-        }
-    }
-    if (!o.err && o.n > 0) record(R, C, o, K);
-    rng_store(R, rng, need_mt);
-    if (lane_id() == 0) R->ctrl[ci] = C;
-    counters_store(R, K, o.err);
-}
 
 // Flags replicas whose binder count is not in mask (bit B set for B present).
 __global__ void k_check_binders(const chromo_replica *reps, int n_reps, int mask)
@@ -544,7 +402,6 @@ int check_reps(const chromo_replica *d_reps, int32_t n_reps)
 
 size_t g_lds_bytes = 0;   // field tape: LDS move arena + MT block
 int g_lds_bp1 = 0;        // largest binder count + 1 the tape's arena fits
-size_t g_mc_bytes = 0;    // Monte Carlo kernels: evaluator block + MT block, for B = 4
 
 // Dynamic LDS per workgroup, sized for the largest binder count that fits the
 // device's per-workgroup limit, set once per process.
@@ -557,13 +414,11 @@ int ensure_lds()
     int bp1 = CHROMO_MAX_BINDERS + 1;
     while (bp1 > 1 && lds_bytes_for(bp1) + 1024 > (size_t)lim) --bp1;
     if (bp1 < 2) return set_err(-2, "device LDS per workgroup too small for the move arena");
-    const size_t mc = mc_lds_bytes(CHROMO_MAX_BINDERS + 1);
-    if (mc + 1024 > (size_t)lim) return set_err(-2, "device LDS per workgroup too small for the evaluator");
-    HIPC(hipFuncSetAttribute((const void *)k_mc_run, hipFuncAttributeMaxDynamicSharedMemorySize, (int)mc));
-    HIPC(hipFuncSetAttribute((const void *)k_mc_step, hipFuncAttributeMaxDynamicSharedMemorySize, (int)mc));
+    const hipError_t e = chromo::step_setup(lim);
+    if (e == hipErrorInvalidValue) return set_err(-2, "device LDS per workgroup too small for the evaluator");
+    HIPC(e);
     HIPC(hipFuncSetAttribute((const void *)k_field_tape, hipFuncAttributeMaxDynamicSharedMemorySize,
                              (int)lds_bytes_for(bp1)));
-    g_mc_bytes = mc;
     g_lds_bp1 = bp1;
     g_lds_bytes = lds_bytes_for(bp1);
     return 0;
@@ -759,9 +614,7 @@ int chromo_mc_run(const chromo_replica *d_reps, int32_t n_reps, int64_t num_step
     if (num_steps < 0) return set_err(-1, "num_steps < 0");
     rc = ensure_lds();
     if (rc) return rc;
-    hipLaunchKernelGGL(k_mc_run, dim3(n_reps), dim3(64), g_mc_bytes, (hipStream_t)stream, d_reps,
-                       n_reps, num_steps, CHROMO_MAX_BINDERS + 1);
-    HIPC(launch_err());
+    HIPC(chromo::run_any_launch(d_reps, n_reps, num_steps, (hipStream_t)stream));
     return 0;
 }
 
@@ -781,32 +634,27 @@ int chromo_mc_run_tuned(const chromo_replica *d_reps, int32_t n_reps, int64_t nu
     if (W != 1 && W != 2) return set_err(-1, "waves_per_replica must be 1 or 2");
     rc = ensure_lds();
     if (rc) return rc;
-    int bp1 = 0;
-    for (int b = 1; b <= CHROMO_MAX_BINDERS; ++b)
-        if (binder_mask & (1 << b)) bp1 = b + 1;
     hipStream_t st = (hipStream_t)stream;
     // replicas whose binder count is not in binder_mask fail with ERR_NBINDERS
     hipLaunchKernelGGL(k_check_binders, dim3((n_reps + 63) / 64), dim3(64), 0, st, d_reps, n_reps,
                        binder_mask);
     HIPC(launch_err());
-    if (W == 1) {
-        // one kernel per binder count (and twist flag) present
-        hipError_t e = hipSuccess;
-        if ((binder_mask & 2) && e == hipSuccess) e = launch_run_nb<1, false>(d_reps, n_reps, num_steps, st);
-        if ((binder_mask & 4) && e == hipSuccess) e = launch_run_nb<2, false>(d_reps, n_reps, num_steps, st);
-        if ((binder_mask & 8) && e == hipSuccess) e = launch_run_nb<3, false>(d_reps, n_reps, num_steps, st);
-        if ((binder_mask & 16) && e == hipSuccess) e = launch_run_nb<4, false>(d_reps, n_reps, num_steps, st);
-        if ((binder_mask & 0x200) && e == hipSuccess) e = launch_run_nb<1, true>(d_reps, n_reps, num_steps, st);
-        if ((binder_mask & 0x400) && e == hipSuccess) e = launch_run_nb<2, true>(d_reps, n_reps, num_steps, st);
-        if ((binder_mask & 0x800) && e == hipSuccess) e = launch_run_nb<3, true>(d_reps, n_reps, num_steps, st);
-        if ((binder_mask & 0x1000) && e == hipSuccess) e = launch_run_nb<4, true>(d_reps, n_reps, num_steps, st);
+    using RunFn = hipError_t (*)(const chromo_replica *, int, int64_t, bool, hipStream_t);
+    using SpecFn = hipError_t (*)(const chromo_replica *, int, int64_t, hipStream_t);
+    static const RunFn run_fn[] = {chromo::run_launch_1, chromo::run_launch_2, chromo::run_launch_3,
+                                   chromo::run_launch_4};
+    static const SpecFn spec_fn[] = {chromo::spec_launch_1, chromo::spec_launch_2, chromo::spec_launch_3,
+                                     chromo::spec_launch_4};
+    // one kernel per binder count (and, with one wavefront, twist flag) present
+    for (int b = 1; b <= CHROMO_MAX_BINDERS; ++b) {
+        if (!(binder_mask & (1 << b))) continue;
+        hipError_t e = W == 1 ? run_fn[b - 1](d_reps, n_reps, num_steps, false, st)
+                              : spec_fn[b - 1](d_reps, n_reps, num_steps, st);
+        if (e == hipSuccess && W == 1 && (binder_mask & (1 << (8 + b))))
+            e = run_fn[b - 1](d_reps, n_reps, num_steps, true, st);
+        if (e == hipErrorInvalidValue) return set_err(-1, "LDS of this launch shape exceeds the device limit");
         HIPC(e);
-        return 0;
     }
-    hipError_t e = chromo::spec_launch_w2(d_reps, n_reps, num_steps, binder_mask & 0x1e, st);
-    if (e == hipErrorInvalidValue)
-        return set_err(-1, "LDS of this launch shape exceeds the device limit");
-    HIPC(e);
     return 0;
 }
 
@@ -815,9 +663,7 @@ int chromo_mc_step(const chromo_replica *d_reps, int32_t rep, int32_t ctrl, void
     if (d_reps == nullptr || rep < 0) return set_err(-1, "bad replica");
     int rc = ensure_lds();
     if (rc) return rc;
-    hipLaunchKernelGGL(k_mc_step, dim3(1), dim3(64), g_mc_bytes, (hipStream_t)stream, d_reps, rep,
-                       ctrl, CHROMO_MAX_BINDERS + 1);
-    HIPC(launch_err());
+    HIPC(chromo::step_launch(d_reps, rep, ctrl, (hipStream_t)stream));
     return 0;
 }
 
@@ -847,8 +693,7 @@ int chromo_mc_run_plain(const chromo_replica *d_reps, int32_t rep, int64_t num_s
         for (int ci = 0; ci < h.n_ctrl; ++ci) {
             if (c[ci].on == 1)
                 for (int j = 0; j < c[ci].num_per_cycle; ++j)
-                    hipLaunchKernelGGL(k_mc_step, dim3(1), dim3(64), g_mc_bytes, st, d_reps, rep, ci,
-                                       CHROMO_MAX_BINDERS + 1);
+                    HIPC(chromo::step_launch(d_reps, rep, ci, st));
             hipLaunchKernelGGL(k_update_amplitudes, dim3(1), dim3(64), 0, st, d_reps, rep, ci);
         }
         HIPC(launch_err());

@@ -1,14 +1,14 @@
 // chromo_mc.hpp -- device code of one Monte Carlo move, shared by the kernels.
 //
 // One wavefront runs a replica's sequential Markov chain
-// (chromo/mc/mc_sim.pyx:26-182).  Moves of at most SEG_MAX beads are evaluated
-// by seg_eval (chromo_seg.hpp).  Larger ones spread their 16*n voxel
-// contributions (2 configurations x 8 corners per bead) over the 64 lanes and
-// group them per voxel in the replica's global scratch arena through a hash
-// table, ordered by contribution index and folded per voxel in the reference's
-// order, so each voxel's delta density is the reference's left fold
-// (chromo/fields.pyx:1491-1520) bit for bit.  Energy terms are reduced across the
-// wavefront in a fixed order; no global atomics are used.
+// (chromo/mc/mc_sim.pyx:26-182).  ev_eval (chromo_eval.hpp) evaluates a move in LDS.
+// A move that touches more voxels than its block holds, and tangent or binding moves
+// of more than EV_LANES beads, spread their 16*n voxel contributions (2
+// configurations x 8 corners per bead) over the 64 lanes and group them per voxel in
+// the replica's global scratch arena through a hash table, ordered by contribution
+// index and folded per voxel in the reference's order, so each voxel's delta density
+// is the reference's left fold (chromo/fields.pyx:1491-1520) bit for bit.  Energy
+// terms are reduced across the wavefront in a fixed order; no global atomics are used.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -35,8 +35,7 @@ struct Proposal {
 
 }  // namespace
 
-#include "chromo_seg.hpp"
-#include "chromo_big.hpp"
+#include "chromo_eval.hpp"
 
 namespace {
 
@@ -168,16 +167,9 @@ inline size_t lds_bytes_for(int Bp1)
     return L.total + MT_LDS_BYTES;
 }
 
-// Dynamic LDS of the one-wavefront Monte Carlo kernels: one evaluator block for
-// moves of up to SEG_WIDE beads (its start doubles as the SEG_MAX block), then the
-// MT19937 state.
-// The wide block of the one-at-a-time path: a SEG_WIDE evaluator block or two
-// SEG_MAX ones, whichever is larger; the long-move evaluator uses all of it.
-__host__ __device__ inline size_t wide_lds_bytes(int Bp1)
-{
-    const size_t a = seg_layout<SEG_WIDE>(Bp1).total, b = 2 * seg_layout<SEG_MAX>(Bp1).total;
-    return a > b ? a : b;
-}
+// Dynamic LDS of the one-wavefront Monte Carlo kernels: the evaluator's one-at-a-time
+// block, then the MT19937 state.
+__host__ __device__ inline size_t wide_lds_bytes(int Bp1) { return ev_layout(Bp1, true).total; }
 
 inline size_t mc_lds_bytes(int Bp1) { return wide_lds_bytes(Bp1) + MT_LDS_BYTES; }
 
@@ -878,51 +870,26 @@ __device__ __forceinline__ void track_acceptance(chromo_ctrl &C, bool accepted)
     }
 }
 
-// mc_step's evaluation of proposal P with Metropolis draw u: the evaluator that
-// holds it, the commit of an accepted move, the acceptance tracker.  G: the
-// caller's SEG_MAX evaluator block.  wide: the start of an LDS region that holds a
-// SEG_WIDE block (nullptr if none) and overlaps nstd SEG_MAX blocks, whose hashes
-// are emptied again after it is used.
+// mc_step's evaluation of proposal P with Metropolis draw u in the one-at-a-time block
+// S (its hash empty on entry and on return), the commit of an accepted move, the
+// acceptance tracker; the global arena for what ev_eval does not hold.
 template <int NB, bool TW = false>
-__device__ __forceinline__ void mc_evaluate(const chromo_replica *R, chromo_ctrl &C, MoveOut &out, const Proposal &P,
-                                            double u, const SegLds &G, char *wide, int nstd)
+__device__ __forceinline__ void mc_evaluate(const chromo_replica *R, const EvConst &EC, chromo_ctrl &C, MoveOut &out,
+                                            const Proposal &P, double u, const EvLds &S)
 {
     const int64_t n = P.n;
-    {
-        SegRes sr;
-        sr.overflow = 1;
-        if (n <= SEG_MAX) {
-            SegKeep<NB> K;
-            seg_eval<NB, SEG_MAX, TW>(R, P, u, G, sr, K);
-            if (!sr.overflow) {
-                if (sr.accepted) seg_commit<NB>(R, P.move, n, P.binder, P.mynew, K, G, sr.U);
-                wave_sync_global();
-            }
-        } else if (n <= SEG_WIDE && wide != nullptr) {
-            const SegLds GW = seg_lds<SEG_WIDE>(wide, NB + 1);
-            seg_clear<SEG_WIDE>(GW);
-            SegKeep<NB> K;
-            seg_eval<NB, SEG_WIDE, TW>(R, P, u, GW, sr, K);
-            if (!sr.overflow) {
-                if (sr.accepted) seg_commit<NB>(R, P.move, n, P.binder, P.mynew, K, GW, sr.U);
-                wave_sync_global();
-            }
-            // the wide block covered the SEG_MAX blocks: their hashes must be empty again
-            for (int b = 0; b < nstd; ++b)
-                seg_clear<SEG_MAX>(seg_lds<SEG_MAX>(wide + (size_t)b * seg_layout<SEG_MAX>(NB + 1).total, NB + 1));
-        } else if (wide != nullptr && big_move(P.move)) {
-            const BigLds GB = big_lds(wide, NB + 1, wide_lds_bytes(NB + 1));
-            if (GB.ucap > 0) {
-                big_eval<NB, TW>(R, P, u, GB, sr);
-                if (!sr.overflow) {
-                    if (sr.accepted) big_commit<NB>(R, P, GB, sr.U);
-                    wave_sync_global();
-                }
-                for (int b = 0; b < nstd; ++b)
-                    seg_clear<SEG_MAX>(seg_lds<SEG_MAX>(wide + (size_t)b * seg_layout<SEG_MAX>(NB + 1).total, NB + 1));
-            }
-        }
+    EvRes sr;
+    sr.overflow = 1;
+    const bool lanes = P.move == CHROMO_TANGENT_ROTATION || P.move == CHROMO_CHANGE_BINDING_STATE;
+    if (!lanes || n <= EV_LANES) {
+        EvKeep K;
+        EvBeads<NB> B;
+        ev_load<NB, TW>(R, P.move, n, P.ind0, P.indf, 0, lanes ? __shfl(P.mypick, lane_id() & 31) : 0, B);
+        ev_eval<NB, TW>(R, EC, P, u, S, sr, K, B);
         if (!sr.overflow) {
+            if (sr.accepted) ev_commit<NB>(R, P, K, S, sr.U);
+            ev_release(S, sr.U);
+            wave_sync_global();
             out.dEp = sr.dEp;
             out.dEf = sr.dEf;
             out.u = u;
@@ -930,16 +897,15 @@ __device__ __forceinline__ void mc_evaluate(const chromo_replica *R, chromo_ctrl
             out.accepted = sr.accepted;
             out.nbins = sr.U;
         }
-        // larger moves, and the rare small one with too many voxels for seg_eval
-        if (sr.overflow) {
-            const bool uses_field = R->field_on && P.move != CHROMO_TANGENT_ROTATION;
-            if (n > R->bead_cap || (uses_field && n > R->seg_cap)) {
-                out.err = ERR_SEGCAP;
-                out.n = 0;
-                return;
-            }
-            move_body<1, NB, TW>(R, u, P, out);
+    }
+    if (sr.overflow) {
+        const bool uses_field = R->field_on && P.move != CHROMO_TANGENT_ROTATION;
+        if (n > R->bead_cap || (uses_field && n > R->seg_cap)) {
+            out.err = ERR_SEGCAP;
+            out.n = 0;
+            return;
         }
+        move_body<1, NB, TW>(R, u, P, out);
     }
     if (out.err) {
         out.n = 0;
@@ -950,12 +916,12 @@ __device__ __forceinline__ void mc_evaluate(const chromo_replica *R, chromo_ctrl
 
 // mc_step (mc_sim.pyx:106-182) on one wavefront: mc_propose, then mc_evaluate.
 template <int NB, bool TW = false>
-__device__ __forceinline__ void mc_step_dev(const chromo_replica *R, WaveRng &rng, chromo_ctrl &C, MoveOut &out,
-                                            const SegLds &G, char *wide, int nstd)
+__device__ __forceinline__ void mc_step_dev(const chromo_replica *R, const EvConst &EC, WaveRng &rng, chromo_ctrl &C,
+                                            MoveOut &out, const EvLds &S)
 {
     Proposal P;
     double u = 0;
-    if (mc_propose<NB>(R, rng, C, out, P, u)) mc_evaluate<NB, TW>(R, C, out, P, u, G, wide, nstd);
+    if (mc_propose<NB>(R, rng, C, out, P, u)) mc_evaluate<NB, TW>(R, EC, C, out, P, u, S);
 }
 
 // SimpleControl.update_amplitudes (mc_controller.py:126-213)
@@ -1136,8 +1102,8 @@ __device__ __forceinline__ bool any_binding(const chromo_replica *R)
 // ---------------------------------------------------------------------------
 
 template <int NB, bool TW = false>
-__device__ __forceinline__ void run_steps(const chromo_replica *R, WaveRng &rng, Counters &K, chromo_ctrl *sctrl,
-                          int nc, int64_t steps, int &err, const SegLds &G, char *wide)
+__device__ __forceinline__ void run_steps(const chromo_replica *R, const EvConst &EC, WaveRng &rng, Counters &K,
+                          chromo_ctrl *sctrl, int nc, int64_t steps, int &err, const EvLds &S)
 {
     for (int64_t s = 0; s < steps && !err; ++s) {
         for (int ci = 0; ci < nc && !err; ++ci) {
@@ -1145,7 +1111,7 @@ __device__ __forceinline__ void run_steps(const chromo_replica *R, WaveRng &rng,
             if (c.on == 1) {
                 for (int j = 0; j < c.num_per_cycle; ++j) {
                     MoveOut o;
-                    mc_step_dev<NB, TW>(R, rng, c, o, G, wide, 1);
+                    mc_step_dev<NB, TW>(R, EC, rng, c, o, S);
                     if (o.err) {
                         err = o.err;
                         break;

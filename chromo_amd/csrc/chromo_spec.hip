@@ -1,12 +1,12 @@
 // chromo_spec.hip -- the speculative persistent kernel k_mc_spec<W, NB> for one
-// W = CHROMO_SPEC_W (wavefronts per replica); built once per W so that the
-// instantiations compile in parallel.
+// NB = CHROMO_NB (binder types); built once per NB so that the instantiations compile
+// in parallel.
 #include <hip/hip_runtime.h>
 
 #include "chromo_spec.hpp"
 
-#ifndef CHROMO_SPEC_W
-#error "compile with -DCHROMO_SPEC_W=2, 4 or 8"
+#ifndef CHROMO_NB
+#error "compile with -DCHROMO_NB=1 .. 4"
 #endif
 
 #define CHROMO_CAT2(a, b) a##b
@@ -16,15 +16,15 @@ namespace {
 
 // Persistent mc_sim with W wavefronts per replica (one workgroup per replica),
 // for the replicas with NB binder types; the others are left to the launch of
-// their own NB.  Two workgroups share a compute unit (LDS), so a SIMD runs W / 2
-// wavefronts: the register budget is sized for that.
+// their own NB.  One wavefront per SIMD: the full register file.
 template <int W, int NB>
-__global__ void __launch_bounds__(WAVE * W) __attribute__((amdgpu_waves_per_eu(W / 2 > 1 ? W / 2 : 1)))
+__global__ void __launch_bounds__(WAVE * W) __attribute__((amdgpu_waves_per_eu(1)))
 k_mc_spec(const chromo_replica *__restrict__ reps, int n_reps, int64_t steps)
 {
     const int r = blockIdx.x;
     if (r >= n_reps) return;
     __shared__ chromo_replica Rs;
+    __shared__ EvConst EC;
     load_record(&Rs, &reps[r]);
     __syncthreads();
     const chromo_replica *R = &Rs;
@@ -32,24 +32,28 @@ k_mc_spec(const chromo_replica *__restrict__ reps, int n_reps, int64_t steps)
     if (R->counters[CHROMO_CNT_ERROR] != 0) return;
     if (R->twist) {
         // the speculative evaluator has no twist terms: a twisting chain runs
-        // with one wavefront (k_mc_run)
+        // with one wavefront (k_mc_run_nb)
         counters_error(R, ERR_TWIST_WAVES);
         return;
     }
-    spec_run<NB, W>(R, steps);
+    ev_const(&EC, R);
+    __syncthreads();
+    spec_run<NB, W>(R, EC, steps);
 }
 
-template <int NB>
-hipError_t launch_nb(const chromo_replica *d_reps, int n_reps, int64_t steps, hipStream_t st, int lim)
+template <int W, int NB>
+hipError_t launch(const chromo_replica *d_reps, int n_reps, int64_t steps, hipStream_t st)
 {
-    constexpr int W = CHROMO_SPEC_W;
-    const size_t bytes = spec_layout(NB + 1, W).total;
-    if (bytes > (size_t)lim) return hipErrorInvalidValue;
+    const size_t bytes = spec_layout<W>(NB + 1).total;
     // the attribute is set once per process: setting it costs far more than a launch
     static bool attr_set = false;
     if (!attr_set) {
-        hipError_t e = hipFuncSetAttribute((const void *)k_mc_spec<W, NB>,
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+        int dev = 0, lim = 0;
+        hipError_t e = hipGetDevice(&dev);
+        if (e == hipSuccess) e = hipDeviceGetAttribute(&lim, hipDeviceAttributeMaxSharedMemoryPerBlock, dev);
+        if (e != hipSuccess) return e;
+        if (bytes > (size_t)lim) return hipErrorInvalidValue;
+        e = hipFuncSetAttribute((const void *)k_mc_spec<W, NB>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
         if (e != hipSuccess) return e;
         attr_set = true;
     }
@@ -61,25 +65,10 @@ hipError_t launch_nb(const chromo_replica *d_reps, int n_reps, int64_t steps, hi
 
 namespace chromo {
 
-// Launches k_mc_spec<CHROMO_SPEC_W, B> for every binder count B whose bit is set
-// in binder_mask (bit B for B = 1..4).  Returns hipErrorInvalidValue when the
-// LDS of a launch exceeds the device limit.
-hipError_t CHROMO_CAT(spec_launch_w, CHROMO_SPEC_W)(const chromo_replica *d_reps, int n_reps, int64_t steps,
-                                                    int binder_mask, hipStream_t st)
+hipError_t CHROMO_CAT(spec_launch_, CHROMO_NB)(const chromo_replica *d_reps, int n_reps, int64_t steps,
+                                               hipStream_t st)
 {
-    static int lim = 0;
-    hipError_t e = hipSuccess;
-    if (lim == 0) {
-        int dev = 0;
-        if ((e = hipGetDevice(&dev)) != hipSuccess) return e;
-        if ((e = hipDeviceGetAttribute(&lim, hipDeviceAttributeMaxSharedMemoryPerBlock, dev)) != hipSuccess)
-            return e;
-    }
-    if ((binder_mask & 2) && (e = launch_nb<1>(d_reps, n_reps, steps, st, lim)) != hipSuccess) return e;
-    if ((binder_mask & 4) && (e = launch_nb<2>(d_reps, n_reps, steps, st, lim)) != hipSuccess) return e;
-    if ((binder_mask & 8) && (e = launch_nb<3>(d_reps, n_reps, steps, st, lim)) != hipSuccess) return e;
-    if ((binder_mask & 16) && (e = launch_nb<4>(d_reps, n_reps, steps, st, lim)) != hipSuccess) return e;
-    return hipSuccess;
+    return launch<2, CHROMO_NB>(d_reps, n_reps, steps, st);
 }
 
 }  // namespace chromo

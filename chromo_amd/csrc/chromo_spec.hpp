@@ -6,28 +6,39 @@
 namespace {
 
 // ===========================================================================
-// Speculative rounds: W proposals of one controller block evaluated at once.
+// Speculative rounds: several proposals of one controller block evaluated at once.
 //
 // Inside a controller block the amplitudes are fixed, so the random draws of each
 // proposal -- the proposal itself and its Metropolis draw -- do not depend on the
 // accept/reject outcomes before it.  (The exception, a crank-shaft axis shorter
 // than 1e-5 which draws a random axis, is detected and redone one at a time.)
-// Wavefront 0 generates up to W proposals; wavefront w evaluates proposal w
-// against the current state with seg_eval, in its own LDS block.  Resolution
-// walks the proposals in order: proposal s keeps its evaluated dE unless an
-// accepted proposal s' < s of the same round wrote a bead or a voxel that s
-// reads; then s and all later proposals go to the next round and are evaluated
-// again.  Each chain therefore is the reference's sequential chain; only the
-// number of rounds depends on conflicts.  Moves of more than SPEC_NMAX beads run
-// one at a time through mc_step_dev.
+// One wavefront (Shape::GEN) draws proposals ahead into a ring of slots; wavefront w <
+// Shape::EV evaluates slot w of the round against the current state with ev_eval, in
+// its own LDS block.  Resolution walks the slots in order: slot s keeps its evaluated
+// dE unless an accepted slot s' < s of the same round wrote a bead or a voxel that s
+// reads; then s and all later slots go to the next round and are evaluated again.
+// Each chain therefore is the reference's sequential chain; only the number of rounds
+// depends on conflicts.  What a slot cannot hold runs one at a time through
+// mc_step_dev.
+//
+// Two shapes.  W = 2 (more replicas than compute units): wavefront 0 both draws and
+// evaluates, two workgroups share a compute unit.  W = 4 (a compute unit per replica):
+// three evaluators and one wavefront that only draws and keeps the books, so drawing
+// leaves the evaluators' critical path.
 // ===========================================================================
 
-constexpr int SPEC_NMAX = SEG_MAX;    // beads (tangent picks) one wavefront evaluates
-constexpr int SPEC_WMAX = 2;          // wavefronts per replica
-constexpr int SPEC_HASH = 1024;       // conflict-table entries
-constexpr int SPEC_HASH_SHIFT = 22;   // 32 - log2(SPEC_HASH)
-constexpr int SPEC_HASH_SOFT = 512;   // insertions by wavefronts 1.. (wavefront 0 adds <= SEG_UMAX)
-static_assert(SPEC_HASH_SOFT + SEG_UMAX <= SPEC_HASH, "the conflict table must never fill");
+template <int W>
+struct Shape {
+    static_assert(W == 2 || W == 4, "two or four wavefronts");
+    static constexpr int EV = W == 2 ? 2 : 3;       // evaluating wavefronts
+    static constexpr int GEN = W == 2 ? 0 : 3;      // the wavefront that draws
+    static constexpr int BOOK = W == 2 ? 1 : 3;     // the wavefront that books a round
+    static constexpr int RING = W == 2 ? 4 : 8;     // slots
+};
+
+constexpr int SPEC_NMAX = SEG_MAX;    // tangent picks or binding beads of a slot
+constexpr int SPEC_BEADS = 192;       // beads of a crank-shaft, end-pivot or slide slot
+constexpr int SPEC_EVMAX = 3;
 enum : int { SLOT_SMALL = 0, SLOT_EMPTY = 1, SLOT_SEQ = 2 };
 constexpr int CK_WORDS = 40;
 
@@ -51,50 +62,42 @@ struct SpecRes {
 };
 
 struct SpecCtl {
-    int32_t nq, cnt, remaining, err;
-    int32_t used;                             // conflict-table insertions this round
+    int32_t cnt, remaining, err;
     int32_t head;                             // ring position of the round's first slot
     int32_t tag;                              // the round's number in the launch (never repeats)
-    int32_t ready;                            // = tag once the later slots' conflict masks are set
-    int32_t ins;                              // = tag once slot 0's voxels are in the conflict table
-    int32_t stall;                            // = tag when a later wavefront gave up waiting for ins
+    int32_t stall;                            // = tag when a wait passed its bound
+    int32_t done[SPEC_EVMAX];                 // = tag once slot s's result and voxels are published
+    int32_t chk[SPEC_EVMAX];                  // = tag once slot s's conflict mask is set
 };
 
-// LDS exchange area of the one-at-a-time path (seq_step, seq_step_coop).
+// LDS exchange area of the one-at-a-time path (seq_step).
 struct SeqIO {
     uint32_t ck[CK_WORDS];
     int32_t mti, pad0;
     chromo_ctrl C;
     MoveOut out;
-    int32_t coop, pad1;      // seq_step_coop: 0 wavefront 0 alone, 1 both in seg_eval, 2 both in big_eval
-    double u;                // its Metropolis draw
-    int32_t move, binder;    // its wave-uniform fields
-    int64_t n, ind0, indf;
-    double T[12];
 };
 
 struct SpecLayout {
-    size_t seg, seg_bytes, mt, slots, res, hkey, hmask, ctl, seq, total;
+    size_t seg, seg_bytes, mt, slots, res, ctl, seq, total;
 };
 
-// LDS: one evaluator block per wavefront, the MT19937 block, two slot buffers,
-// per-wavefront results, the conflict table and the control words.
-__host__ __device__ inline SpecLayout spec_layout(int Bp1, int W)
+// LDS: one evaluator block per evaluating wavefront (together they serve as the
+// one-at-a-time block), the MT19937 block, the slot ring, per-slot results, the
+// control words.
+template <int W>
+__host__ __device__ inline SpecLayout spec_layout(int Bp1)
 {
     SpecLayout S;
     S.seg = 0;
-    S.seg_bytes = seg_layout(Bp1).total;
-    size_t o = S.seg_bytes * (size_t)W;
+    S.seg_bytes = ev_layout(Bp1, false).total;
+    size_t o = S.seg_bytes * (size_t)Shape<W>::EV;
     S.mt = o;
     o = align_up(o + MT_LDS_BYTES, 16);
     S.slots = o;
-    o += sizeof(SpecSlot) * 2 * (size_t)W;
+    o += sizeof(SpecSlot) * (size_t)Shape<W>::RING;
     S.res = o;
-    o += sizeof(SpecRes) * (size_t)W;
-    S.hkey = o;
-    o += sizeof(int32_t) * SPEC_HASH;
-    S.hmask = o;
-    o += sizeof(uint32_t) * SPEC_HASH;
+    o += sizeof(SpecRes) * (size_t)Shape<W>::EV;
     S.ctl = o;
     o += sizeof(SpecCtl);
     o = align_up(o, 16);
@@ -105,16 +108,12 @@ __host__ __device__ inline SpecLayout spec_layout(int Bp1, int W)
 }
 
 struct SpecLds {
-    SpecSlot *slots[2];
+    SpecSlot *ring;
     SpecRes *res;
-    int32_t *hkey;
-    uint32_t *hmask;
     SpecCtl *ctl;
     SeqIO *seq;
     uint32_t *mt;
-    SegLds mine;    // this wavefront's evaluator block
-    SegLds first;   // wavefront 0's (the one-at-a-time path)
-    char *wide;     // the W blocks as one wide block (wide_lds_bytes), or nullptr if they are too small
+    char *blocks;   // the evaluator blocks
 };
 // A stream checkpoint in LDS: the glibc words and indices, and the Philox position
 // (counter, index in block; words 35-38 are not used: rng_restore needs the
@@ -180,8 +179,15 @@ __device__ __forceinline__ int64_t from_point_once(int32_t x_side, int32_t x_exp
     return cexp_once(x_exp, ws, ws, ok) + ind0;
 }
 
+// Whether a slot holds a crank-shaft, end-pivot or slide window of n beads: windows the
+// replica's arena does not hold are left to mc_step_dev, which reports them.
+__device__ __forceinline__ bool slot_holds(const chromo_replica *R, int64_t n)
+{
+    return n <= SEG_MAX || (n <= SPEC_BEADS && n <= R->bead_cap && (!R->field_on || n <= R->seg_cap));
+}
+
 // Philox, crank-shaft / end-pivot / slide: the usual proposal -- every capped
-// exponential accepted at its first draw, a window of 1..SPEC_NMAX beads, no extra
+// exponential accepted at its first draw, a window that a slot holds, no extra
 // axis draws -- from the next eight words of the batch, read in one LDS round
 // trip instead of one per draw.  The same words, in the same order and with the
 // same arithmetic, as gen_slot's draw-at-a-time code.  Consumes nothing and returns
@@ -241,7 +247,7 @@ __device__ __forceinline__ bool gen_fast(const chromo_replica *R, WaveRng &rng, 
         used = 7;
     }
     const int64_t n = indf - ind0;
-    if (!ok || n < 1 || n > SPEC_NMAX) return false;
+    if (!ok || n < 1 || !slot_holds(R, n)) return false;
     rng.pidx = p + used;
     if (lane_id() == 0) {
         S.kind = SLOT_SMALL;
@@ -293,7 +299,7 @@ __device__ __forceinline__ int gen_slot(const chromo_replica *R, WaveRng &rng, c
                 rnd31(rng);
             }
         }
-        seq = err || n > SPEC_NMAX;
+        seq = err || !slot_holds(R, n);
     } else if (mv == CHROMO_END_PIVOT) {
         ang = amp_move * (((double)rnd31(rng) / RMAX) - 0.5);
         lhs = (int32_t)(rnd31(rng) & 1);
@@ -306,7 +312,7 @@ __device__ __forceinline__ int gen_slot(const chromo_replica *R, WaveRng &rng, c
         }
         if (!err && indf > N) err = ERR_WINDOW;
         n = indf - ind0;
-        seq = err || n > SPEC_NMAX;
+        seq = err || !slot_holds(R, n);
         if (!seq) {
             s1 = rnd31(rng);
             s2 = rnd31(rng);
@@ -321,7 +327,7 @@ __device__ __forceinline__ int gen_slot(const chromo_replica *R, WaveRng &rng, c
             check_bead_bounds(b0, b1, N, ind0, indf);
             n = indf - ind0;
         }
-        seq = err || n > SPEC_NMAX;
+        seq = err || !slot_holds(R, n);
     } else if (mv == CHROMO_TANGENT_ROTATION) {
         ang = amp_move * (((double)rnd31(rng) / RMAX) - 0.5);
         int64_t k = draw_mod(rnd31(rng), amp_bead) + 1;
@@ -406,123 +412,43 @@ __device__ __forceinline__ int gen_slot(const chromo_replica *R, WaveRng &rng, c
     return kind;
 }
 
-// One proposal of a sequential round (the RNG, the controller and the result
-// pass through LDS, io).  Inlined: a call boundary here makes the callee save
-// most of the register file on every call and the caller spill around it.
-// Wavefront 0 draws the proposal (mc_propose); a
-// crank-shaft, slide or end-pivot move of more than SEG_MAX beads with the field
-// on is then evaluated by both (up to SEG_WIDE beads seg_eval COOP, in the wide
-// block, exchange area after it; longer ones big_eval COOP), everything else by
-// wavefront 0 alone (mc_evaluate).  The numbers are those of mc_step_dev.  Both
-// wavefronts call it.
+// One proposal of a sequential round by the drawing wavefront alone, in the
+// one-at-a-time block (the slot blocks' LDS: every slot hash is empty again on
+// return).  The RNG, the controller and the result pass through LDS, io.
 template <int NB, int W>
-__device__ __forceinline__ void seq_step_coop(const chromo_replica *R, SeqIO *io, uint32_t *mt, const SegLds &G,
-                                              char *wide)
+__device__ __forceinline__ void seq_step(const chromo_replica *R, const EvConst &EC, SeqIO *io, uint32_t *mt,
+                                         char *blocks)
 {
-    static_assert(W == 2, "two wavefronts");
-    const int wv = wave_id(), lane = lane_id();
+    const int lane = lane_id();
     WaveRng rng;
-    chromo_ctrl C;
+    rng.mode = uni_i32(R->rng_mode);
+    rng.k0 = uni_u32(R->rng[CHROMO_RNG_PHILOX_KEY]);
+    rng.k1 = uni_u32(R->rng[CHROMO_RNG_PHILOX_KEY + 1]);
+    rng.pbase = PHILOX_NONE;
+    rng.pidx = 0;
+    rng.mt = mt;
+    rng_restore(rng, io->ck);
+    rng.mti = uni_i32(io->mti);
+    chromo_ctrl C = io->C;
     MoveOut o;
+    o.err = 0;
+    o.n = 0;
     Proposal P;
     double u = 0;
-    bool go = false;
-    const SegLds GW = seg_lds<SEG_WIDE>(wide, NB + 1);
-    const BigLds GB = big_lds(wide, NB + 1, wide_lds_bytes(NB + 1));
-    if (wv == 0) {
-        rng.mode = uni_i32(R->rng_mode);
-        rng.k0 = uni_u32(R->rng[CHROMO_RNG_PHILOX_KEY]);
-        rng.k1 = uni_u32(R->rng[CHROMO_RNG_PHILOX_KEY + 1]);
-        rng.pbase = PHILOX_NONE;
-        rng.pidx = 0;
-        rng.mt = mt;
-        rng_restore(rng, io->ck);
-        rng.mti = uni_i32(io->mti);
-        C = io->C;
-        o.err = 0;
-        o.n = 0;
-        go = mc_propose<NB>(R, rng, C, o, P, u);
-        // the RNG and the controller go back to LDS now, so that they are not
-        // held in registers through the evaluation
-        rng_save(rng, io->ck);
-        const bool both = go && R->field_on && wide != nullptr && P.n > SEG_MAX && big_move(P.move);
-        const int coop = !both ? 0 : P.n <= SEG_WIDE ? 1 : GB.ucap > 0 ? 2 : 0;
-        if (coop == 1) seg_clear<SEG_WIDE>(GW);
-        if (lane == 0) {
-            io->mti = rng.mti;
-            io->C = C;
-            io->coop = coop;
-            io->u = u;
-            io->move = P.move;
-            io->binder = P.binder;
-            io->n = P.n;
-            io->ind0 = P.ind0;
-            io->indf = P.indf;
-            for (int q = 0; q < 12; ++q) io->T[q] = P.T[q];
-        }
+    const bool go = mc_propose<NB>(R, rng, C, o, P, u);
+    // the RNG goes back to LDS now, so that it is not held through the evaluation
+    rng_save(rng, io->ck);
+    if (lane == 0) io->mti = rng.mti;
+    const EvLds S = ev_lds(blocks, NB + 1, true);
+    ev_clear(S);
+    if (go) mc_evaluate<NB>(R, EC, C, o, P, u, S);
+    const size_t bytes = ev_layout(NB + 1, false).total;
+    for (int b = 0; b < Shape<W>::EV; ++b) ev_clear(ev_lds(blocks + bytes * b, NB + 1, false));
+    if (lane == 0) {
+        io->C = C;
+        io->out = o;
     }
-    __syncthreads();
-    const int coop = io->coop;
-    if (coop) {
-        if (wv != 0) {
-            P.move = io->move;
-            P.binder = io->binder;
-            P.n = io->n;
-            P.ind0 = io->ind0;
-            P.indf = io->indf;
-            for (int q = 0; q < 12; ++q) P.T[q] = io->T[q];
-            P.mypick = 0;
-            P.mynew = 0;
-            for (int q = 0; q < 9; ++q) P.myT[q] = 0;
-            u = io->u;
-        }
-        SegRes sr;
-        if (coop == 1) {
-            SegKeep<NB> K;
-            seg_eval<NB, SEG_WIDE, false, true>(R, P, u, GW, sr, K, wide + seg_layout<SEG_WIDE>(NB + 1).total);
-            if (wv == 0 && !sr.overflow) {
-                if (sr.accepted) seg_commit<NB>(R, P.move, P.n, P.binder, P.mynew, K, GW, sr.U);
-                wave_sync_global();
-            }
-        } else {
-            big_eval<NB, false, true>(R, P, u, GB, sr);
-            if (wv == 0 && !sr.overflow) {
-                if (sr.accepted) big_commit<NB>(R, P, GB, sr.U);
-                wave_sync_global();
-            }
-        }
-        if (wv == 0) {
-            // as mc_evaluate after its SEG_WIDE or long-move evaluation
-            for (int b = 0; b < W; ++b)
-                seg_clear<SEG_MAX>(seg_lds<SEG_MAX>(wide + (size_t)b * seg_layout<SEG_MAX>(NB + 1).total, NB + 1));
-            if (!sr.overflow) {
-                o.dEp = sr.dEp;
-                o.dEf = sr.dEf;
-                o.u = u;
-                o.expdE = sr.expdE;
-                o.accepted = sr.accepted;
-                o.nbins = sr.U;
-            } else if (P.n > R->bead_cap || P.n > R->seg_cap) {
-                o.err = ERR_SEGCAP;
-                o.n = 0;
-            } else {
-                move_body<1, NB>(R, u, P, o);
-            }
-            if (o.err) o.n = 0;
-            if (lane == 0) {
-                if (!o.err) track_acceptance(io->C, o.accepted);
-                io->out = o;
-            }
-            wave_sync();
-        }
-    } else if (wv == 0) {
-        if (go) mc_evaluate<NB>(R, C, o, P, u, G, wide, W);
-        if (lane == 0) {
-            io->C = C;
-            io->out = o;
-        }
-        wave_sync();
-    }
+    wave_sync();
 }
 
 // The proposal of slot S from its stored draws: the arithmetic of mc_step_dev's
@@ -532,7 +458,7 @@ __device__ __forceinline__ void seq_step_coop(const chromo_replica *R, SeqIO *io
 // one-at-a-time path can do in stream order.
 template <int NB>
 __device__ __forceinline__ bool slot_proposal(const chromo_replica *R, const SpecSlot &S, Proposal &P,
-                                              const SegBeads<NB> &B)
+                                              const EvBeads<NB> &B)
 {
     const int lane = lane_id();
     const int64_t N = R->N;
@@ -566,9 +492,9 @@ __device__ __forceinline__ bool slot_proposal(const chromo_replica *R, const Spe
         else ifc = ind0_m1;
         const double sa = sin(S.ang), ca = cos(S.ang);
         double ra[3], rb[3], pt[3], dir[3];
-        seg_r3(B, ia, ind0, indf, n, ra);
-        seg_r3(B, ib, ind0, indf, n, rb);
-        seg_r3(B, ifc, ind0, indf, n, pt);
+        ev_r3(R, B, ia, ind0, indf, ra);
+        ev_r3(R, B, ib, ind0, indf, rb);
+        ev_r3(R, B, ifc, ind0, indf, pt);
         for (int i = 0; i < 3; ++i) dir[i] = ra[i] - rb[i];
         double mag = sqrt(dir[0] * dir[0] + dir[1] * dir[1] + dir[2] * dir[2]);
         if (mag < 1E-5) return false;
@@ -584,7 +510,7 @@ __device__ __forceinline__ bool slot_proposal(const chromo_replica *R, const Spe
         else ifc = ind0;
         double pt[3], axis[3], sa, ca;
         sphere_from_uni(S.s1, S.s2, S.ang, axis, sa, ca);
-        seg_r3(B, ifc, ind0, indf, n, pt);
+        ev_r3(R, B, ifc, ind0, indf, pt);
         axis_rotation_cs(axis, pt, ca, sa, P.T);
     } else if (mv == CHROMO_SLIDE) {
         double dir[3], sa, ca;
@@ -610,13 +536,12 @@ __device__ __forceinline__ bool slot_proposal(const chromo_replica *R, const Spe
     return true;
 }
 
-// Wavefront `slot` evaluates slot S into res, keeps the trial state in K and in
-// its evaluator block, and publishes the voxels it reads to the conflict table
-// (their table slots replace the first-position entries of G.uaux).  Returns
-// whether it inserted into the table.
+// Evaluates slot S into res, its trial state in K, P and the block G, whose hash then
+// holds the slot's voxels (returned: how many; 0 and an empty hash when the slot has to
+// be redone one at a time).
 template <int NB>
-__device__ __forceinline__ bool eval_slot(const chromo_replica *R, const SpecSlot &S, SpecRes &res, SegKeep<NB> &K,
-                                          const SpecLds &L, const SegLds &G, int slot)
+__device__ __forceinline__ int eval_slot(const chromo_replica *R, const EvConst &EC, const SpecSlot &S, SpecRes &res,
+                                         Proposal &P, EvKeep &K, const EvLds &G)
 {
     const int lane = lane_id();
     const int64_t ind0 = S.ind0, indf = S.indf;
@@ -630,127 +555,79 @@ __device__ __forceinline__ bool eval_slot(const chromo_replica *R, const SpecSlo
         res.wlo = ind0;
         res.whi = indf;
     }
-    // every load of the evaluation but the densities', issued before its arithmetic
-    SegBeads<NB> B;
-    const int64_t pick = (S.move == CHROMO_TANGENT_ROTATION && lane < S.n) ? S.picks[lane] : 0;
-    seg_load<NB>(R, S.move, S.n, ind0, indf, pick, B);
-    Proposal P;
+    // every load of the first chunk but the densities', issued before the proposal's
+    // arithmetic
+    EvBeads<NB> B;
+    const int64_t pick = (S.move == CHROMO_TANGENT_ROTATION && (lane & 31) < S.n) ? S.picks[lane & 31] : 0;
+    ev_load<NB, false>(R, S.move, S.n, ind0, indf, 0, pick, B);
     if (!slot_proposal<NB>(R, S, P, B)) {
         if (lane == 0) res.resample = 1;
         wave_sync();
-        return false;
+        return 0;
     }
-    SegRes sr;
+    EvRes sr;
     const double u = (double)S.ud / RMAX;
-    seg_eval_loaded<NB>(R, P, u, G, sr, K, B);
+    ev_eval<NB, false>(R, EC, P, u, G, sr, K, B);
     if (sr.overflow) {
-        // more voxels than seg_eval holds: the one-at-a-time path evaluates it
+        // more voxels than the block holds: the one-at-a-time path evaluates it
         if (lane == 0) res.overflow = 1;
         wave_sync();
-        return false;
+        return 0;
     }
-    const int U = sr.U;
-    bool inserted = false;
-    int full = 0;
-    if (U > 0) {
-        int base = 0;
-        if (lane == 0) base = atomicAdd(&L.ctl->used, U);
-        base = bcast0(base);
-        if (slot > 0 && base + U > SPEC_HASH_SOFT) {
-            full = 1;
-        } else {
-            inserted = true;
-            for (int q = lane; q < U; q += WAVE) {
-                const int32_t v = G.uvox[q];
-                uint32_t h = ((uint32_t)v * 2654435761u) >> SPEC_HASH_SHIFT;
-                int probes = 0;
-                for (;;) {
-                    int old = atomicCAS(&L.hkey[h], HKEY_EMPTY, v);
-                    if (old == HKEY_EMPTY || old == v) break;
-                    h = (h + 1) & (uint32_t)(SPEC_HASH - 1);
-                    if (++probes >= SPEC_HASH) {
-                        full = 1;
-                        break;
-                    }
-                }
-                if (probes >= SPEC_HASH) {
-                    G.uaux[q] = -1;
-                    continue;
-                }
-                atomicOr(&L.hmask[h], 1u << slot);
-                G.uaux[q] = (int32_t)h;
-            }
-        }
-    }
-    full = wave_any(full);
     if (lane == 0) {
         res.dEp = sr.dEp;
         res.dEf = sr.dEf;
         res.u = u;
         res.expdE = sr.expdE;
         res.accepted = sr.accepted;
-        res.nbins = U;
-        res.overflow = full;
+        res.nbins = sr.U;
     }
     wave_sync();
-    return inserted;
+    return sr.U;
 }
 
-// Earlier slots of this round whose writes slot s reads: shared voxels through
-// the conflict table, shared beads through the bead ranges (tangent rotation:
-// picks within one bead of each other).
 template <int RING>
 __device__ __forceinline__ const SpecSlot &ring_at(const SpecSlot *ring, int head, int s)
 {
     return ring[(head + s) & (RING - 1)];
 }
 
+// Whether slot s (its voxels numbered in block G, U of them) reads what the accepted
+// slot a < s of the round writes: a shared bead (tangent rotation: picks within one
+// bead of each other), or a shared voxel, looked up in a's own hash (block A).
 template <int RING>
-__device__ __forceinline__ void spec_conflicts(const SpecSlot *ring, int head, SpecRes *res, const SpecLds &L,
-                                               const SegLds &G, int s)
+__device__ __forceinline__ bool spec_conflict(const SpecSlot *ring, int head, const SpecRes *res, const EvLds &G, int U,
+                                              int s, const EvLds &A, int a)
 {
-    static_assert((SPEC_WMAX - 1) * SPEC_NMAX <= WAVE, "one lane per (earlier slot, pick)");
     const int lane = lane_id();
-    const uint32_t low = (1u << s) - 1u;
-    uint32_t m = 0;
-    const int U = res[s].nbins;
-    for (int q = lane; q < U; q += WAVE) {
-        const int h = G.uaux[q];
-        if (h >= 0) m |= L.hmask[h] & low;
-    }
-    const SpecSlot &S = ring_at<RING>(ring, head, s);
+    const SpecSlot &S = ring_at<RING>(ring, head, s), &Q = ring_at<RING>(ring, head, a);
+    bool hit = false;
     if (S.move == CHROMO_TANGENT_ROTATION) {
-        const int a = lane / SPEC_NMAX, c = lane % SPEC_NMAX;
-        if (a < s && ring_at<RING>(ring, head, a).kind == SLOT_SMALL && c < S.n) {
-            const SpecSlot &A = ring_at<RING>(ring, head, a);
-            const int64_t mine = S.picks[c];
-            for (int64_t q = 0; q < A.n; ++q) {
-                const int64_t d = A.picks[q] - mine;
-                if (d >= -1 && d <= 1) m |= 1u << a;
+        if (lane < S.n) {
+            const int64_t mine = S.picks[lane];
+            for (int64_t q = 0; q < Q.n; ++q) {
+                const int64_t d = Q.picks[q] - mine;
+                hit |= d >= -1 && d <= 1;
             }
         }
-    } else if (lane < s && ring_at<RING>(ring, head, lane).kind == SLOT_SMALL) {
-        const SpecRes &o = res[lane];
-        if (o.wlo <= res[s].rhi && res[s].rlo < o.whi) m |= 1u << lane;
+    } else {
+        hit = res[a].wlo <= res[s].rhi && res[s].rlo < res[a].whi;
+        if (res[a].nbins > 0)
+            for (int q = lane; q < U; q += WAVE) {
+                const int2 v = G.uv[q];
+                int h = (int)((uint32_t)v.y >> 16);
+                for (int probes = 0; probes < A.hsize; ++probes) {
+                    const int key = A.hkey[h];
+                    hit |= key == v.x;
+                    if (key == v.x || key == HKEY_EMPTY) break;
+                    h = (h + 1) & (A.hsize - 1);
+                }
+            }
     }
-    m = wave_or(m);
-    if (lane == 0) res[s].cmask = m;
+    return wave_any(hit);
 }
 
-// Clears this wavefront's conflict-table entries (after every wavefront has read
-// the table this round).
-__device__ __forceinline__ void spec_release(const SpecLds &L, const SegLds &G, int U)
-{
-    for (int q = lane_id(); q < U; q += WAVE) {
-        const int h = G.uaux[q];
-        if (h >= 0) {
-            L.hkey[h] = HKEY_EMPTY;
-            L.hmask[h] = 0;
-        }
-    }
-}
-
-// Wavefront 0: appends proposals to the queue of `q` slots starting at ring
+// The drawing wavefront: appends proposals to the queue of `q` slots starting at ring
 // position head until it holds `limit`, or `remaining` (the block's unresolved
 // proposals), or ends with a SLOT_SEQ one.  Returns the new queue length.
 template <int NB, int RING>
@@ -790,7 +667,7 @@ __device__ __forceinline__ void spec_book(const chromo_replica *R, chromo_ctrl &
     const uint64_t live_m = __ballot(live);
     const uint64_t acc_m = __ballot(live && acc);
     const uint64_t tie_m = __ballot(live && tie);
-    static_assert(SPEC_WMAX <= 8, "bookkeeping sums over the first eight lanes");
+    static_assert(SPEC_EVMAX <= 8, "bookkeeping sums over the first eight lanes");
     const int64_t sn = sum_lanes8_i64(n), sb = sum_lanes8_i64(nb), sy = sum_lanes8_i64(bytes);
     const int64_t logged = K.logged;
     const int nlive = __popcll(live_m);
@@ -838,52 +715,80 @@ __device__ __forceinline__ void spec_book(const chromo_replica *R, chromo_ctrl &
     wave_sync();
 }
 
-// One controller block.  C and K live in LDS: only wavefront 0 touches them, and
-// keeping them out of registers leaves those to the evaluation.
-//
-// The slots wait in a ring of 2W.  A round evaluates the first min(W, queued)
-// of them.  Slot 0 of a round stands whatever the others do (nothing precedes
-// it), so wavefront 0 commits it as soon as it is evaluated -- a later slot that
-// reads what it writes is redone anyway -- and then draws the following
-// proposals into the ring while the other wavefronts finish.
-template <int NB, int W>
-__device__ __forceinline__ void spec_block(const chromo_replica *R, WaveRng &rng, chromo_ctrl &C, Counters &K,
-                                           const SpecLds &L)
+// Raises a flag of the round for the other wavefronts: what this wavefront wrote to
+// LDS before is visible to who sees it.
+__device__ __forceinline__ void flag_raise(int32_t *f, int32_t tag)
 {
-    constexpr int RING = 2 * W;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    if (lane_id() == 0) __hip_atomic_store(f, tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// Waits for a flag; false when it did not come within SPIN_LIMIT looks.
+__device__ __forceinline__ bool flag_wait(const int32_t *f, int32_t tag)
+{
+    int spins = 0;
+    while (uni_i32(__hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) != tag)
+        if (++spins >= SPIN_LIMIT) break;
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    return spins < SPIN_LIMIT;
+}
+
+// One controller block.  C and K live in LDS: only the booking wavefront touches them
+// between two barriers, and keeping them out of registers leaves those to the
+// evaluation.
+//
+// A round, between two barriers:
+//  * wavefront s < cnt evaluates slot s and raises done[s]; slot 0 stands whatever the
+//    others do (nothing precedes it), so it is committed at once -- a later slot that
+//    reads what it writes is redone anyway;
+//  * slot s waits for done[a] of every a < s, looks its voxels and beads up in the
+//    accepted ones', and raises chk[s];
+//  * the drawing wavefront meanwhile draws the following proposals into the ring;
+//  * every wavefront resolves the slots it needs from the published results, in the
+//    same way: slot s commits if nothing before it ends the round.
+// A slot's hash is emptied at the start of its wavefront's next evaluation, when
+// nobody looks into it any more.  The flag waits are bounded; a wait that passes its
+// bound stops the replica with ERR_SPIN at the next round's top.
+template <int NB, int W>
+__device__ __forceinline__ void spec_block(const chromo_replica *R, const EvConst &EC, WaveRng &rng, chromo_ctrl &C,
+                                           Counters &K, const SpecLds &L, int &held)
+{
+    using SH = Shape<W>;
+    constexpr int RING = SH::RING, EV = SH::EV, Bp1 = NB + 1;
     static_assert((RING & (RING - 1)) == 0, "ring positions wrap by mask");
     const int wv = wave_id(), lane = lane_id();
-    SpecSlot *ring = L.slots[0];
-    int head = 0;                      // wavefront 0: ring position of the first queued slot
-    int nq = 0;                        // wavefront 0: slots queued
-    int remaining = C.num_per_cycle;   // wavefront 0: proposals of the block not yet resolved
-    int pend = 0;                      // wavefront 0: error to publish before the next barrier
-    int32_t tag = uni_i32(L.ctl->tag); // wavefront 0: the round's number in the launch
+    const size_t seg_bytes = ev_layout(Bp1, false).total;
+    const EvLds G = ev_lds(L.blocks + seg_bytes * (wv < EV ? wv : 0), Bp1, false);
+    SpecSlot *ring = L.ring;
+    // the drawing wavefront's
+    int head = 0;                      // ring position of the first queued slot
+    int nq = 0;                        // slots queued
+    int remaining = C.num_per_cycle;   // proposals of the block not yet resolved
+    int pend = 0;                      // error to publish before the next barrier
+    int32_t tag = uni_i32(L.ctl->tag); // the round's number in the launch
     int64_t rounds = 0;
     // every round resolves a proposal or turns its first slot into a sequential one
     const int64_t max_rounds = 2 * (int64_t)C.num_per_cycle + 64;
     // drawing ahead is off where a redone proposal would have to rewind MT19937
     const bool ahead = !(rng.mode == CHROMO_RNG_GLIBC && C.move == CHROMO_CHANGE_BINDING_STATE);
     for (;;) {
-        if (wv == 0) {
+        if (wv == SH::GEN) {
             // L.ctl->err is written only here, before the barrier after which every
             // wavefront reads it
             if (++rounds > max_rounds) pend = ERR_SPIN;
+            if (uni_i32(L.ctl->stall) >= 0) pend = ERR_SPIN;
             if (pend && lane == 0) L.ctl->err = pend;
-            // only wavefront 0 writes L.ctl->err and L.ctl->tag: pend and tag are their values
             if (!pend) {
                 tag += 1;
-                nq = spec_gen<NB, RING>(R, rng, C, ring, head, nq, W, remaining);
-                const int nr = nq < W ? nq : W;
+                nq = spec_gen<NB, RING>(R, rng, C, ring, head, nq, EV, remaining);
+                const int nr = nq < EV ? nq : EV;
                 // leading slots that are not SLOT_SEQ, all kinds read at once
                 const int kd = lane < nr ? ring_at<RING>(ring, head, lane).kind : SLOT_SEQ;
                 const uint64_t seqm = __ballot(kd == SLOT_SEQ);
                 const int cnt = seqm ? (int)__builtin_ctzll(seqm) : nr;
                 if (lane == 0) {
-                    L.ctl->nq = nr;
                     L.ctl->cnt = cnt;
                     L.ctl->remaining = remaining;
-                    L.ctl->used = 0;
                     L.ctl->head = head;
                     L.ctl->tag = tag;
                 }
@@ -891,9 +796,12 @@ __device__ __forceinline__ void spec_block(const chromo_replica *R, WaveRng &rng
         }
         __syncthreads();
         if (L.ctl->err || L.ctl->remaining <= 0) break;
-        const int cnt = L.ctl->cnt, h = L.ctl->head;
+        const int cnt = uni_i32(L.ctl->cnt), h = uni_i32(L.ctl->head);
         if (ring_at<RING>(ring, h, 0).kind == SLOT_SEQ) {
-            if (wv == 0) {
+            held = 0;   // the one-at-a-time block lies over the slot blocks and leaves them empty
+            if (wv == SH::GEN) {
+                // the slot hashes may still hold the last round's voxels: seq_step clears
+                // what it uses, before and after
                 SeqIO *io = L.seq;
                 const SpecSlot &S0 = ring_at<RING>(ring, h, 0);
                 for (int i = lane; i < CK_WORDS; i += WAVE) io->ck[i] = S0.ck[i];
@@ -902,12 +810,7 @@ __device__ __forceinline__ void spec_block(const chromo_replica *R, WaveRng &rng
                     io->C = C;
                 }
                 wave_sync();
-            }
-            // the W evaluator blocks serve as one wide block; both wavefronts
-            // enter, and evaluate a long crank-shaft, slide or end-pivot together
-            seq_step_coop<NB, W>(R, L.seq, L.mt, L.first, L.wide);
-            if (wv == 0) {
-                SeqIO *io = L.seq;
+                seq_step<NB, W>(R, EC, io, L.mt, L.blocks);
                 rng_restore(rng, io->ck);
                 rng.mti = uni_i32(io->mti);
                 if (lane == 0) C = io->C;
@@ -924,66 +827,54 @@ __device__ __forceinline__ void spec_block(const chromo_replica *R, WaveRng &rng
                 nq = 0;
             }
         } else {
-            SegKeep<NB> keep;
-            const SpecSlot &mys = ring_at<RING>(ring, h, wv < W ? wv : 0);
-            const bool mine = wv < cnt && mys.kind == SLOT_SMALL;
-            bool inserted = false;
-            if (mine) inserted = eval_slot<NB>(R, mys, L.res[wv], keep, L, L.mine, wv);
-            bool committed = false;
-            static_assert(W <= 2, "one wavefront on each side of the round's flags");
-            if (wv == 0) {
-                // slot 0's voxels are in the conflict table: the later slot may check
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-                if (lane == 0) __hip_atomic_store(&L.ctl->ins, L.ctl->tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                if (mine && L.res[0].accepted && !L.res[0].resample && !L.res[0].overflow) {
-                    const int mynew = lane < mys.n ? mys.newst[lane] : 0;
-                    seg_commit<NB>(R, mys.move, mys.n, mys.binder, mynew, keep, L.mine, L.res[0].nbins);
-                    committed = true;
-                }
+            const int32_t now = uni_i32(L.ctl->tag);
+            const bool evaluates = wv < EV && wv < cnt;
+            const SpecSlot &mys = ring_at<RING>(ring, h, evaluates ? wv : 0);
+            const bool mine = evaluates && mys.kind == SLOT_SMALL;
+            bool stalled = false, committed = false;
+            EvKeep keep;
+            Proposal P;
+            if (mine) {
+                ev_release(G, held);
+                held = eval_slot<NB>(R, EC, mys, L.res[wv], P, keep, G);
             }
-            if (wv > 0) {
-                // wait for slot 0's table entries, set the later slot's conflict mask,
-                // then the flag wavefront 0 waits on
-                const int32_t tag = uni_i32(L.ctl->tag);
-                int spins = 0;
-                while (uni_i32(__hip_atomic_load(&L.ctl->ins, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) != tag) {
-                    if (++spins >= SPIN_LIMIT) break;
-                }
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-                // a table that did not arrive: the slot waits for the next round, and
-                // since this wavefront may then read slot 0's result before it is
-                // written, wavefront 0 stops the replica (ERR_SPIN) rather than let
-                // the two resolve the round differently
-                if (spins >= SPIN_LIMIT && lane == 0) {
-                    if (mine) L.res[wv].overflow = 1;
-                    L.ctl->stall = tag;
-                }
-                wave_sync();
-                if (mine && !L.res[wv].resample && !L.res[wv].overflow)
-                    spec_conflicts<RING>(ring, h, L.res, L, L.mine, wv);
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-                if (lane == 0) __hip_atomic_store(&L.ctl->ready, tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            } else {
-                // draw the following proposals while the other wavefronts check
-                // conflicts, commit and book
-                if (ahead && !pend) nq = spec_gen<NB, RING>(R, rng, C, ring, head, nq, RING, remaining);
-                if (W > 1) {
-                    int spins = 0;
-                    while (uni_i32(__hip_atomic_load(&L.ctl->ready, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) !=
-                           tag) {
-                        if (++spins >= SPIN_LIMIT) {
-                            pend = ERR_SPIN;
-                            break;
-                        }
+            if (evaluates) flag_raise(&L.ctl->done[wv], now);
+            if (wv == 0 && mine && L.res[0].accepted && !L.res[0].resample && !L.res[0].overflow) {
+                ev_commit<NB>(R, P, keep, G, held);
+                committed = true;
+            }
+            if (evaluates && wv > 0) {
+                uint32_t m = 0;
+                const bool look = mine && !L.res[wv].resample && !L.res[wv].overflow;
+                for (int a = 0; a < wv; ++a) {
+                    if (!flag_wait(&L.ctl->done[a], now)) {
+                        stalled = true;
+                        break;
                     }
-                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-                    if (uni_i32(L.ctl->stall) == tag) pend = ERR_SPIN;
+                    if (!look || ring_at<RING>(ring, h, a).kind != SLOT_SMALL) continue;
+                    const SpecRes &q = L.res[a];
+                    if (!q.accepted || q.resample || q.overflow) continue;
+                    if (spec_conflict<RING>(ring, h, L.res, G, held, wv, ev_lds(L.blocks + seg_bytes * a, Bp1, false), a))
+                        m |= 1u << a;
                 }
+                if (lane == 0) L.res[wv].cmask = m;
+                if (stalled && lane == 0) L.ctl->stall = now;
+                flag_raise(&L.ctl->chk[wv], now);
             }
+            // the following proposals
+            if (wv == SH::GEN && ahead && !pend) nq = spec_gen<NB, RING>(R, rng, C, ring, head, nq, RING, remaining);
+            // the results this wavefront resolves: all for the drawing and booking ones,
+            // the slots before its own for the others
+            const bool all = wv == SH::GEN || wv == SH::BOOK;
+            const int upto = all ? cnt : (evaluates ? wv + 1 : 0);
+            if (upto > 0 && !evaluates) stalled |= !flag_wait(&L.ctl->done[0], now);
+            for (int s = 1; s < upto; ++s)
+                if (s != wv) stalled |= !flag_wait(&L.ctl->chk[s], now);
+            if (stalled && lane == 0) L.ctl->stall = now;
             // resolution, identical in every wavefront; lane s reads slot s's result,
             // all slots in one LDS round trip
             uint32_t kd = SLOT_EMPTY, cmk = 0, ov = 0, rs = 0, ac = 0;
-            if (lane < cnt) {
+            if (lane < upto) {
                 const SpecRes &q = L.res[lane];
                 kd = (uint32_t)ring_at<RING>(ring, h, lane).kind;
                 cmk = q.cmask;
@@ -991,16 +882,16 @@ __device__ __forceinline__ void spec_block(const chromo_replica *R, WaveRng &rng
                 rs = (uint32_t)q.resample;
                 ac = (uint32_t)q.accepted;
             }
-            int F = cnt, rew = 0;
+            int F = upto, rew = 0;
             uint32_t accm = 0;
-            for (int s = 0; s < cnt; ++s) {
+            for (int s = 0; s < upto; ++s) {
                 if ((int)readlane_u32(kd, s) == SLOT_EMPTY) continue;
                 const uint32_t q_cmask = readlane_u32(cmk, s), q_overflow = readlane_u32(ov, s);
-                if ((q_cmask & accm) || (q_overflow && s > 0)) {
+                if (q_cmask & accm) {
                     F = s;
                     break;
                 }
-                // the first slot always fits the conflict table; if it did not, the
+                // an axis to be drawn again, or more voxels than a block holds: the
                 // sequential path redoes it
                 if (readlane_u32(rs, s) || q_overflow) {
                     F = s;
@@ -1009,15 +900,10 @@ __device__ __forceinline__ void spec_block(const chromo_replica *R, WaveRng &rng
                 }
                 if (readlane_u32(ac, s)) accm |= 1u << s;
             }
-            if (mine && !committed && wv < F && L.res[wv].accepted) {
-                const int mynew = lane < mys.n ? mys.newst[lane] : 0;
-                seg_commit<NB>(R, mys.move, mys.n, mys.binder, mynew, keep, L.mine, L.res[wv].nbins);
-            }
-            if (inserted) spec_release(L, L.mine, L.res[wv].nbins);
-            // the last wavefront books the round; only the barrier below orders C
-            // and K for the next reader
-            if (wv == W - 1) spec_book<RING>(R, C, K, ring, h, L.res, F);
-            if (wv == 0) {
+            if (mine && !committed && wv < F && L.res[wv].accepted) ev_commit<NB>(R, P, keep, G, held);
+            // only the barrier below orders C and K for the next reader
+            if (wv == SH::BOOK) spec_book<RING>(R, C, K, ring, h, L.res, F);
+            if (wv == SH::GEN) {
                 if (rew) {
                     // slot F is redone one at a time; what was drawn after it is
                     // dropped (the sequential path rewinds the streams to it)
@@ -1034,34 +920,27 @@ __device__ __forceinline__ void spec_block(const chromo_replica *R, WaveRng &rng
 }
 
 template <int NB, int W>
-__device__ __forceinline__ void spec_run(const chromo_replica *R, int64_t steps)
+__device__ __forceinline__ void spec_run(const chromo_replica *R, const EvConst &EC, int64_t steps)
 {
+    using SH = Shape<W>;
     constexpr int Bp1 = NB + 1;
-    const SpecLayout SL = spec_layout(Bp1, W);
+    const SpecLayout SL = spec_layout<W>(Bp1);
     const int wv = wave_id(), lane = lane_id();
     SpecLds L;
-    L.mine = seg_lds(lds_dyn + SL.seg + SL.seg_bytes * wv, Bp1);
-    L.first = seg_lds(lds_dyn + SL.seg, Bp1);
-    L.wide = SL.seg_bytes * W >= wide_lds_bytes(Bp1) ? lds_dyn + SL.seg : nullptr;
-    seg_clear(L.mine);
-    L.slots[0] = (SpecSlot *)(lds_dyn + SL.slots);
-    L.slots[1] = L.slots[0] + W;
+    L.blocks = lds_dyn + SL.seg;
+    L.ring = (SpecSlot *)(lds_dyn + SL.slots);
     L.res = (SpecRes *)(lds_dyn + SL.res);
-    L.hkey = (int32_t *)(lds_dyn + SL.hkey);
-    L.hmask = (uint32_t *)(lds_dyn + SL.hmask);
     L.ctl = (SpecCtl *)(lds_dyn + SL.ctl);
     L.seq = (SeqIO *)(lds_dyn + SL.seq);
     L.mt = (uint32_t *)(lds_dyn + SL.mt);
+    if (wv < SH::EV) ev_clear(ev_lds(L.blocks + SL.seg_bytes * wv, Bp1, false));
     __shared__ chromo_ctrl sctrl[MAX_CTRL];
     __shared__ Counters sK;
-    for (int i = (int)threadIdx.x; i < SPEC_HASH; i += WAVE * W) {
-        L.hkey[i] = HKEY_EMPTY;
-        L.hmask[i] = 0;
-    }
     const int nc = R->n_ctrl < MAX_CTRL ? R->n_ctrl : MAX_CTRL;
     WaveRng rng;
+    rng.mode = uni_i32(R->rng_mode);
     bool need_mt = false;
-    if (wv == 0) {
+    if (wv == SH::GEN) {
         need_mt = any_binding(R);
         rng_load(R, rng, L.mt, need_mt);
         if (lane == 0) {
@@ -1069,22 +948,22 @@ __device__ __forceinline__ void spec_run(const chromo_replica *R, int64_t steps)
             for (int i = 0; i < nc; ++i) sctrl[i] = R->ctrl[i];
             L.ctl->err = 0;
             L.ctl->tag = 0;
-            L.ctl->ready = -1;
-            L.ctl->ins = -1;
             L.ctl->stall = -1;
+            for (int s = 0; s < SPEC_EVMAX; ++s) L.ctl->done[s] = L.ctl->chk[s] = -1;
         }
     }
     __syncthreads();
+    int held = 0;   // voxels in this wavefront's hash
     for (int64_t s = 0; s < steps; ++s) {
         for (int ci = 0; ci < nc; ++ci) {
-            if (sctrl[ci].on == 1) spec_block<NB, W>(R, rng, sctrl[ci], sK, L);
+            if (sctrl[ci].on == 1) spec_block<NB, W>(R, EC, rng, sctrl[ci], sK, L, held);
             if (wv == 0 && lane == 0 && !L.ctl->err) update_amplitudes_dev(sctrl[ci]);
             __syncthreads();
             if (L.ctl->err) break;
         }
         if (L.ctl->err) break;
     }
-    if (wv == 0) {
+    if (wv == SH::GEN) {
         rng_store(R, rng, need_mt);
         if (lane == 0)
             for (int i = 0; i < nc; ++i) R->ctrl[i] = sctrl[i];
