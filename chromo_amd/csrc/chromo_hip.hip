@@ -19,14 +19,14 @@ using namespace chromo;
 
 namespace chromo {
 // chromo_run.hip and chromo_spec.hip, one translation unit per binder count
-hipError_t run_launch_1(const chromo_replica *, int, int64_t, bool, hipStream_t);
-hipError_t run_launch_2(const chromo_replica *, int, int64_t, bool, hipStream_t);
-hipError_t run_launch_3(const chromo_replica *, int, int64_t, bool, hipStream_t);
-hipError_t run_launch_4(const chromo_replica *, int, int64_t, bool, hipStream_t);
-hipError_t spec_launch_1(const chromo_replica *, int, int64_t, hipStream_t);
-hipError_t spec_launch_2(const chromo_replica *, int, int64_t, hipStream_t);
-hipError_t spec_launch_3(const chromo_replica *, int, int64_t, hipStream_t);
-hipError_t spec_launch_4(const chromo_replica *, int, int64_t, hipStream_t);
+hipError_t run_launch_1(const chromo_replica *, int, int64_t, hipStream_t);
+hipError_t run_launch_2(const chromo_replica *, int, int64_t, hipStream_t);
+hipError_t run_launch_3(const chromo_replica *, int, int64_t, hipStream_t);
+hipError_t run_launch_4(const chromo_replica *, int, int64_t, hipStream_t);
+hipError_t spec_launch_1(const chromo_replica *, int, int64_t, bool, hipStream_t);
+hipError_t spec_launch_2(const chromo_replica *, int, int64_t, bool, hipStream_t);
+hipError_t spec_launch_3(const chromo_replica *, int, int64_t, bool, hipStream_t);
+hipError_t spec_launch_4(const chromo_replica *, int, int64_t, bool, hipStream_t);
 // chromo_step.hip
 hipError_t step_setup(int lds_limit);
 hipError_t step_launch(const chromo_replica *, int rep, int ctrl, hipStream_t);
@@ -629,8 +629,8 @@ int chromo_mc_run_tuned(const chromo_replica *d_reps, int32_t n_reps, int64_t nu
                            "(binder counts with twisting chains)");
     const int W = waves_per_replica;
     if (W == 4 || W == 8)
-        return set_err(-1, "waves_per_replica = 4 and 8 are not built: the speculative round has "
-                           "one wavefront on each side of its flags");
+        return set_err(-1, "waves_per_replica = 4 and 8 are not offered: 2 is the speculative kernel, which "
+                           "sets its own number of wavefronts by the replica count");
     if (W != 1 && W != 2) return set_err(-1, "waves_per_replica must be 1 or 2");
     rc = ensure_lds();
     if (rc) return rc;
@@ -639,19 +639,21 @@ int chromo_mc_run_tuned(const chromo_replica *d_reps, int32_t n_reps, int64_t nu
     hipLaunchKernelGGL(k_check_binders, dim3((n_reps + 63) / 64), dim3(64), 0, st, d_reps, n_reps,
                        binder_mask);
     HIPC(launch_err());
-    using RunFn = hipError_t (*)(const chromo_replica *, int, int64_t, bool, hipStream_t);
-    using SpecFn = hipError_t (*)(const chromo_replica *, int, int64_t, hipStream_t);
+    using RunFn = hipError_t (*)(const chromo_replica *, int, int64_t, hipStream_t);
+    using SpecFn = hipError_t (*)(const chromo_replica *, int, int64_t, bool, hipStream_t);
     static const RunFn run_fn[] = {chromo::run_launch_1, chromo::run_launch_2, chromo::run_launch_3,
                                    chromo::run_launch_4};
     static const SpecFn spec_fn[] = {chromo::spec_launch_1, chromo::spec_launch_2, chromo::spec_launch_3,
                                      chromo::spec_launch_4};
-    // one kernel per binder count (and, with one wavefront, twist flag) present
+    // one kernel per binder count present, and with waves_per_replica = 1 one per binder
+    // count among the twisting chains: those have no one-at-a-time kernel, the
+    // speculative one gives the same chains sooner
     for (int b = 1; b <= CHROMO_MAX_BINDERS; ++b) {
         if (!(binder_mask & (1 << b))) continue;
-        hipError_t e = W == 1 ? run_fn[b - 1](d_reps, n_reps, num_steps, false, st)
-                              : spec_fn[b - 1](d_reps, n_reps, num_steps, st);
+        hipError_t e = W == 1 ? run_fn[b - 1](d_reps, n_reps, num_steps, st)
+                              : spec_fn[b - 1](d_reps, n_reps, num_steps, false, st);
         if (e == hipSuccess && W == 1 && (binder_mask & (1 << (8 + b))))
-            e = run_fn[b - 1](d_reps, n_reps, num_steps, true, st);
+            e = spec_fn[b - 1](d_reps, n_reps, num_steps, true, st);
         if (e == hipErrorInvalidValue) return set_err(-1, "LDS of this launch shape exceeds the device limit");
         HIPC(e);
     }

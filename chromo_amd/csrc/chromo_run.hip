@@ -1,4 +1,4 @@
-// chromo_run.hip -- the one-wavefront persistent kernel k_mc_run_nb<NB, TW> for one
+// chromo_run.hip -- the one-wavefront persistent kernel k_mc_run_nb<NB> for one
 // NB = CHROMO_NB (binder types); built once per NB so that the instantiations compile
 // in parallel.
 #include <hip/hip_runtime.h>
@@ -15,10 +15,9 @@
 namespace {
 
 // Persistent mc_sim, one workgroup of one wavefront per replica, for the replicas with
-// NB binder types and twist flag TW only; the others are left to the launch of their
-// own kind.  One instantiation per kernel, so that its registers are allocated for
-// that one alone.
-template <int NB, bool TW>
+// NB binder types and no twist; the others are left to the launch of their own kind.
+// One instantiation per kernel, so that its registers are allocated for that one alone.
+template <int NB>
 __global__ void __launch_bounds__(64) k_mc_run_nb(const chromo_replica *__restrict__ reps, int n_reps,
                                                   int64_t steps)
 {
@@ -29,7 +28,7 @@ __global__ void __launch_bounds__(64) k_mc_run_nb(const chromo_replica *__restri
     load_record(&Rs, &reps[r]);
     wave_sync();
     const chromo_replica *R = &Rs;
-    if (R->B != NB || (R->twist != 0) != TW) return;
+    if (R->B != NB || R->twist) return;
     if (R->counters[CHROMO_CNT_ERROR] != 0) return;
     constexpr int Bp1 = NB + 1;
     ev_const(&EC, R);
@@ -47,26 +46,26 @@ __global__ void __launch_bounds__(64) k_mc_run_nb(const chromo_replica *__restri
         for (int i = 0; i < nc; ++i) sctrl[i] = R->ctrl[i];
     __syncthreads();
     int err = 0;
-    run_steps<NB, TW>(R, EC, rng, K, sctrl, nc, steps, err, S);
+    run_steps<NB>(R, EC, rng, K, sctrl, nc, steps, err, S);
     rng_store(R, rng, need_mt);
     if (lane_id() == 0)
         for (int i = 0; i < nc; ++i) R->ctrl[i] = sctrl[i];
     counters_store(R, K, err);
 }
 
-template <int NB, bool TW>
+template <int NB>
 hipError_t launch_nb(const chromo_replica *d_reps, int n_reps, int64_t steps, hipStream_t st)
 {
     // the attribute is set once per process: setting it costs far more than a launch
     static bool attr_set = false;
     const size_t bytes = mc_lds_bytes(NB + 1);
     if (!attr_set) {
-        hipError_t e = hipFuncSetAttribute((const void *)k_mc_run_nb<NB, TW>,
+        hipError_t e = hipFuncSetAttribute((const void *)k_mc_run_nb<NB>,
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
         if (e != hipSuccess) return e;
         attr_set = true;
     }
-    hipLaunchKernelGGL((k_mc_run_nb<NB, TW>), dim3(n_reps), dim3(WAVE), bytes, st, d_reps, n_reps, steps);
+    hipLaunchKernelGGL((k_mc_run_nb<NB>), dim3(n_reps), dim3(WAVE), bytes, st, d_reps, n_reps, steps);
     return hipGetLastError();
 }
 
@@ -74,11 +73,9 @@ hipError_t launch_nb(const chromo_replica *d_reps, int n_reps, int64_t steps, hi
 
 namespace chromo {
 
-hipError_t CHROMO_CAT(run_launch_, CHROMO_NB)(const chromo_replica *d_reps, int n_reps, int64_t steps, bool twist,
-                                              hipStream_t st)
+hipError_t CHROMO_CAT(run_launch_, CHROMO_NB)(const chromo_replica *d_reps, int n_reps, int64_t steps, hipStream_t st)
 {
-    return twist ? launch_nb<CHROMO_NB, true>(d_reps, n_reps, steps, st)
-                 : launch_nb<CHROMO_NB, false>(d_reps, n_reps, steps, st);
+    return launch_nb<CHROMO_NB>(d_reps, n_reps, steps, st);
 }
 
 }  // namespace chromo

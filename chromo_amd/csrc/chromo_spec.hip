@@ -1,4 +1,4 @@
-// chromo_spec.hip -- the speculative persistent kernel k_mc_spec<W, NB> for one
+// chromo_spec.hip -- the speculative persistent kernel k_mc_spec<W, NB, TW> for one
 // NB = CHROMO_NB (binder types); built once per NB so that the instantiations compile
 // in parallel.
 #include <hip/hip_runtime.h>
@@ -14,10 +14,12 @@
 
 namespace {
 
-// Persistent mc_sim with W wavefronts per replica (one workgroup per replica),
-// for the replicas with NB binder types; the others are left to the launch of
-// their own NB.  One wavefront per SIMD: the full register file.
-template <int W, int NB>
+// Persistent mc_sim with W wavefronts per replica (one workgroup per replica), for the
+// replicas with NB binder types; the others are left to the launch of their own NB.
+// One wavefront per SIMD: the full register file.  TW: the twisting chains' kernel,
+// which passes over the others; the other kernel refuses a twisting chain with
+// ERR_TWIST_WAVES (the caller asked for more wavefronts than such a chain may be given).
+template <int W, int NB, bool TW>
 __global__ void __launch_bounds__(WAVE * W) __attribute__((amdgpu_waves_per_eu(1)))
 k_mc_spec(const chromo_replica *__restrict__ reps, int n_reps, int64_t steps)
 {
@@ -30,18 +32,16 @@ k_mc_spec(const chromo_replica *__restrict__ reps, int n_reps, int64_t steps)
     const chromo_replica *R = &Rs;
     if (R->B != NB) return;
     if (R->counters[CHROMO_CNT_ERROR] != 0) return;
-    if (R->twist) {
-        // the speculative evaluator has no twist terms: a twisting chain runs
-        // with one wavefront (k_mc_run_nb)
-        counters_error(R, ERR_TWIST_WAVES);
+    if ((R->twist != 0) != TW) {
+        if (!TW) counters_error(R, ERR_TWIST_WAVES);
         return;
     }
     ev_const(&EC, R);
     __syncthreads();
-    spec_run<NB, W>(R, EC, steps);
+    spec_run<NB, W, TW>(R, EC, steps);
 }
 
-template <int W, int NB>
+template <int W, int NB, bool TW>
 hipError_t launch(const chromo_replica *d_reps, int n_reps, int64_t steps, hipStream_t st)
 {
     const size_t bytes = spec_layout<W>(NB + 1).total;
@@ -53,22 +53,42 @@ hipError_t launch(const chromo_replica *d_reps, int n_reps, int64_t steps, hipSt
         if (e == hipSuccess) e = hipDeviceGetAttribute(&lim, hipDeviceAttributeMaxSharedMemoryPerBlock, dev);
         if (e != hipSuccess) return e;
         if (bytes > (size_t)lim) return hipErrorInvalidValue;
-        e = hipFuncSetAttribute((const void *)k_mc_spec<W, NB>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+        e = hipFuncSetAttribute((const void *)k_mc_spec<W, NB, TW>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
         if (e != hipSuccess) return e;
         attr_set = true;
     }
-    hipLaunchKernelGGL((k_mc_spec<W, NB>), dim3(n_reps), dim3(WAVE * W), bytes, st, d_reps, n_reps, steps);
+    hipLaunchKernelGGL((k_mc_spec<W, NB, TW>), dim3(n_reps), dim3(WAVE * W), bytes, st, d_reps, n_reps, steps);
     return hipGetLastError();
+}
+
+// Four wavefronts per replica where every replica can have a compute unit of its own
+// (the block of three evaluators takes most of a unit's LDS), two otherwise.  128
+// replicas of 1,500-9,000 beads, B = 3, initial windows, 10 sweeps: 13.8 ms with one
+// wavefront each, 9.5 with two, 6.4 with four; one twisting chain, steady-state
+// windows: 19.2 ms with one, 11.1 with four.
+template <bool TW>
+hipError_t launch_shape(const chromo_replica *d_reps, int n_reps, int64_t steps, hipStream_t st)
+{
+    static int units = 0;
+    if (units == 0) {
+        int dev = 0, n = 0;
+        hipError_t e = hipGetDevice(&dev);
+        if (e == hipSuccess) e = hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev);
+        if (e != hipSuccess) return e;
+        units = n;
+    }
+    return n_reps <= units ? launch<4, CHROMO_NB, TW>(d_reps, n_reps, steps, st)
+                           : launch<2, CHROMO_NB, TW>(d_reps, n_reps, steps, st);
 }
 
 }  // namespace
 
 namespace chromo {
 
-hipError_t CHROMO_CAT(spec_launch_, CHROMO_NB)(const chromo_replica *d_reps, int n_reps, int64_t steps,
+hipError_t CHROMO_CAT(spec_launch_, CHROMO_NB)(const chromo_replica *d_reps, int n_reps, int64_t steps, bool twist,
                                                hipStream_t st)
 {
-    return launch<2, CHROMO_NB>(d_reps, n_reps, steps, st);
+    return twist ? launch_shape<true>(d_reps, n_reps, steps, st) : launch_shape<false>(d_reps, n_reps, steps, st);
 }
 
 }  // namespace chromo

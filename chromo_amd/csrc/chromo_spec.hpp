@@ -415,7 +415,7 @@ __device__ __forceinline__ int gen_slot(const chromo_replica *R, WaveRng &rng, c
 // One proposal of a sequential round by the drawing wavefront alone, in the
 // one-at-a-time block (the slot blocks' LDS: every slot hash is empty again on
 // return).  The RNG, the controller and the result pass through LDS, io.
-template <int NB, int W>
+template <int NB, int W, bool TW>
 __device__ __forceinline__ void seq_step(const chromo_replica *R, const EvConst &EC, SeqIO *io, uint32_t *mt,
                                          char *blocks)
 {
@@ -441,7 +441,7 @@ __device__ __forceinline__ void seq_step(const chromo_replica *R, const EvConst 
     if (lane == 0) io->mti = rng.mti;
     const EvLds S = ev_lds(blocks, NB + 1, true);
     ev_clear(S);
-    if (go) mc_evaluate<NB>(R, EC, C, o, P, u, S);
+    if (go) mc_evaluate<NB, TW>(R, EC, C, o, P, u, S);
     const size_t bytes = ev_layout(NB + 1, false).total;
     for (int b = 0; b < Shape<W>::EV; ++b) ev_clear(ev_lds(blocks + bytes * b, NB + 1, false));
     if (lane == 0) {
@@ -539,7 +539,7 @@ __device__ __forceinline__ bool slot_proposal(const chromo_replica *R, const Spe
 // Evaluates slot S into res, its trial state in K, P and the block G, whose hash then
 // holds the slot's voxels (returned: how many; 0 and an empty hash when the slot has to
 // be redone one at a time).
-template <int NB>
+template <int NB, bool TW>
 __device__ __forceinline__ int eval_slot(const chromo_replica *R, const EvConst &EC, const SpecSlot &S, SpecRes &res,
                                          Proposal &P, EvKeep &K, const EvLds &G)
 {
@@ -559,7 +559,7 @@ __device__ __forceinline__ int eval_slot(const chromo_replica *R, const EvConst 
     // arithmetic
     EvBeads<NB> B;
     const int64_t pick = (S.move == CHROMO_TANGENT_ROTATION && (lane & 31) < S.n) ? S.picks[lane & 31] : 0;
-    ev_load<NB, false>(R, S.move, S.n, ind0, indf, 0, pick, B);
+    ev_load<NB, TW>(R, S.move, S.n, ind0, indf, 0, pick, B);
     if (!slot_proposal<NB>(R, S, P, B)) {
         if (lane == 0) res.resample = 1;
         wave_sync();
@@ -567,7 +567,7 @@ __device__ __forceinline__ int eval_slot(const chromo_replica *R, const EvConst 
     }
     EvRes sr;
     const double u = (double)S.ud / RMAX;
-    ev_eval<NB, false>(R, EC, P, u, G, sr, K, B);
+    ev_eval<NB, TW>(R, EC, P, u, G, sr, K, B);
     if (sr.overflow) {
         // more voxels than the block holds: the one-at-a-time path evaluates it
         if (lane == 0) res.overflow = 1;
@@ -749,7 +749,7 @@ __device__ __forceinline__ bool flag_wait(const int32_t *f, int32_t tag)
 // A slot's hash is emptied at the start of its wavefront's next evaluation, when
 // nobody looks into it any more.  The flag waits are bounded; a wait that passes its
 // bound stops the replica with ERR_SPIN at the next round's top.
-template <int NB, int W>
+template <int NB, int W, bool TW>
 __device__ __forceinline__ void spec_block(const chromo_replica *R, const EvConst &EC, WaveRng &rng, chromo_ctrl &C,
                                            Counters &K, const SpecLds &L, int &held)
 {
@@ -810,7 +810,7 @@ __device__ __forceinline__ void spec_block(const chromo_replica *R, const EvCons
                     io->C = C;
                 }
                 wave_sync();
-                seq_step<NB, W>(R, EC, io, L.mt, L.blocks);
+                seq_step<NB, W, TW>(R, EC, io, L.mt, L.blocks);
                 rng_restore(rng, io->ck);
                 rng.mti = uni_i32(io->mti);
                 if (lane == 0) C = io->C;
@@ -836,7 +836,7 @@ __device__ __forceinline__ void spec_block(const chromo_replica *R, const EvCons
             Proposal P;
             if (mine) {
                 ev_release(G, held);
-                held = eval_slot<NB>(R, EC, mys, L.res[wv], P, keep, G);
+                held = eval_slot<NB, TW>(R, EC, mys, L.res[wv], P, keep, G);
             }
             if (evaluates) flag_raise(&L.ctl->done[wv], now);
             if (wv == 0 && mine && L.res[0].accepted && !L.res[0].resample && !L.res[0].overflow) {
@@ -919,7 +919,7 @@ __device__ __forceinline__ void spec_block(const chromo_replica *R, const EvCons
     }
 }
 
-template <int NB, int W>
+template <int NB, int W, bool TW>
 __device__ __forceinline__ void spec_run(const chromo_replica *R, const EvConst &EC, int64_t steps)
 {
     using SH = Shape<W>;
@@ -956,7 +956,7 @@ __device__ __forceinline__ void spec_run(const chromo_replica *R, const EvConst 
     int held = 0;   // voxels in this wavefront's hash
     for (int64_t s = 0; s < steps; ++s) {
         for (int ci = 0; ci < nc; ++ci) {
-            if (sctrl[ci].on == 1) spec_block<NB, W>(R, EC, rng, sctrl[ci], sK, L, held);
+            if (sctrl[ci].on == 1) spec_block<NB, W, TW>(R, EC, rng, sctrl[ci], sK, L, held);
             if (wv == 0 && lane == 0 && !L.ctl->err) update_amplitudes_dev(sctrl[ci]);
             __syncthreads();
             if (L.ctl->err) break;

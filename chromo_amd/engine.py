@@ -161,7 +161,11 @@ class DeviceReplicas:
     CTRL_SLOTS = 8
     SEG_MAX = 32       # beads per move of the one-wavefront evaluator (chromo_seg.hpp)
     WAVE_CHOICES = (1, 2)
-    waves = 1              # wavefronts per replica used by run(); see chromo_amd.autotune
+    # launch shape used by run() (chromo_mc_run_tuned's waves_per_replica); see
+    # chromo_amd.autotune.  2, the speculative kernel, is the faster one from one
+    # replica to 512 and at initial and steady-state windows alike (16 replicas, 10
+    # sweeps: 20.2 ms with 1, see chromo_spec.hip for the speculative shapes).
+    waves = 2
     sweeps_per_launch = 1  # sweeps per captured graph launch chosen by chromo_amd.autotune
 
     def __init__(self, chains: Sequence[ChainSpec], fields: Sequence[FieldSpec],
