@@ -135,6 +135,10 @@ _SIGNATURES = {
     "chromo_energy_adjoint": (ctypes.c_int, [ctypes.POINTER(ChromoEnergyModel), _c_void_p,
                                              _c_void_p, _c_void_p, _c_void_p, _c_void_p,
                                              _c_void_p]),
+    "chromo_energy_adjoint_bytes": (_c_i64, [ctypes.POINTER(ChromoEnergyModel)]),
+    "chromo_energy_adjoint_ws": (ctypes.c_int, [ctypes.POINTER(ChromoEnergyModel), _c_void_p,
+                                                _c_void_p, _c_void_p, _c_void_p, _c_void_p,
+                                                _c_void_p, _c_i64, _c_void_p]),
     "chromo_energy_adjoint_noalloc": (ctypes.c_int, [ctypes.POINTER(ChromoEnergyModel), _c_void_p,
                                                      _c_void_p, _c_void_p, _c_void_p, _c_void_p,
                                                      _c_void_p]),

@@ -116,6 +116,10 @@ __device__ __forceinline__ uint64_t uni_u64(uint64_t x)
 {
     return ((uint64_t)uni_u32((uint32_t)(x >> 32)) << 32) | uni_u32((uint32_t)x);
 }
+__device__ __forceinline__ double uni_f64(double x)
+{
+    return __longlong_as_double((long long)uni_u64((uint64_t)__double_as_longlong(x)));
+}
 __device__ __forceinline__ int64_t bcast0(int64_t x) { return readlane_i64(x, 0); }
 __device__ __forceinline__ int bcast0(int x) { return (int)readlane_u32((uint32_t)x, 0); }
 
@@ -623,6 +627,20 @@ __device__ __forceinline__ double pymod(double a, double b)
     else r = fmod(a, b);
     r += (double)((r != 0) & ((r < 0) ^ (b < 0))) * b;
     return r;
+}
+
+// Divisors div_by takes.
+__host__ __device__ inline bool recip_range(double b) { return b > 0x1p-200 && b < 0x1p200; }
+
+// a / b, correctly rounded, from y = 1 / b correctly rounded: two residual corrections
+// of a y (Markstein's theorem: a quotient within one ulp and an exact residual give the
+// rounded quotient).  For b in recip_range and a zero or far from the ends of the
+// exponent range; 5 operations against the ~12 of a division that must also scale.
+__device__ __forceinline__ double div_by(double a, double b, double y)
+{
+    double q = a * y;
+    q = fma(fma(-b, q, a), y, q);
+    return fma(fma(-b, q, a), y, q);
 }
 
 // ---------------------------------------------------------------------------

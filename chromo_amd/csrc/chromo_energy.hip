@@ -19,8 +19,7 @@
 // that function separately.)  Gradients: with respect to bead positions
 // through the trilinear weights (dw/dx = -+1/dx) and the SSWLC bond energy, and
 // with respect to theta = (chi, eps_ij for i <= j, mu_j).  Densities are
-// recomputed (deterministic scatter) rather than stored; all sums use fixed-
-// order block reductions.
+// recomputed rather than stored; every sum is exact or in a fixed order.
 #include <hip/hip_runtime.h>
 
 #include <math.h>
@@ -32,6 +31,7 @@
 
 #include "chromo_density.hpp"
 #include "chromo_device.hpp"
+#include "chromo_tiles.hpp"
 
 using namespace chromo;
 
@@ -125,11 +125,11 @@ __device__ inline Coef coef_of(const EModel &M, const double *th)
 // final sums read each term's partials contiguously.
 
 // Fixed-order block sum of NT partial values per thread: a butterfly within each
-// wavefront, then the EB / 64 wavefront sums in wavefront order.
-template <int NT>
+// wavefront, then the wavefront sums in wavefront order.
+template <int NT, int THREADS = EB>
 __device__ void block_reduce_store(const double (&vals)[NT], double *part)
 {
-    __shared__ double sh[EB / 64][NT];
+    __shared__ double sh[THREADS / 64][NT];
     const int wv = threadIdx.x / 64, lane = threadIdx.x % 64;
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
@@ -140,7 +140,7 @@ __device__ void block_reduce_store(const double (&vals)[NT], double *part)
     __syncthreads();
     if ((int)threadIdx.x < NT) {
         double s = sh[0][threadIdx.x];
-        for (int w = 1; w < EB / 64; ++w) s += sh[w][threadIdx.x];
+        for (int w = 1; w < THREADS / 64; ++w) s += sh[w][threadIdx.x];
         part[(int64_t)threadIdx.x * gridDim.x + blockIdx.x] = s;
     }
 }
@@ -161,47 +161,219 @@ __device__ void block_reduce_store(double *vals, int nt, double *part)
     }
 }
 
-// ---- voxel terms -----------------------------------------------------------
-// slots: [0..B) S_jj, [B..B+B(B-1)/2) S_jk (j<k), then sum g, sum dg/dchi
-template <int B>
-__global__ void __launch_bounds__(EB) k_e_voxel(EModel M, const double *theta, const double *rho, double *dEdrho,
-                                                double *part)
+// ---- field terms: densities, voxel energies, gradient at the beads ---------------
+//
+// The adjoint needs a deterministic density, not the reference's bead-order fold.
+// Each corner weight w (in [0, 1]) becomes the integer nearest to w 2^60, a high word of
+// 29 bits and a signed low word of 32, and the words are summed in 64 bits each, times
+// the binder state for the binder rows: the sums are exact, so they do not depend on
+// the order in which the LDS takes them.  A voxel's total is rounded to double once and
+// divided by its volume.  Sums stay in range for 2^30 beads (states up to 3).
+
+// The double nearest (hi 2^32 + lo) 2^-60; exact before the one rounding for words
+// below 2^53 (2^23 beads and more in one voxel round once more).
+__device__ __forceinline__ double from_fixed60(uint64_t hi, uint64_t lo)
+{
+    return fma((double)hi, 0x1p32, (double)(int64_t)lo) * 0x1p-60;
+}
+
+// Slots of the block partials: [0..B) S_jj, [B..B+B(B-1)/2) S_jk (j<k), then sum g,
+// sum dg/dchi.
+template <int B, bool GRAD>
+__global__ void __launch_bounds__(TILE_THREADS, 4)
+k_e_tile(EModel M, TileGeom T, const double *theta, const double *r, const int32_t *cnt, const int32_t *base,
+         const int32_t *list, double *grad, double *part)
 {
     constexpr int Bp1 = B + 1, NT = B + B * (B - 1) / 2 + 2;
-    const Coef c = coef_of<B>(M, theta);
-    const int64_t nb = M.G.nx * M.G.ny * M.G.nz;
+    // [species][low, high][voxel]; a voxel's dE/drho overwrites its low words
+    __shared__ unsigned long long sums[Bp1][2][TILE_VOX];
+    __shared__ int32_t owned[TILE_OWN], nown;
+    const int t = threadIdx.x;
     double acc[NT];
 #pragma unroll
-    for (int t = 0; t < NT; ++t) acc[t] = 0;
+    for (int q = 0; q < NT; ++q) acc[q] = 0;
     const double V = M.bead_vol, vb = M.G.vol_bin;
-    for (int64_t v = (int64_t)blockIdx.x * EB + threadIdx.x; v < nb; v += (int64_t)gridDim.x * EB) {
-        double r[Bp1];
-#pragma unroll
-        for (int j = 0; j < Bp1; ++j) r[j] = rho[v * Bp1 + j];
-        int s = B;
+    // the coefficients in scalar registers: held in vector registers through the tile
+    // loop they spill
+    double pref2[B], XX[B * B], gphi, dphi;
+    {
+        const Coef c = coef_of<B>(M, theta);
+        gphi = uni_f64(c.chi * T.vbV);
+        dphi = uni_f64(2 * c.chi * T.vbV);
 #pragma unroll
         for (int j = 0; j < B; ++j) {
-            acc[j] += r[j + 1] * r[j + 1];
+            pref2[j] = uni_f64(2 * c.pref[j]);
 #pragma unroll
-            for (int k = j + 1; k < B; ++k) acc[s++] += r[j + 1] * r[k + 1];
-        }
-        double phi = r[0] * V;
-        bool huge = phi > M.vf_limit;
-        acc[s] += huge ? E_HUGE_FIELD * phi : c.chi * (vb / V) * (phi * phi);
-        acc[s + 1] += huge ? 0.0 : (vb / V) * (phi * phi);
-        if (dEdrho) {
-            double *d = dEdrho + v * Bp1;
-            d[0] = V * (huge ? E_HUGE_FIELD : 2 * c.chi * (vb / V) * phi);
-#pragma unroll
-            for (int j = 0; j < B; ++j) {
-                double g = 2 * c.pref[j] * r[j + 1];
-#pragma unroll
-                for (int k = 0; k < B; ++k) g += (c.X[j * B + k] + c.X[k * B + j]) * r[k + 1];
-                d[j + 1] = g;
-            }
+            for (int k = 0; k < B; ++k) XX[j * B + k] = uni_f64(c.X[j * B + k] + c.X[k * B + j]);
         }
     }
-    block_reduce_store<NT>(acc, part);
+    for (int tile = blockIdx.x; tile < T.ntiles; tile += gridDim.x) {
+        const int tt[3] = {tile % T.nt[0], (tile / T.nt[0]) % T.nt[1], tile / (T.nt[0] * T.nt[1])};
+        int start[3], size[3];
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            start[j] = tile_start(T.n[j], T.nt[j], tt[j]);
+            size[j] = tile_start(T.n[j], T.nt[j], tt[j] + 1) - start[j];
+        }
+        const int len = cnt[tile];
+        const int32_t *mine = list + base[tile];
+        for (int i = t; i < Bp1 * 2 * TILE_VOX; i += TILE_THREADS) (&sums[0][0][0])[i] = 0;
+        if (t == 0) nown = 0;
+        __syncthreads();
+        // the beads' corner weights.  Lists hold runs of the chain, whose neighbours share
+        // voxels: the lanes of a wavefront take entries far apart, so that their adds
+        // meet different voxels
+        const int per = (len + TILE_THREADS - 1) / TILE_THREADS;
+        for (int k = 0; k < per; ++k) {
+            const int i = ((t & 63) * (TILE_THREADS / 64) + (t >> 6)) * per + k;
+            if (i >= len) continue;
+            const int32_t b = mine[i];
+            double x[3], w[3];
+            int ix[3];
+#pragma unroll
+            for (int j = 0; j < 3; ++j) x[j] = r[3 * b + j];
+            int st[B];
+#pragma unroll
+            for (int j = 0; j < B; ++j) st[j] = M.states[(int64_t)j * M.N + b];
+            tile_lower(M.G, T, x, ix, w);
+            int at[3][2];       // voxel place of the lower and upper corner, -1: not this tile's
+            bool own = true;
+            const int stride[3] = {1, TILE_SX, TILE_SX * TILE_SY};
+#pragma unroll
+            for (int j = 0; j < 3; ++j) {
+                if (T.nt[j] == 1) {
+                    at[j][0] = ix[j] * stride[j];
+                    at[j][1] = (ix[j] + 1 == T.n[j] ? 0 : ix[j] + 1) * stride[j];
+                } else {
+                    const int l = tile_local(T.n[j], start[j], size[j], ix[j]);
+                    own = own && l >= 0 && l < size[j];
+                    at[j][0] = l >= 0 ? l * stride[j] : -1;
+                    at[j][1] = l < size[j] ? (l + 1) * stride[j] : -1;
+                }
+            }
+            if (GRAD && own) {
+                const int o = atomicAdd(&nown, 1);
+                if (o < TILE_OWN) owned[o] = b;
+            }
+            // corner_weight's products, the last factor scaled, and the nearest integers:
+            // adding 1.5 2^52 leaves them in the low word
+            const double ux = 1 - w[0], uy = 1 - w[1], uz = (1 - w[2]) * 0x1p28, wz = w[2] * 0x1p28;
+            const double xy[4] = {w[0] * w[1], ux * w[1], w[0] * uy, ux * uy};
+#pragma unroll
+            for (int l = 0; l < 8; ++l) {
+                const int vx = at[0][l & 1], vy = at[1][(l >> 1) & 1], vz = at[2][l >> 2];
+                if ((vx | vy | vz) < 0) continue;
+                const int v = vx + vy + vz;
+                const double wl = xy[l & 3] * ((l & 4) ? uz : wz);
+                const double mh = wl + 0x1.8p52;
+                const double ml = fma(wl - (mh - 0x1.8p52), 0x1p32, 0x1.8p52);
+                const uint32_t hi = (uint32_t)__double_as_longlong(mh);
+                const long long lo = (int32_t)__double_as_longlong(ml);
+                atomicAdd(&sums[0][0][v], (unsigned long long)lo);
+                atomicAdd(&sums[0][1][v], (unsigned long long)hi);
+#pragma unroll
+                for (int j = 0; j < B; ++j) {
+                    if (st[j] != 0) {
+                        atomicAdd(&sums[j + 1][0][v], (unsigned long long)(lo * st[j]));
+                        atomicAdd(&sums[j + 1][1][v], (unsigned long long)(hi * (uint32_t)st[j]));
+                    }
+                }
+            }
+        }
+        __syncthreads();
+        // densities, energy terms of the tile's own voxels, dE/drho in place
+        for (int v = t; v < TILE_VOX; v += TILE_THREADS) {
+            const int vx = v % TILE_SX, vy = (v / TILE_SX) % TILE_SY, vz = v / (TILE_SX * TILE_SY);
+            double rho[Bp1];
+#pragma unroll
+            for (int j = 0; j < Bp1; ++j) {
+                const double f = from_fixed60(sums[j][1][v], sums[j][0][v]);
+                rho[j] = T.recip ? div_by(f, vb, T.rvol) : f / vb;
+            }
+            const double phi = rho[0] * V;
+            const bool huge = phi > M.vf_limit;
+            if (vx < size[0] && vy < size[1] && vz < size[2]) {
+                int s = B;
+#pragma unroll
+                for (int j = 0; j < B; ++j) {
+                    acc[j] += rho[j + 1] * rho[j + 1];
+#pragma unroll
+                    for (int k = j + 1; k < B; ++k) acc[s++] += rho[j + 1] * rho[k + 1];
+                }
+                acc[s] += huge ? E_HUGE_FIELD * phi : gphi * (phi * phi);
+                acc[s + 1] += huge ? 0.0 : T.vbV * (phi * phi);
+            }
+            if (GRAD) {
+                double d[Bp1];
+                d[0] = V * (huge ? E_HUGE_FIELD : dphi * phi);
+#pragma unroll
+                for (int j = 0; j < B; ++j) {
+                    double g = pref2[j] * rho[j + 1];
+#pragma unroll
+                    for (int k = 0; k < B; ++k) g += XX[j * B + k] * rho[k + 1];
+                    d[j + 1] = g;
+                }
+#pragma unroll
+                for (int j = 0; j < Bp1; ++j) sums[j][0][v] = (unsigned long long)__double_as_longlong(d[j]);
+            }
+        }
+        __syncthreads();
+        if (GRAD) {
+            // trilinear chain rule at the beads of the tile's own cells
+            const int no = nown;
+            const bool noted = no <= TILE_OWN;
+            for (int i = t; i < (noted ? no : len); i += TILE_THREADS) {
+                const int32_t b = noted ? owned[i] : mine[i];
+                double x[3], w[3];
+                int ix[3];
+#pragma unroll
+                for (int j = 0; j < 3; ++j) x[j] = r[3 * b + j];
+                tile_lower(M.G, T, x, ix, w);
+                int at[3][2];
+                bool own = true;
+                const int stride[3] = {1, TILE_SX, TILE_SX * TILE_SY};
+#pragma unroll
+                for (int j = 0; j < 3; ++j) {
+                    const int l = ix[j] - start[j];
+                    own = own && l >= 0 && l < size[j];
+                    at[j][0] = l * stride[j];
+                    at[j][1] = (T.nt[j] == 1 && l + 1 == size[j] ? 0 : l + 1) * stride[j];
+                }
+                if (!own) continue;
+                double st[B];
+#pragma unroll
+                for (int j = 0; j < B; ++j) st[j] = (double)M.states[(int64_t)j * M.N + b];
+                // along x first: A the interpolated value, D the difference, for each
+                // (y, z); then along y and z
+                const double ux = 1 - w[0], uy = 1 - w[1], uz = 1 - w[2];
+                double A[4], D[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    double h[2];
+#pragma unroll
+                    for (int e = 0; e < 2; ++e) {
+                        const int v = at[0][e] + at[1][q & 1] + at[2][q >> 1];
+                        h[e] = __longlong_as_double((long long)sums[0][0][v]);
+#pragma unroll
+                        for (int j = 0; j < B; ++j)
+                            h[e] += st[j] * __longlong_as_double((long long)sums[j + 1][0][v]);
+                    }
+                    A[q] = w[0] * h[0] + ux * h[1];
+                    D[q] = h[1] - h[0];
+                }
+                double g[3];
+                g[0] = (w[2] * (w[1] * D[0] + uy * D[1]) + uz * (w[1] * D[2] + uy * D[3])) * T.rd[0];
+                g[1] = (w[2] * (A[1] - A[0]) + uz * (A[3] - A[2])) * T.rd[1];
+                g[2] = ((w[1] * A[2] + uy * A[3]) - (w[1] * A[0] + uy * A[1])) * T.rd[2];
+#pragma unroll
+                for (int j = 0; j < 3; ++j) g[j] = T.recip ? div_by(g[j], vb, T.rvol) : g[j] / vb;
+#pragma unroll
+                for (int j = 0; j < 3; ++j) grad[3 * b + j] = g[j];
+            }
+            __syncthreads();
+        }
+    }
+    block_reduce_store<NT, TILE_THREADS>(acc, part);
 }
 
 // ---- bead / bond terms -------------------------------------------------------
@@ -228,22 +400,18 @@ __device__ inline double E_pair_and_grad(const Bond &bd, const double *r0, const
 }
 
 // slots: [0] E_elastic, [1] E_bind, [2..2+B) D_j, [2+B..2+2B) sum s_j
-// cell and brec: each bead's lower-corner voxel and weights from the density
-// scatter of the same positions (grid_lower's values, not recomputed).
+// grad: the field's gradient on entry (k_e_tile), the whole gradient on return.
 template <int B>
-__global__ void __launch_bounds__(EB) k_e_bead(EModel M, const double *theta, const double *r,
-                                               const double *dEdrho, const int32_t *cell, const BeadRec *brec,
-                                               double *grad, double *part)
+__global__ void __launch_bounds__(EB) k_e_bead(EModel M, const double *theta, const double *r, double *grad,
+                                               double *part)
 {
-    constexpr int Bp1 = B + 1, NT = 2 + 2 * B;
+    constexpr int NT = 2 + 2 * B;
     const int64_t N = M.N;
     const Coef c = coef_of<B>(M, theta);
     double acc[NT];
 #pragma unroll
     for (int t = 0; t < NT; ++t) acc[t] = 0;
     const double f = M.mu_adjust;
-    // +-1 / dx is exactly +-(1 / dx)
-    const double inv_d[3] = {1.0 / M.G.dxyz[0], 1.0 / M.G.dxyz[1], 1.0 / M.G.dxyz[2]};
     // bond i = (i, i + 1): each is evaluated once, by thread i - b0 of the block
     // that holds bead i (the block's first bond (b0 - 1, b0) by its last thread);
     // the derivatives meet in LDS, where beads b and b + 1 read them
@@ -253,6 +421,9 @@ __global__ void __launch_bounds__(EB) k_e_bead(EModel M, const double *theta, co
         const int64_t b = b0 + t;
         const double *rb = r + 3 * b;
         const double *tb = M.t3 + 3 * b;
+        double g[3] = {0, 0, 0};
+        if (grad && b < N)
+            for (int j = 0; j < 3; ++j) g[j] = grad[3 * b + j];
         if (b + 1 < N) {
             Bond bd = load_bond(M.bonds, N, b);
             double gd[3];
@@ -266,14 +437,10 @@ __global__ void __launch_bounds__(EB) k_e_bead(EModel M, const double *theta, co
             E_pair_and_grad(bd, r + 3 * (b0 - 1), r + 3 * b0, M.t3 + 3 * (b0 - 1), M.t3 + 3 * b0, true, gd);
             for (int j = 0; j < 3; ++j) gbond[0][j] = gd[j];
         }
-        double g[3] = {0, 0, 0};
         if (b < N) {
-            int st[B];
-#pragma unroll
-            for (int j = 0; j < B; ++j) st[j] = M.states[(int64_t)j * N + b];
 #pragma unroll
             for (int j = 0; j < B; ++j) {
-                const int s = st[j];
+                const int s = M.states[(int64_t)j * N + b];
                 int m = M.marks[(int64_t)j * N + b];
                 double mu = c.mu[j];
                 double e = M.F[j][m][s];
@@ -281,35 +448,6 @@ __global__ void __launch_bounds__(EB) k_e_bead(EModel M, const double *theta, co
                 acc[1] += e;
                 acc[2 + j] += (s == 2);
                 acc[2 + B + j] += (double)s * ((mu > 0) ? (2 - f) : f);
-            }
-            if (grad && dEdrho) {
-                // 32-bit index arithmetic: the grids hold fewer than 2^31 voxels
-                const int32_t nx = (int32_t)M.G.nx, ny = (int32_t)M.G.ny, nz = (int32_t)M.G.nz;
-                const uint32_t c = (uint32_t)cell[b], cq = c / (uint32_t)nx;
-                const int32_t ix[3] = {(int32_t)(c - cq * (uint32_t)nx), (int32_t)(cq % (uint32_t)ny),
-                                       (int32_t)(cq / (uint32_t)ny)};
-                const double w[3] = {brec[b].w[0], brec[b].w[1], brec[b].w[2]};
-                for (int l = 0; l < 8; ++l) {
-                    int32_t x = ix[0] + (l & 1), y = ix[1] + ((l >> 1) & 1), z = ix[2] + ((l >> 2) & 1);
-                    if (x >= nx) x -= nx;
-                    if (y >= ny) y -= ny;
-                    if (z >= nz) z -= nz;
-                    const int64_t v = x + nx * (y + ny * z);
-                    const double *d = dEdrho + v * Bp1;
-                    double h = d[0];
-#pragma unroll
-                    for (int j = 0; j < B; ++j) h += (double)st[j] * d[j + 1];
-                    h /= M.G.vol_bin;
-                    double a[3];
-                    for (int j = 0; j < 3; ++j) a[j] = ((l >> j) & 1) ? (1 - w[j]) : w[j];
-                    for (int j = 0; j < 3; ++j) {
-                        double dw = ((l >> j) & 1) ? inv_d[j] : -inv_d[j];
-                        double prod = dw;
-                        for (int q = 0; q < 3; ++q)
-                            if (q != j) prod *= a[q];
-                        g[j] += prod * h;
-                    }
-                }
             }
         }
         if (grad) {
@@ -326,16 +464,6 @@ __global__ void __launch_bounds__(EB) k_e_bead(EModel M, const double *theta, co
         }
     }
     block_reduce_store<NT>(acc, part);
-}
-
-// The voxel and bead kernels of one energy evaluation, for B binders.
-template <int B>
-void launch_energy_terms(const EModel &M, const double *theta, const double *rho, double *dEdrho, double *vpart,
-                         int gv, const double *r, const DensityScratch &S, double *grad, double *bpart, int gb,
-                         hipStream_t st)
-{
-    hipLaunchKernelGGL(k_e_voxel<B>, dim3(gv), dim3(EB), 0, st, M, theta, rho, dEdrho, vpart);
-    hipLaunchKernelGGL(k_e_bead<B>, dim3(gb), dim3(EB), 0, st, M, theta, r, dEdrho, S.cell, S.brec, grad, bpart);
 }
 
 // Sums of the block partials of ntv voxel terms and ntb bead terms, by one block of
@@ -429,15 +557,6 @@ k_e_final(EModel M, const double *theta, const double *vpart, int nbv, int ntv, 
 #pragma unroll
         for (int j = 0; j < B; ++j) gtheta[1 + B * (B + 1) / 2 + j] = -sb[2 + B + j];
     }
-}
-
-// The final reduction and assembly of one energy evaluation, for B binders.
-template <int B>
-void launch_energy_final(const EModel &M, const double *theta, const double *vpart, int gv, int ntv,
-                         const double *bpart, int gb, int ntb, double *E, double *gtheta, hipStream_t st)
-{
-    hipLaunchKernelGGL(k_e_final<B>, dim3(1), dim3(FINAL_THREADS), 0, st, M, theta, vpart, gv, ntv, bpart, gb, ntb,
-                       E, gtheta);
 }
 
 // ---- the reference's compute_E (fields.pyx:1939-2286, polymers.pyx:1348-1381) ----
@@ -584,23 +703,32 @@ int make_model(const chromo_energy_model *m, EModel &M)
     return 0;
 }
 
-// Device buffers of one energy evaluation, carved from one allocation (or from
-// the file-scope scratch array of chromo_energy_adjoint_noalloc).
+// make_model and the argument checks of the energy adjoint's entry points.
+int make_adjoint_model(const chromo_energy_model *m, const double *d_r, const double *d_theta, const double *d_E,
+                       EModel &M)
+{
+    const int rc = make_model(m, M);
+    if (rc) return rc;
+    if (M.twist) return eset(-1, "the energy adjoint has no twist term (SSTWLC)");
+    if (!d_r || !d_theta || !d_E) return eset(-1, "NULL argument");
+    return 0;
+}
+
+// Device buffers of one evaluation of the reference energies, carved from one
+// allocation.
 struct EnergyBufs {
     DensityScratch S;
-    double *rho = nullptr, *dEdrho = nullptr, *vpart = nullptr, *bpart = nullptr;
+    double *rho = nullptr, *vpart = nullptr, *bpart = nullptr;
     int gv = 0, gb = 0;
 };
 
 // Carves the buffers of an evaluation of M from base (nullptr: sizes only) and
 // returns the bytes used.  rho_given: the density goes to the caller's array.
-// fixed_order: the adjoint's density (k_dens_gather_fixed); otherwise the
-// reference's bead-order fold.
-size_t energy_carve(const EModel &M, bool grad, bool rho_given, bool fixed_order, char *base, EnergyBufs &Bf)
+size_t energy_carve(const EModel &M, bool rho_given, char *base, EnergyBufs &Bf)
 {
     const int64_t nb = M.G.nx * M.G.ny * M.G.nz;
     const int Bp1 = M.B + 1;
-    size_t o = density_scratch_carve(Bf.S, base, M.N, nb, fixed_order);
+    size_t o = density_scratch_carve(Bf.S, base, M.N, nb);
     auto take = [&](size_t bytes) {
         double *p = base ? (double *)(base + o) : nullptr;
         o = align_scratch(o + bytes);
@@ -609,9 +737,36 @@ size_t energy_carve(const EModel &M, bool grad, bool rho_given, bool fixed_order
     Bf.gv = grid_blocks(nb);
     Bf.gb = grid_blocks(M.N);
     Bf.rho = rho_given ? nullptr : take(sizeof(double) * nb * Bp1);
-    Bf.dEdrho = grad ? take(sizeof(double) * nb * Bp1) : nullptr;
     Bf.vpart = take(sizeof(double) * MAXT * Bf.gv);
     Bf.bpart = take(sizeof(double) * MAXT * Bf.gb);
+    return o;
+}
+
+// The same for the energy and its adjoint: the tiles' lists and the block partials.
+struct AdjointBufs {
+    int32_t *cnt = nullptr, *fill = nullptr, *base = nullptr, *cursor = nullptr, *cell = nullptr, *list = nullptr;
+    double *vpart = nullptr, *bpart = nullptr;
+    int gt = 0, gb = 0;
+};
+
+size_t adjoint_carve(const EModel &M, const TileGeom &T, char *base, AdjointBufs &Bf)
+{
+    size_t o = 0;
+    auto take = [&](size_t bytes) {
+        char *p = base ? base + o : nullptr;
+        o = align_scratch(o + bytes);
+        return p;
+    };
+    Bf.gt = T.ntiles < TILE_BLOCKS ? T.ntiles : TILE_BLOCKS;
+    Bf.gb = grid_blocks(M.N);
+    Bf.cnt = (int32_t *)take(sizeof(int32_t) * T.ntiles);
+    Bf.fill = (int32_t *)take(sizeof(int32_t) * T.ntiles);
+    Bf.base = (int32_t *)take(sizeof(int32_t) * T.ntiles);
+    Bf.cursor = (int32_t *)take(sizeof(int32_t));
+    Bf.cell = (int32_t *)take(sizeof(int32_t) * M.N);
+    Bf.list = (int32_t *)take(sizeof(int32_t) * M.N * tile_images(T));
+    Bf.vpart = (double *)take(sizeof(double) * MAXT * Bf.gt);
+    Bf.bpart = (double *)take(sizeof(double) * MAXT * Bf.gb);
     return o;
 }
 
@@ -625,32 +780,55 @@ struct StreamBuffer {
     }
 };
 
-// E, dE/dr and dE/dtheta of M at (r, theta) with the buffers Bf.
-int energy_adjoint_run(const EModel &M, const double *d_r, const double *d_theta, double *d_E, double *d_grad_r,
-                       double *d_grad_theta, EnergyBufs &Bf, hipStream_t st)
+template <int B>
+void launch_adjoint(const EModel &M, const TileGeom &T, const double *r, const double *theta, double *E, double *grad,
+                    double *gtheta, const AdjointBufs &Bf, hipStream_t st)
 {
-    const int B = M.B, Bp1 = B + 1;
-    PosView P{d_r, 1, 3};
-    // a deterministic density, not the reference's bead-order fold (nothing compares
-    // the adjoint's densities with the reference's bit for bit)
-    hipError_t e = density_scatter(M.G, M.N, Bp1, P, M.states, Bf.rho, 0, Bf.S, st, true);
-    if (e != hipSuccess) return eset(-2, std::string("density scatter: ") + hipGetErrorString(e));
-    const int ntv = B + B * (B - 1) / 2 + 2, ntb = 2 + 2 * B;
-    const int gv = Bf.gv, gb = Bf.gb;
-    switch (B) {
-    case 1: launch_energy_terms<1>(M, d_theta, Bf.rho, Bf.dEdrho, Bf.vpart, gv, d_r, Bf.S, d_grad_r, Bf.bpart, gb, st); break;
-    case 2: launch_energy_terms<2>(M, d_theta, Bf.rho, Bf.dEdrho, Bf.vpart, gv, d_r, Bf.S, d_grad_r, Bf.bpart, gb, st); break;
-    case 3: launch_energy_terms<3>(M, d_theta, Bf.rho, Bf.dEdrho, Bf.vpart, gv, d_r, Bf.S, d_grad_r, Bf.bpart, gb, st); break;
-    default: launch_energy_terms<4>(M, d_theta, Bf.rho, Bf.dEdrho, Bf.vpart, gv, d_r, Bf.S, d_grad_r, Bf.bpart, gb, st); break;
-    }
-    switch (B) {
-    case 1: launch_energy_final<1>(M, d_theta, Bf.vpart, gv, ntv, Bf.bpart, gb, ntb, d_E, d_grad_theta, st); break;
-    case 2: launch_energy_final<2>(M, d_theta, Bf.vpart, gv, ntv, Bf.bpart, gb, ntb, d_E, d_grad_theta, st); break;
-    case 3: launch_energy_final<3>(M, d_theta, Bf.vpart, gv, ntv, Bf.bpart, gb, ntb, d_E, d_grad_theta, st); break;
-    default: launch_energy_final<4>(M, d_theta, Bf.vpart, gv, ntv, Bf.bpart, gb, ntb, d_E, d_grad_theta, st); break;
+    if (grad)
+        hipLaunchKernelGGL((k_e_tile<B, true>), dim3(Bf.gt), dim3(TILE_THREADS), 0, st, M, T, theta, r, Bf.cnt, Bf.base,
+                           Bf.list, grad, Bf.vpart);
+    else
+        hipLaunchKernelGGL((k_e_tile<B, false>), dim3(Bf.gt), dim3(TILE_THREADS), 0, st, M, T, theta, r, Bf.cnt,
+                           Bf.base, Bf.list, grad, Bf.vpart);
+    hipLaunchKernelGGL(k_e_bead<B>, dim3(Bf.gb), dim3(EB), 0, st, M, theta, r, grad, Bf.bpart);
+    hipLaunchKernelGGL(k_e_final<B>, dim3(1), dim3(FINAL_THREADS), 0, st, M, theta, Bf.vpart, Bf.gt,
+                       B + B * (B - 1) / 2 + 2, Bf.bpart, Bf.gb, 2 + 2 * B, E, gtheta);
+}
+
+// E, dE/dr and dE/dtheta of M at (r, theta) with the buffers Bf.
+int energy_adjoint_run(const EModel &M, const TileGeom &T, const double *d_r, const double *d_theta, double *d_E,
+                       double *d_grad_r, double *d_grad_theta, const AdjointBufs &Bf, hipStream_t st)
+{
+    const unsigned gb = (unsigned)((M.N + BIN_THREADS - 1) / BIN_THREADS), gt = (unsigned)((T.ntiles + 255) / 256);
+    // cleared by a kernel rather than hipMemsetAsync: a caller may capture this
+    // sequence in a HIP graph
+    hipLaunchKernelGGL(k_tile_clear, dim3(gt), dim3(256), 0, st, Bf.cnt, Bf.fill, Bf.cursor, T.ntiles);
+    hipLaunchKernelGGL(k_tile_bin<false>, dim3(gb), dim3(BIN_THREADS), 0, st, M.G, T, M.N, d_r, Bf.cell, Bf.cnt,
+                       (const int32_t *)nullptr, (int32_t *)nullptr);
+    hipLaunchKernelGGL(k_tile_base, dim3(gt), dim3(256), 0, st, Bf.cnt, Bf.base, Bf.cursor, T.ntiles);
+    hipLaunchKernelGGL(k_tile_bin<true>, dim3(gb), dim3(BIN_THREADS), 0, st, M.G, T, M.N, d_r, Bf.cell, Bf.fill, Bf.base,
+                       Bf.list);
+    switch (M.B) {
+    case 1: launch_adjoint<1>(M, T, d_r, d_theta, d_E, d_grad_r, d_grad_theta, Bf, st); break;
+    case 2: launch_adjoint<2>(M, T, d_r, d_theta, d_E, d_grad_r, d_grad_theta, Bf, st); break;
+    case 3: launch_adjoint<3>(M, T, d_r, d_theta, d_E, d_grad_r, d_grad_theta, Bf, st); break;
+    default: launch_adjoint<4>(M, T, d_r, d_theta, d_E, d_grad_r, d_grad_theta, Bf, st); break;
     }
     HIPE(hipGetLastError());
     return 0;
+}
+
+// The scratch chromo_energy_adjoint_noalloc documents and checks: a limit on sizes
+// that does not move with the kernels.
+size_t noalloc_bytes(const EModel &M, bool grad)
+{
+    const size_t nb = (size_t)(M.G.nx * M.G.ny * M.G.nz), Bp1 = (size_t)M.B + 1, N = (size_t)M.N;
+    size_t o = 0;
+    for (size_t x : {4 * N, 4 * N, 32 * N, 32 * N, 4 * nb, 4 * nb, 4 * nb, (size_t)8192, (size_t)8192, (size_t)8,
+                     8 * nb * Bp1, grad ? 8 * nb * Bp1 : (size_t)0, 8 * MAXT * (size_t)grid_blocks((int64_t)nb),
+                     8 * MAXT * (size_t)grid_blocks(M.N)})
+        o = align_scratch(o + x);
+    return o;
 }
 
 // ---- the allocation-free evaluation -----------------------------------------
@@ -691,38 +869,62 @@ int chromo_energy_adjoint(const chromo_energy_model *model, const double *d_r, c
                           double *d_E, double *d_grad_r, double *d_grad_theta, void *stream)
 {
     EModel M;
-    int rc = make_model(model, M);
+    int rc = make_adjoint_model(model, d_r, d_theta, d_E, M);
     if (rc) return rc;
-    if (M.twist) return eset(-1, "the energy adjoint has no twist term (SSTWLC)");
-    if (!d_r || !d_theta || !d_E) return eset(-1, "NULL argument");
     hipStream_t st = (hipStream_t)stream;
-    EnergyBufs Bf;
-    const size_t bytes = energy_carve(M, d_grad_r != nullptr, false, true, nullptr, Bf);
+    const TileGeom T = tile_geom(M.G, M.bead_vol);
+    AdjointBufs Bf;
     StreamBuffer buf;
     buf.st = st;
-    HIPE(hipMallocAsync((void **)&buf.p, bytes, st));
-    energy_carve(M, d_grad_r != nullptr, false, true, buf.p, Bf);
-    return energy_adjoint_run(M, d_r, d_theta, d_E, d_grad_r, d_grad_theta, Bf, st);
+    HIPE(hipMallocAsync((void **)&buf.p, adjoint_carve(M, T, nullptr, Bf), st));
+    adjoint_carve(M, T, buf.p, Bf);
+    return energy_adjoint_run(M, T, d_r, d_theta, d_E, d_grad_r, d_grad_theta, Bf, st);
+}
+
+int64_t chromo_energy_adjoint_bytes(const chromo_energy_model *model)
+{
+    EModel M;
+    const int rc = make_model(model, M);
+    if (rc) return rc;
+    AdjointBufs Bf;
+    return (int64_t)adjoint_carve(M, tile_geom(M.G, M.bead_vol), nullptr, Bf);
+}
+
+int chromo_energy_adjoint_ws(const chromo_energy_model *model, const double *d_r, const double *d_theta,
+                             double *d_E, double *d_grad_r, double *d_grad_theta, void *d_ws, int64_t ws_bytes,
+                             void *stream)
+{
+    EModel M;
+    int rc = make_adjoint_model(model, d_r, d_theta, d_E, M);
+    if (rc) return rc;
+    const TileGeom T = tile_geom(M.G, M.bead_vol);
+    AdjointBufs Bf;
+    const size_t bytes = adjoint_carve(M, T, nullptr, Bf);
+    if (!d_ws || ws_bytes < 0 || (size_t)ws_bytes < bytes)
+        return eset(-1, "the workspace holds fewer bytes than chromo_energy_adjoint_bytes");
+    if ((uintptr_t)d_ws % 16) return eset(-1, "the workspace must be 16-byte aligned");
+    adjoint_carve(M, T, (char *)d_ws, Bf);
+    return energy_adjoint_run(M, T, d_r, d_theta, d_E, d_grad_r, d_grad_theta, Bf, (hipStream_t)stream);
 }
 
 int chromo_energy_adjoint_noalloc(const chromo_energy_model *model, const double *d_r, const double *d_theta,
                                   double *d_E, double *d_grad_r, double *d_grad_theta, void *stream)
 {
     EModel M;
-    int rc = make_model(model, M);
+    int rc = make_adjoint_model(model, d_r, d_theta, d_E, M);
     if (rc) return rc;
-    if (M.twist) return eset(-1, "the energy adjoint has no twist term (SSTWLC)");
-    if (!d_r || !d_theta || !d_E) return eset(-1, "NULL argument");
-    EnergyBufs Bf;
-    const size_t bytes = energy_carve(M, d_grad_r != nullptr, false, true, nullptr, Bf);
+    const TileGeom T = tile_geom(M.G, M.bead_vol);
+    AdjointBufs Bf;
+    const size_t doc = noalloc_bytes(M, d_grad_r != nullptr), own = adjoint_carve(M, T, nullptr, Bf);
+    const size_t bytes = doc > own ? doc : own;
     if (bytes > NOALLOC_BYTES)
         return eset(-1, "the evaluation needs " + std::to_string(bytes) + " bytes of scratch; the allocation-free "
                         "entry point holds " + std::to_string(NOALLOC_BYTES) + " (use chromo_energy_adjoint)");
     char *base = nullptr;
     rc = noalloc_scratch(&base);
     if (rc) return rc;
-    energy_carve(M, d_grad_r != nullptr, false, true, base, Bf);
-    return energy_adjoint_run(M, d_r, d_theta, d_E, d_grad_r, d_grad_theta, Bf, (hipStream_t)stream);
+    adjoint_carve(M, T, base, Bf);
+    return energy_adjoint_run(M, T, d_r, d_theta, d_E, d_grad_r, d_grad_theta, Bf, (hipStream_t)stream);
 }
 
 int chromo_energy_reference(const chromo_energy_model *model, const double *d_pos, int32_t soa,
@@ -736,11 +938,11 @@ int chromo_energy_reference(const chromo_energy_model *model, const double *d_po
     hipStream_t st = (hipStream_t)stream;
     const int B = M.B, Bp1 = B + 1;
     EnergyBufs Bf;
-    const size_t bytes = energy_carve(M, false, d_density_out != nullptr, false, nullptr, Bf);
+    const size_t bytes = energy_carve(M, d_density_out != nullptr, nullptr, Bf);
     StreamBuffer buf;
     buf.st = st;
     HIPE(hipMallocAsync((void **)&buf.p, bytes, st));
-    energy_carve(M, false, d_density_out != nullptr, false, buf.p, Bf);
+    energy_carve(M, d_density_out != nullptr, buf.p, Bf);
     double *rho = d_density_out ? d_density_out : Bf.rho;
     const int gv = Bf.gv, gb = Bf.gb;
     // UniformDensityField.update_all_densities: bead-order scatter without the 1e-18 clean-up

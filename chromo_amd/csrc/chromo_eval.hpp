@@ -135,8 +135,6 @@ struct EvConst {
     int32_t n[3], fast, recip, cross;
 };
 
-__device__ __forceinline__ bool recip_range(double b) { return b > 0x1p-200 && b < 0x1p200; }
-
 // Fills the constants; the first four threads of the workgroup, the caller synchronises.
 __device__ __forceinline__ void ev_const(EvConst *C, const chromo_replica *R)
 {
@@ -170,17 +168,6 @@ __device__ __forceinline__ void ev_const(EvConst *C, const chromo_replica *R)
         for (int j = 0; j < R->B * R->B; ++j) x = x || R->cross[j] != 0;
         C->cross = x;
     }
-}
-
-// a / b, correctly rounded, from y = 1 / b correctly rounded: two residual corrections
-// of a y (Markstein's theorem: a quotient within one ulp and an exact residual give the
-// rounded quotient).  For b in recip_range and a zero or far from the ends of the
-// exponent range; 5 operations against the ~12 of a division that must also scale.
-__device__ __forceinline__ double div_by(double a, double b, double y)
-{
-    double q = a * y;
-    q = fma(fma(-b, q, a), y, q);
-    return fma(fma(-b, q, a), y, q);
 }
 
 // Lower voxel indices and lower-corner weights of one position: voxel_lower's values

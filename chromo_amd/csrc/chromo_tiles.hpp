@@ -1,0 +1,228 @@
+// chromo_tiles.hpp -- voxel densities, field energy and its gradient of the energy
+// adjoint, tile by tile in LDS.
+//
+// The grid is cut into tiles of at most 8 x 8 x 8 voxels.  Every bead is listed in
+// the tile of its lower-corner cell and in the tiles that cell is a neighbour of
+// (at most one per axis), so a tile's list holds every bead that reaches its voxels
+// and their upper neighbours.  One block per tile then does what took four passes over
+// memory: it adds the beads' corner weights into LDS, turns each voxel's density into
+// its energy terms and dE/drho in place, and gathers dE/drho back at the beads of its
+// own cells.  Neither the densities nor dE/drho ever reach HBM.
+//
+// What bounds it: at 10^6 beads, B = 4, 128^3 voxels a third of the time is the adds (8
+// corners x species x 2 words per bead and tile, a third of them conflicting), a quarter
+// turning sums into dE/drho, a sixth the gather at the beads, the rest loads, weights and
+// the barriers between; two blocks of eight wavefronts share a compute unit's LDS.
+// Tiles of 8 x 8 x 4 with four smaller blocks take the same time (less waiting, more
+// halo).  One evaluation there: 417 us as bucketed records, a gather of every record by
+// its eight voxels and passes for the voxel and bead terms; 280 us so.
+#pragma once
+
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include "chromo_density.hpp"
+#include "chromo_device.hpp"
+
+namespace chromo {
+namespace {
+
+// Tiles of at most 8 x 8 x 8 voxels.  Tile t of an axis of n voxels cut into nt tiles
+// starts at t n / nt: tiles of at least half the size when there are several, so a cell
+// touches at most one face per axis and the lists hold at most twice the beads per axis.
+// An axis that fits one tile is one tile that wraps onto itself.
+constexpr int TILE_MAX[3] = {8, 8, 8};
+constexpr int TILE_SX = 9, TILE_SY = 9, TILE_SZ = 9;    // a tile's voxels and their upper neighbours
+constexpr int TILE_VOX = TILE_SX * TILE_SY * TILE_SZ;
+constexpr int TILE_THREADS = 512;
+constexpr int TILE_OWN = 1024;              // beads of its own cells a tile notes down in LDS
+constexpr int TILE_BLOCKS = 1024;           // blocks of the tile kernel, at most
+
+struct TileGeom {
+    int32_t n[3], nt[3], ntiles;
+    int32_t recip;                          // the divisors below suit div_by
+    double rw[3], rd[3], rvol;              // 1 / width, 1 / voxel side, 1 / vol_bin
+    double vbV;                             // vol_bin / bead_vol
+};
+
+inline TileGeom tile_geom(const GridGeom &G, double bead_vol)
+{
+    TileGeom T;
+    const int64_t n[3] = {G.nx, G.ny, G.nz};
+    T.ntiles = 1;
+    T.recip = recip_range(G.vol_bin);
+    T.rvol = 1.0 / G.vol_bin;
+    T.vbV = G.vol_bin / bead_vol;
+    for (int j = 0; j < 3; ++j) {
+        T.n[j] = (int32_t)n[j];
+        T.nt[j] = (int32_t)((n[j] + TILE_MAX[j] - 1) / TILE_MAX[j]);
+        T.ntiles *= T.nt[j];
+        T.recip = T.recip && recip_range(G.width[j]) && recip_range(G.dxyz[j]);
+        T.rw[j] = 1.0 / G.width[j];
+        T.rd[j] = 1.0 / G.dxyz[j];
+    }
+    return T;
+}
+
+// Tiles that list one bead, at most.
+inline int tile_images(const TileGeom &T)
+{
+    int k = 1;
+    for (int j = 0; j < 3; ++j) k *= T.nt[j] > 1 ? 2 : 1;
+    return k;
+}
+
+__device__ __forceinline__ int tile_start(int n, int nt, int t) { return (int)((int64_t)t * n / nt); }
+__device__ __forceinline__ int tile_of(int n, int nt, int c) { return (int)(((int64_t)(c + 1) * nt - 1) / n); }
+
+// grid_lower's cell and weights (chromo_density.hpp), bit for bit, with the exact
+// divisions from reciprocals where the grid allows.
+__device__ __forceinline__ void tile_lower(const GridGeom &G, const TileGeom &T, const double *x, int ix[3],
+                                           double w[3])
+{
+    double a[3];
+    bool far = !T.recip;
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        a[j] = x[j] + G.half_width[j];
+        far = far || !(fabs(a[j]) < 0x1p40 * G.width[j]);
+    }
+    if (far) {
+        int64_t i64[3];
+        grid_lower(G, x[0], x[1], x[2], i64, w);
+#pragma unroll
+        for (int j = 0; j < 3; ++j) ix[j] = (int)i64[j];
+        return;
+    }
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        const double W = G.width[j];
+        double q = trunc(a[j] * T.rw[j]);
+        double r = fma(-q, W, a[j]);
+        q += (a[j] >= 0) ? ((r < 0) ? -1.0 : (r >= W ? 1.0 : 0.0)) : ((r > 0) ? 1.0 : (r <= -W ? -1.0 : 0.0));
+        r = fma(-q, W, a[j]);
+        r += (r < 0) ? W : 0.0;
+        double u = div_by(r - G.half_step[j], G.dxyz[j], T.rd[j]);
+        if (!(u >= -1.0 && u < (double)T.n[j])) u = 0.0;
+        const double f = floor(u);
+        ix[j] = (f == -1.0) ? T.n[j] - 1 : (int)f;
+        w[j] = 1 - (u - f);
+    }
+}
+
+// The tiles of one axis that list a bead of cell c: its own and, when the cell lies on
+// a face, the neighbour behind that face.  Returns how many.
+__device__ __forceinline__ int axis_tiles(int n, int nt, int c, int t[2])
+{
+    t[0] = nt == 1 ? 0 : tile_of(n, nt, c);
+    t[1] = t[0];
+    if (nt == 1) return 1;
+    if (c == tile_start(n, nt, t[0])) {
+        t[1] = t[0] == 0 ? nt - 1 : t[0] - 1;
+        return 2;
+    }
+    if (c + 1 == tile_start(n, nt, t[0] + 1)) {
+        t[1] = t[0] + 1 == nt ? 0 : t[0] + 1;
+        return 2;
+    }
+    return 1;
+}
+
+// Clears the lists' counters and the list cursor.
+__global__ void k_tile_clear(int32_t *cnt, int32_t *fill, int32_t *cursor, int n)
+{
+    const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    if (i < n) cnt[i] = fill[i] = 0;
+    if (i == 0) *cursor = 0;
+}
+
+// Room for every list: a wavefront's lists in a row, the wavefronts in the order they
+// arrive (nothing depends on where a list lies).
+__global__ void k_tile_base(const int32_t *cnt, int32_t *base, int32_t *cursor, int n)
+{
+    const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    const int k = i < n ? cnt[i] : 0;
+    int tot;
+    const int off = wave_excl_scan(k, tot);
+    int at = 0;
+    if (lane_id() == 0) at = atomicAdd(cursor, tot);
+    at = bcast0(at);
+    if (i < n) base[i] = at + off;
+}
+
+// PLACE false: each bead's cell into cell[], and the lists' lengths into num.  PLACE
+// true: the beads into their lists, num counting the entries placed.  A block counts its beads per
+// list in LDS first (consecutive beads lie in a few tiles), so that a list costs it one
+// global atomic; a list that finds no room in the block's table takes its entries from
+// the global counter one by one.  The order within a list does not matter.
+constexpr int TILE_TABLE = 512, TILE_PROBES = 16, BIN_THREADS = 256;
+
+template <bool PLACE>
+__global__ void __launch_bounds__(BIN_THREADS) k_tile_bin(GridGeom G, TileGeom T, int64_t N, const double *r, int32_t *cell,
+                                                  int32_t *num, const int32_t *base, int32_t *list)
+{
+    __shared__ int32_t key[TILE_TABLE], cntl[TILE_TABLE], from[TILE_TABLE];
+    for (int i = threadIdx.x; i < TILE_TABLE; i += BIN_THREADS) {
+        key[i] = -1;
+        cntl[i] = 0;
+    }
+    __syncthreads();
+    const int64_t b = (int64_t)blockIdx.x * BIN_THREADS + threadIdx.x;
+    int slot[8], rank[8], tile[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) tile[q] = -1;
+    if (b < N) {
+        int ix[3];
+        if (PLACE) {
+            const uint32_t c = (uint32_t)cell[b], q = c / (uint32_t)T.n[0];
+            ix[0] = (int)(c - q * (uint32_t)T.n[0]);
+            ix[1] = (int)(q % (uint32_t)T.n[1]);
+            ix[2] = (int)(q / (uint32_t)T.n[1]);
+        } else {
+            double x[3], w[3];
+            for (int j = 0; j < 3; ++j) x[j] = r[3 * b + j];
+            tile_lower(G, T, x, ix, w);
+            cell[b] = ix[0] + T.n[0] * (ix[1] + T.n[1] * ix[2]);
+        }
+        int t[3][2], k[3];
+#pragma unroll
+        for (int j = 0; j < 3; ++j) k[j] = axis_tiles(T.n[j], T.nt[j], ix[j], t[j]);
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            if ((q & 1) >= k[0] || ((q >> 1) & 1) >= k[1] || (q >> 2) >= k[2]) continue;
+            tile[q] = t[0][q & 1] + T.nt[0] * (t[1][(q >> 1) & 1] + T.nt[1] * t[2][q >> 2]);
+            int h = tile[q] & (TILE_TABLE - 1);
+            slot[q] = -1;
+            for (int p = 0; p < TILE_PROBES; ++p) {
+                const int old = atomicCAS(&key[h], -1, tile[q]);
+                if (old == -1 || old == tile[q]) {
+                    slot[q] = h;
+                    break;
+                }
+                h = (h + 1) & (TILE_TABLE - 1);
+            }
+            rank[q] = slot[q] >= 0 ? atomicAdd(&cntl[slot[q]], 1) : atomicAdd(&num[tile[q]], 1);
+        }
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < TILE_TABLE; i += BIN_THREADS)
+        if (key[i] >= 0) from[i] = atomicAdd(&num[key[i]], cntl[i]);
+    if (!PLACE) return;
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 8; ++q)
+        if (tile[q] >= 0) list[base[tile[q]] + (slot[q] >= 0 ? from[slot[q]] : 0) + rank[q]] = (int32_t)b;
+}
+
+// Place of a cell on one axis of a tile of `size` voxels from `start`: 0 .. size - 1
+// inside, -1 and size for the neighbours below and above.
+__device__ __forceinline__ int tile_local(int n, int start, int size, int c)
+{
+    int d = c - start;
+    if (d >= 0 && d < size) return d;
+    if (d < 0) d += n;
+    return d == size ? size : -1;
+}
+
+}  // namespace
+}  // namespace chromo

@@ -298,15 +298,23 @@ int chromo_energy_adjoint(const chromo_energy_model *model, const double *d_r,
                           const double *d_theta, double *d_E, double *d_grad_r,
                           double *d_grad_theta, void *stream);
 
+/* chromo_energy_adjoint with a workspace of the caller's: device memory of at least
+ * chromo_energy_adjoint_bytes(model) bytes (negative: an error code), 16-byte aligned,
+ * free for other use once the work on the stream is done.  Same results bit for bit;
+ * allocates nothing, and calls on different workspaces may overlap. */
+int64_t chromo_energy_adjoint_bytes(const chromo_energy_model *model);
+int chromo_energy_adjoint_ws(const chromo_energy_model *model, const double *d_r,
+                             const double *d_theta, double *d_E, double *d_grad_r,
+                             double *d_grad_theta, void *d_ws, int64_t ws_bytes, void *stream);
+
 /* No counterpart in the reference.  chromo_energy_adjoint for callers that cannot
  * allocate device memory: code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc.  Same arguments, same results bit for bit.
- * Its scratch (the density scatter's buckets, the voxel densities and their
- * adjoint, the block partials) lives in one file-scope device array of 32 MiB
- * per GPU, held until the process ends; it calls no hipMalloc / hipFree.  An
- * evaluation that needs more is rejected (-1, the bytes it needs in the message):
- * 72 B per bead plus 12 + 8 (B+1) B per voxel (12 + 16 (B+1) with gradients),
- * e.g. 20,000 beads and 48^3 voxels with B = 3 take 10 MiB.  Every call on one GPU shares that
+ * Its scratch (the tiles' bead lists, the block partials) lives in one file-scope
+ * device array of 32 MiB per GPU, held until the process ends; it calls no
+ * hipMalloc / hipFree.  An evaluation is rejected (-1, the bytes in the message)
+ * when 72 B per bead plus 12 + 8 (B+1) B per voxel (12 + 16 (B+1) with gradients)
+ * exceed that, e.g. 20,000 beads and 48^3 voxels with B = 3 count as 10 MiB.  Every call on one GPU shares that
  * array and it keeps the last call's contents: calls that overlap on one GPU
  * (two streams, two host threads) race. */
 int chromo_energy_adjoint_noalloc(const chromo_energy_model *model, const double *d_r,
