@@ -6,7 +6,7 @@
   hand-written adjoint kernel, dE/dr and dE/dtheta, with
   theta = (chi, eps_ij for i <= j, mu_j).
 * ``ChromoEnergy`` wraps it as a ``torch.autograd.Function``: forward returns E,
-  backward recomputes the voxel densities and returns dE/dr, dE/dtheta.
+  backward returns dE/dr, dE/dtheta.
 * ``elastic_energy`` / ``field_energy`` are the reference's own
   ``SSWLC.compute_E`` and ``UniformDensityField.compute_E`` on the GPU.
 * ``ReweightingAccumulator`` turns sampled (O, dE/dtheta) pairs into
@@ -111,35 +111,50 @@ def energy(model: EnergyModel, r: torch.Tensor, theta: torch.Tensor, grad: bool 
     theta = theta.detach().to(model.device, torch.float64).contiguous()
     if r.shape != (model.N, 3) or theta.numel() != n_theta(model.B):
         raise ValueError("r must be (N, 3) and theta (1 + B(B+1)/2 + B,)")
-    E = torch.zeros(4, dtype=torch.float64, device=model.device)
+    E = torch.empty(4, dtype=torch.float64, device=model.device)
     gr = torch.empty_like(r) if grad else None
     gt = torch.empty_like(theta) if grad else None
-    L.check(model.lib.chromo_energy_adjoint(ctypes.byref(model.m), r.data_ptr(), theta.data_ptr(),
-                                            E.data_ptr(), gr.data_ptr() if grad else None,
-                                            gt.data_ptr() if grad else None, _current_stream()),
-            "chromo_energy_adjoint")
+    # scratch from torch's allocator, which keeps freed blocks of the stream at hand: a
+    # stream-ordered hipMalloc per evaluation costs up to 350 us after a synchronisation
+    nb = model.lib.chromo_energy_adjoint_bytes(ctypes.byref(model.m))
+    if nb < 0:
+        L.check(int(nb), "chromo_energy_adjoint_bytes")
+    ws = torch.empty(int(nb), dtype=torch.uint8, device=model.device)
+    L.check(model.lib.chromo_energy_adjoint_ws(ctypes.byref(model.m), r.data_ptr(), theta.data_ptr(),
+                                               E.data_ptr(), gr.data_ptr() if grad else None,
+                                               gt.data_ptr() if grad else None, ws.data_ptr(), int(nb),
+                                               _current_stream()),
+            "chromo_energy_adjoint_ws")
     return E, gr, gt
 
 
 class ChromoEnergy(torch.autograd.Function):
-    """E(r, theta) with the adjoint kernel as backward (densities recomputed)."""
+    """E(r, theta) with the adjoint kernel as backward.
+
+    ``with_grad``: the forward evaluation also takes the gradients (one evaluation for a
+    forward and its backward instead of two; the kernels share all but the last step).
+    Without it backward evaluates again.
+    """
 
     @staticmethod
-    def forward(ctx, r, theta, model):
-        E, _, _ = energy(model, r, theta, grad=False)
+    def forward(ctx, r, theta, model, with_grad=False):
+        E, gr, gt = energy(model, r, theta, grad=with_grad)
         ctx.model = model
-        ctx.save_for_backward(r, theta)
+        # r and theta stay saved either way: autograd refuses a backward after either
+        # was changed in place
+        ctx.save_for_backward(r, theta, gr, gt)
         return E[0]
 
     @staticmethod
     def backward(ctx, gout):
-        r, theta = ctx.saved_tensors
-        _, gr, gt = energy(ctx.model, r, theta, grad=True)
-        return gout * gr.to(r.dtype), gout * gt.to(theta.dtype), None
+        r, theta, gr, gt = ctx.saved_tensors
+        if gr is None:
+            _, gr, gt = energy(ctx.model, r, theta, grad=True)
+        return gout * gr.to(r.dtype), gout * gt.to(theta.dtype), None, None
 
 
 def chromo_energy(r: torch.Tensor, theta: torch.Tensor, model: EnergyModel) -> torch.Tensor:
-    return ChromoEnergy.apply(r, theta, model)
+    return ChromoEnergy.apply(r, theta, model, torch.is_grad_enabled() and (r.requires_grad or theta.requires_grad))
 
 
 # ---------------------------------------------------------------------------
