@@ -4,9 +4,8 @@
 // UniformDensityField.update_all_densities_for_all_polymers
 // (chromo/fields.pyx:2041-2106) adds every bead's eight trilinear weights to
 // the grid in bead order.  To reproduce those per-voxel sums bit for bit in
-// parallel, beads are bucketed by their lower-corner voxel (counting sort with
-// sorted buckets) and every voxel then gathers from the <= 8 buckets that reach
-// it, merging them in ascending bead index.  No floating-point atomics.
+// parallel, beads are listed per tile of voxels, and one wavefront per tile folds its
+// list in bead order into LDS.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -48,370 +47,383 @@ __device__ __forceinline__ void grid_lower(const GridGeom &G, double x0, double 
     }
 }
 
-// What the gather reads of one bead, in one 32-byte record (one cache line per
-// merge step instead of one per weight and per state row).
-struct BeadRec {
-    double w[3];
-    int8_t st[CHROMO_MAX_BINDERS];
-    int32_t pad;
-};
-static_assert(sizeof(BeadRec) == 32, "one bead record is 32 bytes");
-
-__global__ void k_dens_cells(GridGeom G, int64_t N, PosView P, int B, const int8_t *states, int32_t *cell,
-                             BeadRec *brec, int32_t *cnt)
-{
-    int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= N) return;
-    int64_t ix[3];
-    double w[3];
-    grid_lower(G, P.p[b * P.sb], P.p[P.sc + b * P.sb], P.p[2 * P.sc + b * P.sb], ix, w);
-    int32_t c = (int32_t)(ix[0] + ix[1] * G.nx + ix[2] * G.nx * G.ny);
-    cell[b] = c;
-    BeadRec q;
-    q.w[0] = w[0];
-    q.w[1] = w[1];
-    q.w[2] = w[2];
-#pragma unroll
-    for (int m = 0; m < CHROMO_MAX_BINDERS; ++m) q.st[m] = m < B ? states[(int64_t)m * N + b] : (int8_t)0;
-    q.pad = 0;
-    brec[b] = q;
-    atomicAdd(&cnt[c], 1);
-}
-
-// exclusive scan: one block of 1024 threads per 2048 elements, block totals in bsum
-__global__ void k_scan_blocks(const int32_t *in, int32_t *out, int32_t *bsum, int64_t n)
-{
-    __shared__ int32_t s[2048];
-    int64_t base = (int64_t)blockIdx.x * 2048;
-    int t = threadIdx.x;
-    for (int i = t; i < 2048; i += 1024) s[i] = (base + i < n) ? in[base + i] : 0;
-    __syncthreads();
-    for (int d = 1; d < 2048; d <<= 1) {
-        int32_t v0 = 0, v1 = 0;
-        int i0 = t, i1 = t + 1024;
-        if (i0 >= d) v0 = s[i0 - d];
-        if (i1 >= d) v1 = s[i1 - d];
-        __syncthreads();
-        s[i0] += v0;
-        s[i1] += v1;
-        __syncthreads();
-    }
-    for (int i = t; i < 2048; i += 1024) {
-        if (base + i < n) out[base + i] = s[i] - in[base + i];
-    }
-    if (t == 0) bsum[blockIdx.x] = s[2047];
-}
-
-__global__ void k_scan_add(int32_t *out, const int32_t *boff, int64_t n)
-{
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) out[i] += boff[i / 2048];
-}
-
-__global__ void k_dens_place(int64_t N, const int32_t *cell, const int32_t *off, int32_t *fill,
-                             int32_t *list)
-{
-    int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= N) return;
-    int32_t c = cell[b];
-    int32_t pos = off[c] + atomicAdd(&fill[c], 1);
-    list[pos] = (int32_t)b;
-}
-
-// Puts each bucket (filled in atomic order by k_dens_place) in bead order.  Small
-// buckets, the usual case, by insertion sort; large ones (dense voxels: compact
-// or collapsed chains, coarse grids) by heapsort, so the cost stays k log k.
-__device__ __forceinline__ void sift_down(int32_t *a, int32_t i, int32_t n)
-{
-    const int32_t x = a[i];
-    for (;;) {
-        int32_t c = 2 * i + 1;
-        if (c >= n) break;
-        if (c + 1 < n && a[c + 1] > a[c]) ++c;
-        if (a[c] <= x) break;
-        a[i] = a[c];
-        i = c;
-    }
-    a[i] = x;
-}
-
-__global__ void k_dens_sort(int64_t nbins, const int32_t *off, const int32_t *cnt, int32_t *list)
-{
-    int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= nbins) return;
-    const int32_t s0 = off[c], k = cnt[c];
-    int32_t *a = list + s0;
-    if (k <= 32) {
-        for (int32_t p = 1; p < k; ++p) {
-            const int32_t x = a[p];
-            int32_t q = p - 1;
-            while (q >= 0 && a[q] > x) {
-                a[q + 1] = a[q];
-                --q;
-            }
-            a[q + 1] = x;
-        }
-        return;
-    }
-    for (int32_t i = k / 2 - 1; i >= 0; --i) sift_down(a, i, k);
-    for (int32_t e = k - 1; e > 0; --e) {
-        const int32_t t = a[0];
-        a[0] = a[e];
-        a[e] = t;
-        sift_down(a, 0, e);
-    }
-}
-
-// The buckets that reach voxel v: cell[l] holds the beads of which v is corner l;
-// a bucket reached by several corners (grids one or two voxels wide) is kept once,
-// in its first slot, whose mask collects every such corner.
-__device__ __forceinline__ void voxel_cells(const GridGeom &G, int64_t v, int32_t (&cell)[8], int (&msk)[8])
-{
-    const int64_t nx = G.nx, ny = G.ny, nz = G.nz;
-    const int64_t x = v % nx, y = (v / nx) % ny, z = v / (nx * ny);
-#pragma unroll
-    for (int l = 0; l < 8; ++l) {
-        int64_t cx = x - (l & 1), cy = y - ((l >> 1) & 1), cz = z - ((l >> 2) & 1);
-        if (cx < 0) cx += nx;
-        if (cy < 0) cy += ny;
-        if (cz < 0) cz += nz;
-        cell[l] = (int32_t)(cx + cy * nx + cz * nx * ny);
-        msk[l] = 0;
-    }
-#pragma unroll
-    for (int l = 0; l < 8; ++l) {
-        bool placed = false;
-#pragma unroll
-        for (int k = 0; k < l; ++k) {
-            if (!placed && cell[k] == cell[l]) {
-                msk[k] |= 1 << l;
-                placed = true;
-            }
-        }
-        if (!placed) msk[l] |= 1 << l;
-    }
-}
-
-// On large grids (at least GATHER_BIG_BLOCKS blocks of 1024 voxels) one gather
-// block takes 1024 consecutive voxels and hands them to its threads in order of
-// merge length (the beads of their buckets, keys clamped to GATHER_KEYS - 1), so
-// that the lanes of a wavefront have merges of similar length.  Smaller grids run
-// in one round of 256-thread blocks, voxel t of the block on thread t: there the
-// ranking's extra phase costs more than the balance saves.
-constexpr int GATHER_KEYS = 64, GATHER_BIG_BLOCKS = 512;
-
-// density[v * Bp1 + m]: m = 0 beads, m >= 1 binder m-1 (weight x state).  Voxel v
-// is corner l of the beads whose lower-corner cell is v - (l & 1, l >> 1 & 1,
-// l >> 2 & 1), wrapped.  Those <= 8 sorted buckets are merged in ascending bead
-// index, and the corners of one bead that land on v (several only on grids one or
-// two voxels wide, where buckets coincide) are folded in corner order: the
-// reference's bead loop.  Every per-bucket value is indexed at compile time, so
-// the merge state stays in registers.  Which thread merges which voxel of the
-// block does not change any voxel's sum.
-template <int T, bool RANK>
-__global__ void __launch_bounds__(T)
-k_dens_gather(GridGeom G, int Bp1, const int32_t *off, const int32_t *cnt, const int32_t *list,
-              const BeadRec *brec, double *density, int cleanup)
-{
-    constexpr int32_t NONE = 0x7fffffff;
-    __shared__ int32_t hist[GATHER_KEYS], hoff[GATHER_KEYS], perm[T];
-    const int t = threadIdx.x;
-    const int64_t nbv = G.nx * G.ny * G.nz, base = (int64_t)blockIdx.x * T;
-    const int nreal = (int)(nbv - base < T ? nbv - base : T);
-    int32_t cell[8], pos[8], end[8], head[8];
-    int msk[8];
-    int64_t v = base + t;
-    if constexpr (RANK) {
-        if (t < GATHER_KEYS) hist[t] = 0;
-        __syncthreads();
-        int key = 0;
-        if (t < nreal) {
-            voxel_cells(G, base + t, cell, msk);
-            int64_t n = 0;
-#pragma unroll
-            for (int k = 0; k < 8; ++k) n += msk[k] ? cnt[cell[k]] : 0;
-            key = (int)(n < GATHER_KEYS - 1 ? n : GATHER_KEYS - 1);
-            atomicAdd(&hist[key], 1);
-        }
-        __syncthreads();
-        if (t < GATHER_KEYS) {
-            static_assert(GATHER_KEYS == 64, "one wavefront scans the key counts");
-            const int c = hist[t];
-            int incl = c;
-            for (int o = 1; o < GATHER_KEYS; o <<= 1) {
-                const int y = __shfl_up(incl, o);
-                if (t >= o) incl += y;
-            }
-            hoff[t] = incl - c;
-        }
-        __syncthreads();
-        if (t < nreal) perm[atomicAdd(&hoff[key], 1)] = t;
-        __syncthreads();
-        if (t < nreal) v = base + perm[t];
-    }
-    if (t >= nreal) return;
-    voxel_cells(G, v, cell, msk);
-    const double vvol = G.access_vol ? G.access_vol[v] : G.vol_bin;
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-        pos[k] = msk[k] ? off[cell[k]] : 0;
-        end[k] = msk[k] ? pos[k] + cnt[cell[k]] : 0;
-    }
-#pragma unroll
-    for (int k = 0; k < 8; ++k) head[k] = pos[k] < end[k] ? list[pos[k]] : NONE;
-    double acc[CHROMO_MAX_BINDERS + 1];
-#pragma unroll
-    for (int m = 0; m <= CHROMO_MAX_BINDERS; ++m) acc[m] = 0;
-    for (;;) {
-        // the smallest bead index at the buckets' heads; a bead lies in one bucket only
-        int32_t bb = NONE;
-        int bm = 0;
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            if (head[k] < bb) {
-                bb = head[k];
-                bm = msk[k];
-            }
-        }
-        if (bb == NONE) break;
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            if (head[k] == bb) {
-                ++pos[k];
-                head[k] = pos[k] < end[k] ? list[pos[k]] : NONE;
-            }
-        }
-        const BeadRec q = brec[bb];
-        const double wx = q.w[0], wy = q.w[1], wz = q.w[2];
-        double st[CHROMO_MAX_BINDERS];
-#pragma unroll
-        for (int m = 1; m <= CHROMO_MAX_BINDERS; ++m) st[m - 1] = m < Bp1 ? (double)q.st[m - 1] : 0.0;
-#pragma unroll
-        for (int l = 0; l < 8; ++l) {
-            if (!(bm >> l & 1)) continue;
-            const double d = corner_weight(l, wx, wy, wz) / vvol;
-            acc[0] += d;
-#pragma unroll
-            for (int m = 1; m <= CHROMO_MAX_BINDERS; ++m)
-                if (m < Bp1) acc[m] += d * st[m - 1];
-        }
-    }
-#pragma unroll
-    for (int m = 0; m <= CHROMO_MAX_BINDERS; ++m) {
-        if (m < Bp1) {
-            double a = acc[m];
-            if (cleanup && fabs(a) < 1E-18) a = 0;
-            density[v * Bp1 + m] = a;
-        }
-    }
-}
-
-// Scratch for one scatter: sized by the largest chain and grid.
-struct DensityScratch {
-    int32_t *cell = nullptr, *list = nullptr, *cnt = nullptr, *off = nullptr, *fill = nullptr;
-    int32_t *bsum = nullptr, *boff = nullptr, *bsum2 = nullptr;
-    BeadRec *brec = nullptr;
-    int64_t maxN = 0, maxBins = 0;
-};
-
 constexpr size_t SCRATCH_ALIGN = 256;
 
 inline size_t align_scratch(size_t o) { return (o + SCRATCH_ALIGN - 1) / SCRATCH_ALIGN * SCRATCH_ALIGN; }
 
-// The scatter's scratch carved from one buffer at base (nullptr: sizes only);
-// returns the bytes used, a multiple of SCRATCH_ALIGN.
-inline size_t density_scratch_carve(DensityScratch &S, char *base, int64_t maxN, int64_t maxBins)
+}  // namespace
+}  // namespace chromo
+
+#include "chromo_tiles.hpp"
+
+namespace chromo {
+namespace {
+
+// One scatter: a chain's beads into its density grid.
+struct ScatterJob {
+    GridGeom G;
+    TileGeom T;
+    int64_t N;
+    PosView P;
+    const int8_t *states;
+    double *density;                // n_bins x Bp1
+    int32_t *cell, *list;           // per bead; the tiles' bead lists
+    int32_t *cnt, *fill, *base;     // per tile
+    int32_t *cursor;
+    int32_t Bp1, cleanup;
+};
+
+// A job's scratch carved from base (nullptr: sizes only); returns the bytes used, a
+// multiple of SCRATCH_ALIGN.  cnt, fill and cursor lie in a row, the first of them.
+inline size_t scatter_carve(ScatterJob &J, char *base)
 {
     size_t o = 0;
-    auto take = [&](size_t bytes) {
-        char *p = base ? base + o : nullptr;
-        o = align_scratch(o + bytes);
+    auto take = [&](size_t n) {
+        int32_t *p = base ? (int32_t *)(base + o) : nullptr;
+        o = align_scratch(o + sizeof(int32_t) * n);
         return p;
     };
-    S.maxN = maxN;
-    S.maxBins = maxBins;
-    S.cell = (int32_t *)take(sizeof(int32_t) * maxN);
-    S.list = (int32_t *)take(sizeof(int32_t) * maxN);
-    S.brec = (BeadRec *)take(sizeof(BeadRec) * maxN);
-    S.cnt = (int32_t *)take(sizeof(int32_t) * maxBins);
-    S.off = (int32_t *)take(sizeof(int32_t) * maxBins);
-    S.fill = (int32_t *)take(sizeof(int32_t) * maxBins);
-    S.bsum = (int32_t *)take(sizeof(int32_t) * 2048);
-    S.boff = (int32_t *)take(sizeof(int32_t) * 2048);
-    S.bsum2 = (int32_t *)take(sizeof(int32_t) * 2);
+    J.cnt = take((size_t)J.T.ntiles);
+    J.fill = take((size_t)J.T.ntiles);
+    J.cursor = take(1);
+    J.base = take((size_t)J.T.ntiles);
+    J.cell = take((size_t)J.N);
+    J.list = take((size_t)J.N * tile_images(J.T));
     return o;
 }
 
-inline hipError_t density_scratch_alloc(DensityScratch &S, int64_t maxN, int64_t maxBins,
-                                        hipStream_t st)
+inline ScatterJob scatter_job(const GridGeom &G, int64_t N, int Bp1, PosView P, const int8_t *states, double *density,
+                              int cleanup)
 {
-    hipError_t e;
-    S.maxN = maxN;
-    S.maxBins = maxBins;
-#define CHROMO_ALLOC(ptr, bytes) \
-    if ((e = hipMallocAsync((void **)&ptr, bytes, st)) != hipSuccess) return e
-    CHROMO_ALLOC(S.cell, sizeof(int32_t) * maxN);
-    CHROMO_ALLOC(S.list, sizeof(int32_t) * maxN);
-    CHROMO_ALLOC(S.brec, sizeof(BeadRec) * maxN);
-    CHROMO_ALLOC(S.cnt, sizeof(int32_t) * maxBins);
-    CHROMO_ALLOC(S.off, sizeof(int32_t) * maxBins);
-    CHROMO_ALLOC(S.fill, sizeof(int32_t) * maxBins);
-    CHROMO_ALLOC(S.bsum, sizeof(int32_t) * 2048);
-    CHROMO_ALLOC(S.boff, sizeof(int32_t) * 2048);
-    CHROMO_ALLOC(S.bsum2, sizeof(int32_t) * 2);
-#undef CHROMO_ALLOC
-    return hipSuccess;
+    ScatterJob J{};
+    J.G = G;
+    J.T = fold_geom(G);
+    J.N = N;
+    J.P = P;
+    J.states = states;
+    J.density = density;
+    J.Bp1 = Bp1;
+    J.cleanup = cleanup;
+    return J;
 }
 
-inline void density_scratch_free(DensityScratch &S, hipStream_t st)
+// The kernels take job blockIdx.y of a table in device memory, or (TABLE false) the one
+// in `one`: both are read with scalar loads.
+template <bool TABLE>
+__global__ void k_scatter_clear(const ScatterJob *__restrict__ jobs, const ScatterJob one)
 {
-    int32_t *ip[] = {S.cell, S.list, S.cnt, S.off, S.fill, S.bsum, S.boff, S.bsum2};
-    for (auto p : ip)
-        if (p) (void)hipFreeAsync(p, st);
-    if (S.brec) (void)hipFreeAsync(S.brec, st);
-    S = DensityScratch();
+    const ScatterJob &J = TABLE ? jobs[blockIdx.y] : one;
+    const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    if (i < J.T.ntiles) J.cnt[i] = J.fill[i] = 0;
+    if (i == 0) *J.cursor = 0;
 }
 
-// Clears two int32 arrays of n elements.
-__global__ void k_fill2_i32(int32_t *p, int32_t *q, int64_t n)
+template <bool TABLE>
+__global__ void k_scatter_base(const ScatterJob *__restrict__ jobs, const ScatterJob one)
 {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) {
-        p[i] = 0;
-        q[i] = 0;
+    const ScatterJob &J = TABLE ? jobs[blockIdx.y] : one;
+    if ((int)(blockIdx.x * blockDim.x) >= J.T.ntiles) return;
+    tile_bases(J.cnt, J.base, J.cursor, J.T.ntiles);
+}
+
+template <bool TABLE, bool PLACE>
+__global__ void __launch_bounds__(BIN_THREADS) k_scatter_bin(const ScatterJob *__restrict__ jobs, const ScatterJob one)
+{
+    const ScatterJob &J = TABLE ? jobs[blockIdx.y] : one;
+    if ((int64_t)blockIdx.x * BIN_THREADS >= J.N) return;
+    tile_bin<PLACE, false, true>(J.G, J.T, J.N, J.P, J.cell, PLACE ? J.fill : J.cnt, J.base, J.list);
+}
+
+// Ascending sort of a[0 .. n) in global memory by one wavefront: a bitonic network whose
+// comparators all point the same way (each merge starts with a mirrored step), so that
+// the places past n, which would hold the largest keys, need not exist.
+__device__ __forceinline__ void wave_sort(int32_t *a, int n)
+{
+    const uint32_t lane = (uint32_t)lane_id(), un = (uint32_t)n;
+    for (int kb = 1; kb <= 31 && (1u << (kb - 1)) < un; ++kb) {
+        for (int db = kb - 1; db >= 0; --db) {
+            // pair t: groups of 2^db pairs over 2^(db + 1) places
+            for (uint32_t t = lane; ((t >> db) << (db + 1)) < un; t += WAVE) {
+                const uint32_t g = (t >> db) << (db + 1), o = t & ((1u << db) - 1);
+                const uint32_t i = g + o, j = db == kb - 1 ? g + (2u << db) - 1 - o : i + (1u << db);
+                if (j < un) {
+                    const int32_t x = a[i], y = a[j];
+                    if (x > y) {
+                        a[i] = y;
+                        a[j] = x;
+                    }
+                }
+            }
+            wave_sync_global();
+        }
     }
 }
 
-// Scatter N beads into density (n_bins x Bp1) by the reference's bead-order fold.
-// Requires N <= S.maxN, n_bins <= S.maxBins <= 2048 * 2048.  cleanup: the 1e-18 rule of
-// the initial densities.
-inline hipError_t density_scatter(const GridGeom &G, int64_t N, int Bp1, PosView P,
-                                  const int8_t *states, double *density, int cleanup,
-                                  DensityScratch &S, hipStream_t st)
+// A tile's list in bead order, without sorting it: the placement leaves it as runs in
+// bead order (what one block placed), so only the runs are ordered, by their first bead.
+// Run k of that order starts at list place from[k] and at position off[k] of the order;
+// off[runs] = len.  When there are more than RUNS_MAX runs, or runs that overlap (entries
+// a block had to place one by one), the list itself is sorted and is one run.  One
+// wavefront; returns the number of runs.
+constexpr int RUNS_MAX = 128;
+
+__device__ __forceinline__ int list_runs(int32_t *list, int len, int32_t *from, int32_t *off, int32_t *key)
 {
-    const int64_t nb = G.nx * G.ny * G.nz;
-    hipError_t e;
-    unsigned gb = (unsigned)((N + 255) / 256);
-    unsigned gv = (unsigned)((nb + 255) / 256);
-    // cleared by a kernel rather than hipMemsetAsync: a caller may capture this
-    // sequence in a HIP graph
-    hipLaunchKernelGGL(k_fill2_i32, dim3(gv), dim3(256), 0, st, S.cnt, S.fill, nb);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-    hipLaunchKernelGGL(k_dens_cells, dim3(gb), dim3(256), 0, st, G, N, P, Bp1 - 1, states, S.cell, S.brec,
-                       S.cnt);
-    int64_t nbl = (nb + 2047) / 2048;
-    hipLaunchKernelGGL(k_scan_blocks, dim3((unsigned)nbl), dim3(1024), 0, st, S.cnt, S.off, S.bsum, nb);
-    hipLaunchKernelGGL(k_scan_blocks, dim3(1), dim3(1024), 0, st, S.bsum, S.boff, S.bsum2, nbl);
-    hipLaunchKernelGGL(k_scan_add, dim3(gv), dim3(256), 0, st, S.off, S.boff, nb);
-    hipLaunchKernelGGL(k_dens_place, dim3(gb), dim3(256), 0, st, N, S.cell, S.off, S.fill, S.list);
-    hipLaunchKernelGGL(k_dens_sort, dim3(gv), dim3(256), 0, st, nb, S.off, S.cnt, S.list);
-    if (nb >= (int64_t)1024 * GATHER_BIG_BLOCKS)
-        hipLaunchKernelGGL((k_dens_gather<1024, true>), dim3((unsigned)((nb + 1023) / 1024)), dim3(1024), 0, st, G, Bp1,
-                           S.off, S.cnt, S.list, S.brec, density, cleanup);
-    else
-        hipLaunchKernelGGL((k_dens_gather<256, false>), dim3(gv), dim3(256), 0, st, G, Bp1, S.off, S.cnt, S.list, S.brec,
-                           density, cleanup);
+    const int lane = lane_id();
+    int runs = 0;
+    for (int i0 = 0; i0 < len && runs <= RUNS_MAX; i0 += WAVE) {
+        const int i = i0 + lane;
+        const int x = i < len ? list[i] : 0, y = i > 0 && i < len ? list[i - 1] : 0;
+        const bool head = i < len && (i == 0 || x < y || (x ^ y) >> 8 != 0);
+        static_assert(BIN_THREADS == 256, "a run's beads share their upper bits");
+        int cnt;
+        const int k = runs + wave_excl_count(head, cnt);
+        if (head && k < RUNS_MAX) {
+            from[k] = i;
+            key[k] = x;
+        }
+        runs += cnt;
+    }
+    wave_sync();
+    bool bad = runs > RUNS_MAX;
+    if (!bad) {
+        // ranks by counting; a run's length from the next run's start
+        int lens[RUNS_MAX / WAVE], rank[RUNS_MAX / WAVE], keep[RUNS_MAX / WAVE];
+#pragma unroll
+        for (int q = 0; q < RUNS_MAX / WAVE; ++q) {
+            lens[q] = rank[q] = keep[q] = 0;
+            const int k = q * WAVE + lane;
+            if (q * WAVE >= runs) continue;
+            if (k < runs) {
+                const int mine = key[k], end = k + 1 < runs ? from[k + 1] : len;
+                keep[q] = from[k];
+                lens[q] = end - keep[q];
+                for (int j = 0; j < runs; ++j) rank[q] += key[j] < mine;
+                // no other run starts between this one's first and last bead
+                const int last = list[end - 1];
+                for (int j = 0; j < runs; ++j) bad = bad || (key[j] > mine && key[j] <= last);
+            }
+        }
+        bad = wave_any(bad);
+        wave_sync();
+        if (!bad) {
+#pragma unroll
+            for (int q = 0; q < RUNS_MAX / WAVE; ++q) {
+                const int k = q * WAVE + lane;
+                if (q * WAVE < runs && k < runs) {
+                    from[rank[q]] = keep[q];
+                    off[rank[q]] = lens[q];
+                }
+            }
+            wave_sync();
+            int at = 0;
+            for (int k0 = 0; k0 < runs; k0 += WAVE) {
+                const int k = k0 + lane, n = k < runs ? off[k] : 0;
+                int tot;
+                const int o = wave_excl_scan(n, tot);
+                if (k < runs) off[k] = at + o;
+                at += tot;
+            }
+            if (lane == 0) off[runs] = len;
+            wave_sync();
+            return runs;
+        }
+    }
+    wave_sort(list, len);
+    if (lane == 0) {
+        from[0] = 0;
+        off[0] = 0;
+        off[1] = len;
+    }
+    wave_sync();
+    return 1;
+}
+
+// The density of one tile's voxels: the reference's bead-order fold
+// (fields.pyx:2063-2106) by one wavefront.  The tile's beads go through 64 at a time in
+// bead order, each lane working out its bead's weights / volume and voxel places; then
+// one LDS floating-point add per bead, its lanes the corners times the species, issued
+// in bead order: the LDS executes a wavefront's operations in order, so each voxel's sum
+// is the reference's left fold bit for bit.  (On a grid with a one-voxel axis corners of
+// a bead share a voxel and are issued one after the other.)
+// What bounds it: each wavefront's chain of loads and LDS round trips (27,000 cycles for
+// a tile of 60 listed beads) at three to four wavefronts per SIMD.  10^6 beads, B = 4,
+// 128^3: 171 us, of 262 us a scatter; the merge of eight sorted buckets per voxel it
+// replaces took 311 us, of 700.  With 8 x 8 x 4 tiles the longest list decides (241 us).
+template <bool TABLE, int NB>
+__global__ void __launch_bounds__(WAVE) k_scatter_fold(const ScatterJob *__restrict__ jobs, const ScatterJob one)
+{
+    constexpr int Bp1 = NB + 1, LP = 8 * Bp1, PB = WAVE / LP, UN = PB == 1 ? 8 : 4;
+    constexpr int VOX = FOLD_MAX[0] * FOLD_MAX[1] * FOLD_MAX[2];
+    // the sums of the tile's voxels, then a row per corner that nobody reads for corners
+    // outside the tile (one row for all would make their adds wait for each other)
+    __shared__ double sum[(VOX + 8) * Bp1], c0[8 * WAVE];
+    __shared__ uint16_t vox[8 * WAVE];      // byte offset of a corner's sums
+    __shared__ uint8_t fac[8 * WAVE];       // factor m of bead p at 8 p + m: 1, then the binder states
+    __shared__ int32_t from[RUNS_MAX], off[RUNS_MAX + 1];
+    static_assert(sizeof(c0) >= sizeof(int32_t) * RUNS_MAX, "the runs' keys use c0 before its first use");
+    constexpr uint32_t ROW = sizeof(double) * Bp1;
+    static_assert((VOX + 8) * ROW < 65536, "byte offsets fit 16 bits");
+    const ScatterJob &J = TABLE ? jobs[blockIdx.y] : one;
+    const int tile = (int)blockIdx.x;
+    if (tile >= J.T.ntiles || J.Bp1 != Bp1) return;
+    const TileGeom &T = J.T;
+    const int lane = lane_id();
+    const int tt[3] = {tile % T.nt[0], (tile / T.nt[0]) % T.nt[1], tile / (T.nt[0] * T.nt[1])};
+    int start[3], size[3];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        start[j] = tile_start(T.n[j], T.nt[j], tt[j]);
+        size[j] = tile_start(T.n[j], T.nt[j], tt[j] + 1) - start[j];
+    }
+    const bool degen = T.n[0] == 1 || T.n[1] == 1 || T.n[2] == 1;
+    const int stride[3] = {1, FOLD_MAX[0], FOLD_MAX[0] * FOLD_MAX[1]};
+    for (int i = lane; i < VOX * Bp1; i += WAVE) sum[i] = 0;
+    const int len = J.cnt[tile];
+    int32_t *list = J.list + J.base[tile];
+    const int runs = len > 0 ? list_runs(list, len, from, off, (int32_t *)c0) : 0;
+    const bool in = lane < PB * LP;
+    const int pj = in ? lane / LP : 0, m = in ? (lane % LP) >> 3 : 0, l8 = lane & 7;
+    char *acc = (char *)(sum + m);
+    const double *avol = J.G.access_vol;
+    for (int i0 = 0; i0 < len; i0 += WAVE) {
+        const int n = len - i0 < WAVE ? len - i0 : WAVE;
+        if (lane < n) {
+            // the run that holds position i0 + lane of the order
+            int lo = 0, hi = runs;
+            while (hi - lo > 1) {
+                const int mid = (lo + hi) >> 1;
+                if (off[mid] <= i0 + lane) lo = mid;
+                else hi = mid;
+            }
+            const int64_t b = list[from[lo] + (i0 + lane - off[lo])];
+            double x[3], w[3];
+            int ix[3];
+#pragma unroll
+            for (int j = 0; j < 3; ++j) x[j] = J.P.p[j * J.P.sc + b * J.P.sb];
+            uint64_t st = 1;
+#pragma unroll
+            for (int j = 0; j < NB; ++j) st |= (uint64_t)(uint8_t)J.states[(int64_t)j * J.N + b] << (8 * (j + 1));
+            tile_lower(J.G, T, x, ix, w);
+            int at[3][2], ax[3][2];     // place of the lower and upper corner in the tile (-1: outside), on the grid
+#pragma unroll
+            for (int j = 0; j < 3; ++j) {
+                ax[j][0] = ix[j];
+                ax[j][1] = ix[j] + 1 == T.n[j] ? 0 : ix[j] + 1;
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    const int d = ax[j][e] - start[j];
+                    at[j][e] = d >= 0 && d < size[j] ? d * stride[j] : -1;
+                }
+            }
+            const double u[3] = {1 - w[0], 1 - w[1], 1 - w[2]};
+            const double xy[4] = {w[0] * w[1], u[0] * w[1], w[0] * u[1], u[0] * u[1]};
+            uint32_t q[8];
+#pragma unroll
+            for (int l = 0; l < 8; ++l) {
+                const int vx = at[0][l & 1], vy = at[1][(l >> 1) & 1], vz = at[2][l >> 2];
+                q[l] = ((vx | vy | vz) < 0 ? (uint32_t)(VOX + l) : (uint32_t)(vx + vy + vz)) * ROW;
+                const double c = xy[l & 3] * ((l & 4) ? u[2] : w[2]);
+                double d;
+                if (avol)
+                    d = c / avol[(int64_t)ax[0][l & 1] +
+                                 (int64_t)T.n[0] * (ax[1][(l >> 1) & 1] + (int64_t)T.n[1] * ax[2][l >> 2])];
+                else
+                    d = T.recip ? div_by(c, J.G.vol_bin, T.rvol) : c / J.G.vol_bin;
+                c0[8 * lane + l] = d;
+            }
+            *(uint4 *)&vox[8 * lane] = make_uint4(q[0] | q[1] << 16, q[2] | q[3] << 16, q[4] | q[5] << 16,
+                                                  q[6] | q[7] << 16);
+            *(uint64_t *)&fac[8 * lane] = st;
+        } else {
+            // the steps below run over whole groups: rows past the last bead add nothing
+#pragma unroll
+            for (int l = 0; l < 8; ++l) vox[8 * lane + l] = (uint16_t)((VOX + l) * ROW);
+#pragma unroll
+            for (int l = 0; l < 8; ++l) c0[8 * lane + l] = 0;
+            *(uint64_t *)&fac[8 * lane] = 0;
+        }
+        wave_sync();
+        for (int p0 = 0; p0 < n; p0 += PB * UN) {
+            static_assert(WAVE % (PB * UN) == 0, "whole steps");
+            double t[UN];
+            char *to[UN];
+#pragma unroll
+            for (int k = 0; k < UN; ++k) {
+                const int p = p0 + k * PB + pj;
+                t[k] = c0[8 * p + l8] * (double)(int8_t)fac[8 * p + m];
+                to[k] = acc + vox[8 * p + l8];
+            }
+            if (!degen) {
+#pragma unroll
+                for (int k = 0; k < UN; ++k) {
+#pragma unroll
+                    for (int j = 0; j < PB; ++j) {
+                        if (in && pj == j) lds_add((double *)to[k], t[k]);
+                        __builtin_amdgcn_wave_barrier();
+                    }
+                }
+            } else {
+#pragma unroll
+                for (int k = 0; k < UN; ++k)
+                    for (int s = 0; s < 8 * PB; ++s) {
+                        if (in && pj == (s >> 3) && l8 == (s & 7)) lds_add((double *)to[k], t[k]);
+                        __builtin_amdgcn_wave_barrier();
+                    }
+            }
+        }
+        wave_sync();
+    }
+    wave_sync();
+    for (int i = lane; i < VOX * Bp1; i += WAVE) {
+        const int v = i / Bp1, s = i % Bp1;
+        const int x = v % FOLD_MAX[0], y = (v / FOLD_MAX[0]) % FOLD_MAX[1], z = v / (FOLD_MAX[0] * FOLD_MAX[1]);
+        if (x >= size[0] || y >= size[1] || z >= size[2]) continue;
+        const int64_t gv = (start[0] + x) + (int64_t)T.n[0] * ((start[1] + y) + (int64_t)T.n[1] * (start[2] + z));
+        double a = sum[i];
+        if (J.cleanup && fabs(a) < 1E-18) a = 0;
+        J.density[gv * Bp1 + s] = a;
+    }
+}
+
+// Largest sizes among the jobs of one launch, and the binder counts present (bit B).
+struct ScatterSpan {
+    int64_t N = 0;
+    int32_t ntiles = 0;
+    int binders = 0;
+    void add(const ScatterJob &J)
+    {
+        N = J.N > N ? J.N : N;
+        ntiles = J.T.ntiles > ntiles ? J.T.ntiles : ntiles;
+        binders |= 1 << (J.Bp1 - 1);
+    }
+};
+
+template <bool TABLE>
+hipError_t scatter_launch(const ScatterJob *jobs, const ScatterJob &one, int njobs, const ScatterSpan &X, hipStream_t st)
+{
+    const unsigned y = (unsigned)njobs;
+    const dim3 gt((unsigned)((X.ntiles + 255) / 256), y), gb((unsigned)((X.N + BIN_THREADS - 1) / BIN_THREADS), y);
+    const dim3 gf((unsigned)X.ntiles, y), bin(BIN_THREADS), wave(WAVE);
+    hipLaunchKernelGGL((k_scatter_clear<TABLE>), gt, dim3(256), 0, st, jobs, one);
+    hipLaunchKernelGGL((k_scatter_bin<TABLE, false>), gb, bin, 0, st, jobs, one);
+    hipLaunchKernelGGL((k_scatter_base<TABLE>), gt, dim3(256), 0, st, jobs, one);
+    hipLaunchKernelGGL((k_scatter_bin<TABLE, true>), gb, bin, 0, st, jobs, one);
+    if (X.binders & 1) hipLaunchKernelGGL((k_scatter_fold<TABLE, 0>), gf, wave, 0, st, jobs, one);
+    if (X.binders & 2) hipLaunchKernelGGL((k_scatter_fold<TABLE, 1>), gf, wave, 0, st, jobs, one);
+    if (X.binders & 4) hipLaunchKernelGGL((k_scatter_fold<TABLE, 2>), gf, wave, 0, st, jobs, one);
+    if (X.binders & 8) hipLaunchKernelGGL((k_scatter_fold<TABLE, 3>), gf, wave, 0, st, jobs, one);
+    if (X.binders & 16) hipLaunchKernelGGL((k_scatter_fold<TABLE, 4>), gf, wave, 0, st, jobs, one);
     return hipGetLastError();
+}
+
+// Runs the jobs (a table of njobs in device memory, or jobs == nullptr and `one`),
+// their scratch carved: five launches and one per further binder count.  Cleared by a
+// kernel rather than hipMemsetAsync: a caller may capture this sequence in a HIP graph.
+inline hipError_t scatter_run(const ScatterJob *jobs, const ScatterJob &one, int njobs, const ScatterSpan &X,
+                              hipStream_t st)
+{
+    return jobs ? scatter_launch<true>(jobs, one, njobs, X, st) : scatter_launch<false>(nullptr, one, 1, X, st);
 }
 
 }  // namespace

@@ -257,6 +257,13 @@ __device__ __forceinline__ int wave_excl_scan(int x, int &total)
     return v - x;
 }
 
+// *p += v for the active lanes, in LDS, rounded as a double add; the LDS executes a
+// wavefront's operations in issue order.
+__device__ __forceinline__ void lds_add(double *p, double v)
+{
+    (void)__builtin_amdgcn_ds_atomic_fadd_f64((double __attribute__((address_space(3))) *)p, v);
+}
+
 // ---------------------------------------------------------------------------
 // Random streams (wave-uniform)
 // ---------------------------------------------------------------------------

@@ -31,7 +31,6 @@
 
 #include "chromo_density.hpp"
 #include "chromo_device.hpp"
-#include "chromo_tiles.hpp"
 
 using namespace chromo;
 
@@ -717,18 +716,20 @@ int make_adjoint_model(const chromo_energy_model *m, const double *d_r, const do
 // Device buffers of one evaluation of the reference energies, carved from one
 // allocation.
 struct EnergyBufs {
-    DensityScratch S;
-    double *rho = nullptr, *vpart = nullptr, *bpart = nullptr;
+    ScatterJob J;
+    double *vpart = nullptr, *bpart = nullptr;
     int gv = 0, gb = 0;
 };
 
 // Carves the buffers of an evaluation of M from base (nullptr: sizes only) and
-// returns the bytes used.  rho_given: the density goes to the caller's array.
-size_t energy_carve(const EModel &M, bool rho_given, char *base, EnergyBufs &Bf)
+// returns the bytes used.  rho: the caller's density array, or nullptr: one of its own.
+size_t energy_carve(const EModel &M, const PosView &P, double *rho, char *base, EnergyBufs &Bf)
 {
     const int64_t nb = M.G.nx * M.G.ny * M.G.nz;
     const int Bp1 = M.B + 1;
-    size_t o = density_scratch_carve(Bf.S, base, M.N, nb);
+    // UniformDensityField.update_all_densities: no 1e-18 clean-up
+    Bf.J = scatter_job(M.G, M.N, Bp1, P, M.states, rho, 0);
+    size_t o = scatter_carve(Bf.J, base);
     auto take = [&](size_t bytes) {
         double *p = base ? (double *)(base + o) : nullptr;
         o = align_scratch(o + bytes);
@@ -736,7 +737,7 @@ size_t energy_carve(const EModel &M, bool rho_given, char *base, EnergyBufs &Bf)
     };
     Bf.gv = grid_blocks(nb);
     Bf.gb = grid_blocks(M.N);
-    Bf.rho = rho_given ? nullptr : take(sizeof(double) * nb * Bp1);
+    if (!rho) Bf.J.density = take(sizeof(double) * nb * Bp1);
     Bf.vpart = take(sizeof(double) * MAXT * Bf.gv);
     Bf.bpart = take(sizeof(double) * MAXT * Bf.gb);
     return o;
@@ -799,14 +800,15 @@ void launch_adjoint(const EModel &M, const TileGeom &T, const double *r, const d
 int energy_adjoint_run(const EModel &M, const TileGeom &T, const double *d_r, const double *d_theta, double *d_E,
                        double *d_grad_r, double *d_grad_theta, const AdjointBufs &Bf, hipStream_t st)
 {
+    const PosView P{d_r, 1, 3};
     const unsigned gb = (unsigned)((M.N + BIN_THREADS - 1) / BIN_THREADS), gt = (unsigned)((T.ntiles + 255) / 256);
     // cleared by a kernel rather than hipMemsetAsync: a caller may capture this
     // sequence in a HIP graph
     hipLaunchKernelGGL(k_tile_clear, dim3(gt), dim3(256), 0, st, Bf.cnt, Bf.fill, Bf.cursor, T.ntiles);
-    hipLaunchKernelGGL(k_tile_bin<false>, dim3(gb), dim3(BIN_THREADS), 0, st, M.G, T, M.N, d_r, Bf.cell, Bf.cnt,
+    hipLaunchKernelGGL(k_tile_bin<false>, dim3(gb), dim3(BIN_THREADS), 0, st, M.G, T, M.N, P, Bf.cell, Bf.cnt,
                        (const int32_t *)nullptr, (int32_t *)nullptr);
     hipLaunchKernelGGL(k_tile_base, dim3(gt), dim3(256), 0, st, Bf.cnt, Bf.base, Bf.cursor, T.ntiles);
-    hipLaunchKernelGGL(k_tile_bin<true>, dim3(gb), dim3(BIN_THREADS), 0, st, M.G, T, M.N, d_r, Bf.cell, Bf.fill, Bf.base,
+    hipLaunchKernelGGL(k_tile_bin<true>, dim3(gb), dim3(BIN_THREADS), 0, st, M.G, T, M.N, P, Bf.cell, Bf.fill, Bf.base,
                        Bf.list);
     switch (M.B) {
     case 1: launch_adjoint<1>(M, T, d_r, d_theta, d_E, d_grad_r, d_grad_theta, Bf, st); break;
@@ -872,7 +874,7 @@ int chromo_energy_adjoint(const chromo_energy_model *model, const double *d_r, c
     int rc = make_adjoint_model(model, d_r, d_theta, d_E, M);
     if (rc) return rc;
     hipStream_t st = (hipStream_t)stream;
-    const TileGeom T = tile_geom(M.G, M.bead_vol);
+    const TileGeom T = tile_geom(M.G, TILE_MAX, M.bead_vol);
     AdjointBufs Bf;
     StreamBuffer buf;
     buf.st = st;
@@ -887,7 +889,7 @@ int64_t chromo_energy_adjoint_bytes(const chromo_energy_model *model)
     const int rc = make_model(model, M);
     if (rc) return rc;
     AdjointBufs Bf;
-    return (int64_t)adjoint_carve(M, tile_geom(M.G, M.bead_vol), nullptr, Bf);
+    return (int64_t)adjoint_carve(M, tile_geom(M.G, TILE_MAX, M.bead_vol), nullptr, Bf);
 }
 
 int chromo_energy_adjoint_ws(const chromo_energy_model *model, const double *d_r, const double *d_theta,
@@ -897,7 +899,7 @@ int chromo_energy_adjoint_ws(const chromo_energy_model *model, const double *d_r
     EModel M;
     int rc = make_adjoint_model(model, d_r, d_theta, d_E, M);
     if (rc) return rc;
-    const TileGeom T = tile_geom(M.G, M.bead_vol);
+    const TileGeom T = tile_geom(M.G, TILE_MAX, M.bead_vol);
     AdjointBufs Bf;
     const size_t bytes = adjoint_carve(M, T, nullptr, Bf);
     if (!d_ws || ws_bytes < 0 || (size_t)ws_bytes < bytes)
@@ -913,7 +915,7 @@ int chromo_energy_adjoint_noalloc(const chromo_energy_model *model, const double
     EModel M;
     int rc = make_adjoint_model(model, d_r, d_theta, d_E, M);
     if (rc) return rc;
-    const TileGeom T = tile_geom(M.G, M.bead_vol);
+    const TileGeom T = tile_geom(M.G, TILE_MAX, M.bead_vol);
     AdjointBufs Bf;
     const size_t doc = noalloc_bytes(M, d_grad_r != nullptr), own = adjoint_carve(M, T, nullptr, Bf);
     const size_t bytes = doc > own ? doc : own;
@@ -936,19 +938,19 @@ int chromo_energy_reference(const chromo_energy_model *model, const double *d_po
     if (rc) return rc;
     if (!d_pos || !d_pref || !d_intra || !d_out) return eset(-1, "NULL argument");
     hipStream_t st = (hipStream_t)stream;
-    const int B = M.B, Bp1 = B + 1;
+    const int B = M.B;
+    const int64_t sc = soa ? M.N : 1, sbd = soa ? 1 : 9;
+    const PosView P{d_pos, sc, sbd};
     EnergyBufs Bf;
-    const size_t bytes = energy_carve(M, d_density_out != nullptr, nullptr, Bf);
     StreamBuffer buf;
     buf.st = st;
-    HIPE(hipMallocAsync((void **)&buf.p, bytes, st));
-    energy_carve(M, d_density_out != nullptr, buf.p, Bf);
-    double *rho = d_density_out ? d_density_out : Bf.rho;
+    HIPE(hipMallocAsync((void **)&buf.p, energy_carve(M, P, d_density_out, nullptr, Bf), st));
+    energy_carve(M, P, d_density_out, buf.p, Bf);
+    const double *rho = Bf.J.density;
     const int gv = Bf.gv, gb = Bf.gb;
-    // UniformDensityField.update_all_densities: bead-order scatter without the 1e-18 clean-up
-    const int64_t sc = soa ? M.N : 1, sbd = soa ? 1 : 9;
-    PosView P{d_pos, sc, sbd};
-    hipError_t e = density_scatter(M.G, M.N, Bp1, P, M.states, rho, 0, Bf.S, st);
+    ScatterSpan X;
+    X.add(Bf.J);
+    hipError_t e = scatter_run(nullptr, Bf.J, 1, X, st);
     if (e != hipSuccess) return eset(-2, std::string("density scatter: ") + hipGetErrorString(e));
     hipLaunchKernelGGL(k_ref_voxel, dim3(gv), dim3(EB), 0, st, M, d_pref, chi, rho, Bf.vpart, B + 1);
     hipLaunchKernelGGL(k_ref_bead, dim3(gb), dim3(EB), 0, st, M, d_pos, sc, sbd, Bf.bpart, B + 1);

@@ -384,13 +384,6 @@ __device__ __forceinline__ double bond_E(const Bond &bd, const double *r0, const
     return E_pair(bd, be, par, drp);
 }
 
-// *p += v for the active lanes, in LDS, rounded as a double add; the LDS executes a
-// wavefront's operations in issue order.
-__device__ __forceinline__ void lds_add(double *p, double v)
-{
-    (void)__builtin_amdgcn_ds_atomic_fadd_f64((double __attribute__((address_space(3))) *)p, v);
-}
-
 // The fold of one chunk's npos positions into S.acc (fields.pyx:1491-1520): lanes
 // 8 m + l of a position's group hold species m of corner l; PB positions share the
 // arithmetic of one step, and their adds are issued one position after the other.

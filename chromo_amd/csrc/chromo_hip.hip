@@ -505,6 +505,81 @@ int read_table(const chromo_replica *d_reps, int32_t n_reps, hipStream_t st, std
     return 0;
 }
 
+// ---- density initialisation ------------------------------------------------------
+
+// The scatters of the replicas that have a field (chromo_density.hpp).
+int density_jobs(const chromo_replica *h, int32_t n_reps, std::vector<ScatterJob> &jobs)
+{
+    for (int32_t i = 0; i < n_reps; ++i) {
+        const chromo_replica &r = h[i];
+        if (r.field_on == 0) continue;
+        if (r.B < 0 || r.B > CHROMO_MAX_BINDERS) return set_err(-1, "B out of range");
+        if (r.nx * r.ny * r.nz > 2048LL * 2048LL || r.N > 0x7fffffff)
+            return set_err(-1, "grid or chain too large for the density scatter");
+        if (r.nx < 1 || r.ny < 1 || r.nz < 1) return set_err(-1, "a grid axis without voxels");
+        jobs.push_back(scatter_job(grid_of(r), r.N, r.B + 1, PosView{r.pos, r.N, 1}, r.states, r.density, 1));
+    }
+    return 0;
+}
+
+// Jobs run together while their scratch stays below this (a single larger one alone),
+// at most 65535 (grid rows) at a time: a run's scratch is bounded by its largest job or
+// this, not by the number of replicas.
+constexpr size_t DENSITY_GROUP_BYTES = size_t(1) << 30;
+constexpr size_t DENSITY_GROUP_JOBS = 4096;
+
+// The group of jobs from i on: its end, and the bytes of its scratch.
+size_t density_group(std::vector<ScatterJob> &jobs, size_t i, size_t &bytes)
+{
+    bytes = 0;
+    size_t k = i;
+    for (; k < jobs.size() && k - i < DENSITY_GROUP_JOBS; ++k) {
+        const size_t b = scatter_carve(jobs[k], nullptr);
+        if (k > i && bytes + b > DENSITY_GROUP_BYTES) break;
+        bytes += b;
+    }
+    return k;
+}
+
+// The workspace of density_run: the largest group's scratch and the table of all jobs.
+size_t density_bytes(std::vector<ScatterJob> &jobs)
+{
+    size_t most = 0, b = 0;
+    for (size_t i = 0; i < jobs.size();) {
+        i = density_group(jobs, i, b);
+        most = b > most ? b : most;
+    }
+    return align_scratch(sizeof(ScatterJob) * jobs.size()) + most;
+}
+
+int density_run(std::vector<ScatterJob> &jobs, char *ws, hipStream_t st)
+{
+    ScatterJob *table = (ScatterJob *)ws;
+    char *scratch = ws + align_scratch(sizeof(ScatterJob) * jobs.size());
+    for (size_t i = 0, end = 0, b = 0; i < jobs.size(); i = end) {
+        end = density_group(jobs, i, b);
+        size_t o = 0;
+        for (size_t k = i; k < end; ++k) o += scatter_carve(jobs[k], scratch + o);
+    }
+    // one job travels as a kernel argument; a table is copied, and waited for, since it
+    // leaves with this call
+    if (jobs.size() > 1) {
+        HIPC(hipMemcpyAsync(table, jobs.data(), sizeof(ScatterJob) * jobs.size(), hipMemcpyHostToDevice, st));
+        HIPC(hipStreamSynchronize(st));
+    }
+    for (size_t i = 0, end = 0, b = 0; i < jobs.size(); i = end) {
+        end = density_group(jobs, i, b);
+        size_t o = 0;
+        ScatterSpan X;
+        for (size_t k = i; k < end; ++k) {
+            o += scatter_carve(jobs[k], scratch + o);
+            X.add(jobs[k]);
+        }
+        HIPC(scatter_run(jobs.size() > 1 ? table + i : nullptr, jobs[i], (int)(end - i), X, st));
+    }
+    return 0;
+}
+
 }  // namespace
 
 extern "C" {
@@ -564,37 +639,42 @@ int chromo_np_seed(const chromo_replica *d_reps, int32_t n_reps, const uint32_t 
 
 int chromo_density_init(const chromo_replica *d_reps, int32_t n_reps, void *stream)
 {
-    int rc = check_reps(d_reps, n_reps);
+    std::vector<chromo_replica> h;
+    int rc = read_table(d_reps, n_reps, (hipStream_t)stream, h);
     if (rc) return rc;
+    std::vector<ScatterJob> jobs;
+    rc = density_jobs(h.data(), n_reps, jobs);
+    if (rc || jobs.empty()) return rc;
     hipStream_t st = (hipStream_t)stream;
-    std::vector<chromo_replica> h(n_reps);
-    HIPC(hipMemcpyAsync(h.data(), d_reps, sizeof(chromo_replica) * n_reps, hipMemcpyDeviceToHost, st));
-    HIPC(hipStreamSynchronize(st));
-    int64_t maxN = 0, maxBins = 0;
-    for (auto &r : h) {
-        if (r.field_on == 0) continue;
-        if (r.B < 0 || r.B > CHROMO_MAX_BINDERS) return set_err(-1, "B out of range");
-        int64_t nb = r.nx * r.ny * r.nz;
-        if (nb > 2048LL * 2048LL || r.N > 0x7fffffff)
-            return set_err(-1, "grid or chain too large for the density scatter");
-        maxN = r.N > maxN ? r.N : maxN;
-        maxBins = nb > maxBins ? nb : maxBins;
-    }
-    if (maxN == 0) return 0;
-    DensityScratch S;
-    HIPC(density_scratch_alloc(S, maxN, maxBins, st));
-    for (int i = 0; i < n_reps; ++i) {
-        const chromo_replica &r = h[i];
-        if (r.field_on == 0) continue;
-        PosView P{r.pos, r.N, 1};
-        hipError_t e = density_scatter(grid_of(r), r.N, r.B + 1, P, r.states, r.density, 1, S, st);
-        if (e != hipSuccess) {
-            density_scratch_free(S, st);
-            return set_err(-2, std::string("density scatter: ") + hipGetErrorString(e));
-        }
-    }
-    density_scratch_free(S, st);
-    return 0;
+    char *ws = nullptr;
+    const size_t bytes = density_bytes(jobs);
+    HIPC(hipMallocAsync((void **)&ws, bytes, st));
+    rc = density_run(jobs, ws, st);
+    (void)hipFreeAsync(ws, st);
+    return rc;
+}
+
+int64_t chromo_density_init_bytes(const chromo_replica *h_reps, int32_t n_reps)
+{
+    int rc = check_reps(h_reps, n_reps);
+    if (rc) return rc;
+    std::vector<ScatterJob> jobs;
+    rc = density_jobs(h_reps, n_reps, jobs);
+    if (rc) return rc;
+    return jobs.empty() ? 0 : (int64_t)density_bytes(jobs);
+}
+
+int chromo_density_init_ws(const chromo_replica *h_reps, int32_t n_reps, void *d_ws, int64_t ws_bytes, void *stream)
+{
+    int rc = check_reps(h_reps, n_reps);
+    if (rc) return rc;
+    std::vector<ScatterJob> jobs;
+    rc = density_jobs(h_reps, n_reps, jobs);
+    if (rc || jobs.empty()) return rc;
+    if (!d_ws || ws_bytes < 0 || (size_t)ws_bytes < density_bytes(jobs))
+        return set_err(-1, "the workspace holds fewer bytes than chromo_density_init_bytes");
+    if ((uintptr_t)d_ws % 16) return set_err(-1, "the workspace must be 16-byte aligned");
+    return density_run(jobs, (char *)d_ws, (hipStream_t)stream);
 }
 
 int chromo_scratch_init(const chromo_replica *d_reps, int32_t n_reps, void *stream)

@@ -1,7 +1,8 @@
-// chromo_tiles.hpp -- voxel densities, field energy and its gradient of the energy
-// adjoint, tile by tile in LDS.
+// chromo_tiles.hpp -- a density grid in tiles and the bead lists of the tiles, for the
+// scatter (chromo_density.hpp, which includes this file) and the energy adjoint's tile
+// kernel (chromo_energy.hip): voxel densities, field energy and gradient in LDS.
 //
-// The grid is cut into tiles of at most 8 x 8 x 8 voxels.  Every bead is listed in
+// For the adjoint the grid is cut into tiles of at most 8 x 8 x 8 voxels.  Every bead is listed in
 // the tile of its lower-corner cell and in the tiles that cell is a neighbour of
 // (at most one per axis), so a tile's list holds every bead that reaches its voxels
 // and their upper neighbours.  One block per tile then does what took four passes over
@@ -21,7 +22,6 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#include "chromo_density.hpp"
 #include "chromo_device.hpp"
 
 namespace chromo {
@@ -31,7 +31,10 @@ namespace {
 // starts at t n / nt: tiles of at least half the size when there are several, so a cell
 // touches at most one face per axis and the lists hold at most twice the beads per axis.
 // An axis that fits one tile is one tile that wraps onto itself.
+// The scatter needs no upper neighbours, and smaller tiles keep more wavefronts on a
+// compute unit.
 constexpr int TILE_MAX[3] = {8, 8, 8};
+constexpr int FOLD_MAX[3] = {4, 4, 4};
 constexpr int TILE_SX = 9, TILE_SY = 9, TILE_SZ = 9;    // a tile's voxels and their upper neighbours
 constexpr int TILE_VOX = TILE_SX * TILE_SY * TILE_SZ;
 constexpr int TILE_THREADS = 512;
@@ -45,7 +48,7 @@ struct TileGeom {
     double vbV;                             // vol_bin / bead_vol
 };
 
-inline TileGeom tile_geom(const GridGeom &G, double bead_vol)
+inline TileGeom tile_geom(const GridGeom &G, const int (&most)[3], double bead_vol)
 {
     TileGeom T;
     const int64_t n[3] = {G.nx, G.ny, G.nz};
@@ -55,11 +58,28 @@ inline TileGeom tile_geom(const GridGeom &G, double bead_vol)
     T.vbV = G.vol_bin / bead_vol;
     for (int j = 0; j < 3; ++j) {
         T.n[j] = (int32_t)n[j];
-        T.nt[j] = (int32_t)((n[j] + TILE_MAX[j] - 1) / TILE_MAX[j]);
+        T.nt[j] = (int32_t)((n[j] + most[j] - 1) / most[j]);
         T.ntiles *= T.nt[j];
         T.recip = T.recip && recip_range(G.width[j]) && recip_range(G.dxyz[j]);
         T.rw[j] = 1.0 / G.width[j];
         T.rd[j] = 1.0 / G.dxyz[j];
+    }
+    return T;
+}
+
+// The scatter's tiles: the largest of these shapes that still gives every compute unit
+// several wavefronts, one per tile.  A tile's beads are folded one after the other, so a
+// small grid with many beads wants small tiles, and a large one large tiles (fewer beads
+// listed twice).
+constexpr int FOLD_TILES = 2048;
+
+inline TileGeom fold_geom(const GridGeom &G)
+{
+    constexpr int shapes[4][3] = {{FOLD_MAX[0], FOLD_MAX[1], FOLD_MAX[2]}, {4, 4, 2}, {2, 2, 2}, {1, 1, 1}};
+    TileGeom T;
+    for (const auto &most : shapes) {
+        T = tile_geom(G, most, 1.0);
+        if (T.ntiles >= FOLD_TILES) break;
     }
     return T;
 }
@@ -111,13 +131,16 @@ __device__ __forceinline__ void tile_lower(const GridGeom &G, const TileGeom &T,
 }
 
 // The tiles of one axis that list a bead of cell c: its own and, when the cell lies on
-// a face, the neighbour behind that face.  Returns how many.
+// a face, the neighbour behind that face (UPPER: behind either face, for tiles that
+// need their voxels' upper neighbours; else only behind the upper one, whose voxels the
+// bead's upper corners reach).  Returns how many.
+template <bool UPPER>
 __device__ __forceinline__ int axis_tiles(int n, int nt, int c, int t[2])
 {
     t[0] = nt == 1 ? 0 : tile_of(n, nt, c);
     t[1] = t[0];
     if (nt == 1) return 1;
-    if (c == tile_start(n, nt, t[0])) {
+    if (UPPER && c == tile_start(n, nt, t[0])) {
         t[1] = t[0] == 0 ? nt - 1 : t[0] - 1;
         return 2;
     }
@@ -138,7 +161,7 @@ __global__ void k_tile_clear(int32_t *cnt, int32_t *fill, int32_t *cursor, int n
 
 // Room for every list: a wavefront's lists in a row, the wavefronts in the order they
 // arrive (nothing depends on where a list lies).
-__global__ void k_tile_base(const int32_t *cnt, int32_t *base, int32_t *cursor, int n)
+__device__ __forceinline__ void tile_bases(const int32_t *cnt, int32_t *base, int32_t *cursor, int n)
 {
     const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
     const int k = i < n ? cnt[i] : 0;
@@ -150,27 +173,43 @@ __global__ void k_tile_base(const int32_t *cnt, int32_t *base, int32_t *cursor, 
     if (i < n) base[i] = at + off;
 }
 
+__global__ void k_tile_base(const int32_t *cnt, int32_t *base, int32_t *cursor, int n)
+{
+    tile_bases(cnt, base, cursor, n);
+}
+
 // PLACE false: each bead's cell into cell[], and the lists' lengths into num.  PLACE
 // true: the beads into their lists, num counting the entries placed.  A block counts its beads per
 // list in LDS first (consecutive beads lie in a few tiles), so that a list costs it one
 // global atomic; a list that finds no room in the block's table takes its entries from
-// the global counter one by one.  The order within a list does not matter.
+// the global counter one by one.  STABLE: what a block places in a list through its
+// table is in bead order (a bit per bead and list in LDS, the rank the bits below).
+// Otherwise the order within a list is any.
 constexpr int TILE_TABLE = 512, TILE_PROBES = 16, BIN_THREADS = 256;
 
-template <bool PLACE>
-__global__ void __launch_bounds__(BIN_THREADS) k_tile_bin(GridGeom G, TileGeom T, int64_t N, const double *r, int32_t *cell,
-                                                  int32_t *num, const int32_t *base, int32_t *list)
+template <bool PLACE, bool UPPER, bool STABLE>
+__device__ __forceinline__ void tile_bin(const GridGeom &G, const TileGeom &T, int64_t N, const PosView &P,
+                                         int32_t *cell, int32_t *num, const int32_t *base, int32_t *list)
 {
+    constexpr int W = BIN_THREADS / WAVE;
     __shared__ int32_t key[TILE_TABLE], cntl[TILE_TABLE], from[TILE_TABLE];
-    for (int i = threadIdx.x; i < TILE_TABLE; i += BIN_THREADS) {
+    __shared__ unsigned long long bits[STABLE && PLACE ? TILE_TABLE * W : 1];
+    const int t = (int)threadIdx.x, wv = t / WAVE, lane = t % WAVE;
+    for (int i = t; i < TILE_TABLE; i += BIN_THREADS) {
         key[i] = -1;
         cntl[i] = 0;
     }
+    if (STABLE && PLACE)
+        for (int i = t; i < TILE_TABLE * W; i += BIN_THREADS) bits[i] = 0;
     __syncthreads();
-    const int64_t b = (int64_t)blockIdx.x * BIN_THREADS + threadIdx.x;
+    const int64_t b = (int64_t)blockIdx.x * BIN_THREADS + t;
     int slot[8], rank[8], tile[8];
 #pragma unroll
-    for (int q = 0; q < 8; ++q) tile[q] = -1;
+    for (int q = 0; q < 8; ++q) {
+        tile[q] = -1;
+        slot[q] = -1;
+        rank[q] = 0;
+    }
     if (b < N) {
         int ix[3];
         if (PLACE) {
@@ -180,19 +219,18 @@ __global__ void __launch_bounds__(BIN_THREADS) k_tile_bin(GridGeom G, TileGeom T
             ix[2] = (int)(q / (uint32_t)T.n[1]);
         } else {
             double x[3], w[3];
-            for (int j = 0; j < 3; ++j) x[j] = r[3 * b + j];
+            for (int j = 0; j < 3; ++j) x[j] = P.p[j * P.sc + b * P.sb];
             tile_lower(G, T, x, ix, w);
             cell[b] = ix[0] + T.n[0] * (ix[1] + T.n[1] * ix[2]);
         }
-        int t[3][2], k[3];
+        int s[3][2], k[3];
 #pragma unroll
-        for (int j = 0; j < 3; ++j) k[j] = axis_tiles(T.n[j], T.nt[j], ix[j], t[j]);
+        for (int j = 0; j < 3; ++j) k[j] = axis_tiles<UPPER>(T.n[j], T.nt[j], ix[j], s[j]);
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
             if ((q & 1) >= k[0] || ((q >> 1) & 1) >= k[1] || (q >> 2) >= k[2]) continue;
-            tile[q] = t[0][q & 1] + T.nt[0] * (t[1][(q >> 1) & 1] + T.nt[1] * t[2][q >> 2]);
+            tile[q] = s[0][q & 1] + T.nt[0] * (s[1][(q >> 1) & 1] + T.nt[1] * s[2][q >> 2]);
             int h = tile[q] & (TILE_TABLE - 1);
-            slot[q] = -1;
             for (int p = 0; p < TILE_PROBES; ++p) {
                 const int old = atomicCAS(&key[h], -1, tile[q]);
                 if (old == -1 || old == tile[q]) {
@@ -201,17 +239,41 @@ __global__ void __launch_bounds__(BIN_THREADS) k_tile_bin(GridGeom G, TileGeom T
                 }
                 h = (h + 1) & (TILE_TABLE - 1);
             }
-            rank[q] = slot[q] >= 0 ? atomicAdd(&cntl[slot[q]], 1) : atomicAdd(&num[tile[q]], 1);
+            if (slot[q] < 0) rank[q] = atomicAdd(&num[tile[q]], 1);
+            else if (STABLE && PLACE) atomicOr(&bits[slot[q] * W + wv], 1ull << lane);
+            else rank[q] = atomicAdd(&cntl[slot[q]], 1);
         }
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < TILE_TABLE; i += BIN_THREADS)
-        if (key[i] >= 0) from[i] = atomicAdd(&num[key[i]], cntl[i]);
+    for (int i = t; i < TILE_TABLE; i += BIN_THREADS)
+        if (key[i] >= 0) {
+            int n = cntl[i];
+            if (STABLE && PLACE)
+                for (int w = 0; w < W; ++w) n += __popcll(bits[i * W + w]);
+            from[i] = atomicAdd(&num[key[i]], n);
+        }
     if (!PLACE) return;
     __syncthreads();
 #pragma unroll
-    for (int q = 0; q < 8; ++q)
-        if (tile[q] >= 0) list[base[tile[q]] + (slot[q] >= 0 ? from[slot[q]] : 0) + rank[q]] = (int32_t)b;
+    for (int q = 0; q < 8; ++q) {
+        if (tile[q] < 0) continue;
+        int at = rank[q];
+        if (slot[q] >= 0) {
+            at += from[slot[q]];
+            if (STABLE) {
+                for (int w = 0; w < wv; ++w) at += __popcll(bits[slot[q] * W + w]);
+                at += __popcll(bits[slot[q] * W + wv] & ((1ull << lane) - 1));
+            }
+        }
+        list[base[tile[q]] + at] = (int32_t)b;
+    }
+}
+
+template <bool PLACE>
+__global__ void __launch_bounds__(BIN_THREADS) k_tile_bin(GridGeom G, TileGeom T, int64_t N, PosView P, int32_t *cell,
+                                                          int32_t *num, const int32_t *base, int32_t *list)
+{
+    tile_bin<PLACE, true, false>(G, T, N, P, cell, num, base, list);
 }
 
 // Place of a cell on one axis of a tile of `size` voxels from `start`: 0 .. size - 1

@@ -363,7 +363,7 @@ class DeviceReplicas:
         L.check(self.lib.chromo_scratch_init(self.tab_ptr, n, stream), "chromo_scratch_init")
         self.seed(seeds if seeds is not None else [1] * n, streams)
         if any(f.field_on for f in fields):
-            L.check(self.lib.chromo_density_init(self.tab_ptr, n, stream), "chromo_density_init")
+            self.density_init()
 
     # -- RNG -----------------------------------------------------------------
     def seed(self, seeds: Sequence[int], streams: Optional[Sequence[int]] = None) -> None:
@@ -484,8 +484,14 @@ class DeviceReplicas:
         return d.view(self.nbins[i], self.Bs[i] + 1).cpu().numpy().copy()
 
     def density_init(self) -> None:
-        L.check(self.lib.chromo_density_init(self.tab_ptr, self.n, _current_stream()),
-                "chromo_density_init")
+        """Every replica's densities from its chain (the reference's bead-order scatter)."""
+        h = ctypes.addressof(self._tab_host)
+        nb = int(self.lib.chromo_density_init_bytes(h, self.n))
+        if nb < 0:
+            L.check(nb, "chromo_density_init_bytes")
+        ws = torch.empty(max(nb, 1), dtype=torch.uint8, device=self.device)
+        L.check(self.lib.chromo_density_init_ws(h, self.n, ws.data_ptr(), nb, _current_stream()),
+                "chromo_density_init_ws")
 
     def controllers(self, i: int) -> List[CtrlSpec]:
         cs = ctypes.sizeof(L.ChromoCtrl)

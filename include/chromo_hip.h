@@ -199,6 +199,14 @@ int chromo_np_seed(const chromo_replica *d_reps, int32_t n_reps, const uint32_t 
  * (chromo/fields.pyx:2041-2106): deterministic, bitwise equal to the
  * reference's sequential bead-order scatter, including the 1e-18 clean-up. */
 int chromo_density_init(const chromo_replica *d_reps, int32_t n_reps, void *stream);
+/* The same from the host's copy of the replica table (the pointers in it are device
+ * pointers), with a workspace of the caller's: device memory of at least
+ * chromo_density_init_bytes(h_reps, n_reps) bytes (negative: an error code), 16-byte
+ * aligned, free for other use once the work on the stream is done.  Reads nothing back
+ * and allocates nothing; with one replica that has a field it does not wait either. */
+int64_t chromo_density_init_bytes(const chromo_replica *h_reps, int32_t n_reps);
+int chromo_density_init_ws(const chromo_replica *h_reps, int32_t n_reps, void *d_ws, int64_t ws_bytes,
+                           void *stream);
 
 /* ---- Monte Carlo -------------------------------------------------------- */
 
