@@ -52,6 +52,8 @@ constexpr int EV_NUM = (int)0x80000000;         // hash value of voxel number q:
 // workgroups on a compute unit.
 __host__ __device__ inline int ev_slot_ucap(int Bp1) { return Bp1 <= 3 ? 640 : (Bp1 == 4 ? 512 : 416); }
 __host__ __device__ inline int ev_wide_ucap(int Bp1) { return Bp1 <= 2 ? 1024 : (Bp1 == 3 ? 896 : (Bp1 == 4 ? 704 : 576)); }
+static_assert(1024 * 2 * 8 < 65536 && 896 * 3 * 8 < 65536 && 704 * 4 * 8 < 65536 && 576 * 5 * 8 < 65536,
+              "byte offsets of the deltas fit 16 bits");
 
 struct EvLayout {
     size_t c0, eq, pst, ends, tmat, hkey, hval, uv, acc, total;
@@ -63,10 +65,10 @@ __host__ __device__ inline EvLayout ev_layout(int Bp1, bool wide)
     EvLayout L;
     size_t o = 0;
     L.c0 = o;   o += sizeof(double) * 8 * EV_POS;      // corner weight / volume per contribution
-    L.eq = o;   o += sizeof(uint16_t) * 8 * EV_POS;    // its voxel number
+    L.eq = o;   o += sizeof(uint16_t) * 8 * EV_POS;    // byte offset of its voxel's deltas
     L.ends = o; o += sizeof(double) * 2 * 2 * 9;       // end beads: [first / last][current / trial][r, t3, t2]
     L.tmat = o; o += sizeof(double) * 12;              // the proposal's transform, for the commit
-    L.pst = o;  o += sizeof(int32_t) * EV_POS;         // binder states per position
+    L.pst = o;  o += sizeof(uint64_t) * EV_POS;        // weight factors per position: 1, then the binder states
     L.uv = o;   o += sizeof(int2) * U;                 // voxel, its hash slot | its first probe << 16
     L.acc = o;  o += sizeof(double) * U * Bp1;         // delta densities, then new densities
     L.hkey = o; o += sizeof(int32_t) * H;              // voxel
@@ -78,7 +80,8 @@ __host__ __device__ inline EvLayout ev_layout(int Bp1, bool wide)
 struct EvLds {
     double *c0, *ends, *tmat, *acc;
     uint16_t *eq;
-    int32_t *pst, *hkey, *hval;
+    uint8_t *pst;       // factor m of position p at 8 p + m
+    int32_t *hkey, *hval;
     int2 *uv;
     int hsize, ymask, zshift, ucap;
 };
@@ -91,7 +94,7 @@ __device__ __forceinline__ EvLds ev_lds(char *base, int Bp1, bool wide)
     S.eq = (uint16_t *)(base + L.eq);
     S.ends = (double *)(base + L.ends);
     S.tmat = (double *)(base + L.tmat);
-    S.pst = (int32_t *)(base + L.pst);
+    S.pst = (uint8_t *)(base + L.pst);
     S.uv = (int2 *)(base + L.uv);
     S.acc = (double *)(base + L.acc);
     S.hkey = (int32_t *)(base + L.hkey);
@@ -386,36 +389,37 @@ __device__ __forceinline__ double bond_E(const Bond &bd, const double *r0, const
 
 // The fold of one chunk's npos positions into S.acc (fields.pyx:1491-1520): lanes
 // 8 m + l of a position's group hold species m of corner l; PB positions share the
-// arithmetic of one step, and their adds are issued one position after the other.
-template <int NB>
-__device__ __forceinline__ void ev_fold(const EvLds &S, int npos, bool thr, bool degen)
+// arithmetic of one step, and their adds are issued one position after the other.  Every
+// row of the chunk's arrays is written (a position past npos with weights of zero), so
+// the steps need no bounds.  THR: the 1e-18 rule; without it a zero weight alone is
+// passed over.
+template <int NB, bool THR>
+__device__ __forceinline__ void ev_fold(const EvLds &S, int npos, bool degen)
 {
     constexpr int Bp1 = NB + 1, LP = 8 * Bp1, PB = WAVE / LP, UN = PB == 1 ? 8 : 4;
-    const int lane = lane_id(), pj = lane / LP, m = (lane % LP) >> 3, l = lane & 7;
-    const bool in = pj < PB;
+    static_assert(EV_POS % (PB * UN) == 0, "whole steps");
+    const int lane = lane_id(), l = lane & 7;
+    const bool in = lane < PB * LP;
+    const int pj = in ? lane / LP : 0, m = in ? (lane % LP) >> 3 : 0;
+    char *acc = (char *)(S.acc + m);
     for (int p0 = 0; p0 < npos; p0 += PB * UN) {
         double t[UN];
-        double *to[UN];
+        char *to[UN];
         bool go[UN];
 #pragma unroll
         for (int k = 0; k < UN; ++k) {
             const int p = p0 + k * PB + pj;
-            const bool ok = in && p < npos;
-            const int pc = ok ? p : 0;
-            const double c = S.c0[8 * pc + l];
-            const int q = S.eq[8 * pc + l];
-            const int st = S.pst[pc];
-            const double v = m == 0 ? c : c * (double)((st >> (8 * (m - 1) & 31)) & 0xff);
-            t[k] = (p & 1) ? v : -v;
-            go[k] = ok && (!thr || fabs(t[k]) > 1E-18);
-            to[k] = &S.acc[q * Bp1 + m];
+            // species 0 has the factor 1: no branch, so the steps' loads go out together
+            t[k] = S.c0[8 * p + l] * (double)S.pst[8 * p + m];
+            to[k] = acc + S.eq[8 * p + l];
+            go[k] = in && (THR ? fabs(t[k]) > 1E-18 : !(fabs(t[k]) <= 0));
         }
         if (!degen) {
 #pragma unroll
             for (int k = 0; k < UN; ++k) {
 #pragma unroll
                 for (int j = 0; j < PB; ++j) {
-                    if (go[k] && pj == j) lds_add(to[k], t[k]);
+                    if (go[k] && pj == j) lds_add((double *)to[k], t[k]);
                     __builtin_amdgcn_wave_barrier();
                 }
             }
@@ -423,7 +427,7 @@ __device__ __forceinline__ void ev_fold(const EvLds &S, int npos, bool thr, bool
 #pragma unroll
             for (int k = 0; k < UN; ++k) {
                 for (int s = 0; s < 8 * PB; ++s) {
-                    if (go[k] && pj == (s >> 3) && l == (s & 7)) lds_add(to[k], t[k]);
+                    if (go[k] && pj == (s >> 3) && l == (s & 7)) lds_add((double *)to[k], t[k]);
                     __builtin_amdgcn_wave_barrier();
                 }
             }
@@ -640,10 +644,10 @@ __device__ __forceinline__ void ev_eval(const chromo_replica *R, const EvConst &
         const int p = 2 * i32 + k;
         int v8[8], h8[8];
         double c8[8];
-        int32_t sp = 0;
+        uint64_t sp = 1;
         int ties = 0;
 #pragma unroll
-        for (int m = 0; m < NB; ++m) sp |= ((int32_t)(uint8_t)(k == 0 ? B.so[m] : sn[m])) << (8 * m);
+        for (int m = 0; m < NB; ++m) sp |= (uint64_t)(uint8_t)(k == 0 ? B.so[m] : sn[m]) << (8 * (m + 1));
         uint32_t bad = 0;
         int hb[8];
         if (act) {
@@ -725,15 +729,19 @@ __device__ __forceinline__ void ev_eval(const chromo_replica *R, const EvConst &
         }
         for (int t = U0 * Bp1 + lane; t < U * Bp1; t += WAVE) S.acc[t] = 0;
         wave_sync();
-        if (act) {
+        {
+            // the position's rows; the current position takes its weights away
             uint32_t qq[8];
 #pragma unroll
-            for (int l = 0; l < 8; ++l) qq[l] = (uint32_t)(S.hval[h8[l]] - EV_NUM);
+            for (int l = 0; l < 8; ++l)
+                qq[l] = act ? (uint32_t)(S.hval[h8[l]] - EV_NUM) * (uint32_t)(sizeof(double) * Bp1) : 0u;
             *(uint4 *)&S.eq[8 * p] = make_uint4(qq[0] | qq[1] << 16, qq[2] | qq[3] << 16, qq[4] | qq[5] << 16,
                                                 qq[6] | qq[7] << 16);
 #pragma unroll
-            for (int l = 0; l < 8; l += 2) *(double2 *)&S.c0[8 * p + l] = make_double2(c8[l], c8[l + 1]);
-            S.pst[p] = sp;
+            for (int l = 0; l < 8; l += 2)
+                *(double2 *)&S.c0[8 * p + l] = act ? make_double2(k ? c8[l] : -c8[l], k ? c8[l + 1] : -c8[l + 1])
+                                                   : make_double2(0, 0);
+            *(uint64_t *)&S.pst[8 * p] = sp;
         }
         wave_sync();
         if (c == nchunks - 1) {
@@ -746,7 +754,8 @@ __device__ __forceinline__ void ev_eval(const chromo_replica *R, const EvConst &
                 for (int m = 0; m < Bp1; ++m) rho[a][m] = q < U ? rho_g[(int64_t)v * Bp1 + m] : 0.0;
             }
         }
-        ev_fold<NB>(S, 2 * nb, thr, degen);
+        if (thr) ev_fold<NB, true>(S, 2 * nb, degen);
+        else ev_fold<NB, false>(S, 2 * nb, degen);
     }
 
     if (!state_change) {
