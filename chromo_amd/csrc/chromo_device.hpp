@@ -414,21 +414,25 @@ __device__ __forceinline__ void philox_set(WaveRng &R, uint64_t ctr, int bi)
     }
 }
 
-// MT19937 regeneration of the 624-word block (lane 0, LDS), then tempering.
-__device__ void mt_twist(uint32_t *mt)
+// MT19937 regeneration of the 624-word block in LDS, 64 words at a time: word i takes
+// words i and i + 1 of the old block (word 0 of the new one after the last) and word
+// i + 397, which wraps to word i - 227 of the new block, of an earlier group.
+__device__ __forceinline__ void mt_twist(uint32_t *mt)
 {
     wave_sync();
-    if (lane_id() == 0) {
-        for (int i = 0; i < 624; ++i) {
-            uint32_t y = (mt[i] & 0x80000000u) | (mt[i + 1 == 624 ? 0 : i + 1] & 0x7fffffffu);
-            int j = i + 397;
-            if (j >= 624) j -= 624;
-            uint32_t v = mt[j] ^ (y >> 1);
+    for (int i0 = 0; i0 < 624; i0 += WAVE) {
+        const int i = i0 + lane_id();
+        const bool in = i < 624;
+        uint32_t v = 0;
+        if (in) {
+            const uint32_t y = (mt[i] & 0x80000000u) | (mt[i + 1 == 624 ? 0 : i + 1] & 0x7fffffffu);
+            v = mt[i + 397 < 624 ? i + 397 : i - 227] ^ (y >> 1);
             if (y & 1u) v ^= 0x9908b0dfu;
-            mt[i] = v;
         }
+        wave_sync();
+        if (in) mt[i] = v;
+        wave_sync();
     }
-    wave_sync();
 }
 
 __device__ __forceinline__ uint32_t mt_draw(WaveRng &R)

@@ -131,44 +131,50 @@ __device__ __forceinline__ void ev_release(const EvLds &S, int U)
 
 // Grid constants with the reciprocals the exact divisions below use, worked out once
 // per launch and kept in LDS.
+enum : int { EC_WIDTH = 0, EC_D = 3, EC_SUB = 6, EC_NSUB = 9, EC_LEN = 12 };
 struct EvConst {
-    double width[3], rwidth[3], hw[3], hs[3], d[3], rd[3];
-    double sw[3], rsw[3], nsub[3], rnsub[3], half_points;
+    double len[EC_LEN], rec[EC_LEN];  // per axis: box width, voxel size, sub-bin width, sub-bins; their reciprocals
+    double hw[3], hs[3], half_points;
     double vol, rvol, vbV, cphi;      // vol_bin, its reciprocal, vol_bin / bead_vol, chi (vol_bin / bead_vol)
     int32_t n[3], fast, recip, cross;
 };
 
-// Fills the constants; the first four threads of the workgroup, the caller synchronises.
+// Fills the constants; the first wavefront of the workgroup, the caller synchronises.
+// One division per lane, so the launch waits for one: in three lanes of four divisions
+// each they took 0.4 us of a launch that evaluates one proposal.
 __device__ __forceinline__ void ev_const(EvConst *C, const chromo_replica *R)
 {
     const int t = (int)threadIdx.x;
+    if (t >= WAVE) return;
+    const bool axis = t < EC_LEN;
+    const int j = t % 3;
+    const double *const row = t < EC_D ? R->width : (t < EC_SUB ? R->dxyz : R->sub_width);
+    double den = R->vol_bin;
+    if (axis) den = t < EC_NSUB ? row[j] : (double)R->n_sub[j];
+    if (t == EC_LEN + 1) den = R->bead_vol;
+    const double q = (t == EC_LEN + 1 ? R->vol_bin : 1.0) / den;
+    if (axis) {
+        C->len[t] = den;
+        C->rec[t] = q;
+    } else if (t == EC_LEN) {
+        C->vol = den;
+        C->rvol = q;
+        C->half_points = R->half_points;
+        C->fast = R->fast_field;
+    } else if (t == EC_LEN + 1) {
+        C->vbV = q;
+        C->cphi = R->chi * q;
+    }
     if (t < 3) {
-        const double W = R->width[t], d = R->dxyz[t], sw = R->sub_width[t], ns = (double)R->n_sub[t];
-        C->width[t] = W;
-        C->rwidth[t] = 1.0 / W;
         C->hw[t] = R->half_width[t];
         C->hs[t] = R->half_step[t];
-        C->d[t] = d;
-        C->rd[t] = 1.0 / d;
-        C->sw[t] = sw;
-        C->rsw[t] = 1.0 / sw;
-        C->nsub[t] = ns;
-        C->rnsub[t] = 1.0 / ns;
         C->n[t] = (int32_t)(t == 0 ? R->nx : (t == 1 ? R->ny : R->nz));
-    } else if (t == 3) {
-        C->half_points = R->half_points;
-        C->vol = R->vol_bin;
-        C->rvol = 1.0 / R->vol_bin;
-        C->vbV = R->vol_bin / R->bead_vol;
-        C->cphi = R->chi * (R->vol_bin / R->bead_vol);
-        C->fast = R->fast_field;
-        bool ok = recip_range(R->vol_bin);
-        for (int j = 0; j < 3; ++j)
-            ok = ok && recip_range(R->dxyz[j]) && recip_range(R->width[j]) &&
-                 (!R->fast_field || recip_range(R->sub_width[j]));
-        C->recip = ok;
-        bool x = false;
-        for (int j = 0; j < R->B * R->B; ++j) x = x || R->cross[j] != 0;
+    }
+    const bool used = t < EC_SUB || (t < EC_NSUB && R->fast_field) || t == EC_LEN;
+    const bool out = wave_any(used && !recip_range(den));
+    const bool x = wave_any(t < R->B * R->B && R->cross[t] != 0);
+    if (t == 0) {
+        C->recip = !out;
         C->cross = x;
     }
 }
@@ -183,7 +189,7 @@ __device__ __forceinline__ void ev_lower(const chromo_replica *R, const EvConst 
 #pragma unroll
     for (int j = 0; j < 3; ++j) {
         a[j] = pos[j] + C.hw[j];
-        far = far || !(fabs(a[j]) < 0x1p40 * (C.fast ? C.sw[j] : C.width[j]));
+        far = far || !(fabs(a[j]) < 0x1p40 * C.len[(C.fast ? EC_SUB : EC_WIDTH) + j]);
     }
     if (wave_any(far)) {
         // a coordinate far outside the box, or a grid of extreme size: the general path
@@ -196,14 +202,14 @@ __device__ __forceinline__ void ev_lower(const chromo_replica *R, const EvConst 
     if (C.fast) {
 #pragma unroll
         for (int j = 0; j < 3; ++j) {
-            const double qs = div_by(a[j], C.sw[j], C.rsw[j]);
+            const double qs = div_by(a[j], C.len[EC_SUB + j], C.rec[EC_SUB + j]);
             const double sb = floor(qs);
             ties += fabs(qs - rint(qs)) < TIE_VOXEL_EPS;
             // sb mod n_sub, whole numbers below 2^41: exact
-            double i = fma(-floor(sb * C.rnsub[j]), C.nsub[j], sb);
-            if (i < 0) i += C.nsub[j];
-            if (i >= C.nsub[j]) i -= C.nsub[j];
-            const double u = div_by((i - C.half_points) * C.sw[j], C.d[j], C.rd[j]);
+            double i = fma(-floor(sb * C.rec[EC_NSUB + j]), C.len[EC_NSUB + j], sb);
+            if (i < 0) i += C.len[EC_NSUB + j];
+            if (i >= C.len[EC_NSUB + j]) i -= C.len[EC_NSUB + j];
+            const double u = div_by((i - C.half_points) * C.len[EC_SUB + j], C.len[EC_D + j], C.rec[EC_D + j]);
             const double ind = floor(u);
             ix[j] = (ind == -1.0) ? C.n[j] - 1 : (int)ind;
             w[j] = 1 - (u - ind);
@@ -214,14 +220,14 @@ __device__ __forceinline__ void ev_lower(const chromo_replica *R, const EvConst 
     for (int j = 0; j < 3; ++j) {
         // Python's a % W: the quotient from the reciprocal is off by at most one, which
         // the first remainder's sign and range show; the second is exact (fmod_exact)
-        const double W = C.width[j];
-        double q = trunc(a[j] * C.rwidth[j]);
+        const double W = C.len[EC_WIDTH + j];
+        double q = trunc(a[j] * C.rec[EC_WIDTH + j]);
         double r = fma(-q, W, a[j]);
         q += (a[j] >= 0) ? ((r < 0) ? -1.0 : (r >= W ? 1.0 : 0.0)) : ((r > 0) ? 1.0 : (r <= -W ? -1.0 : 0.0));
         r = fma(-q, W, a[j]);
         r = (r == 0) ? copysign(0.0, a[j]) : r;
         r += (r < 0) ? W : 0.0;
-        double x = div_by(r - C.hs[j], C.d[j], C.rd[j]);
+        double x = div_by(r - C.hs[j], C.len[EC_D + j], C.rec[EC_D + j]);
         if (!(x >= -1.0 && x < (double)C.n[j])) x = 0.0;
         const double f = floor(x);
         ix[j] = (f == -1.0) ? C.n[j] - 1 : (int)f;

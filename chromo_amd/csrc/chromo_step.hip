@@ -72,22 +72,25 @@ __global__ void __launch_bounds__(64) k_mc_step(const chromo_replica *__restrict
     load_record(&Rs, &reps[rep]);
     wave_sync();
     const chromo_replica *R = &Rs;
-    if (R->counters[CHROMO_CNT_ERROR] != 0) return;
+    // the replica's state travels while the constants and the hash are set up; nothing
+    // is written before the error check
+    const int64_t failed = R->counters[CHROMO_CNT_ERROR];
+    chromo_ctrl C = R->ctrl[ci];
+    Counters K;
+    counters_load(R, K);
+    const int Bp1 = R->B < 1 || R->B + 1 > max_bp1 ? max_bp1 : R->B + 1;
+    uint32_t *mt_lds = (uint32_t *)(lds_dyn + wide_lds_bytes(Bp1));
+    const bool need_mt = (C.move == CHROMO_CHANGE_BINDING_STATE);
+    WaveRng rng;
+    rng_load(R, rng, mt_lds, need_mt);
+    ev_const(&EC, R);
+    const EvLds S = ev_lds(lds_dyn, Bp1, true);
+    ev_clear(S);
+    if (failed != 0) return;
     if (R->B < 1 || R->B + 1 > max_bp1) {
         counters_error(R, ERR_NBINDERS);
         return;
     }
-    const int Bp1 = R->B + 1;
-    ev_const(&EC, R);
-    const EvLds S = ev_lds(lds_dyn, Bp1, true);
-    ev_clear(S);
-    uint32_t *mt_lds = (uint32_t *)(lds_dyn + wide_lds_bytes(Bp1));
-    chromo_ctrl C = R->ctrl[ci];
-    const bool need_mt = (C.move == CHROMO_CHANGE_BINDING_STATE);
-    WaveRng rng;
-    rng_load(R, rng, mt_lds, need_mt);
-    Counters K;
-    counters_load(R, K);
     MoveOut o;
     if (R->twist) {
         switch (R->B) {
