@@ -47,10 +47,9 @@ constexpr int EV_WAVES = 4;       // wavefronts of a workgroup, at most
 constexpr int EV_FREE = 0x7fffffff;             // hash value: no contribution yet
 constexpr int EV_NUM = (int)0x80000000;         // hash value of voxel number q: EV_NUM + q
 
-// Voxels a block holds.  A speculative slot's block (hash of 1024): two per workgroup
-// and two workgroups on a compute unit.  The one-at-a-time block (hash of 2048): three
-// workgroups on a compute unit.
-__host__ __device__ inline int ev_slot_ucap(int Bp1) { return Bp1 <= 3 ? 640 : (Bp1 == 4 ? 512 : 416); }
+// Voxels a block holds.  The one-at-a-time block (hash of 2048): three workgroups on a
+// compute unit.  A speculative evaluator's block (hash of 1024, the voxel list kept
+// apart from it) takes what its workgroup's shape leaves it.
 __host__ __device__ inline int ev_wide_ucap(int Bp1) { return Bp1 <= 2 ? 1024 : (Bp1 == 3 ? 896 : (Bp1 == 4 ? 704 : 576)); }
 static_assert(1024 * 2 * 8 < 65536 && 896 * 3 * 8 < 65536 && 704 * 4 * 8 < 65536 && 576 * 5 * 8 < 65536,
               "byte offsets of the deltas fit 16 bits");
@@ -59,9 +58,11 @@ struct EvLayout {
     size_t c0, eq, pst, ends, tmat, hkey, hval, uv, acc, total;
 };
 
-__host__ __device__ inline EvLayout ev_layout(int Bp1, bool wide)
+// slot_ucap: voxels of a speculative evaluator's block, 0 for the one-at-a-time block.
+__host__ __device__ inline EvLayout ev_layout(int Bp1, int slot_ucap)
 {
-    const size_t H = wide ? 2048 : 1024, U = (size_t)(wide ? ev_wide_ucap(Bp1) : ev_slot_ucap(Bp1));
+    const bool wide = slot_ucap == 0;
+    const size_t H = wide ? 2048 : 1024, U = (size_t)(wide ? ev_wide_ucap(Bp1) : slot_ucap);
     EvLayout L;
     size_t o = 0;
     L.c0 = o;   o += sizeof(double) * 8 * EV_POS;      // corner weight / volume per contribution
@@ -69,7 +70,7 @@ __host__ __device__ inline EvLayout ev_layout(int Bp1, bool wide)
     L.ends = o; o += sizeof(double) * 2 * 2 * 9;       // end beads: [first / last][current / trial][r, t3, t2]
     L.tmat = o; o += sizeof(double) * 12;              // the proposal's transform, for the commit
     L.pst = o;  o += sizeof(uint64_t) * EV_POS;        // weight factors per position: 1, then the binder states
-    L.uv = o;   o += sizeof(int2) * U;                 // voxel, its hash slot | its first probe << 16
+    L.uv = o;   o += wide ? sizeof(int2) * U : 0;      // voxel, its hash slot | its first probe << 16
     L.acc = o;  o += sizeof(double) * U * Bp1;         // delta densities, then new densities
     L.hkey = o; o += sizeof(int32_t) * H;              // voxel
     L.hval = o; o += sizeof(int32_t) * H;              // smallest contribution, then number
@@ -86,9 +87,11 @@ struct EvLds {
     int hsize, ymask, zshift, ucap;
 };
 
-__device__ __forceinline__ EvLds ev_lds(char *base, int Bp1, bool wide)
+// A speculative evaluator sets uv to the list of the slot it evaluates.
+__device__ __forceinline__ EvLds ev_lds(char *base, int Bp1, int slot_ucap)
 {
-    const EvLayout L = ev_layout(Bp1, wide);
+    const bool wide = slot_ucap == 0;
+    const EvLayout L = ev_layout(Bp1, slot_ucap);
     EvLds S;
     S.c0 = (double *)(base + L.c0);
     S.eq = (uint16_t *)(base + L.eq);
@@ -102,7 +105,7 @@ __device__ __forceinline__ EvLds ev_lds(char *base, int Bp1, bool wide)
     S.hsize = wide ? 2048 : 1024;
     S.ymask = wide ? 15 : 7;
     S.zshift = wide ? 8 : 7;
-    S.ucap = wide ? ev_wide_ucap(Bp1) : ev_slot_ucap(Bp1);
+    S.ucap = wide ? ev_wide_ucap(Bp1) : slot_ucap;
     return S;
 }
 

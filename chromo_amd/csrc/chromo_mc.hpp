@@ -169,7 +169,7 @@ inline size_t lds_bytes_for(int Bp1)
 
 // Dynamic LDS of the one-wavefront Monte Carlo kernels: the evaluator's one-at-a-time
 // block, then the MT19937 state.
-__host__ __device__ inline size_t wide_lds_bytes(int Bp1) { return ev_layout(Bp1, true).total; }
+__host__ __device__ inline size_t wide_lds_bytes(int Bp1) { return ev_layout(Bp1, 0).total; }
 
 inline size_t mc_lds_bytes(int Bp1) { return wide_lds_bytes(Bp1) + MT_LDS_BYTES; }
 

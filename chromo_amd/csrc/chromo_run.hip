@@ -32,7 +32,7 @@ __global__ void __launch_bounds__(64) k_mc_run_nb(const chromo_replica *__restri
     if (R->counters[CHROMO_CNT_ERROR] != 0) return;
     constexpr int Bp1 = NB + 1;
     ev_const(&EC, R);
-    const EvLds S = ev_lds(lds_dyn, Bp1, true);
+    const EvLds S = ev_lds(lds_dyn, Bp1, 0);
     ev_clear(S);
     uint32_t *mt_lds = (uint32_t *)(lds_dyn + wide_lds_bytes(Bp1));
     const bool need_mt = any_binding(R);

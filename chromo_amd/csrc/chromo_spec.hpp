@@ -6,34 +6,50 @@
 namespace {
 
 // ===========================================================================
-// Speculative rounds: several proposals of one controller block evaluated at once.
+// Speculative evaluation: several proposals of a chain in flight at once.
 //
-// Inside a controller block the amplitudes are fixed, so the random draws of each
-// proposal -- the proposal itself and its Metropolis draw -- do not depend on the
-// accept/reject outcomes before it.  (The exception, a crank-shaft axis shorter
-// than 1e-5 which draws a random axis, is detected and redone one at a time.)
-// One wavefront (Shape::GEN) draws proposals ahead into a ring of slots; wavefront w <
-// Shape::EV evaluates slot w of the round against the current state with ev_eval, in
-// its own LDS block.  Resolution walks the slots in order: slot s keeps its evaluated
-// dE unless an accepted slot s' < s of the same round wrote a bead or a voxel that s
-// reads; then s and all later slots go to the next round and are evaluated again.
-// Each chain therefore is the reference's sequential chain; only the number of rounds
-// depends on conflicts.  What a slot cannot hold runs one at a time through
-// mc_step_dev.
+// Inside a controller block the amplitudes are fixed, and a controller's amplitudes
+// change only at the end of its own block, so the random draws of each proposal -- the
+// proposal itself and its Metropolis draw -- do not depend on the accept/reject outcomes
+// before it.  (The exception, a crank-shaft axis shorter than 1e-5 which draws a random
+// axis, is detected and redone one at a time.)
+//
+// Proposals are numbered through the launch.  The drawing wavefront (Shape::GEN) draws
+// them in order into a ring of slots.  Each of Shape::EV evaluating wavefronts takes the
+// next number, evaluates that slot against the committed state with ev_eval in its own
+// LDS block, and then waits for its turn: slots are resolved in order.  Meanwhile it
+// looks each earlier slot that is resolved as accepted up in its own hash: a slot that
+// reads a bead or a voxel written since its evaluation began is evaluated again at
+// once.  At its turn it commits an accepted proposal and passes the turn on.  The
+// chain therefore is the reference's sequential chain, whatever the schedule; and no
+// wavefront waits for the slowest evaluation of a group, nor at the end of a block.
+// What a slot cannot hold runs one at a time through mc_step_dev, when it is its turn
+// and nothing else is in flight.
 //
 // Two shapes.  W = 2 (more replicas than compute units): wavefront 0 both draws and
 // evaluates, two workgroups share a compute unit.  W = 4 (a compute unit per replica):
-// three evaluators and one wavefront that only draws and keeps the books, so drawing
-// leaves the evaluators' critical path.
+// three evaluators and one wavefront that only draws and keeps the books.
 // ===========================================================================
 
 template <int W>
 struct Shape {
     static_assert(W == 2 || W == 4, "two or four wavefronts");
     static constexpr int EV = W == 2 ? 2 : 3;       // evaluating wavefronts
-    static constexpr int GEN = W == 2 ? 0 : 3;      // the wavefront that draws
-    static constexpr int BOOK = W == 2 ? 1 : 3;     // the wavefront that books a round
-    static constexpr int RING = W == 2 ? 4 : 8;     // slots
+    static constexpr int GEN = W == 2 ? 0 : 3;      // the wavefront that draws and books
+    static constexpr int RING = 8;                  // slots
+    // Slots drawn past the first unresolved one, at most: slot d takes the place of slot
+    // d - RING, which a slot in flight (numbers below first + EV) may still look at when
+    // it is among the EV - 1 before that one.
+    static constexpr int AHEAD = RING - EV + 1;
+    // Voxel lists: slot a's is looked at by the next EV - 1 slots, which can be in flight
+    // together with the EV - 1 after them.
+    static constexpr int LISTS = 2 * EV - 1;
+    // Voxels of a block: two workgroups on a compute unit, or one.
+    __host__ __device__ static constexpr int ucap(int Bp1)
+    {
+        return W == 2 ? (Bp1 <= 2 ? 640 : (Bp1 == 3 ? 560 : (Bp1 == 4 ? 448 : 384)))
+                      : (Bp1 <= 4 ? 704 : 640);
+    }
 };
 
 constexpr int SPEC_NMAX = SEG_MAX;    // tangent picks or binding beads of a slot
@@ -41,13 +57,16 @@ constexpr int SPEC_BEADS = 192;       // beads of a crank-shaft, end-pivot or sl
 constexpr int SPEC_EVMAX = 3;
 enum : int { SLOT_SMALL = 0, SLOT_EMPTY = 1, SLOT_SEQ = 2 };
 constexpr int CK_WORDS = 40;
+// a binding slot always fits a block: it is never given back (its MT19937 draws could
+// not be)
+static_assert(8 * SPEC_NMAX <= 384, "voxels of a binding slot");
 
 struct SpecSlot {
     int32_t kind, move, binder, lhs;
-    int32_t ud, s1, s2, pad0;
+    int32_t ud, s1, s2, list;                 // list: which voxel list is the slot's
     int64_t n, ind0, indf;
     double ang;                               // angle; slide: amplitude
-    int64_t picks[SPEC_NMAX];                 // tangent rotation beads
+    int32_t picks[SPEC_NMAX];                 // tangent rotation beads (31-bit draws)
     int32_t ps1[SPEC_NMAX], ps2[SPEC_NMAX];   // their unit-sphere draws
     int32_t newst[SPEC_NMAX];                 // binding: new states
     uint32_t ck[CK_WORDS];                    // RNG state before the proposal
@@ -57,17 +76,18 @@ struct SpecRes {
     double dEp, dEf, u, expdE;
     int32_t accepted, nbins, resample, overflow;
     int64_t rlo, rhi, wlo, whi;               // beads read [rlo, rhi], written [wlo, whi)
-    uint32_t cmask;                           // earlier slots whose writes this one reads
-    int32_t pad1;
 };
 
+// The launch's state, slots by their number in it (numbers wrap: compared by difference).
 struct SpecCtl {
-    int32_t cnt, remaining, err;
-    int32_t head;                             // ring position of the round's first slot
-    int32_t tag;                              // the round's number in the launch (never repeats)
-    int32_t stall;                            // = tag when a wait passed its bound
-    int32_t done[SPEC_EVMAX];                 // = tag once slot s's result and voxels are published
-    int32_t chk[SPEC_EVMAX];                  // = tag once slot s's conflict mask is set
+    uint32_t next;                            // next slot to take
+    uint32_t drawn;                           // slots before it are in the ring
+    uint32_t resolved;                        // slots before it are committed or rejected
+    int32_t back;                             // 1: slot back_at, then the first unresolved one, has to be
+    uint32_t back_at;                         //    redone one at a time
+    int32_t alone;                            // 1: the drawing wavefront runs a slot one at a time
+    int32_t stop, err;
+    int32_t idle[SPEC_EVMAX];                 // evaluating wavefront holds nothing in its block
 };
 
 // LDS exchange area of the one-at-a-time path (seq_step).
@@ -79,28 +99,28 @@ struct SeqIO {
 };
 
 struct SpecLayout {
-    size_t seg, seg_bytes, mt, slots, res, ctl, seq, total;
+    size_t seg_bytes, lists, mt, slots, res, ctl, seq, total;
 };
 
 // LDS: one evaluator block per evaluating wavefront (together they serve as the
-// one-at-a-time block), the MT19937 block, the slot ring, per-slot results, the
-// control words.
+// one-at-a-time block), the voxel lists, the MT19937 block, the slot ring, per-slot
+// results, the control words.
 template <int W>
 __host__ __device__ inline SpecLayout spec_layout(int Bp1)
 {
     SpecLayout S;
-    S.seg = 0;
-    S.seg_bytes = ev_layout(Bp1, false).total;
+    S.seg_bytes = ev_layout(Bp1, Shape<W>::ucap(Bp1)).total;
     size_t o = S.seg_bytes * (size_t)Shape<W>::EV;
+    S.lists = o;
+    o += sizeof(int2) * (size_t)(Shape<W>::LISTS * Shape<W>::ucap(Bp1));
     S.mt = o;
     o = align_up(o + MT_LDS_BYTES, 16);
     S.slots = o;
     o += sizeof(SpecSlot) * (size_t)Shape<W>::RING;
     S.res = o;
-    o += sizeof(SpecRes) * (size_t)Shape<W>::EV;
+    o += sizeof(SpecRes) * (size_t)Shape<W>::RING;
     S.ctl = o;
-    o += sizeof(SpecCtl);
-    o = align_up(o, 16);
+    o = align_up(o + sizeof(SpecCtl), 16);
     S.seq = o;
     o += sizeof(SeqIO);
     S.total = align_up(o, 256);
@@ -113,8 +133,10 @@ struct SpecLds {
     SpecCtl *ctl;
     SeqIO *seq;
     uint32_t *mt;
+    int2 *lists;
     char *blocks;   // the evaluator blocks
 };
+
 // A stream checkpoint in LDS: the glibc words and indices, and the Philox position
 // (counter, index in block; words 35-38 are not used: rng_restore needs the
 // position only).
@@ -266,7 +288,7 @@ __device__ __forceinline__ bool gen_fast(const chromo_replica *R, WaveRng &rng, 
     return true;
 }
 
-// Draws one proposal into slot S (wavefront 0), in the draw order of
+// Draws one proposal into slot S (the drawing wavefront), in the draw order of
 // mc_step_dev.  A proposal that is too large for one wavefront, or that fails,
 // is marked SLOT_SEQ with its draws given back: mc_step_dev redoes it.
 template <int NB>
@@ -337,7 +359,7 @@ __device__ __forceinline__ int gen_slot(const chromo_replica *R, WaveRng &rng, c
         int32_t fd1 = 0, fd2 = 0;
         if (!seq && tangent_draws_at_once(rng, k, N, fpick, fd1, fd2)) {
             if (lane < k) {
-                S.picks[lane] = fpick;
+                S.picks[lane] = (int32_t)fpick;
                 S.ps1[lane] = fd1;
                 S.ps2[lane] = fd2;
             }
@@ -357,7 +379,7 @@ __device__ __forceinline__ int gen_slot(const chromo_replica *R, WaveRng &rng, c
                     }
                 }
             }
-            if (lane < k) S.picks[lane] = mine;
+            if (lane < k) S.picks[lane] = (int32_t)mine;
             for (int64_t i = 0; i < k && !seq; ++i) {
                 int32_t a = rnd31(rng);
                 int32_t b = rnd31(rng);
@@ -439,11 +461,12 @@ __device__ __forceinline__ void seq_step(const chromo_replica *R, const EvConst 
     // the RNG goes back to LDS now, so that it is not held through the evaluation
     rng_save(rng, io->ck);
     if (lane == 0) io->mti = rng.mti;
-    const EvLds S = ev_lds(blocks, NB + 1, true);
+    const EvLds S = ev_lds(blocks, NB + 1, 0);
     ev_clear(S);
     if (go) mc_evaluate<NB, TW>(R, EC, C, o, P, u, S);
-    const size_t bytes = ev_layout(NB + 1, false).total;
-    for (int b = 0; b < Shape<W>::EV; ++b) ev_clear(ev_lds(blocks + bytes * b, NB + 1, false));
+    constexpr int U = Shape<W>::ucap(NB + 1);
+    const size_t bytes = ev_layout(NB + 1, U).total;
+    for (int b = 0; b < Shape<W>::EV; ++b) ev_clear(ev_lds(blocks + bytes * b, NB + 1, U));
     if (lane == 0) {
         io->C = C;
         io->out = o;
@@ -546,7 +569,6 @@ __device__ __forceinline__ int eval_slot(const chromo_replica *R, const EvConst 
     const int lane = lane_id();
     const int64_t ind0 = S.ind0, indf = S.indf;
     if (lane == 0) {
-        res.cmask = 0;
         res.resample = 0;
         res.overflow = 0;
         res.nbins = 0;
@@ -586,78 +608,63 @@ __device__ __forceinline__ int eval_slot(const chromo_replica *R, const EvConst 
     return sr.U;
 }
 
-template <int RING>
-__device__ __forceinline__ const SpecSlot &ring_at(const SpecSlot *ring, int head, int s)
-{
-    return ring[(head + s) & (RING - 1)];
-}
-
-// Whether slot s (its voxels numbered in block G, U of them) reads what the accepted
-// slot a < s of the round writes: a shared bead (tangent rotation: picks within one
-// bead of each other), or a shared voxel, looked up in a's own hash (block A).
-template <int RING>
-__device__ __forceinline__ bool spec_conflict(const SpecSlot *ring, int head, const SpecRes *res, const EvLds &G, int U,
-                                              int s, const EvLds &A, int a)
+// Whether slot S (result s, its voxels in the hash of block G) reads what the accepted
+// slot Q (result a, its voxels in list) wrote.  Beads: a window reads its beads and one
+// on either side, a tangent rotation its picks and their neighbours; a window writes its
+// beads, a tangent rotation its picks (tangents only, which binding moves do not read).
+// Voxels: Q's are looked up in S's hash.
+__device__ __forceinline__ bool spec_conflict(const SpecSlot &S, const SpecRes &s, const EvLds &G, const SpecSlot &Q,
+                                              const SpecRes &a, const int2 *list)
 {
     const int lane = lane_id();
-    const SpecSlot &S = ring_at<RING>(ring, head, s), &Q = ring_at<RING>(ring, head, a);
+    const bool st = S.move == CHROMO_TANGENT_ROTATION, qt = Q.move == CHROMO_TANGENT_ROTATION;
     bool hit = false;
-    if (S.move == CHROMO_TANGENT_ROTATION) {
+    if (st) {
         if (lane < S.n) {
             const int64_t mine = S.picks[lane];
-            for (int64_t q = 0; q < Q.n; ++q) {
-                const int64_t d = Q.picks[q] - mine;
-                hit |= d >= -1 && d <= 1;
+            if (qt) {
+                for (int q = 0; q < (int)Q.n; ++q) {
+                    const int64_t d = Q.picks[q] - mine;
+                    hit |= d >= -1 && d <= 1;
+                }
+            } else {
+                hit = mine >= a.wlo - 1 && mine <= a.whi;
             }
         }
+    } else if (qt) {
+        if (lane < Q.n) hit = Q.picks[lane] >= s.rlo && Q.picks[lane] <= s.rhi;
     } else {
-        hit = res[a].wlo <= res[s].rhi && res[s].rlo < res[a].whi;
-        if (res[a].nbins > 0)
-            for (int q = lane; q < U; q += WAVE) {
-                const int2 v = G.uv[q];
+        hit = a.wlo <= s.rhi && s.rlo < a.whi;
+        if (s.nbins > 0)
+            for (int q = lane; q < a.nbins; q += WAVE) {
+                const int2 v = list[q];
                 int h = (int)((uint32_t)v.y >> 16);
-                for (int probes = 0; probes < A.hsize; ++probes) {
-                    const int key = A.hkey[h];
+                for (int probes = 0; probes < G.hsize; ++probes) {
+                    const int key = G.hkey[h];
                     hit |= key == v.x;
                     if (key == v.x || key == HKEY_EMPTY) break;
-                    h = (h + 1) & (A.hsize - 1);
+                    h = (h + 1) & (G.hsize - 1);
                 }
             }
     }
     return wave_any(hit);
 }
 
-// The drawing wavefront: appends proposals to the queue of `q` slots starting at ring
-// position head until it holds `limit`, or `remaining` (the block's unresolved
-// proposals), or ends with a SLOT_SEQ one.  Returns the new queue length.
-template <int NB, int RING>
-__device__ __forceinline__ int spec_gen(const chromo_replica *R, WaveRng &rng, const chromo_ctrl &C, SpecSlot *ring,
-                                        int head, int q, int limit, int remaining)
-{
-    if (q >= limit || q >= remaining) return q;
-    bool stop = q > 0 && ring_at<RING>(ring, head, q - 1).kind == SLOT_SEQ;
-    while (!stop && q < limit && q < remaining) {
-        const int kind = gen_slot<NB>(R, rng, C, ring[(head + q) & (RING - 1)]);
-        ++q;
-        stop = kind == SLOT_SEQ;
-    }
-    return q;
-}
-
 // One wavefront: AcceptanceTracker updates (mc_stat.py:190-208), controller counts,
-// replica counters and log records of the resolved slots 0..F-1, one slot per
-// lane; the same totals as record() called once per slot in order.
+// replica counters and log records of the F resolved slots from number s0 on, one slot
+// per lane; the same totals as record() called once per slot in order.
 template <int RING>
 __device__ __forceinline__ void spec_book(const chromo_replica *R, chromo_ctrl &C, Counters &K,
-                                          const SpecSlot *ring, int head, const SpecRes *res, int F)
+                                          const SpecSlot *ring, const SpecRes *res, uint32_t s0, int F)
 {
     const int lane = lane_id();
-    const bool live = lane < F && ring_at<RING>(ring, head, lane < F ? lane : 0).kind != SLOT_EMPTY;
+    const int at_ring = (int)((s0 + (uint32_t)(lane < F ? lane : 0)) & (RING - 1));
+    const SpecSlot &S = ring[at_ring];
+    const SpecRes &q = res[at_ring];
+    const bool live = lane < F && S.kind != SLOT_EMPTY;
     int64_t n = 0, nb = 0, bytes = 0;
     int acc = 0, tie = 0;
     if (live) {
-        const SpecSlot &S = ring_at<RING>(ring, head, lane);
-        const SpecRes &q = res[lane];
         n = S.n;
         nb = q.nbins;
         acc = q.accepted;
@@ -667,15 +674,13 @@ __device__ __forceinline__ void spec_book(const chromo_replica *R, chromo_ctrl &
     const uint64_t live_m = __ballot(live);
     const uint64_t acc_m = __ballot(live && acc);
     const uint64_t tie_m = __ballot(live && tie);
-    static_assert(SPEC_EVMAX <= 8, "bookkeeping sums over the first eight lanes");
+    static_assert(RING <= 8, "bookkeeping sums over the first eight lanes");
     const int64_t sn = sum_lanes8_i64(n), sb = sum_lanes8_i64(nb), sy = sum_lanes8_i64(bytes);
     const int64_t logged = K.logged;
     const int nlive = __popcll(live_m);
     if (R->log != nullptr && live) {
         const int64_t at = logged + __popcll(live_m & ((1ull << lane) - 1));
         if (at < R->log_cap) {
-            const SpecSlot &S = ring_at<RING>(ring, head, lane);
-            const SpecRes &q = res[lane];
             chromo_move_log &Lg = R->log[at];
             Lg.move = S.move;
             Lg.accepted = q.accepted;
@@ -715,259 +720,351 @@ __device__ __forceinline__ void spec_book(const chromo_replica *R, chromo_ctrl &
     wave_sync();
 }
 
-// Raises a flag of the round for the other wavefronts: what this wavefront wrote to
-// LDS before is visible to who sees it.
-__device__ __forceinline__ void flag_raise(int32_t *f, int32_t tag)
+// Words of SpecCtl: what a wavefront wrote before it sets one is visible to who reads
+// it there.
+template <typename T>
+__device__ __forceinline__ void ctl_set(T *f, T v)
 {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-    if (lane_id() == 0) __hip_atomic_store(f, tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    if (lane_id() == 0) __hip_atomic_store(f, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-// Waits for a flag; false when it did not come within SPIN_LIMIT looks.
-__device__ __forceinline__ bool flag_wait(const int32_t *f, int32_t tag)
+template <typename T>
+__device__ __forceinline__ T ctl_get(const T *f)
 {
-    int spins = 0;
-    while (uni_i32(__hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) != tag)
-        if (++spins >= SPIN_LIMIT) break;
+    const T v = (T)uni_i32((int)__hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-    return spins < SPIN_LIMIT;
+    return v;
 }
 
-// One controller block.  C and K live in LDS: only the booking wavefront touches them
-// between two barriers, and keeping them out of registers leaves those to the
-// evaluation.
-//
-// A round, between two barriers:
-//  * wavefront s < cnt evaluates slot s and raises done[s]; slot 0 stands whatever the
-//    others do (nothing precedes it), so it is committed at once -- a later slot that
-//    reads what it writes is redone anyway;
-//  * slot s waits for done[a] of every a < s, looks its voxels and beads up in the
-//    accepted ones', and raises chk[s];
-//  * the drawing wavefront meanwhile draws the following proposals into the ring;
-//  * every wavefront resolves the slots it needs from the published results, in the
-//    same way: slot s commits if nothing before it ends the round.
-// A slot's hash is emptied at the start of its wavefront's next evaluation, when
-// nobody looks into it any more.  The flag waits are bounded; a wait that passes its
-// bound stops the replica with ERR_SPIN at the next round's top.
+// A wait's next look: false (and the replica's error) once it passed its bound.
+__device__ __forceinline__ bool spin_on(SpecCtl *ctl, int &spins)
+{
+    __builtin_amdgcn_s_sleep(1);
+    if (++spins < SPIN_LIMIT) return true;
+    ctl_set(&ctl->err, (int32_t)ERR_SPIN);
+    return false;
+}
+
+// A controller block of the launch: controller ci in step `step`, slots start .. start + n - 1.
+struct SpecBlock {
+    int64_t step;
+    int ci;
+    uint32_t start;
+    int n;
+};
+
+// What the drawing wavefront keeps.
+struct SpecGen {
+    WaveRng rng;
+    SpecBlock book, draw;       // the block being booked; the one being drawn: that one or the next
+    uint32_t drawn, booked;
+    int list;                   // voxel list of the last slot drawn
+    int64_t steps;
+    int nc;
+};
+
+// Moves b to the next controller that makes proposals; step = steps when there is none.
+__device__ __forceinline__ void block_next(SpecBlock &b, const chromo_ctrl *sctrl, int nc, int64_t steps)
+{
+    const uint32_t start = b.start + (uint32_t)b.n;
+    b.start = start;
+    b.n = 0;
+    while (b.step < steps) {
+        if (++b.ci >= nc) {
+            b.ci = 0;
+            if (++b.step >= steps) break;
+        }
+        if (sctrl[b.ci].on == 1 && sctrl[b.ci].num_per_cycle > 0) {
+            b.n = uni_i32(sctrl[b.ci].num_per_cycle);
+            break;
+        }
+    }
+}
+
+// The booked slots end a block: the amplitudes of its controller, and of the controllers
+// without proposals that follow, are updated.
+__device__ __forceinline__ void block_done(SpecGen &g, chromo_ctrl *sctrl)
+{
+    const int c0 = g.book.ci;
+    const int64_t s0 = g.book.step;
+    const bool same = g.draw.step == s0 && g.draw.ci == c0;
+    block_next(g.book, sctrl, g.nc, g.steps);
+    wave_sync();
+    if (lane_id() == 0) {
+        int64_t s = s0;
+        int c = c0;
+        while (s < g.book.step || (s == g.book.step && c < g.book.ci)) {
+            if (s >= g.steps) break;
+            update_amplitudes_dev(sctrl[c]);
+            if (++c >= g.nc) {
+                c = 0;
+                ++s;
+            }
+        }
+    }
+    wave_sync();
+    if (same) g.draw = g.book;
+}
+
+// The drawing wavefront's work that is at hand: books the resolved slots, runs the first
+// unresolved slot one at a time where that is needed (alone: only while this wavefront
+// holds nothing in a block), draws further slots.  True when there was something to do.
 template <int NB, int W, bool TW>
-__device__ __forceinline__ void spec_block(const chromo_replica *R, const EvConst &EC, WaveRng &rng, chromo_ctrl &C,
-                                           Counters &K, const SpecLds &L, int &held)
+__device__ __forceinline__ bool spec_serve(const chromo_replica *R, const EvConst &EC, SpecGen &g, chromo_ctrl *sctrl,
+                                           Counters &K, const SpecLds &L, bool alone)
 {
     using SH = Shape<W>;
-    constexpr int RING = SH::RING, EV = SH::EV, Bp1 = NB + 1;
-    static_assert((RING & (RING - 1)) == 0, "ring positions wrap by mask");
-    const int wv = wave_id(), lane = lane_id();
-    const size_t seg_bytes = ev_layout(Bp1, false).total;
-    const EvLds G = ev_lds(L.blocks + seg_bytes * (wv < EV ? wv : 0), Bp1, false);
-    SpecSlot *ring = L.ring;
-    // the drawing wavefront's
-    int head = 0;                      // ring position of the first queued slot
-    int nq = 0;                        // slots queued
-    int remaining = C.num_per_cycle;   // proposals of the block not yet resolved
-    int pend = 0;                      // error to publish before the next barrier
-    int32_t tag = uni_i32(L.ctl->tag); // the round's number in the launch
-    int64_t rounds = 0;
-    // every round resolves a proposal or turns its first slot into a sequential one
-    const int64_t max_rounds = 2 * (int64_t)C.num_per_cycle + 64;
-    // drawing ahead is off where a redone proposal would have to rewind MT19937
-    const bool ahead = !(rng.mode == CHROMO_RNG_GLIBC && C.move == CHROMO_CHANGE_BINDING_STATE);
-    for (;;) {
-        if (wv == SH::GEN) {
-            // L.ctl->err is written only here, before the barrier after which every
-            // wavefront reads it
-            if (++rounds > max_rounds) pend = ERR_SPIN;
-            if (uni_i32(L.ctl->stall) >= 0) pend = ERR_SPIN;
-            if (pend && lane == 0) L.ctl->err = pend;
-            if (!pend) {
-                tag += 1;
-                nq = spec_gen<NB, RING>(R, rng, C, ring, head, nq, EV, remaining);
-                const int nr = nq < EV ? nq : EV;
-                // leading slots that are not SLOT_SEQ, all kinds read at once
-                const int kd = lane < nr ? ring_at<RING>(ring, head, lane).kind : SLOT_SEQ;
-                const uint64_t seqm = __ballot(kd == SLOT_SEQ);
-                const int cnt = seqm ? (int)__builtin_ctzll(seqm) : nr;
-                if (lane == 0) {
-                    L.ctl->cnt = cnt;
-                    L.ctl->remaining = remaining;
-                    L.ctl->head = head;
-                    L.ctl->tag = tag;
-                }
-            }
-        }
-        __syncthreads();
-        if (L.ctl->err || L.ctl->remaining <= 0) break;
-        const int cnt = uni_i32(L.ctl->cnt), h = uni_i32(L.ctl->head);
-        if (ring_at<RING>(ring, h, 0).kind == SLOT_SEQ) {
-            held = 0;   // the one-at-a-time block lies over the slot blocks and leaves them empty
-            if (wv == SH::GEN) {
-                // the slot hashes may still hold the last round's voxels: seq_step clears
-                // what it uses, before and after
-                SeqIO *io = L.seq;
-                const SpecSlot &S0 = ring_at<RING>(ring, h, 0);
-                for (int i = lane; i < CK_WORDS; i += WAVE) io->ck[i] = S0.ck[i];
-                if (lane == 0) {
-                    io->mti = rng.mti;
-                    io->C = C;
-                }
-                wave_sync();
-                seq_step<NB, W, TW>(R, EC, io, L.mt, L.blocks);
-                rng_restore(rng, io->ck);
-                rng.mti = uni_i32(io->mti);
-                if (lane == 0) C = io->C;
-                wave_sync();
-                const MoveOut o = io->out;
-                if (o.err) {
-                    pend = o.err;
-                } else if (o.n > 0) {
-                    record(R, C, o, K);
-                }
-                remaining -= 1;
-                // nothing is drawn past a SLOT_SEQ slot
-                head = (head + 1) & (RING - 1);
-                nq = 0;
-            }
-        } else {
-            const int32_t now = uni_i32(L.ctl->tag);
-            const bool evaluates = wv < EV && wv < cnt;
-            const SpecSlot &mys = ring_at<RING>(ring, h, evaluates ? wv : 0);
-            const bool mine = evaluates && mys.kind == SLOT_SMALL;
-            bool stalled = false, committed = false;
-            EvKeep keep;
-            Proposal P;
-            if (mine) {
-                ev_release(G, held);
-                held = eval_slot<NB, TW>(R, EC, mys, L.res[wv], P, keep, G);
-            }
-            if (evaluates) flag_raise(&L.ctl->done[wv], now);
-            if (wv == 0 && mine && L.res[0].accepted && !L.res[0].resample && !L.res[0].overflow) {
-                ev_commit<NB>(R, P, keep, G, held);
-                committed = true;
-            }
-            if (evaluates && wv > 0) {
-                uint32_t m = 0;
-                const bool look = mine && !L.res[wv].resample && !L.res[wv].overflow;
-                for (int a = 0; a < wv; ++a) {
-                    if (!flag_wait(&L.ctl->done[a], now)) {
-                        stalled = true;
-                        break;
-                    }
-                    if (!look || ring_at<RING>(ring, h, a).kind != SLOT_SMALL) continue;
-                    const SpecRes &q = L.res[a];
-                    if (!q.accepted || q.resample || q.overflow) continue;
-                    if (spec_conflict<RING>(ring, h, L.res, G, held, wv, ev_lds(L.blocks + seg_bytes * a, Bp1, false), a))
-                        m |= 1u << a;
-                }
-                if (lane == 0) L.res[wv].cmask = m;
-                if (stalled && lane == 0) L.ctl->stall = now;
-                flag_raise(&L.ctl->chk[wv], now);
-            }
-            // the following proposals
-            if (wv == SH::GEN && ahead && !pend) nq = spec_gen<NB, RING>(R, rng, C, ring, head, nq, RING, remaining);
-            // the results this wavefront resolves: all for the drawing and booking ones,
-            // the slots before its own for the others
-            const bool all = wv == SH::GEN || wv == SH::BOOK;
-            const int upto = all ? cnt : (evaluates ? wv + 1 : 0);
-            if (upto > 0 && !evaluates) stalled |= !flag_wait(&L.ctl->done[0], now);
-            for (int s = 1; s < upto; ++s)
-                if (s != wv) stalled |= !flag_wait(&L.ctl->chk[s], now);
-            if (stalled && lane == 0) L.ctl->stall = now;
-            // resolution, identical in every wavefront; lane s reads slot s's result,
-            // all slots in one LDS round trip
-            uint32_t kd = SLOT_EMPTY, cmk = 0, ov = 0, rs = 0, ac = 0;
-            if (lane < upto) {
-                const SpecRes &q = L.res[lane];
-                kd = (uint32_t)ring_at<RING>(ring, h, lane).kind;
-                cmk = q.cmask;
-                ov = (uint32_t)q.overflow;
-                rs = (uint32_t)q.resample;
-                ac = (uint32_t)q.accepted;
-            }
-            int F = upto, rew = 0;
-            uint32_t accm = 0;
-            for (int s = 0; s < upto; ++s) {
-                if ((int)readlane_u32(kd, s) == SLOT_EMPTY) continue;
-                const uint32_t q_cmask = readlane_u32(cmk, s), q_overflow = readlane_u32(ov, s);
-                if (q_cmask & accm) {
-                    F = s;
-                    break;
-                }
-                // an axis to be drawn again, or more voxels than a block holds: the
-                // sequential path redoes it
-                if (readlane_u32(rs, s) || q_overflow) {
-                    F = s;
-                    rew = 1;
-                    break;
-                }
-                if (readlane_u32(ac, s)) accm |= 1u << s;
-            }
-            if (mine && !committed && wv < F && L.res[wv].accepted) ev_commit<NB>(R, P, keep, G, held);
-            // only the barrier below orders C and K for the next reader
-            if (wv == SH::BOOK) spec_book<RING>(R, C, K, ring, h, L.res, F);
-            if (wv == SH::GEN) {
-                if (rew) {
-                    // slot F is redone one at a time; what was drawn after it is
-                    // dropped (the sequential path rewinds the streams to it)
-                    if (lane == 0) ring[(head + F) & (RING - 1)].kind = SLOT_SEQ;
-                    nq = F + 1;
-                }
-                head = (head + F) & (RING - 1);
-                nq -= F;
-                remaining -= F;
-            }
-        }
-        __syncthreads();
+    constexpr int RING = SH::RING;
+    SpecCtl *ctl = L.ctl;
+    const int lane = lane_id();
+    bool did = false;
+    const uint32_t r = ctl_get(&ctl->resolved);
+    while (g.booked != r) {
+        const int left = g.book.n - (int)(g.booked - g.book.start), have = (int)(r - g.booked);
+        const int F = have < left ? have : left;
+        spec_book<RING>(R, sctrl[g.book.ci], K, L.ring, L.res, g.booked, F);
+        g.booked += (uint32_t)F;
+        if (F == left) block_done(g, sctrl);
+        did = true;
     }
+    if (g.book.step >= g.steps) {
+        ctl_set(&ctl->stop, 1);
+        return true;
+    }
+    // (a slot given back after r was read is a later one: left to the next call)
+    if (r != g.drawn &&
+        (L.ring[r & (RING - 1)].kind == SLOT_SEQ || (ctl_get(&ctl->back) && ctl_get(&ctl->back_at) == r))) {
+        if (!alone) return did;
+        // what was drawn after slot r is dropped, and drawn again after it: the wavefronts
+        // that evaluate it fall back to waiting for it
+        if (g.drawn != r + 1) {
+            g.drawn = r + 1;
+            g.draw = g.book;
+            g.list = uni_i32(L.ring[r & (RING - 1)].list);
+            ctl_set(&ctl->drawn, g.drawn);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+        for (int w = 0; w < SH::EV; ++w)
+            if (!ctl_get(&ctl->idle[w])) return did;
+        SeqIO *io = L.seq;
+        const SpecSlot &S0 = L.ring[r & (RING - 1)];
+        chromo_ctrl &C = sctrl[g.book.ci];
+        for (int i = lane; i < CK_WORDS; i += WAVE) io->ck[i] = S0.ck[i];
+        if (lane == 0) {
+            io->mti = g.rng.mti;
+            io->C = C;
+        }
+        wave_sync();
+        ctl_set(&ctl->alone, 1);
+        seq_step<NB, W, TW>(R, EC, io, L.mt, L.blocks);
+        rng_restore(g.rng, io->ck);
+        g.rng.mti = uni_i32(io->mti);
+        if (lane == 0) C = io->C;
+        wave_sync();
+        const MoveOut o = io->out;
+        if (o.err) {
+            ctl_set(&ctl->err, (int32_t)o.err);
+            return true;
+        }
+        if (o.n > 0) record(R, C, o, K);
+        wave_sync_global();
+        g.booked = r + 1;
+        // in this order: who holds number r goes on before anything may start again
+        ctl_set(&ctl->resolved, r + 1);
+        ctl_set(&ctl->back, 0);
+        ctl_set(&ctl->alone, 0);
+        if (g.booked - g.book.start == (uint32_t)g.book.n) block_done(g, sctrl);
+        if (g.book.step >= g.steps) ctl_set(&ctl->stop, 1);
+        return true;
+    }
+    // nothing is drawn past a SLOT_SEQ slot
+    if (g.drawn != r && L.ring[(g.drawn - 1) & (RING - 1)].kind == SLOT_SEQ) return did;
+    while ((int)(g.drawn - r) < SH::AHEAD) {
+        if (g.drawn - g.draw.start == (uint32_t)g.draw.n) {
+            // the next block, one ahead of the booked one, unless its controller's
+            // amplitudes still depend on that one
+            if (g.draw.start != g.book.start) break;
+            SpecBlock b = g.draw;
+            block_next(b, sctrl, g.nc, g.steps);
+            if (b.step >= g.steps || b.ci == g.book.ci) break;
+            g.draw = b;
+        }
+        const chromo_ctrl &C = sctrl[g.draw.ci];
+        // MT19937 is not rewound: no binding slot is drawn behind one that may be given back
+        if (g.rng.mode == CHROMO_RNG_GLIBC && C.move == CHROMO_CHANGE_BINDING_STATE && (int)(r - g.draw.start) < 0) break;
+        SpecSlot &S = L.ring[g.drawn & (RING - 1)];
+        const int kind = gen_slot<NB>(R, g.rng, C, S);
+        g.list = g.list + 1 == SH::LISTS ? 0 : g.list + 1;
+        if (lane == 0) S.list = g.list;
+        g.drawn += 1;
+        ctl_set(&ctl->drawn, g.drawn);
+        did = true;
+        if (kind == SLOT_SEQ) break;
+    }
+    return did;
 }
 
 template <int NB, int W, bool TW>
 __device__ __forceinline__ void spec_run(const chromo_replica *R, const EvConst &EC, int64_t steps)
 {
     using SH = Shape<W>;
-    constexpr int Bp1 = NB + 1;
+    constexpr int Bp1 = NB + 1, RING = SH::RING, EV = SH::EV, U = SH::ucap(Bp1);
+    static_assert((RING & (RING - 1)) == 0 && RING > SH::AHEAD, "ring positions wrap by mask");
+    static_assert(U * Bp1 * 8 < 65536, "byte offsets of the deltas fit 16 bits");
     const SpecLayout SL = spec_layout<W>(Bp1);
     const int wv = wave_id(), lane = lane_id();
     SpecLds L;
-    L.blocks = lds_dyn + SL.seg;
+    L.blocks = lds_dyn;
+    L.lists = (int2 *)(lds_dyn + SL.lists);
     L.ring = (SpecSlot *)(lds_dyn + SL.slots);
     L.res = (SpecRes *)(lds_dyn + SL.res);
     L.ctl = (SpecCtl *)(lds_dyn + SL.ctl);
     L.seq = (SeqIO *)(lds_dyn + SL.seq);
     L.mt = (uint32_t *)(lds_dyn + SL.mt);
-    if (wv < SH::EV) ev_clear(ev_lds(L.blocks + SL.seg_bytes * wv, Bp1, false));
+    EvLds G = ev_lds(L.blocks + SL.seg_bytes * (wv < EV ? wv : 0), Bp1, U);
+    if (wv < EV) ev_clear(G);
     __shared__ chromo_ctrl sctrl[MAX_CTRL];
     __shared__ Counters sK;
-    const int nc = R->n_ctrl < MAX_CTRL ? R->n_ctrl : MAX_CTRL;
-    WaveRng rng;
-    rng.mode = uni_i32(R->rng_mode);
+    SpecCtl *ctl = L.ctl;
+    const bool gen = wv == SH::GEN;
+    constexpr bool DRAWS = SH::GEN < EV;   // an evaluating wavefront draws
     bool need_mt = false;
-    if (wv == SH::GEN) {
+    SpecGen g;
+    g.rng.mode = uni_i32(R->rng_mode);
+    g.nc = R->n_ctrl < MAX_CTRL ? R->n_ctrl : MAX_CTRL;
+    g.steps = steps;
+    g.drawn = g.booked = 0;
+    g.list = SH::LISTS - 1;
+    if (gen) {
         need_mt = any_binding(R);
-        rng_load(R, rng, L.mt, need_mt);
+        rng_load(R, g.rng, L.mt, need_mt);
         if (lane == 0) {
             counters_load(R, sK);
-            for (int i = 0; i < nc; ++i) sctrl[i] = R->ctrl[i];
-            L.ctl->err = 0;
-            L.ctl->tag = 0;
-            L.ctl->stall = -1;
-            for (int s = 0; s < SPEC_EVMAX; ++s) L.ctl->done[s] = L.ctl->chk[s] = -1;
+            for (int i = 0; i < g.nc; ++i) sctrl[i] = R->ctrl[i];
+            ctl->next = ctl->drawn = ctl->resolved = 0;
+            ctl->back = ctl->alone = ctl->stop = ctl->err = 0;
+            for (int w = 0; w < SPEC_EVMAX; ++w) ctl->idle[w] = 1;
+        }
+        wave_sync();
+        // the controllers before the first with proposals are updated like the others
+        g.book = SpecBlock{0, 0, 0, 0};
+        if (g.nc < 1 || steps < 1) g.book.step = steps;
+        else if (sctrl[0].on == 1 && sctrl[0].num_per_cycle > 0) g.book.n = uni_i32(sctrl[0].num_per_cycle);
+        g.draw = g.book;
+        if (g.book.step < steps && g.book.n == 0) block_done(g, sctrl);
+    }
+    __syncthreads();
+    if (wv >= EV) {
+        // draws and books only
+        int spins = 0;
+        while (!ctl_get(&ctl->stop) && !ctl_get(&ctl->err)) {
+            if (spec_serve<NB, W, TW>(R, EC, g, sctrl, sK, L, true)) spins = 0;
+            else if (!spin_on(ctl, spins)) break;
+        }
+    } else {
+        uint32_t t = 0;
+        bool have = false;   // holds number t
+        for (;;) {
+            // take a number, wait for its slot
+            if (!have) {
+                uint32_t v = 0;
+                if (lane == 0) v = atomicAdd(&ctl->next, 1u);
+                t = uni_u32(v);
+                have = true;
+            }
+            SpecSlot &S = L.ring[t & (RING - 1)];
+            bool go = false;
+            for (int spins = 0;;) {
+                if (ctl_get(&ctl->stop) || ctl_get(&ctl->err)) break;
+                if ((int)(ctl_get(&ctl->resolved) - t) > 0) {
+                    have = false;   // it was run one at a time
+                    break;
+                }
+                if ((int)(ctl_get(&ctl->drawn) - t) > 0 && S.kind != SLOT_SEQ && !ctl_get(&ctl->back)) {
+                    // no longer idle, unless the slot was dropped meanwhile, or run one at
+                    // a time between the looks above (`back` falls after `resolved` rises)
+                    ctl_set(&ctl->idle[wv], 0);
+                    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+                    if ((int)(ctl_get(&ctl->drawn) - t) > 0 && !ctl_get(&ctl->back) &&
+                        (int)(ctl_get(&ctl->resolved) - t) <= 0) {
+                        go = true;
+                        break;
+                    }
+                    ctl_set(&ctl->idle[wv], 1);
+                }
+                if (DRAWS && gen) {
+                    if (spec_serve<NB, W, TW>(R, EC, g, sctrl, sK, L, true)) {
+                        spins = 0;
+                        continue;
+                    }
+                }
+                // a slot run one at a time may be of any length
+                if (ctl_get(&ctl->alone)) spins = 0;
+                if (!spin_on(ctl, spins)) break;
+            }
+            if (!have) continue;
+            if (!go) break;
+            SpecRes &res = L.res[t & (RING - 1)];
+            G.uv = L.lists + U * uni_i32(S.list);
+            EvKeep keep;
+            Proposal P;
+            int held = 0;
+            bool turn = false, again = true;
+            uint32_t seen = ctl_get(&ctl->resolved);   // earlier slots up to here are committed or rejected
+            while (again) {
+                again = false;
+                ev_release(G, held);
+                held = 0;
+                if (S.kind == SLOT_SMALL) held = eval_slot<NB, TW>(R, EC, S, res, P, keep, G);
+                for (int spins = 0;;) {
+                    if (ctl_get(&ctl->err)) break;
+                    const uint32_t r = ctl_get(&ctl->resolved);
+                    bool hit = false;
+                    for (; seen != r; ++seen) {
+                        const SpecSlot &Q = L.ring[seen & (RING - 1)];
+                        const SpecRes &q = L.res[seen & (RING - 1)];
+                        if (!hit && S.kind == SLOT_SMALL && Q.kind == SLOT_SMALL && q.accepted)
+                            hit = spec_conflict(S, res, G, Q, q, L.lists + U * uni_i32(Q.list));
+                        spins = 0;
+                    }
+                    if (hit) {
+                        again = true;
+                        break;
+                    }
+                    if (r == t) {
+                        turn = true;
+                        break;
+                    }
+                    if ((int)(ctl_get(&ctl->drawn) - t) <= 0) break;   // dropped
+                    if (DRAWS && gen) {
+                        if (ctl_get(&ctl->back)) break;                // to be dropped, by this wavefront
+                        if (spec_serve<NB, W, TW>(R, EC, g, sctrl, sK, L, false)) continue;
+                    }
+                    if (!spin_on(ctl, spins)) break;
+                }
+            }
+            if (turn && S.kind == SLOT_SMALL && (res.resample || res.overflow)) {
+                // an axis to be drawn again, or more voxels than the block holds
+                if (lane == 0) ctl->back_at = t;
+                ctl_set(&ctl->back, 1);
+                turn = false;
+            }
+            if (turn) {
+                if (S.kind == SLOT_SMALL && res.accepted) ev_commit<NB>(R, P, keep, G, held);
+                ctl_set(&ctl->resolved, t + 1);
+                have = false;
+            }
+            ev_release(G, held);
+            ctl_set(&ctl->idle[wv], 1);
         }
     }
     __syncthreads();
-    int held = 0;   // voxels in this wavefront's hash
-    for (int64_t s = 0; s < steps; ++s) {
-        for (int ci = 0; ci < nc; ++ci) {
-            if (sctrl[ci].on == 1) spec_block<NB, W, TW>(R, EC, rng, sctrl[ci], sK, L, held);
-            if (wv == 0 && lane == 0 && !L.ctl->err) update_amplitudes_dev(sctrl[ci]);
-            __syncthreads();
-            if (L.ctl->err) break;
-        }
-        if (L.ctl->err) break;
-    }
-    if (wv == SH::GEN) {
-        rng_store(R, rng, need_mt);
+    if (gen) {
+        rng_store(R, g.rng, need_mt);
         if (lane == 0)
-            for (int i = 0; i < nc; ++i) R->ctrl[i] = sctrl[i];
-        counters_store(R, sK, L.ctl->err);
+            for (int i = 0; i < g.nc; ++i) R->ctrl[i] = sctrl[i];
+        counters_store(R, sK, ctl->err);
     }
 }
 

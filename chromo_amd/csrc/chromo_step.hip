@@ -26,7 +26,7 @@ __global__ void __launch_bounds__(64) k_mc_run(const chromo_replica *__restrict_
     }
     const int Bp1 = R->B + 1;
     ev_const(&EC, R);
-    const EvLds S = ev_lds(lds_dyn, Bp1, true);
+    const EvLds S = ev_lds(lds_dyn, Bp1, 0);
     ev_clear(S);
     uint32_t *mt_lds = (uint32_t *)(lds_dyn + wide_lds_bytes(Bp1));
     const bool need_mt = any_binding(R);
@@ -84,7 +84,7 @@ __global__ void __launch_bounds__(64) k_mc_step(const chromo_replica *__restrict
     WaveRng rng;
     rng_load(R, rng, mt_lds, need_mt);
     ev_const(&EC, R);
-    const EvLds S = ev_lds(lds_dyn, Bp1, true);
+    const EvLds S = ev_lds(lds_dyn, Bp1, 0);
     ev_clear(S);
     if (failed != 0) return;
     if (R->B < 1 || R->B + 1 > max_bp1) {
