@@ -435,6 +435,15 @@ __device__ __forceinline__ void mt_twist(uint32_t *mt)
     }
 }
 
+__device__ __forceinline__ uint32_t mt_temper(uint32_t y)
+{
+    y ^= y >> 11;
+    y ^= (y << 7) & 0x9d2c5680u;
+    y ^= (y << 15) & 0xefc60000u;
+    y ^= y >> 18;
+    return y;
+}
+
 __device__ __forceinline__ uint32_t mt_draw(WaveRng &R)
 {
     R.mti = uni_i32(R.mti);
@@ -442,12 +451,7 @@ __device__ __forceinline__ uint32_t mt_draw(WaveRng &R)
         mt_twist(R.mt);
         R.mti = 0;
     }
-    uint32_t y = uni_u32(R.mt[R.mti++]);
-    y ^= y >> 11;
-    y ^= (y << 7) & 0x9d2c5680u;
-    y ^= (y << 15) & 0xefc60000u;
-    y ^= y >> 18;
-    return y;
+    return mt_temper(uni_u32(R.mt[R.mti++]));
 }
 
 __device__ __forceinline__ int32_t rnd31(WaveRng &R)

@@ -1,6 +1,8 @@
 // chromo_spec.hpp -- device code of the speculative persistent kernel.
 #pragma once
 
+#include <cstddef>
+
 #include "chromo_mc.hpp"
 
 namespace {
@@ -36,30 +38,35 @@ struct Shape {
     static_assert(W == 2 || W == 4, "two or four wavefronts");
     static constexpr int EV = W == 2 ? 2 : 3;       // evaluating wavefronts
     static constexpr int GEN = W == 2 ? 0 : 3;      // the wavefront that draws and books
-    static constexpr int RING = 8;                  // slots
-    // Slots drawn past the first unresolved one, at most: slot d takes the place of slot
-    // d - RING, which a slot in flight (numbers below first + EV) may still look at when
-    // it is among the EV - 1 before that one.
-    static constexpr int AHEAD = RING - EV + 1;
+    static constexpr int RING = W == 2 ? 8 : 16;    // slots
+    // Slots drawn past the first unresolved one, at most, and slots resolved but not yet
+    // booked.  Slot d takes the place of slot d - RING, which has to be booked, and which a
+    // slot in flight (numbers below first + EV) may still look at when it is among the
+    // EV - 1 before that one.
+    static constexpr int AHEAD = W == 2 ? 6 : 8;
+    static_assert(AHEAD <= RING - EV + 1, "no slot is overwritten while it is looked at");
     // Voxel lists: slot a's is looked at by the next EV - 1 slots, which can be in flight
     // together with the EV - 1 after them.
     static constexpr int LISTS = 2 * EV - 1;
     // Voxels of a block: two workgroups on a compute unit, or one.
     __host__ __device__ static constexpr int ucap(int Bp1)
     {
-        return W == 2 ? (Bp1 <= 2 ? 640 : (Bp1 == 3 ? 560 : (Bp1 == 4 ? 448 : 384)))
-                      : (Bp1 <= 4 ? 704 : 640);
+        return W == 2 ? (Bp1 <= 2 ? 640 : (Bp1 == 3 ? 528 : (Bp1 == 4 ? 432 : 368)))
+                      : (Bp1 <= 4 ? 704 : 576);
     }
 };
 
 constexpr int SPEC_NMAX = SEG_MAX;    // tangent picks or binding beads of a slot
 constexpr int SPEC_BEADS = 192;       // beads of a crank-shaft, end-pivot or slide slot
 constexpr int SPEC_EVMAX = 3;
+constexpr int CTL_WORDS = 16;
 enum : int { SLOT_SMALL = 0, SLOT_EMPTY = 1, SLOT_SEQ = 2 };
 constexpr int CK_WORDS = 40;
+constexpr int GLIBC_BLOCKS = 4;                       // 31-word blocks of the additive generator drawn ahead, at most
+constexpr int GLIBC_BUF = 31 * (GLIBC_BLOCKS + 1);    // its state, oldest word first, then the blocks
 // a binding slot always fits a block: it is never given back (its MT19937 draws could
 // not be)
-static_assert(8 * SPEC_NMAX <= 384, "voxels of a binding slot");
+static_assert(8 * SPEC_NMAX <= 368, "voxels of a binding slot");
 
 struct SpecSlot {
     int32_t kind, move, binder, lhs;
@@ -88,7 +95,9 @@ struct SpecCtl {
     int32_t alone;                            // 1: the drawing wavefront runs a slot one at a time
     int32_t stop, err;
     int32_t idle[SPEC_EVMAX];                 // evaluating wavefront holds nothing in its block
+    int32_t pad[CTL_WORDS - 8 - SPEC_EVMAX];
 };
+static_assert(sizeof(SpecCtl) == 4 * CTL_WORDS, "ctl_look reads it whole");
 
 // LDS exchange area of the one-at-a-time path (seq_step).
 struct SeqIO {
@@ -96,6 +105,7 @@ struct SeqIO {
     int32_t mti, pad0;
     chromo_ctrl C;
     MoveOut out;
+    uint32_t words[GLIBC_BUF + 1];   // gen_batch's
 };
 
 struct SpecLayout {
@@ -137,36 +147,43 @@ struct SpecLds {
     char *blocks;   // the evaluator blocks
 };
 
-// A stream checkpoint in LDS: the glibc words and indices, and the Philox position
-// (counter, index in block; words 35-38 are not used: rng_restore needs the
-// position only).
+// A stream checkpoint in LDS: the additive generator's words and indices, or the Philox
+// position (words 33 and 34 the counter, 39 the index in its block: all rng_restore needs).
 __device__ __forceinline__ void rng_save(const WaveRng &g, uint32_t *ck)
 {
     const int lane = lane_id();
-    uint64_t ctr = 0;
-    int bi = 4;
-    if (g.mode == CHROMO_RNG_PHILOX) philox_pos(g, ctr, bi);
-    if (lane < 31) ck[lane] = g.g;
-    if (lane == 0) {
-        ck[31] = (uint32_t)g.gf;
-        ck[32] = (uint32_t)g.gr;
-        ck[33] = (uint32_t)ctr;
-        ck[34] = (uint32_t)(ctr >> 32);
-        ck[39] = (uint32_t)bi;
+    if (g.mode == CHROMO_RNG_PHILOX) {
+        uint64_t ctr = 0;
+        int bi = 4;
+        philox_pos(g, ctr, bi);
+        if (lane == 0) {
+            ck[33] = (uint32_t)ctr;
+            ck[34] = (uint32_t)(ctr >> 32);
+            ck[39] = (uint32_t)bi;
+        }
+    } else {
+        if (lane < 31) ck[lane] = g.g;
+        if (lane == 0) {
+            ck[31] = (uint32_t)g.gf;
+            ck[32] = (uint32_t)g.gr;
+        }
     }
     wave_sync();
 }
 
-// Restores the glibc and Philox streams (the MT19937 stream is never rewound:
-// no proposal that is redone consumed MT19937 draws).
+// Restores the stream (MT19937 is never rewound: no proposal that is redone consumed
+// MT19937 draws).
 __device__ __forceinline__ void rng_restore(WaveRng &g, const uint32_t *ck)
 {
     wave_sync();
     const int lane = lane_id();
-    g.g = lane < 31 ? ck[lane] : 0u;
-    g.gf = uni_i32((int)ck[31]);
-    g.gr = uni_i32((int)ck[32]);
-    if (g.mode == CHROMO_RNG_PHILOX) philox_set(g, (uint64_t)ck[33] | ((uint64_t)ck[34] << 32), (int)ck[39]);
+    if (g.mode == CHROMO_RNG_PHILOX) {
+        philox_set(g, (uint64_t)ck[33] | ((uint64_t)ck[34] << 32), (int)ck[39]);
+    } else {
+        g.g = lane < 31 ? ck[lane] : 0u;
+        g.gf = uni_i32((int)ck[31]);
+        g.gr = uni_i32((int)ck[32]);
+    }
 }
 
 // capped_exponential (bead_selection.pyx:19-66) with the one draw x: ok is
@@ -208,84 +225,248 @@ __device__ __forceinline__ bool slot_holds(const chromo_replica *R, int64_t n)
     return n <= SEG_MAX || (n <= SPEC_BEADS && n <= R->bead_cap && (!R->field_on || n <= R->seg_cap));
 }
 
-// Philox, crank-shaft / end-pivot / slide: the usual proposal -- every capped
-// exponential accepted at its first draw, a window that a slot holds, no extra
-// axis draws -- from the next eight words of the batch, read in one LDS round
-// trip instead of one per draw.  The same words, in the same order and with the
-// same arithmetic, as gen_slot's draw-at-a-time code.  Consumes nothing and returns
-// false for any other case, which gen_slot then draws one word at a time.
-template <int NB>
-__device__ __forceinline__ bool gen_fast(const chromo_replica *R, WaveRng &rng, const chromo_ctrl &C, SpecSlot &S)
+// The next words of the stream in LDS, in order, as the draw functions would take them
+// (a draw is a word >> 1): Philox words of the batch, or, computed ahead into buf, the
+// reference's additive generator x[n] = x[n - 31] + x[n - 3].  Nothing is consumed.
+struct RngWords {
+    const uint32_t *w;
+    int avail;
+};
+
+// `blocks`: 31-word blocks of the additive generator.  A block is three sums in steps of
+// three: lanes 16 c + t hold word 3 t + c, and a scan over the 16 lanes of a row adds them
+// up -- four adds for 31 words, which cost ~100 cycles each drawn one by one.
+__device__ __forceinline__ RngWords rng_words(WaveRng &g, uint32_t *buf, int blocks)
 {
-    const int mv = C.move;
-    if (rng.mode != CHROMO_RNG_PHILOX ||
-        (mv != CHROMO_CRANK_SHAFT && mv != CHROMO_END_PIVOT && mv != CHROMO_SLIDE))
-        return false;
-    const int p = uni_i32(rng.pidx);
-    if (p + 8 > 4 * WAVE) return false;
-    int32_t d[8];
-#pragma unroll
-    for (int t = 0; t < 8; ++t) d[t] = (int32_t)(uni_u32(rng.mt[p + t]) >> 1);
+    if (g.mode == CHROMO_RNG_PHILOX) {
+        g.pidx = uni_i32(g.pidx);
+        // near the batch's end: the batch again from the current block on
+        if (g.pidx > 4 * WAVE - 128) {
+            philox_fill(g, g.pbase + (uint64_t)(g.pidx >> 2));
+            g.pidx &= 3;
+        }
+        return RngWords{g.mt + g.pidx, 4 * WAVE - g.pidx};
+    }
+    const int lane = lane_id();
+    wave_sync();
+    if (lane < 31) {
+        const int i = lane - g.gf;
+        buf[i < 0 ? i + 31 : i] = g.g;
+    }
+    wave_sync();
+    const int c = lane >> 4, t = lane & 15, i = 3 * t + c;
+    const bool in = c < 3 && i < 31;
+    for (int b = 0; b < blocks; ++b) {
+        const uint32_t *s = buf + 31 * b;
+        int x = in ? (int)(s[i] + (t == 0 ? s[28 + c] : 0u)) : 0;
+        x += dpp_i32<DPP_SHR1>(x);
+        x += dpp_i32<DPP_SHR2>(x);
+        x += dpp_i32<DPP_SHR4>(x);
+        x += dpp_i32<DPP_SHR8>(x);
+        if (in) buf[31 * (b + 1) + i] = (uint32_t)x;
+        wave_sync();
+    }
+    return RngWords{buf + 31, 31 * blocks};
+}
+
+// The stream's checkpoint m words on (rng_save's form, of the words in v).
+__device__ __forceinline__ void rng_mark(const WaveRng &g, const RngWords &v, int m, uint32_t *ck)
+{
+    const int lane = lane_id();
+    if (g.mode == CHROMO_RNG_PHILOX) {
+        WaveRng q = g;
+        q.pidx = g.pidx + m;
+        uint64_t ctr;
+        int bi;
+        philox_pos(q, ctr, bi);
+        if (lane == 0) {
+            ck[33] = (uint32_t)ctr;
+            ck[34] = (uint32_t)(ctr >> 32);
+            ck[39] = (uint32_t)bi;
+        }
+        return;
+    }
+    const int gf = (g.gf + m) % 31, i = lane - gf;
+    if (lane < 31) ck[lane] = v.w[m - 31 + (i < 0 ? i + 31 : i)];
+    if (lane == 0) {
+        ck[31] = (uint32_t)gf;
+        ck[32] = (uint32_t)((g.gr + m) % 31);
+    }
+}
+
+// Consumes m of the words in v.
+__device__ __forceinline__ void rng_take(WaveRng &g, const RngWords &v, int m)
+{
+    if (g.mode == CHROMO_RNG_PHILOX) {
+        g.pidx += m;
+        return;
+    }
+    const int lane = lane_id();
+    g.gf = (g.gf + m) % 31;
+    g.gr = (g.gr + m) % 31;
+    const int i = lane - g.gf;
+    if (lane < 31) g.g = v.w[m - 31 + (i < 0 ? i + 31 : i)];
+}
+
+// The usual proposals of controller C, drawn into the ring from slot number at on: up to
+// `room` crank-shafts, end pivots or slides at once, one per lane, or one tangent rotation
+// or binding move, its beads one per lane.  The same words, in the same order and with
+// the same arithmetic, as gen_slot's draw-at-a-time code.  Returns the slots drawn; none,
+// and nothing consumed, where the first proposal is not a usual one (a capped
+// exponential drawn again, a bead picked twice, extra axis draws, a window that a slot
+// does not hold, MT19937 to be regenerated): gen_slot then draws it one word at a time.
+// Drawn one by one a slot cost the drawing wavefront about 5,000 cycles, most of them
+// the latency of the exponential's logarithm and of one draw after the other.
+template <int NB, int RING>
+__device__ __forceinline__ int gen_batch(const chromo_replica *R, WaveRng &rng, const chromo_ctrl &C, SpecSlot *ring,
+                                         uint32_t at, int room, uint32_t *buf)
+{
+    const int lane = lane_id();
+    const int mv = uni_i32(C.move);
     const int64_t N = R->N;
     const double amp_move = C.amp_move;
     const int64_t amp_bead = C.amp_bead;
-    bool ok = true;
-    int used = 0;
-    int64_t ind0 = 0, indf = 0;
-    double ang = 0;
-    int32_t s1 = 0, s2 = 0, lhs = 0, ud = 0;
-    if (mv == CHROMO_CRANK_SHAFT) {
-        ang = amp_move * (((double)d[0] / RMAX) - 0.5);
-        const int64_t b0 = (int64_t)(int32_t)(((double)d[1] / RMAX) * (double)N);
-        const int64_t b1 = imax64(from_point_once(d[2], d[3], amp_bead, N, b0, ok), 1);
-        check_bead_bounds(b0, b1, N, ind0, indf);
-        ud = d[4];
-        used = 5;
-    } else if (mv == CHROMO_END_PIVOT) {
-        ang = amp_move * (((double)d[0] / RMAX) - 0.5);
-        lhs = (int32_t)(d[1] & 1);
-        if (amp_bead > N) ok = false;
-        const int64_t r = cexp_once(d[2], amp_bead, amp_bead, ok);
-        if (lhs == 1) {
-            ind0 = 0;
-            indf = r + 1;
+    const RngWords v = rng_words(rng, buf, mv == CHROMO_TANGENT_ROTATION ? GLIBC_BLOCKS : 1);
+    if (mv == CHROMO_CRANK_SHAFT || mv == CHROMO_END_PIVOT || mv == CHROMO_SLIDE) {
+        const int used = mv == CHROMO_CRANK_SHAFT ? 5 : (mv == CHROMO_END_PIVOT ? 6 : 7);
+        const int most = v.avail / used < room ? v.avail / used : room;
+        const bool in = lane < most;
+        int32_t d[7];
+#pragma unroll
+        for (int t = 0; t < 7; ++t) d[t] = (int32_t)(v.w[in && t < used ? used * lane + t : 0] >> 1);
+        bool ok = in;
+        int64_t ind0 = 0, indf = 0;
+        double ang = 0;
+        int32_t s1 = 0, s2 = 0, lhs = 0, ud = 0;
+        if (mv == CHROMO_CRANK_SHAFT) {
+            ang = amp_move * (((double)d[0] / RMAX) - 0.5);
+            const int64_t b0 = (int64_t)(int32_t)(((double)d[1] / RMAX) * (double)N);
+            const int64_t b1 = imax64(from_point_once(d[2], d[3], amp_bead, N, b0, ok), 1);
+            check_bead_bounds(b0, b1, N, ind0, indf);
+            ud = d[4];
+        } else if (mv == CHROMO_END_PIVOT) {
+            ang = amp_move * (((double)d[0] / RMAX) - 0.5);
+            lhs = (int32_t)(d[1] & 1);
+            if (amp_bead > N) ok = false;
+            const int64_t r = cexp_once(d[2], amp_bead, amp_bead, ok);
+            ind0 = lhs == 1 ? 0 : N - r;
+            indf = lhs == 1 ? r + 1 : N;
+            if (indf > N) ok = false;
+            s1 = d[3];
+            s2 = d[4];
+            ud = d[5];
         } else {
-            ind0 = N - r;
-            indf = N;
+            ang = amp_move * ((double)d[0] / RMAX);
+            s1 = d[1];
+            s2 = d[2];
+            const int64_t b0 = draw_mod(d[3], N);
+            const int64_t b1 = from_point_once(d[4], d[5], amp_bead, N, b0, ok);
+            check_bead_bounds(b0, b1, N, ind0, indf);
+            ud = d[6];
         }
-        if (indf > N) ok = false;
-        s1 = d[3];
-        s2 = d[4];
-        ud = d[5];
-        used = 6;
-    } else {
-        ang = amp_move * ((double)d[0] / RMAX);
-        s1 = d[1];
-        s2 = d[2];
-        const int64_t b0 = draw_mod(d[3], N);
-        const int64_t b1 = from_point_once(d[4], d[5], amp_bead, N, b0, ok);
-        check_bead_bounds(b0, b1, N, ind0, indf);
-        ud = d[6];
-        used = 7;
+        const int64_t n = indf - ind0;
+        ok = ok && n >= 1 && slot_holds(R, n);
+        const int cnt = (int)__builtin_ctzll(~__ballot(ok));   // the leading usual ones
+        if (lane < cnt) {
+            SpecSlot &S = ring[(at + (uint32_t)lane) & (RING - 1)];
+            S.kind = SLOT_SMALL;
+            S.move = mv;
+            S.binder = 0;
+            S.lhs = lhs;
+            S.ud = ud;
+            S.s1 = s1;
+            S.s2 = s2;
+            S.n = n;
+            S.ind0 = ind0;
+            S.indf = indf;
+            S.ang = ang;
+        }
+        for (int j = 0; j < cnt; ++j) rng_mark(rng, v, used * j, ring[(at + (uint32_t)j) & (RING - 1)].ck);
+        rng_take(rng, v, used * cnt);
+        wave_sync();
+        return cnt;
     }
-    const int64_t n = indf - ind0;
-    if (!ok || n < 1 || !slot_holds(R, n)) return false;
-    rng.pidx = p + used;
-    if (lane_id() == 0) {
+    SpecSlot &S = ring[at & (RING - 1)];
+    int64_t n = 0, ind0 = 0, indf = 0;
+    double ang = 0;
+    int binder = 0, used = 0;
+    int32_t ud = 0;
+    if (mv == CHROMO_TANGENT_ROTATION) {
+        ang = amp_move * (((double)(int32_t)(uni_u32(v.w[0]) >> 1) / RMAX) - 0.5);
+        n = draw_mod((int32_t)(uni_u32(v.w[1]) >> 1), amp_bead) + 1;
+        if (n > N || n > SPEC_NMAX || 3 + 3 * n > v.avail) return 0;
+        const int k = uni_i32((int)n);
+        const bool act = lane < k;
+        const int c = (int)draw_mod((int32_t)(v.w[2 + (act ? lane : 0)] >> 1), N);
+        bool twice = false;
+        for (int j = 0; j + 1 < k; ++j) twice |= act && lane > j && c == (int)readlane_u32((uint32_t)c, j);
+        if (wave_any(twice)) return 0;
+        if (act) {
+            S.picks[lane] = c;
+            S.ps1[lane] = (int32_t)(v.w[2 + k + 2 * lane] >> 1);
+            S.ps2[lane] = (int32_t)(v.w[3 + k + 2 * lane] >> 1);
+        }
+        ud = (int32_t)(uni_u32(v.w[2 + 3 * k]) >> 1);
+        used = 3 + 3 * k;
+    } else {
+        binder = (int)((uni_u32(v.w[0]) >> 1) % (uint32_t)NB);
+        const uint32_t top = (uint32_t)R->sites[binder];
+        const int64_t b0 = draw_mod((int32_t)(uni_u32(v.w[1]) >> 1), N);
+        bool ok = true;
+        const int64_t b1 = from_point_once((int32_t)(uni_u32(v.w[2]) >> 1), (int32_t)(uni_u32(v.w[3]) >> 1), amp_bead,
+                                           N, b0, ok);
+        check_bead_bounds(b0, b1, N, ind0, indf);
+        n = indf - ind0;
+        if (!wave_any(ok) || n < 1 || n > SPEC_NMAX) return 0;
+        // the new states: masked rejection (rnd_randint), 64 words looked at at once
+        used = 4;
+        if (top == 0) {
+            if (lane < n) S.newst[lane] = 0;
+        } else {
+            uint32_t mask = top;
+            mask |= mask >> 1;
+            mask |= mask >> 2;
+            mask |= mask >> 4;
+            mask |= mask >> 8;
+            mask |= mask >> 16;
+            const bool mt = rng.mode == CHROMO_RNG_GLIBC;
+            const int have = mt ? 624 - uni_i32(rng.mti) : v.avail - 4;
+            uint32_t y = 0;
+            if (lane < have) y = mt ? mt_temper(rng.mt[rng.mti + lane]) : v.w[4 + lane];
+            y &= mask;
+            const uint64_t m = __ballot(lane < have && y <= top);
+            const int rank = __popcll(m & ((1ull << lane) - 1));
+            const bool mine = (m >> lane & 1) && rank < n;
+            const uint64_t last = __ballot(mine && rank == n - 1);
+            if (last == 0) return 0;
+            const int words = (int)__builtin_ctzll(last) + 1;
+            if (!mt) {
+                used += words;
+                if (used >= v.avail) return 0;
+            }
+            if (mine) S.newst[rank] = (int32_t)y;
+            if (mt) rng.mti = uni_i32(rng.mti) + words;
+        }
+        ud = (int32_t)(uni_u32(v.w[used]) >> 1);
+        used += 1;
+    }
+    rng_mark(rng, v, 0, S.ck);
+    if (lane == 0) {
         S.kind = SLOT_SMALL;
         S.move = mv;
-        S.binder = 0;
-        S.lhs = lhs;
+        S.binder = binder;
+        S.lhs = 0;
         S.ud = ud;
-        S.s1 = s1;
-        S.s2 = s2;
+        S.s1 = 0;
+        S.s2 = 0;
         S.n = n;
         S.ind0 = ind0;
         S.indf = indf;
         S.ang = ang;
     }
+    rng_take(rng, v, used);
     wave_sync();
-    return true;
+    return 1;
 }
 
 // Draws one proposal into slot S (the drawing wavefront), in the draw order of
@@ -297,7 +478,6 @@ __device__ __forceinline__ int gen_slot(const chromo_replica *R, WaveRng &rng, c
     const int lane = lane_id();
     const int64_t N = R->N;
     rng_save(rng, S.ck);
-    if (gen_fast<NB>(R, rng, C, S)) return SLOT_SMALL;
     const double amp_move = C.amp_move;
     const int64_t amp_bead = C.amp_bead;
     const int mv = C.move;
@@ -446,6 +626,8 @@ __device__ __forceinline__ void seq_step(const chromo_replica *R, const EvConst 
     rng.mode = uni_i32(R->rng_mode);
     rng.k0 = uni_u32(R->rng[CHROMO_RNG_PHILOX_KEY]);
     rng.k1 = uni_u32(R->rng[CHROMO_RNG_PHILOX_KEY + 1]);
+    rng.g = 0;
+    rng.gf = rng.gr = 0;
     rng.pbase = PHILOX_NONE;
     rng.pidx = 0;
     rng.mt = mt;
@@ -674,7 +856,7 @@ __device__ __forceinline__ void spec_book(const chromo_replica *R, chromo_ctrl &
     const uint64_t live_m = __ballot(live);
     const uint64_t acc_m = __ballot(live && acc);
     const uint64_t tie_m = __ballot(live && tie);
-    static_assert(RING <= 8, "bookkeeping sums over the first eight lanes");
+    // sums over the first eight lanes
     const int64_t sn = sum_lanes8_i64(n), sb = sum_lanes8_i64(nb), sy = sum_lanes8_i64(bytes);
     const int64_t logged = K.logged;
     const int nlive = __popcll(live_m);
@@ -735,6 +917,26 @@ __device__ __forceinline__ T ctl_get(const T *f)
     const T v = (T)uni_i32((int)__hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
     return v;
+}
+
+// All of SpecCtl in one LDS read (its words share a read of 16 lanes, so they are of one
+// moment), as scalars.
+struct CtlNow {
+    uint32_t drawn, resolved;
+    int back, alone, over;    // over: stop or err
+};
+__device__ __forceinline__ CtlNow ctl_look(const SpecCtl *ctl)
+{
+    const uint32_t w = __hip_atomic_load((const uint32_t *)ctl + (lane_id() & (CTL_WORDS - 1)), __ATOMIC_RELAXED,
+                                         __HIP_MEMORY_SCOPE_WORKGROUP);
+    CtlNow c;
+    c.drawn = readlane_u32(w, (int)offsetof(SpecCtl, drawn) / 4);
+    c.resolved = readlane_u32(w, (int)offsetof(SpecCtl, resolved) / 4);
+    c.back = (int)readlane_u32(w, (int)offsetof(SpecCtl, back) / 4);
+    c.alone = (int)readlane_u32(w, (int)offsetof(SpecCtl, alone) / 4);
+    c.over = (int)(readlane_u32(w, (int)offsetof(SpecCtl, stop) / 4) | readlane_u32(w, (int)offsetof(SpecCtl, err) / 4));
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    return c;
 }
 
 // A wait's next look: false (and the replica's error) once it passed its bound.
@@ -807,9 +1009,23 @@ __device__ __forceinline__ void block_done(SpecGen &g, chromo_ctrl *sctrl)
     if (same) g.draw = g.book;
 }
 
-// The drawing wavefront's work that is at hand: books the resolved slots, runs the first
-// unresolved slot one at a time where that is needed (alone: only while this wavefront
-// holds nothing in a block), draws further slots.  True when there was something to do.
+// Books the slots before number r.
+template <int RING>
+__device__ __forceinline__ void book_to(const chromo_replica *R, SpecGen &g, chromo_ctrl *sctrl, Counters &K,
+                                        const SpecLds &L, uint32_t r)
+{
+    while (g.booked != r) {
+        const int left = g.book.n - (int)(g.booked - g.book.start), have = (int)(r - g.booked);
+        const int n = have < left ? have : left, F = n < 8 ? n : 8;
+        spec_book<RING>(R, sctrl[g.book.ci], K, L.ring, L.res, g.booked, F);
+        g.booked += (uint32_t)F;
+        if (F == left) block_done(g, sctrl);
+    }
+}
+
+// The drawing wavefront's work that is at hand: draws further slots, books the resolved
+// ones, runs the first unresolved slot one at a time where that is needed (alone: only
+// while this wavefront holds nothing in a block).  True when there was something to do.
 template <int NB, int W, bool TW>
 __device__ __forceinline__ bool spec_serve(const chromo_replica *R, const EvConst &EC, SpecGen &g, chromo_ctrl *sctrl,
                                            Counters &K, const SpecLds &L, bool alone)
@@ -819,23 +1035,16 @@ __device__ __forceinline__ bool spec_serve(const chromo_replica *R, const EvCons
     SpecCtl *ctl = L.ctl;
     const int lane = lane_id();
     bool did = false;
-    const uint32_t r = ctl_get(&ctl->resolved);
-    while (g.booked != r) {
-        const int left = g.book.n - (int)(g.booked - g.book.start), have = (int)(r - g.booked);
-        const int F = have < left ? have : left;
-        spec_book<RING>(R, sctrl[g.book.ci], K, L.ring, L.res, g.booked, F);
-        g.booked += (uint32_t)F;
-        if (F == left) block_done(g, sctrl);
-        did = true;
-    }
     if (g.book.step >= g.steps) {
         ctl_set(&ctl->stop, 1);
         return true;
     }
+    const uint32_t r = ctl_get(&ctl->resolved);
     // (a slot given back after r was read is a later one: left to the next call)
     if (r != g.drawn &&
         (L.ring[r & (RING - 1)].kind == SLOT_SEQ || (ctl_get(&ctl->back) && ctl_get(&ctl->back_at) == r))) {
-        if (!alone) return did;
+        if (!alone) return false;
+        book_to<RING>(R, g, sctrl, K, L, r);
         // what was drawn after slot r is dropped, and drawn again after it: the wavefronts
         // that evaluate it fall back to waiting for it
         if (g.drawn != r + 1) {
@@ -846,7 +1055,7 @@ __device__ __forceinline__ bool spec_serve(const chromo_replica *R, const EvCons
         }
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
         for (int w = 0; w < SH::EV; ++w)
-            if (!ctl_get(&ctl->idle[w])) return did;
+            if (!ctl_get(&ctl->idle[w])) return false;
         SeqIO *io = L.seq;
         const SpecSlot &S0 = L.ring[r & (RING - 1)];
         chromo_ctrl &C = sctrl[g.book.ci];
@@ -875,12 +1084,12 @@ __device__ __forceinline__ bool spec_serve(const chromo_replica *R, const EvCons
         ctl_set(&ctl->back, 0);
         ctl_set(&ctl->alone, 0);
         if (g.booked - g.book.start == (uint32_t)g.book.n) block_done(g, sctrl);
-        if (g.book.step >= g.steps) ctl_set(&ctl->stop, 1);
         return true;
     }
     // nothing is drawn past a SLOT_SEQ slot
-    if (g.drawn != r && L.ring[(g.drawn - 1) & (RING - 1)].kind == SLOT_SEQ) return did;
-    while ((int)(g.drawn - r) < SH::AHEAD) {
+    bool more = g.drawn == r || L.ring[(g.drawn - 1) & (RING - 1)].kind != SLOT_SEQ;
+    const uint32_t room_to = (int)(g.booked + RING - (r + SH::AHEAD)) < 0 ? g.booked + RING : r + SH::AHEAD;
+    while (more && (int)(room_to - g.drawn) > 0) {
         if (g.drawn - g.draw.start == (uint32_t)g.draw.n) {
             // the next block, one ahead of the booked one, unless its controller's
             // amplitudes still depend on that one
@@ -893,14 +1102,26 @@ __device__ __forceinline__ bool spec_serve(const chromo_replica *R, const EvCons
         const chromo_ctrl &C = sctrl[g.draw.ci];
         // MT19937 is not rewound: no binding slot is drawn behind one that may be given back
         if (g.rng.mode == CHROMO_RNG_GLIBC && C.move == CHROMO_CHANGE_BINDING_STATE && (int)(r - g.draw.start) < 0) break;
-        SpecSlot &S = L.ring[g.drawn & (RING - 1)];
-        const int kind = gen_slot<NB>(R, g.rng, C, S);
-        g.list = g.list + 1 == SH::LISTS ? 0 : g.list + 1;
-        if (lane == 0) S.list = g.list;
-        g.drawn += 1;
+        const int left = g.draw.n - (int)(g.drawn - g.draw.start), room = (int)(room_to - g.drawn);
+        int cnt = gen_batch<NB, RING>(R, g.rng, C, L.ring, g.drawn, left < room ? left : room, L.seq->words);
+        if (cnt == 0) {
+            more = gen_slot<NB>(R, g.rng, C, L.ring[g.drawn & (RING - 1)]) != SLOT_SEQ;
+            cnt = 1;
+        }
+        for (int j = 0; j < cnt; ++j) {
+            g.list = g.list + 1 == SH::LISTS ? 0 : g.list + 1;
+            if (lane == 0) L.ring[(g.drawn + (uint32_t)j) & (RING - 1)].list = g.list;
+        }
+        g.drawn += (uint32_t)cnt;
         ctl_set(&ctl->drawn, g.drawn);
         did = true;
-        if (kind == SLOT_SEQ) break;
+    }
+    // several at a time, the last ones of a block at once: the block after the next waits
+    // for them
+    const int waiting = (int)(r - g.booked);
+    if (waiting > 0 && (!did || waiting >= RING / 4 || (int)(r - (g.book.start + (uint32_t)g.book.n)) >= 0)) {
+        book_to<RING>(R, g, sctrl, K, L, r);
+        did = true;
     }
     return did;
 }
@@ -958,7 +1179,7 @@ __device__ __forceinline__ void spec_run(const chromo_replica *R, const EvConst 
     if (wv >= EV) {
         // draws and books only
         int spins = 0;
-        while (!ctl_get(&ctl->stop) && !ctl_get(&ctl->err)) {
+        while (!ctl_look(ctl).over) {
             if (spec_serve<NB, W, TW>(R, EC, g, sctrl, sK, L, true)) spins = 0;
             else if (!spin_on(ctl, spins)) break;
         }
@@ -975,19 +1196,22 @@ __device__ __forceinline__ void spec_run(const chromo_replica *R, const EvConst 
             }
             SpecSlot &S = L.ring[t & (RING - 1)];
             bool go = false;
+            uint32_t seen = 0;   // earlier slots up to here are committed or rejected
             for (int spins = 0;;) {
-                if (ctl_get(&ctl->stop) || ctl_get(&ctl->err)) break;
-                if ((int)(ctl_get(&ctl->resolved) - t) > 0) {
+                const CtlNow c = ctl_look(ctl);
+                if (c.over) break;
+                if ((int)(c.resolved - t) > 0) {
                     have = false;   // it was run one at a time
                     break;
                 }
-                if ((int)(ctl_get(&ctl->drawn) - t) > 0 && S.kind != SLOT_SEQ && !ctl_get(&ctl->back)) {
+                if ((int)(c.drawn - t) > 0 && !c.back && S.kind != SLOT_SEQ) {
                     // no longer idle, unless the slot was dropped meanwhile, or run one at
-                    // a time between the looks above (`back` falls after `resolved` rises)
+                    // a time between the looks (`back` falls after `resolved` rises)
                     ctl_set(&ctl->idle[wv], 0);
                     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
-                    if ((int)(ctl_get(&ctl->drawn) - t) > 0 && !ctl_get(&ctl->back) &&
-                        (int)(ctl_get(&ctl->resolved) - t) <= 0) {
+                    const CtlNow d = ctl_look(ctl);
+                    if ((int)(d.drawn - t) > 0 && !d.back && (int)(d.resolved - t) <= 0) {
+                        seen = d.resolved;
                         go = true;
                         break;
                     }
@@ -1000,7 +1224,7 @@ __device__ __forceinline__ void spec_run(const chromo_replica *R, const EvConst 
                     }
                 }
                 // a slot run one at a time may be of any length
-                if (ctl_get(&ctl->alone)) spins = 0;
+                if (c.alone) spins = 0;
                 if (!spin_on(ctl, spins)) break;
             }
             if (!have) continue;
@@ -1011,15 +1235,15 @@ __device__ __forceinline__ void spec_run(const chromo_replica *R, const EvConst 
             Proposal P;
             int held = 0;
             bool turn = false, again = true;
-            uint32_t seen = ctl_get(&ctl->resolved);   // earlier slots up to here are committed or rejected
             while (again) {
                 again = false;
                 ev_release(G, held);
                 held = 0;
                 if (S.kind == SLOT_SMALL) held = eval_slot<NB, TW>(R, EC, S, res, P, keep, G);
                 for (int spins = 0;;) {
-                    if (ctl_get(&ctl->err)) break;
-                    const uint32_t r = ctl_get(&ctl->resolved);
+                    const CtlNow c = ctl_look(ctl);
+                    if (c.over) break;
+                    const uint32_t r = c.resolved;
                     bool hit = false;
                     for (; seen != r; ++seen) {
                         const SpecSlot &Q = L.ring[seen & (RING - 1)];
@@ -1036,9 +1260,9 @@ __device__ __forceinline__ void spec_run(const chromo_replica *R, const EvConst 
                         turn = true;
                         break;
                     }
-                    if ((int)(ctl_get(&ctl->drawn) - t) <= 0) break;   // dropped
+                    if ((int)(c.drawn - t) <= 0) break;   // dropped
                     if (DRAWS && gen) {
-                        if (ctl_get(&ctl->back)) break;                // to be dropped, by this wavefront
+                        if (c.back) break;                // to be dropped, by this wavefront
                         if (spec_serve<NB, W, TW>(R, EC, g, sctrl, sK, L, false)) continue;
                     }
                     if (!spin_on(ctl, spins)) break;
