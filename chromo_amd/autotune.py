@@ -4,9 +4,9 @@ Two knobs set how the replicas' chains are laid on the GPU; every setting gives
 the same chains bit for bit, so the choice is purely one of speed:
 
 * ``waves`` -- wavefronts per replica (``chromo_mc_run_tuned``): 1 evaluates one
-  proposal at a time; 2 evaluates two proposals of a controller block at once
-  and resolves them in order.  A replica is one workgroup, so with 512 replicas
-  on 256 compute units this also sets the wavefronts resident per SIMD.
+  proposal at a time; 2 evaluates several proposals at once and resolves them
+  in order (on two wavefronts per replica, or four where the launch has a
+  compute unit per replica).
 * ``sweeps_per_launch`` -- sweeps of every replica in one kernel launch (one
   replay of a captured HIP graph).  One sweep per launch ends every launch on
   the slowest replica's sweep; several let each replica run ahead through

@@ -23,7 +23,7 @@ namespace chromo {
 int set_last_error(int code, const std::string &msg);
 
 constexpr int WAVE = 64;
-constexpr int SEG_LDS = 32;                 // moves with n_inds <= SEG_LDS use the LDS arena
+constexpr int SEG_LDS = 32;                 // the field-dE tape's moves of n_inds <= SEG_LDS use the LDS arena
 constexpr int HASH_LDS = 1024;              // >= 2 * 16 * SEG_LDS
 constexpr int MAX_CTRL = 8;
 constexpr double RMAX = 2147483647.0;       // RAND_MAX as a double
@@ -40,7 +40,7 @@ enum : int {
     ERR_NBINDERS = 4,     // binder count outside 1..4 or not in the launch's binder_mask
     ERR_SPIN = 5,         // a rejection or probe loop ran past SPIN_LIMIT iterations
     ERR_ARENA = 6,        // a move-arena index check failed (internal error)
-    ERR_TWIST_WAVES = 7,  // a twisting chain in the speculative (two-wavefront) kernel
+    ERR_TWIST_WAVES = 7,  // a twisting chain launched without its kind's bit (more wavefronts asked for)
 };
 
 // Iteration bound of every data-dependent loop (rejection sampling, distinct-bead
@@ -167,15 +167,6 @@ __device__ __forceinline__ double wave_sum(double x)
     return ((r0 + r1) + r2) + r3;
 }
 
-__device__ __forceinline__ int64_t wave_sum_i64(int64_t x)
-{
-    x += dpp_i64<DPP_XOR1>(x);
-    x += dpp_i64<DPP_XOR2>(x);
-    x += dpp_i64<DPP_HALF_MIRROR>(x);
-    x += dpp_i64<DPP_MIRROR>(x);
-    return readlane_i64(x, 0) + readlane_i64(x, 16) + readlane_i64(x, 32) + readlane_i64(x, 48);
-}
-
 __device__ __forceinline__ int wave_sum_int(int x)
 {
     x += dpp_i32<DPP_XOR1>(x);
@@ -195,18 +186,6 @@ __device__ __forceinline__ int64_t sum_lanes8_i64(int64_t x)
     return readlane_i64(x, 0);
 }
 
-__device__ __forceinline__ uint32_t wave_or(uint32_t m)
-{
-    int x = (int)m;
-    x |= dpp_i32<DPP_XOR1>(x);
-    x |= dpp_i32<DPP_XOR2>(x);
-    x |= dpp_i32<DPP_HALF_MIRROR>(x);
-    x |= dpp_i32<DPP_MIRROR>(x);
-    return readlane_u32((uint32_t)x, 0) | readlane_u32((uint32_t)x, 16) | readlane_u32((uint32_t)x, 32) |
-           readlane_u32((uint32_t)x, 48);
-}
-
-// Exclusive prefix sum over the wave; total receives the wave sum.
 // Exclusive prefix count of a predicate over the wavefront, and its total:
 // wave_excl_scan of 0 / 1 values from one ballot.  Whole wave.
 __device__ __forceinline__ int wave_excl_count(bool pred, int &total)
@@ -216,31 +195,7 @@ __device__ __forceinline__ int wave_excl_count(bool pred, int &total)
     return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
 }
 
-// Fold-length classes, longest first: the positions a voxel's fold visits (1 or
-// 2 -> 7, ..., 15 or more -> 0).
-__device__ __forceinline__ int fold_class(int visits) { return visits >= 15 ? 0 : (16 - visits) >> 1; }
-
-// Ranks of the lane's J items (item j of lane l is item l + 64 j) in the order
-// (class, item) for classes 0..7; items of class 8 or more get no rank.  Items
-// dealt out to lanes in that order give each round of a per-voxel fold loop
-// voxels of similar length: the loop runs as long as its longest voxel.
-// Deterministic.  Whole wave.
-template <int J>
-__device__ __forceinline__ void wave_rank_by_class(const int *cls, int *rank)
-{
-    int off = 0;
-    for (int c = 0; c < 8; ++c) {
-#pragma unroll
-        for (int j = 0; j < J; ++j) {
-            const uint64_t m = __builtin_amdgcn_ballot_w64(cls[j] == c);
-            if (cls[j] == c)
-                rank[j] = off + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
-                                                              __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-            off += __popcll(m);
-        }
-    }
-}
-
+// Exclusive prefix sum over the wave; total receives the wave sum.
 __device__ __forceinline__ int wave_excl_scan(int x, int &total)
 {
     // inclusive scan within rows of 16 (lanes shifted in from outside the row read 0)

@@ -187,19 +187,10 @@ struct MoveOut {
 };
 
 // ---------------------------------------------------------------------------
-// Move body: everything after the bead range is known.  KIND 0 = LDS arena,
-// KIND 1 = global scratch arena.
+// Move body: everything after the bead range is known, in the global scratch arena.
 // ---------------------------------------------------------------------------
 
-// The arena is LDS (KIND 0) or global scratch (KIND 1); one wavefront uses it.
-template <int KIND>
-__device__ __forceinline__ void arena_sync()
-{
-    if (KIND == 0) wave_sync();
-    else wave_sync_global();
-}
-
-template <int KIND, int NB, bool TW = false>
+template <int NB, bool TW = false>
 __device__ __forceinline__ void move_body(const chromo_replica *R, double u, const Proposal &P, MoveOut &out)
 {
     const int lane = lane_id();
@@ -212,12 +203,7 @@ __device__ __forceinline__ void move_body(const chromo_replica *R, double u, con
     const bool check_field = R->field_on && mv != CHROMO_TANGENT_ROTATION;
     const bool state_change = (mv == CHROMO_CHANGE_BINDING_STATE);
 
-    Arena A;
-    if (KIND == 0) {
-        A = make_arena(lds_dyn, lds_layout(Bp1));
-    } else {
-        A = make_arena((char *)R->scratch, global_layout(R->bead_cap, R->seg_cap, Bp1));
-    }
+    const Arena A = make_arena((char *)R->scratch, global_layout(R->bead_cap, R->seg_cap, Bp1));
     const int cap = A.cap;
     double *Pp = R->pos;
 
@@ -359,7 +345,7 @@ __device__ __forceinline__ void move_body(const chromo_replica *R, double u, con
             }
         }
     }
-    arena_sync<KIND>();
+    wave_sync_global();
 
     // ---- polymer dE (SSWLC.compute_dE, polymers.pyx:1024-1082), uniform
     double dEp = 0;
@@ -400,7 +386,7 @@ __device__ __forceinline__ void move_body(const chromo_replica *R, double u, con
             out.err = ERR_ARENA;
             return;
         }
-        arena_sync<KIND>();
+        wave_sync_global();
         // number unique voxels in first-occurrence order
         const int C = (E + WAVE - 1) / WAVE;
         const int e0 = lane * C;
@@ -423,7 +409,7 @@ __device__ __forceinline__ void move_body(const chromo_replica *R, double u, con
                 ++base;
             }
         }
-        arena_sync<KIND>();
+        wave_sync_global();
         // gather current densities of the touched voxels
         const double *rho = R->density;
         for (int q = lane; q < U; q += WAVE) {
@@ -431,7 +417,7 @@ __device__ __forceinline__ void move_body(const chromo_replica *R, double u, con
             for (int m = 0; m < Bp1; ++m) A.urho[m * A.ecap + q] = rho[v * Bp1 + m];
         }
         for (int e = lane; e < E; e += WAVE) atomicAdd(&A.ucnt[A.hu[A.eslot[e]]], 1);
-        arena_sync<KIND>();
+        wave_sync_global();
         {
             const int Cu = (U + WAVE - 1) / WAVE;
             const int q0 = lane * Cu, q1 = min(U, q0 + Cu);
@@ -446,7 +432,7 @@ __device__ __forceinline__ void move_body(const chromo_replica *R, double u, con
             }
             if (lane == 0) A.uoff[U] = E;
         }
-        arena_sync<KIND>();
+        wave_sync_global();
         // counting-sort placement, filling each voxel's list from the front so that
         // it comes out (nearly) in contribution order; the insertion sort below
         // makes it exact
@@ -461,7 +447,7 @@ __device__ __forceinline__ void move_body(const chromo_replica *R, double u, con
             out.err = ERR_ARENA;
             return;
         }
-        arena_sync<KIND>();
+        wave_sync_global();
         // per voxel: order contributions, fold (fields.pyx:1491-1520), energy terms.
         // Lane l handles the voxels whose first contribution e has e % 64 == l, in
         // increasing e: the same partial sums as the register path below.
@@ -905,7 +891,7 @@ __device__ __forceinline__ void mc_evaluate(const chromo_replica *R, const EvCon
             out.n = 0;
             return;
         }
-        move_body<1, NB, TW>(R, u, P, out);
+        move_body<NB, TW>(R, u, P, out);
     }
     if (out.err) {
         out.n = 0;

@@ -159,12 +159,12 @@ class DeviceReplicas:
     """Chains, fields, controllers and RNG streams of ``n`` replicas in HBM."""
 
     CTRL_SLOTS = 8
-    SEG_MAX = 32       # beads per move of the one-wavefront evaluator (chromo_seg.hpp)
+    SEG_MAX = 32       # beads of one chunk of the evaluator (chromo_eval.hpp)
     WAVE_CHOICES = (1, 2)
     # launch shape used by run() (chromo_mc_run_tuned's waves_per_replica); see
     # chromo_amd.autotune.  2, the speculative kernel, is the faster one from one
     # replica to 512 and at initial and steady-state windows alike (16 replicas, 10
-    # sweeps: 20.2 ms with 1, see chromo_spec.hip for the speculative shapes).
+    # sweeps: 20.2 ms with 1, 10.8 ms with 2).
     waves = 2
     sweeps_per_launch = 1  # sweeps per captured graph launch chosen by chromo_amd.autotune
 
@@ -401,7 +401,7 @@ class DeviceReplicas:
         depend on ``waves``."""
         w = int(self.waves if waves is None else waves)
         if self.twist:
-            w = 1       # the speculative evaluator has no twist terms
+            w = 1       # the C entry takes twisting chains only so (their kernel is speculative all the same)
         L.check(self.lib.chromo_mc_run_tuned(self.tab_ptr, self.n, int(num_steps), w, self.binder_mask,
                                              _current_stream()), "chromo_mc_run_tuned")
         if sync:

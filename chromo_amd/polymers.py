@@ -393,7 +393,7 @@ class SSTWLC(SSWLC):
     between the two beads' (t2, t3) frames (compute_twist_angle_omega,
     polymers.pyx:3427-3461), omega_0 = bead_length 2 pi / (10.5 * 0.332 nm) the
     natural twist of DNA, the difference wrapped into [-pi, pi);
-    eps_twist = lt / (delta lp).  Moves run with one wavefront per replica.
+    eps_twist = lt / (delta lp).
     """
 
     def __init__(self, name: str, r, *, bead_length, lp: float, lt: float, bead_rad: float = 5,

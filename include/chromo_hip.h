@@ -111,8 +111,8 @@ enum chromo_replica_error {
     CHROMO_ERR_SPIN = 5,        /* a rejection or probe loop passed its bound (amplitude below one bead:
                                    the reference loops for ever) */
     CHROMO_ERR_ARENA = 6,       /* a scratch-arena index check failed */
-    CHROMO_ERR_TWIST_WAVES = 7  /* a twisting chain (SSTWLC) launched with more than one wavefront
-                                   per replica: it runs with one */
+    CHROMO_ERR_TWIST_WAVES = 7  /* a twisting chain (SSTWLC) launched with waves_per_replica above 1,
+                                   which takes none */
 };
 
 /* Everything the kernels need about one replica (one chain in one field).  The
@@ -217,9 +217,8 @@ int chromo_mc_run(const chromo_replica *d_reps, int32_t n_reps, int64_t num_step
                   void *stream);
 /* chromo_mc_run with an explicit launch shape.  waves_per_replica = 1 runs each
  * chain on one wavefront, one proposal at a time.  2 is the speculative kernel:
- * several proposals of a controller block are evaluated at once and resolved in
- * order, re-evaluating any proposal an earlier accepted one in the same round
- * touched, so the chains (decisions, states, densities, RNG streams) are the same
+ * several proposals are evaluated at once and resolved in order, and one that reads
+ * what a proposal accepted meanwhile wrote is evaluated again, so the chains (decisions, states, densities, RNG streams) are the same
  * for every waves_per_replica; it takes two wavefronts per replica, or four (three
  * evaluating, one drawing) when the launch has at most one replica per compute
  * unit.  binder_mask has bit B set for each binder count B (1..4) among the
