@@ -858,10 +858,11 @@ __device__ __forceinline__ void track_acceptance(chromo_ctrl &C, bool accepted)
 
 // mc_step's evaluation of proposal P with Metropolis draw u in the one-at-a-time block
 // S (its hash empty on entry and on return), the commit of an accepted move, the
-// acceptance tracker; the global arena for what ev_eval does not hold.
+// acceptance tracker; the global arena for what ev_eval does not hold.  loaded: B holds
+// ev_load's data of chunk 0.
 template <int NB, bool TW = false>
 __device__ __forceinline__ void mc_evaluate(const chromo_replica *R, const EvConst &EC, chromo_ctrl &C, MoveOut &out,
-                                            const Proposal &P, double u, const EvLds &S)
+                                            const Proposal &P, double u, const EvLds &S, EvBeads<NB> &B, bool loaded)
 {
     const int64_t n = P.n;
     EvRes sr;
@@ -869,8 +870,7 @@ __device__ __forceinline__ void mc_evaluate(const chromo_replica *R, const EvCon
     const bool lanes = P.move == CHROMO_TANGENT_ROTATION || P.move == CHROMO_CHANGE_BINDING_STATE;
     if (!lanes || n <= EV_LANES) {
         EvKeep K;
-        EvBeads<NB> B;
-        ev_load<NB, TW>(R, P.move, n, P.ind0, P.indf, 0, lanes ? __shfl(P.mypick, lane_id() & 31) : 0, B);
+        if (!loaded) ev_load<NB, TW>(R, P.move, n, P.ind0, P.indf, 0, lanes ? __shfl(P.mypick, lane_id() & 31) : 0, B);
         ev_eval<NB, TW>(R, EC, P, u, S, sr, K, B);
         if (!sr.overflow) {
             if (sr.accepted) ev_commit<NB>(R, P, K, S, sr.U);
@@ -907,7 +907,8 @@ __device__ __forceinline__ void mc_step_dev(const chromo_replica *R, const EvCon
 {
     Proposal P;
     double u = 0;
-    if (mc_propose<NB>(R, rng, C, out, P, u)) mc_evaluate<NB, TW>(R, EC, C, out, P, u, S);
+    EvBeads<NB> B;
+    if (mc_propose<NB>(R, rng, C, out, P, u)) mc_evaluate<NB, TW>(R, EC, C, out, P, u, S, B, false);
 }
 
 // SimpleControl.update_amplitudes (mc_controller.py:126-213)

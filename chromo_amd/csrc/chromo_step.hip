@@ -2,7 +2,7 @@
 // launch (mc_step and the plain path) and the persistent kernel behind chromo_mc_run.
 #include <hip/hip_runtime.h>
 
-#include "chromo_mc.hpp"
+#include "chromo_spec.hpp"
 
 using namespace chromo;
 
@@ -69,6 +69,8 @@ __global__ void __launch_bounds__(64) k_mc_step(const chromo_replica *__restrict
 {
     __shared__ chromo_replica Rs;
     __shared__ EvConst EC;
+    __shared__ SpecSlot slot;
+    __shared__ uint32_t words[GLIBC_BUF + 1];
     load_record(&Rs, &reps[rep]);
     wave_sync();
     const chromo_replica *R = &Rs;
@@ -94,18 +96,18 @@ __global__ void __launch_bounds__(64) k_mc_step(const chromo_replica *__restrict
     MoveOut o;
     if (R->twist) {
         switch (R->B) {
-        case 1: mc_step_dev<1, true>(R, EC, rng, C, o, S); break;
-        case 2: mc_step_dev<2, true>(R, EC, rng, C, o, S); break;
-        case 3: mc_step_dev<3, true>(R, EC, rng, C, o, S); break;
-        case 4: mc_step_dev<4, true>(R, EC, rng, C, o, S); break;
+        case 1: mc_step_slot<1, true>(R, EC, rng, C, o, S, slot, words); break;
+        case 2: mc_step_slot<2, true>(R, EC, rng, C, o, S, slot, words); break;
+        case 3: mc_step_slot<3, true>(R, EC, rng, C, o, S, slot, words); break;
+        case 4: mc_step_slot<4, true>(R, EC, rng, C, o, S, slot, words); break;
         default: o.err = ERR_NBINDERS; o.n = 0; break;
         }
     } else {
         switch (R->B) {
-        case 1: mc_step_dev<1>(R, EC, rng, C, o, S); break;
-        case 2: mc_step_dev<2>(R, EC, rng, C, o, S); break;
-        case 3: mc_step_dev<3>(R, EC, rng, C, o, S); break;
-        case 4: mc_step_dev<4>(R, EC, rng, C, o, S); break;
+        case 1: mc_step_slot<1, false>(R, EC, rng, C, o, S, slot, words); break;
+        case 2: mc_step_slot<2, false>(R, EC, rng, C, o, S, slot, words); break;
+        case 3: mc_step_slot<3, false>(R, EC, rng, C, o, S, slot, words); break;
+        case 4: mc_step_slot<4, false>(R, EC, rng, C, o, S, slot, words); break;
         default: o.err = ERR_NBINDERS; o.n = 0; break;
         }
     }
