@@ -74,3 +74,36 @@ def test_slot_order(kind, mode):
     ca, cb = one.counter_array(), four.counter_array()
     for w in (L.CNT_PROPOSALS, L.CNT_ACCEPTED, L.CNT_SUM_N, L.CNT_SUM_BINS, L.CNT_BYTES):
         assert np.array_equal(ca[:, w], cb[:, w]), w
+
+
+@pytest.mark.parametrize("mode", [L.RNG_PHILOX, L.RNG_GLIBC])
+@pytest.mark.parametrize("kind", ["mixed", "overflow", "short chain", "twist"])
+def test_one_proposal_launches(kind, mode):
+    """One launch per proposal draws the usual proposals at once and the others word by
+    word: the persistent kernel's chains for every binder count."""
+    from chromo_amd.engine import DeviceReplicas
+    k = CASES["mixed" if kind == "twist" else kind]
+    print("one-proposal launches", kind, mode, flush=True)
+    kw = {"voxel": k["voxel"]} if "voxel" in k else {}
+    for B in (1, 2, 3, 4):
+        build = W.make_twist_system if kind == "twist" else W.make_system
+        s = build(k.get("N", 300), B, k.get("grid", 6), seed=950 + B, chi=0.4, per_cycle=k["per_cycle"], **kw)
+        s.field.vf_limit = 1e9
+        for c in s.ctrls:
+            if "amp" in k and c.move in (L.CRANK_SHAFT, L.SLIDE, L.END_PIVOT):
+                c.amp_bead = min(k["amp"], int(c.bead_hi))
+                c.bead_lo = c.bead_hi
+
+        def make():
+            dr = DeviceReplicas([s.chain], [s.field], [copy.deepcopy(s.ctrls)], rng_mode=mode, seeds=[3], streams=[1])
+            dr.np_seed([4])
+            return dr
+        a, b = make(), make()
+        a.run(4, waves=1)
+        b.run_plain(4)
+        for x, y in zip(a.positions(0), b.positions(0)):
+            assert np.array_equal(x, y), B
+        assert np.array_equal(a.binder_states(0), b.binder_states(0))
+        assert np.array_equal(a.density_of(0), b.density_of(0))
+        assert np.array_equal(a.rng_words(0), b.rng_words(0))
+        assert a.controllers(0) == b.controllers(0)
