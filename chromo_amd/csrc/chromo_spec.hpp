@@ -46,7 +46,8 @@ struct Shape {
     static constexpr int AHEAD = W == 2 ? 6 : 8;
     static_assert(AHEAD <= RING - EV + 1, "no slot is overwritten while it is looked at");
     // Voxel lists: slot a's is looked at by the next EV - 1 slots, which can be in flight
-    // together with the EV - 1 after them.
+    // together with the EV - 1 after them.  Its own wavefront reads it up to its turn and
+    // not after: from there on nothing keeps the others from a slot that has this list.
     static constexpr int LISTS = 2 * EV - 1;
     // Voxels of a block: two workgroups on a compute unit, or one.
     __host__ __device__ static constexpr int ucap(int Bp1)
@@ -1314,7 +1315,8 @@ __device__ __forceinline__ void spec_run(const chromo_replica *R, const EvConst 
                 ctl_set(&ctl->resolved, t + 1);
                 have = false;
             }
-            ev_release(G, held);
+            // whole, not by the slot's list: another slot may have that by now
+            if (held) ev_clear(G);
             ctl_set(&ctl->idle[wv], 1);
         }
     }
