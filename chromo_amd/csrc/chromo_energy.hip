@@ -31,6 +31,7 @@
 
 #include "chromo_density.hpp"
 #include "chromo_device.hpp"
+#include "chromo_fixed.hpp"
 
 using namespace chromo;
 
@@ -163,18 +164,10 @@ __device__ void block_reduce_store(double *vals, int nt, double *part)
 // ---- field terms: densities, voxel energies, gradient at the beads ---------------
 //
 // The adjoint needs a deterministic density, not the reference's bead-order fold.
-// Each corner weight w (in [0, 1]) becomes the integer nearest to w 2^60, a high word of
-// 29 bits and a signed low word of 32, and the words are summed in 64 bits each, times
-// the binder state for the binder rows: the sums are exact, so they do not depend on
-// the order in which the LDS takes them.  A voxel's total is rounded to double once and
-// divided by its volume.  Sums stay in range for 2^30 beads (states up to 3).
-
-// The double nearest (hi 2^32 + lo) 2^-60; exact before the one rounding for words
-// below 2^53 (2^23 beads and more in one voxel round once more).
-__device__ __forceinline__ double from_fixed60(uint64_t hi, uint64_t lo)
-{
-    return fma((double)hi, 0x1p32, (double)(int64_t)lo) * 0x1p-60;
-}
+// Each corner weight becomes an integer of two words (chromo_fixed.hpp), and the words are
+// summed in 64 bits each, times the binder state for the binder rows: the sums are exact,
+// so they do not depend on the order in which the LDS takes them.  A voxel's total is
+// rounded to double once and divided by its volume.
 
 // Slots of the block partials: [0..B) S_jj, [B..B+B(B-1)/2) S_jk (j<k), then sum g,
 // sum dg/dchi.
@@ -254,27 +247,22 @@ k_e_tile(EModel M, TileGeom T, const double *theta, const double *r, const int32
                 const int o = atomicAdd(&nown, 1);
                 if (o < TILE_OWN) owned[o] = b;
             }
-            // corner_weight's products, the last factor scaled, and the nearest integers:
-            // adding 1.5 2^52 leaves them in the low word
-            const double ux = 1 - w[0], uy = 1 - w[1], uz = (1 - w[2]) * 0x1p28, wz = w[2] * 0x1p28;
+            // corner_weight's products, the last factor scaled
+            const double ux = 1 - w[0], uy = 1 - w[1], uz = (1 - w[2]) * FIXED60_SCALE, wz = w[2] * FIXED60_SCALE;
             const double xy[4] = {w[0] * w[1], ux * w[1], w[0] * uy, ux * uy};
 #pragma unroll
             for (int l = 0; l < 8; ++l) {
                 const int vx = at[0][l & 1], vy = at[1][(l >> 1) & 1], vz = at[2][l >> 2];
                 if ((vx | vy | vz) < 0) continue;
                 const int v = vx + vy + vz;
-                const double wl = xy[l & 3] * ((l & 4) ? uz : wz);
-                const double mh = wl + 0x1.8p52;
-                const double ml = fma(wl - (mh - 0x1.8p52), 0x1p32, 0x1.8p52);
-                const uint32_t hi = (uint32_t)__double_as_longlong(mh);
-                const long long lo = (int32_t)__double_as_longlong(ml);
-                atomicAdd(&sums[0][0][v], (unsigned long long)lo);
-                atomicAdd(&sums[0][1][v], (unsigned long long)hi);
+                const Fixed60 f = fixed60(xy[l & 3] * ((l & 4) ? uz : wz));
+                atomicAdd(&sums[0][0][v], (unsigned long long)(long long)f.lo);
+                atomicAdd(&sums[0][1][v], (unsigned long long)f.hi);
 #pragma unroll
                 for (int j = 0; j < B; ++j) {
                     if (st[j] != 0) {
-                        atomicAdd(&sums[j + 1][0][v], (unsigned long long)(lo * st[j]));
-                        atomicAdd(&sums[j + 1][1][v], (unsigned long long)(hi * (uint32_t)st[j]));
+                        atomicAdd(&sums[j + 1][0][v], (unsigned long long)(long long)(f.lo * st[j]));
+                        atomicAdd(&sums[j + 1][1][v], (unsigned long long)(f.hi * (uint32_t)st[j]));
                     }
                 }
             }
