@@ -32,6 +32,7 @@
 #include "chromo_density.hpp"
 #include "chromo_device.hpp"
 #include "chromo_fixed.hpp"
+#include "chromo_index.hpp"
 
 using namespace chromo;
 
@@ -207,7 +208,7 @@ k_e_tile(EModel M, TileGeom T, const double *theta, const double *r, const int32
             start[j] = tile_start(T.n[j], T.nt[j], tt[j]);
             size[j] = tile_start(T.n[j], T.nt[j], tt[j] + 1) - start[j];
         }
-        const int len = cnt[tile];
+        const uint32_t len = (uint32_t)cnt[tile];
         const int32_t *mine = list + base[tile];
         for (int i = t; i < Bp1 * 2 * TILE_VOX; i += TILE_THREADS) (&sums[0][0][0])[i] = 0;
         if (t == 0) nown = 0;
@@ -215,15 +216,15 @@ k_e_tile(EModel M, TileGeom T, const double *theta, const double *r, const int32
         // the beads' corner weights.  Lists hold runs of the chain, whose neighbours share
         // voxels: the lanes of a wavefront take entries far apart, so that their adds
         // meet different voxels
-        const int per = (len + TILE_THREADS - 1) / TILE_THREADS;
-        for (int k = 0; k < per; ++k) {
-            const int i = ((t & 63) * (TILE_THREADS / 64) + (t >> 6)) * per + k;
+        const uint32_t per = (len + TILE_THREADS - 1) / TILE_THREADS;
+        for (uint32_t k = 0; k < per; ++k) {
+            const uint32_t i = (uint32_t)((t & 63) * (TILE_THREADS / 64) + (t >> 6)) * per + k;
             if (i >= len) continue;
             const int32_t b = mine[i];
             double x[3], w[3];
             int ix[3];
 #pragma unroll
-            for (int j = 0; j < 3; ++j) x[j] = r[3 * b + j];
+            for (int j = 0; j < 3; ++j) x[j] = r[row3(b, j)];
             int st[B];
 #pragma unroll
             for (int j = 0; j < B; ++j) st[j] = M.states[(int64_t)j * M.N + b];
@@ -307,14 +308,14 @@ k_e_tile(EModel M, TileGeom T, const double *theta, const double *r, const int32
         __syncthreads();
         if (GRAD) {
             // trilinear chain rule at the beads of the tile's own cells
-            const int no = nown;
-            const bool noted = no <= TILE_OWN;
-            for (int i = t; i < (noted ? no : len); i += TILE_THREADS) {
+            const uint32_t no = (uint32_t)nown;
+            const bool noted = no <= (uint32_t)TILE_OWN;
+            for (uint32_t i = (uint32_t)t; i < (noted ? no : len); i += TILE_THREADS) {
                 const int32_t b = noted ? owned[i] : mine[i];
                 double x[3], w[3];
                 int ix[3];
 #pragma unroll
-                for (int j = 0; j < 3; ++j) x[j] = r[3 * b + j];
+                for (int j = 0; j < 3; ++j) x[j] = r[row3(b, j)];
                 tile_lower(M.G, T, x, ix, w);
                 int at[3][2];
                 bool own = true;
@@ -355,7 +356,7 @@ k_e_tile(EModel M, TileGeom T, const double *theta, const double *r, const int32
 #pragma unroll
                 for (int j = 0; j < 3; ++j) g[j] = T.recip ? div_by(g[j], vb, T.rvol) : g[j] / vb;
 #pragma unroll
-                for (int j = 0; j < 3; ++j) grad[3 * b + j] = g[j];
+                for (int j = 0; j < 3; ++j) grad[row3(b, j)] = g[j];
             }
             __syncthreads();
         }
