@@ -12,6 +12,7 @@
 #include <stdint.h>
 
 #include <string>
+#include <type_traits>
 
 #include "chromo_device.hpp"
 
@@ -68,8 +69,8 @@ struct ScatterJob {
     const int8_t *states;
     double *density;                // n_bins x Bp1
     int32_t *cell, *list;           // per bead; the tiles' bead lists
-    int32_t *cnt, *fill, *base;     // per tile
-    int32_t *cursor;
+    int32_t *cnt, *fill;            // per tile
+    ListPlace *base, *cursor;
     int32_t Bp1, cleanup;
 };
 
@@ -78,17 +79,16 @@ struct ScatterJob {
 inline size_t scatter_carve(ScatterJob &J, char *base)
 {
     size_t o = 0;
-    auto take = [&](size_t n) {
-        int32_t *p = base ? (int32_t *)(base + o) : nullptr;
-        o = align_scratch(o + sizeof(int32_t) * n);
-        return p;
+    auto take = [&](auto *&p, size_t n) {
+        p = base ? (std::remove_reference_t<decltype(p)>)(base + o) : nullptr;
+        o = align_scratch(o + sizeof(*p) * n);
     };
-    J.cnt = take((size_t)J.T.ntiles);
-    J.fill = take((size_t)J.T.ntiles);
-    J.cursor = take(1);
-    J.base = take((size_t)J.T.ntiles);
-    J.cell = take((size_t)J.N);
-    J.list = take((size_t)J.N * tile_images(J.T));
+    take(J.cnt, (size_t)J.T.ntiles);
+    take(J.fill, (size_t)J.T.ntiles);
+    take(J.cursor, 1);
+    take(J.base, (size_t)J.T.ntiles);
+    take(J.cell, (size_t)J.N);
+    take(J.list, (size_t)J.N * tile_images(J.T));
     return o;
 }
 
@@ -279,24 +279,25 @@ __global__ void __launch_bounds__(WAVE) k_scatter_fold(const ScatterJob *__restr
     const bool degen = T.n[0] == 1 || T.n[1] == 1 || T.n[2] == 1;
     const int stride[3] = {1, FOLD_MAX[0], FOLD_MAX[0] * FOLD_MAX[1]};
     for (int i = lane; i < VOX * Bp1; i += WAVE) sum[i] = 0;
-    const int len = J.cnt[tile];
+    const uint32_t len = (uint32_t)J.cnt[tile];     // its places and the step past the last in 32 bits
     int32_t *list = J.list + J.base[tile];
-    const int runs = len > 0 ? list_runs(list, len, from, off, (int32_t *)c0) : 0;
+    const int runs = len > 0 ? list_runs(list, (int)len, from, off, (int32_t *)c0) : 0;
     const bool in = lane < PB * LP;
     const int pj = in ? lane / LP : 0, m = in ? (lane % LP) >> 3 : 0, l8 = lane & 7;
     char *acc = (char *)(sum + m);
     const double *avol = J.G.access_vol;
-    for (int i0 = 0; i0 < len; i0 += WAVE) {
-        const int n = len - i0 < WAVE ? len - i0 : WAVE;
+    for (uint32_t i0 = 0; i0 < len; i0 += WAVE) {
+        const int n = len - i0 < (uint32_t)WAVE ? (int)(len - i0) : WAVE;
         if (lane < n) {
+            const int32_t i = (int32_t)(i0 + (uint32_t)lane);
             // the run that holds position i0 + lane of the order
             int lo = 0, hi = runs;
             while (hi - lo > 1) {
                 const int mid = (lo + hi) >> 1;
-                if (off[mid] <= i0 + lane) lo = mid;
+                if (off[mid] <= i) lo = mid;
                 else hi = mid;
             }
-            const int64_t b = list[from[lo] + (i0 + lane - off[lo])];
+            const int64_t b = list[from[lo] + (i - off[lo])];
             double x[3], w[3];
             int ix[3];
 #pragma unroll

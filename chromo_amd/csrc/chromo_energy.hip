@@ -174,7 +174,7 @@ __device__ void block_reduce_store(double *vals, int nt, double *part)
 // sum dg/dchi.
 template <int B, bool GRAD>
 __global__ void __launch_bounds__(TILE_THREADS, 4)
-k_e_tile(EModel M, TileGeom T, const double *theta, const double *r, const int32_t *cnt, const int32_t *base,
+k_e_tile(EModel M, TileGeom T, const double *theta, const double *r, const int32_t *cnt, const ListPlace *base,
          const int32_t *list, double *grad, double *part)
 {
     constexpr int Bp1 = B + 1, NT = B + B * (B - 1) / 2 + 2;
@@ -734,7 +734,8 @@ size_t energy_carve(const EModel &M, const PosView &P, double *rho, char *base, 
 
 // The same for the energy and its adjoint: the tiles' lists and the block partials.
 struct AdjointBufs {
-    int32_t *cnt = nullptr, *fill = nullptr, *base = nullptr, *cursor = nullptr, *cell = nullptr, *list = nullptr;
+    int32_t *cnt = nullptr, *fill = nullptr, *cell = nullptr, *list = nullptr;
+    ListPlace *base = nullptr, *cursor = nullptr;
     double *vpart = nullptr, *bpart = nullptr;
     int gt = 0, gb = 0;
 };
@@ -751,8 +752,8 @@ size_t adjoint_carve(const EModel &M, const TileGeom &T, char *base, AdjointBufs
     Bf.gb = grid_blocks(M.N);
     Bf.cnt = (int32_t *)take(sizeof(int32_t) * T.ntiles);
     Bf.fill = (int32_t *)take(sizeof(int32_t) * T.ntiles);
-    Bf.base = (int32_t *)take(sizeof(int32_t) * T.ntiles);
-    Bf.cursor = (int32_t *)take(sizeof(int32_t));
+    Bf.base = (ListPlace *)take(sizeof(ListPlace) * T.ntiles);
+    Bf.cursor = (ListPlace *)take(sizeof(ListPlace));
     Bf.cell = (int32_t *)take(sizeof(int32_t) * M.N);
     Bf.list = (int32_t *)take(sizeof(int32_t) * M.N * tile_images(T));
     Bf.vpart = (double *)take(sizeof(double) * MAXT * Bf.gt);
@@ -795,7 +796,7 @@ int energy_adjoint_run(const EModel &M, const TileGeom &T, const double *d_r, co
     // sequence in a HIP graph
     hipLaunchKernelGGL(k_tile_clear, dim3(gt), dim3(256), 0, st, Bf.cnt, Bf.fill, Bf.cursor, T.ntiles);
     hipLaunchKernelGGL(k_tile_bin<false>, dim3(gb), dim3(BIN_THREADS), 0, st, M.G, T, M.N, P, Bf.cell, Bf.cnt,
-                       (const int32_t *)nullptr, (int32_t *)nullptr);
+                       (const ListPlace *)nullptr, (int32_t *)nullptr);
     hipLaunchKernelGGL(k_tile_base, dim3(gt), dim3(256), 0, st, Bf.cnt, Bf.base, Bf.cursor, T.ntiles);
     hipLaunchKernelGGL(k_tile_bin<true>, dim3(gb), dim3(BIN_THREADS), 0, st, M.G, T, M.N, P, Bf.cell, Bf.fill, Bf.base,
                        Bf.list);

@@ -151,8 +151,12 @@ __device__ __forceinline__ int axis_tiles(int n, int nt, int c, int t[2])
     return 1;
 }
 
+// Where a list begins in the array of all lists, which hold a bead up to eight times: 64
+// bits (268,435,456 beads in one-voxel tiles pass 2^31 entries).
+using ListPlace = unsigned long long;
+
 // Clears the lists' counters and the list cursor.
-__global__ void k_tile_clear(int32_t *cnt, int32_t *fill, int32_t *cursor, int n)
+__global__ void k_tile_clear(int32_t *cnt, int32_t *fill, ListPlace *cursor, int n)
 {
     const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
     if (i < n) cnt[i] = fill[i] = 0;
@@ -161,19 +165,22 @@ __global__ void k_tile_clear(int32_t *cnt, int32_t *fill, int32_t *cursor, int n
 
 // Room for every list: a wavefront's lists in a row, the wavefronts in the order they
 // arrive (nothing depends on where a list lies).
-__device__ __forceinline__ void tile_bases(const int32_t *cnt, int32_t *base, int32_t *cursor, int n)
+__device__ __forceinline__ void tile_bases(const int32_t *cnt, ListPlace *base, ListPlace *cursor, int n)
 {
-    const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-    const int k = i < n ? cnt[i] : 0;
-    int tot;
-    const int off = wave_excl_scan(k, tot);
-    int at = 0;
-    if (lane_id() == 0) at = atomicAdd(cursor, tot);
-    at = bcast0(at);
-    if (i < n) base[i] = at + off;
+    const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x), lane = lane_id();
+    const int64_t k = i < n ? cnt[i] : 0;
+    int64_t sum = k;    // of the lanes up to this one
+    for (int o = 1; o < WAVE; o <<= 1) {
+        const int64_t below = __shfl_up(sum, o);
+        if (lane >= o) sum += below;
+    }
+    ListPlace at = 0;
+    if (lane == WAVE - 1) at = atomicAdd(cursor, (ListPlace)sum);
+    at = (ListPlace)readlane_i64((int64_t)at, WAVE - 1);
+    if (i < n) base[i] = at + (ListPlace)(sum - k);
 }
 
-__global__ void k_tile_base(const int32_t *cnt, int32_t *base, int32_t *cursor, int n)
+__global__ void k_tile_base(const int32_t *cnt, ListPlace *base, ListPlace *cursor, int n)
 {
     tile_bases(cnt, base, cursor, n);
 }
@@ -189,7 +196,7 @@ constexpr int TILE_TABLE = 512, TILE_PROBES = 16, BIN_THREADS = 256;
 
 template <bool PLACE, bool UPPER, bool STABLE>
 __device__ __forceinline__ void tile_bin(const GridGeom &G, const TileGeom &T, int64_t N, const PosView &P,
-                                         int32_t *cell, int32_t *num, const int32_t *base, int32_t *list)
+                                         int32_t *cell, int32_t *num, const ListPlace *base, int32_t *list)
 {
     constexpr int W = BIN_THREADS / WAVE;
     __shared__ int32_t key[TILE_TABLE], cntl[TILE_TABLE], from[TILE_TABLE];
@@ -257,21 +264,21 @@ __device__ __forceinline__ void tile_bin(const GridGeom &G, const TileGeom &T, i
 #pragma unroll
     for (int q = 0; q < 8; ++q) {
         if (tile[q] < 0) continue;
-        int at = rank[q];
+        ListPlace at = base[tile[q]] + (ListPlace)rank[q];
         if (slot[q] >= 0) {
-            at += from[slot[q]];
+            at += (ListPlace)from[slot[q]];
             if (STABLE) {
-                for (int w = 0; w < wv; ++w) at += __popcll(bits[slot[q] * W + w]);
-                at += __popcll(bits[slot[q] * W + wv] & ((1ull << lane) - 1));
+                for (int w = 0; w < wv; ++w) at += (ListPlace)__popcll(bits[slot[q] * W + w]);
+                at += (ListPlace)__popcll(bits[slot[q] * W + wv] & ((1ull << lane) - 1));
             }
         }
-        list[base[tile[q]] + at] = (int32_t)b;
+        list[at] = (int32_t)b;
     }
 }
 
 template <bool PLACE>
 __global__ void __launch_bounds__(BIN_THREADS) k_tile_bin(GridGeom G, TileGeom T, int64_t N, PosView P, int32_t *cell,
-                                                          int32_t *num, const int32_t *base, int32_t *list)
+                                                          int32_t *num, const ListPlace *base, int32_t *list)
 {
     tile_bin<PLACE, true, false>(G, T, N, P, cell, num, base, list);
 }

@@ -32,3 +32,27 @@ def test_kernels_index_beads_through_it():
     src = (ROOT / "chromo_amd" / "csrc" / "chromo_energy.hip").read_text()
     tile = src[src.index("k_e_tile(EModel"):src.index("// ---- bead / bond terms")]
     assert "3 * b" not in tile and tile.count("row3(b, j)") == 3
+
+
+def test_list_places_have_64_bits():
+    """The workspaces hold, per bead, its cell and its entries in the lists, and per tile
+    two counters of 32 bits and the place of its list in 64: the lists of the largest
+    chains hold more than 2^31 entries."""
+    import ctypes
+
+    from chromo_amd import _lib as L
+    h = L.lib()
+    # a long flat grid: so many tiles that 4 bytes of each outweigh the rest of the scratch
+    n, N = 2 ** 22, 2 ** 31 - 2
+    m = L.ChromoEnergyModel()
+    m.N, m.B, m.nx, m.ny, m.nz = N, 1, n, 1, 1
+    m.x_width, m.y_width, m.z_width, m.bead_vol = 30.0 * n, 30.0, 30.0, 1.0
+    assert h.chromo_energy_adjoint_bytes(ctypes.byref(m)) >= 4 * N + 4 * 2 * N + (4 + 4 + 8) * (n // 8)
+    rep = (L.ChromoReplica * 1)()
+    R = rep[0]
+    R.N, R.B, R.field_on, R.nx, R.ny, R.nz = N, 1, 1, n, 1, 1
+    for j in range(3):
+        R.width[j] = (30.0 * n, 30.0, 30.0)[j]
+        R.dxyz[j], R.half_width[j], R.half_step[j] = 30.0, R.width[j] / 2, 15.0
+    R.vol_bin = 27000.0
+    assert h.chromo_density_init_bytes(ctypes.addressof(rep), 1) >= 4 * N + 4 * 2 * N + (4 + 4 + 8) * (n // 4)
