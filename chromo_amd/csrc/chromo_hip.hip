@@ -516,6 +516,7 @@ int density_jobs(const chromo_replica *h, int32_t n_reps, std::vector<ScatterJob
         if (r.B < 0 || r.B > CHROMO_MAX_BINDERS) return set_err(-1, "B out of range");
         if (r.nx * r.ny * r.nz > 2048LL * 2048LL || r.N > 0x7fffffff)
             return set_err(-1, "grid or chain too large for the density scatter");
+        if (r.N < 1) continue;      // no beads: nothing to scatter
         if (r.nx < 1 || r.ny < 1 || r.nz < 1) return set_err(-1, "a grid axis without voxels");
         jobs.push_back(scatter_job(grid_of(r), r.N, r.B + 1, PosView{r.pos, r.N, 1}, r.states, r.density, 1));
     }
