@@ -151,6 +151,16 @@ def _current_stream() -> int:
     return torch.cuda.current_stream().cuda_stream
 
 
+def kinds_mask(chains) -> int:
+    """Bit B: chains with B binder types present; bit 8 + B: twisting ones among them."""
+    mask = 0
+    for c in chains:
+        mask |= 1 << c.B
+        if c.twist:
+            mask |= 1 << (8 + c.B)
+    return mask
+
+
 # ---------------------------------------------------------------------------
 # Device replicas
 # ---------------------------------------------------------------------------
@@ -203,9 +213,7 @@ class DeviceReplicas:
             if f.field_on and max(int(f.nx), int(f.ny), int(f.nz)) > 32767:
                 raise NotImplementedError("more than 32767 voxels along one axis")
         self.Ns, self.Bs = Ns, Bs
-        # bit B: B binder types present; bit 8 + B: twisting chains among them
-        self.binder_mask = (sum(1 << b for b in set(Bs)) |
-                            sum(1 << (8 + c.B) for c in chains if c.twist))
+        self.binder_mask = kinds_mask(chains)
         nctrl = [len(c) for c in ctrls]
         if max(nctrl) > self.CTRL_SLOTS:
             raise NotImplementedError(f"at most {self.CTRL_SLOTS} controllers per replica")
