@@ -28,6 +28,7 @@
 
 #include <mutex>
 #include <string>
+#include <type_traits>
 
 #include "chromo_density.hpp"
 #include "chromo_device.hpp"
@@ -127,7 +128,8 @@ __device__ inline Coef coef_of(const EModel &M, const double *th)
 
 // Fixed-order block sum of NT partial values per thread: a butterfly within each
 // wavefront, then the wavefront sums in wavefront order.
-template <int NT, int THREADS = EB>
+// SHARED: for another block of the same launch, past the caches of this block's die.
+template <int NT, int THREADS = EB, bool SHARED = false>
 __device__ void block_reduce_store(const double (&vals)[NT], double *part)
 {
     __shared__ double sh[THREADS / 64][NT];
@@ -142,7 +144,9 @@ __device__ void block_reduce_store(const double (&vals)[NT], double *part)
     if ((int)threadIdx.x < NT) {
         double s = sh[0][threadIdx.x];
         for (int w = 1; w < THREADS / 64; ++w) s += sh[w][threadIdx.x];
-        part[(int64_t)threadIdx.x * gridDim.x + blockIdx.x] = s;
+        double *to = &part[(int64_t)threadIdx.x * gridDim.x + blockIdx.x];
+        if (SHARED) __hip_atomic_store(to, s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        else *to = s;
     }
 }
 
@@ -170,25 +174,12 @@ __device__ void block_reduce_store(double *vals, int nt, double *part)
 // so they do not depend on the order in which the LDS takes them.  A voxel's total is
 // rounded to double once and divided by its volume.
 
-// Slots of the block partials: [0..B) S_jj, [B..B+B(B-1)/2) S_jk (j<k), then sum g,
-// sum dg/dchi.
-template <int B, bool GRAD>
-__global__ void __launch_bounds__(TILE_THREADS, 4)
-k_e_tile(EModel M, TileGeom T, const double *theta, const double *r, const int32_t *cnt, const ListPlace *base,
-         const int32_t *list, double *grad, double *part)
-{
-    constexpr int Bp1 = B + 1, NT = B + B * (B - 1) / 2 + 2;
-    // [species][low, high][voxel]; a voxel's dE/drho overwrites its low words
-    __shared__ unsigned long long sums[Bp1][2][TILE_VOX];
-    __shared__ int32_t owned[TILE_OWN], nown;
-    const int t = threadIdx.x;
-    double acc[NT];
-#pragma unroll
-    for (int q = 0; q < NT; ++q) acc[q] = 0;
-    const double V = M.bead_vol, vb = M.G.vol_bin;
-    // the coefficients in scalar registers: held in vector registers through the tile
-    // loop they spill
+// Coefficients of the voxel terms in scalar registers: held in vector registers through
+// the tile loop they spill.
+template <int B>
+struct VoxelCoef {
     double pref2[B], XX[B * B], gphi, dphi;
+    __device__ __forceinline__ VoxelCoef(const EModel &M, const TileGeom &T, const double *theta)
     {
         const Coef c = coef_of<B>(M, theta);
         gphi = uni_f64(c.chi * T.vbV);
@@ -200,17 +191,219 @@ k_e_tile(EModel M, TileGeom T, const double *theta, const double *r, const int32
             for (int k = 0; k < B; ++k) XX[j * B + k] = uni_f64(c.X[j * B + k] + c.X[k * B + j]);
         }
     }
-    for (int tile = blockIdx.x; tile < T.ntiles; tile += gridDim.x) {
-        const int tt[3] = {tile % T.nt[0], (tile / T.nt[0]) % T.nt[1], tile / (T.nt[0] * T.nt[1])};
-        int start[3], size[3];
+};
+
+// The sums of a tile or part: [species][low, high][voxel]; a voxel's dE/drho overwrites
+// its low words.
+// SIDE: places per axis, the tile's or part's voxels and their upper neighbours.
+template <int B, int SIDE>
+using TileSums = unsigned long long[B + 1][2][SIDE * SIDE * SIDE];
+constexpr int TILE_SIDE = 9, PART_SIDE = 5;
+static_assert(TILE_MAX[0] < TILE_SIDE && TILE_MAX[1] < TILE_SIDE && TILE_MAX[2] < TILE_SIDE &&
+              (TILE_SIDE - 1 + 1) / 2 < PART_SIDE, "places of a tile and of half of one");
+
+// A tile's or part's first voxels and sizes.
+struct TileBox {
+    int start[3], size[3];
+};
+
+// Whether X is all of axis j, wrapping onto itself.  (For a tile the same either way; this
+// one keeps the tile kernel's registers in bounds.)
+template <int SIDE>
+__device__ __forceinline__ bool whole_axis(const TileGeom &T, const TileBox &X, int j)
+{
+    return SIDE == TILE_SIDE ? T.nt[j] == 1 : X.size[j] == T.n[j];
+}
+
+// Adds bead b's corner weights to the sums of the box X (its upper neighbours included).
+// b's cell is inside X or a neighbour; note(whether inside).
+template <int B, int SIDE, class F>
+__device__ __forceinline__ void tile_add(const EModel &M, const TileGeom &T, const double *r, int32_t b,
+                                         const TileBox &X, TileSums<B, SIDE> &sums, F note)
+{
+    double x[3], w[3];
+    int ix[3];
 #pragma unroll
-        for (int j = 0; j < 3; ++j) {
-            start[j] = tile_start(T.n[j], T.nt[j], tt[j]);
-            size[j] = tile_start(T.n[j], T.nt[j], tt[j] + 1) - start[j];
+    for (int j = 0; j < 3; ++j) x[j] = r[row3(b, j)];
+    int st[B];
+#pragma unroll
+    for (int j = 0; j < B; ++j) st[j] = M.states[(int64_t)j * M.N + b];
+    tile_lower(M.G, T, x, ix, w);
+    int at[3][2];       // voxel place of the lower and upper corner, -1: not among these voxels
+    bool own = true;
+    const int stride[3] = {1, SIDE, SIDE * SIDE};
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        if (whole_axis<SIDE>(T, X, j)) {
+            at[j][0] = ix[j] * stride[j];
+            at[j][1] = (ix[j] + 1 == T.n[j] ? 0 : ix[j] + 1) * stride[j];
+        } else {
+            const int l = tile_local(T.n[j], X.start[j], X.size[j], ix[j]);
+            own = own && l >= 0 && l < X.size[j];
+            at[j][0] = l >= 0 ? l * stride[j] : -1;
+            at[j][1] = l < X.size[j] ? (l + 1) * stride[j] : -1;
         }
-        const uint32_t len = (uint32_t)cnt[tile];
+    }
+    note(own);
+    // corner_weight's products, the last factor scaled
+    const double ux = 1 - w[0], uy = 1 - w[1], uz = (1 - w[2]) * FIXED60_SCALE, wz = w[2] * FIXED60_SCALE;
+    const double xy[4] = {w[0] * w[1], ux * w[1], w[0] * uy, ux * uy};
+#pragma unroll
+    for (int l = 0; l < 8; ++l) {
+        const int vx = at[0][l & 1], vy = at[1][(l >> 1) & 1], vz = at[2][l >> 2];
+        if ((vx | vy | vz) < 0) continue;
+        const int v = vx + vy + vz;
+        const Fixed60 f = fixed60(xy[l & 3] * ((l & 4) ? uz : wz));
+        atomicAdd(&sums[0][0][v], (unsigned long long)(long long)f.lo);
+        atomicAdd(&sums[0][1][v], (unsigned long long)f.hi);
+#pragma unroll
+        for (int j = 0; j < B; ++j) {
+            if (st[j] != 0) {
+                atomicAdd(&sums[j + 1][0][v], (unsigned long long)(long long)(f.lo * st[j]));
+                atomicAdd(&sums[j + 1][1][v], (unsigned long long)(f.hi * (uint32_t)st[j]));
+            }
+        }
+    }
+}
+
+// Densities, energy terms of the voxels of the tile or part itself, dE/drho in place.
+// acc: [0..B) S_jj, [B..B+B(B-1)/2) S_jk (j<k), then sum g, sum dg/dchi.
+template <int B, bool GRAD, int THREADS, int SIDE, int NT>
+__device__ __forceinline__ void tile_voxels(const EModel &M, const TileGeom &T, const VoxelCoef<B> &c,
+                                            const TileBox &X, TileSums<B, SIDE> &sums, double (&acc)[NT])
+{
+    constexpr int Bp1 = B + 1;
+    const double V = M.bead_vol, vb = M.G.vol_bin;
+    for (int v = threadIdx.x; v < SIDE * SIDE * SIDE; v += THREADS) {
+        const int vx = v % SIDE, vy = (v / SIDE) % SIDE, vz = v / (SIDE * SIDE);
+        double rho[Bp1];
+#pragma unroll
+        for (int j = 0; j < Bp1; ++j) {
+            const double f = from_fixed60(sums[j][1][v], sums[j][0][v]);
+            rho[j] = T.recip ? div_by(f, vb, T.rvol) : f / vb;
+        }
+        const double phi = rho[0] * V;
+        const bool huge = phi > M.vf_limit;
+        if (vx < X.size[0] && vy < X.size[1] && vz < X.size[2]) {
+            int s = B;
+#pragma unroll
+            for (int j = 0; j < B; ++j) {
+                acc[j] += rho[j + 1] * rho[j + 1];
+#pragma unroll
+                for (int k = j + 1; k < B; ++k) acc[s++] += rho[j + 1] * rho[k + 1];
+            }
+            acc[s] += huge ? E_HUGE_FIELD * phi : c.gphi * (phi * phi);
+            acc[s + 1] += huge ? 0.0 : T.vbV * (phi * phi);
+        }
+        if (GRAD) {
+            double d[Bp1];
+            d[0] = V * (huge ? E_HUGE_FIELD : c.dphi * phi);
+#pragma unroll
+            for (int j = 0; j < B; ++j) {
+                double g = c.pref2[j] * rho[j + 1];
+#pragma unroll
+                for (int k = 0; k < B; ++k) g += c.XX[j * B + k] * rho[k + 1];
+                d[j + 1] = g;
+            }
+#pragma unroll
+            for (int j = 0; j < Bp1; ++j) sums[j][0][v] = (unsigned long long)__double_as_longlong(d[j]);
+        }
+    }
+}
+
+// The field's gradient at bead b into grad (ADD: added to it), by the trilinear chain rule,
+// when its cell is inside.
+template <int B, int SIDE, bool ADD>
+__device__ __forceinline__ void tile_gather(const EModel &M, const TileGeom &T, const double *r, int32_t b,
+                                            const TileBox &X, const TileSums<B, SIDE> &sums, double *grad)
+{
+    double x[3], w[3];
+    int ix[3];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) x[j] = r[row3(b, j)];
+    tile_lower(M.G, T, x, ix, w);
+    int at[3][2];
+    bool own = true;
+    const int stride[3] = {1, SIDE, SIDE * SIDE};
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        const int l = ix[j] - X.start[j];
+        own = own && l >= 0 && l < X.size[j];
+        at[j][0] = l * stride[j];
+        at[j][1] = (whole_axis<SIDE>(T, X, j) && l + 1 == X.size[j] ? 0 : l + 1) * stride[j];
+    }
+    if (!own) return;
+    double st[B];
+#pragma unroll
+    for (int j = 0; j < B; ++j) st[j] = (double)M.states[(int64_t)j * M.N + b];
+    // along x first: A the interpolated value, D the difference, for each
+    // (y, z); then along y and z
+    const double ux = 1 - w[0], uy = 1 - w[1], uz = 1 - w[2], vb = M.G.vol_bin;
+    double A[4], D[4], g[3];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        double h[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const int v = at[0][e] + at[1][q & 1] + at[2][q >> 1];
+            h[e] = __longlong_as_double((long long)sums[0][0][v]);
+#pragma unroll
+            for (int j = 0; j < B; ++j) h[e] += st[j] * __longlong_as_double((long long)sums[j + 1][0][v]);
+        }
+        A[q] = w[0] * h[0] + ux * h[1];
+        D[q] = h[1] - h[0];
+    }
+    g[0] = (w[2] * (w[1] * D[0] + uy * D[1]) + uz * (w[1] * D[2] + uy * D[3])) * T.rd[0];
+    g[1] = (w[2] * (A[1] - A[0]) + uz * (A[3] - A[2])) * T.rd[1];
+    g[2] = ((w[1] * A[2] + uy * A[3]) - (w[1] * A[0] + uy * A[1])) * T.rd[2];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) g[j] = T.recip ? div_by(g[j], vb, T.rvol) : g[j] / vb;
+#pragma unroll
+    for (int j = 0; j < 3; ++j) grad[row3(b, j)] = ADD ? grad[row3(b, j)] + g[j] : g[j];
+}
+
+__device__ __forceinline__ TileBox tile_box(const TileGeom &T, int tile)
+{
+    const int tt[3] = {tile % T.nt[0], (tile / T.nt[0]) % T.nt[1], tile / (T.nt[0] * T.nt[1])};
+    TileBox X;
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        X.start[j] = tile_start(T.n[j], T.nt[j], tt[j]);
+        X.size[j] = tile_start(T.n[j], T.nt[j], tt[j] + 1) - X.start[j];
+    }
+    return X;
+}
+
+// Cell c of the grid, by axis.
+__device__ __forceinline__ void cell_axes(const TileGeom &T, int32_t cell, int ix[3])
+{
+    const uint32_t c = (uint32_t)cell, q = c / (uint32_t)T.n[0];
+    ix[0] = (int)(c - q * (uint32_t)T.n[0]);
+    ix[1] = (int)(q % (uint32_t)T.n[1]);
+    ix[2] = (int)(q / (uint32_t)T.n[1]);
+}
+
+// The tiles whose lists are not split.  Block partials: tile_voxels' acc.
+template <int B, bool GRAD>
+__global__ void __launch_bounds__(TILE_THREADS, 4)
+k_e_tile(EModel M, TileGeom T, const double *theta, const double *r, TileCounters C, const ListPlace *base,
+         const int32_t *list, LongTiles L, double *grad, double *part)
+{
+    constexpr int NT = B + B * (B - 1) / 2 + 2;
+    __shared__ TileSums<B, TILE_SIDE> sums;
+    __shared__ int32_t owned[TILE_OWN], nown;
+    const int t = threadIdx.x;
+    double acc[NT];
+#pragma unroll
+    for (int q = 0; q < NT; ++q) acc[q] = 0;
+    const VoxelCoef<B> c(M, T, theta);
+    const int32_t most = split_above(C, L);
+    for (int tile = blockIdx.x; tile < T.ntiles; tile += gridDim.x) {
+        const TileBox X = tile_box(T, tile);
+        uint32_t len = (uint32_t)C.cnt[tile];
+        if (len > (uint32_t)most) len = 0;      // as if it were empty: tile_parts does it
         const int32_t *mine = list + base[tile];
-        for (int i = t; i < Bp1 * 2 * TILE_VOX; i += TILE_THREADS) (&sums[0][0][0])[i] = 0;
+        for (int i = t; i < (int)(sizeof(sums) / 8); i += TILE_THREADS) (&sums[0][0][0])[i] = 0;
         if (t == 0) nown = 0;
         __syncthreads();
         // the beads' corner weights.  Lists hold runs of the chain, whose neighbours share
@@ -221,90 +414,16 @@ k_e_tile(EModel M, TileGeom T, const double *theta, const double *r, const int32
             const uint32_t i = (uint32_t)((t & 63) * (TILE_THREADS / 64) + (t >> 6)) * per + k;
             if (i >= len) continue;
             const int32_t b = mine[i];
-            double x[3], w[3];
-            int ix[3];
-#pragma unroll
-            for (int j = 0; j < 3; ++j) x[j] = r[row3(b, j)];
-            int st[B];
-#pragma unroll
-            for (int j = 0; j < B; ++j) st[j] = M.states[(int64_t)j * M.N + b];
-            tile_lower(M.G, T, x, ix, w);
-            int at[3][2];       // voxel place of the lower and upper corner, -1: not this tile's
-            bool own = true;
-            const int stride[3] = {1, TILE_SX, TILE_SX * TILE_SY};
-#pragma unroll
-            for (int j = 0; j < 3; ++j) {
-                if (T.nt[j] == 1) {
-                    at[j][0] = ix[j] * stride[j];
-                    at[j][1] = (ix[j] + 1 == T.n[j] ? 0 : ix[j] + 1) * stride[j];
-                } else {
-                    const int l = tile_local(T.n[j], start[j], size[j], ix[j]);
-                    own = own && l >= 0 && l < size[j];
-                    at[j][0] = l >= 0 ? l * stride[j] : -1;
-                    at[j][1] = l < size[j] ? (l + 1) * stride[j] : -1;
+            tile_add<B, TILE_SIDE>(M, T, r, b, X, sums, [&](bool own) {
+                if (GRAD && own) {
+                    const int o = atomicAdd(&nown, 1);
+                    if (o < TILE_OWN) owned[o] = b;
                 }
-            }
-            if (GRAD && own) {
-                const int o = atomicAdd(&nown, 1);
-                if (o < TILE_OWN) owned[o] = b;
-            }
-            // corner_weight's products, the last factor scaled
-            const double ux = 1 - w[0], uy = 1 - w[1], uz = (1 - w[2]) * FIXED60_SCALE, wz = w[2] * FIXED60_SCALE;
-            const double xy[4] = {w[0] * w[1], ux * w[1], w[0] * uy, ux * uy};
-#pragma unroll
-            for (int l = 0; l < 8; ++l) {
-                const int vx = at[0][l & 1], vy = at[1][(l >> 1) & 1], vz = at[2][l >> 2];
-                if ((vx | vy | vz) < 0) continue;
-                const int v = vx + vy + vz;
-                const Fixed60 f = fixed60(xy[l & 3] * ((l & 4) ? uz : wz));
-                atomicAdd(&sums[0][0][v], (unsigned long long)(long long)f.lo);
-                atomicAdd(&sums[0][1][v], (unsigned long long)f.hi);
-#pragma unroll
-                for (int j = 0; j < B; ++j) {
-                    if (st[j] != 0) {
-                        atomicAdd(&sums[j + 1][0][v], (unsigned long long)(long long)(f.lo * st[j]));
-                        atomicAdd(&sums[j + 1][1][v], (unsigned long long)(f.hi * (uint32_t)st[j]));
-                    }
-                }
-            }
+            });
         }
         __syncthreads();
         // densities, energy terms of the tile's own voxels, dE/drho in place
-        for (int v = t; v < TILE_VOX; v += TILE_THREADS) {
-            const int vx = v % TILE_SX, vy = (v / TILE_SX) % TILE_SY, vz = v / (TILE_SX * TILE_SY);
-            double rho[Bp1];
-#pragma unroll
-            for (int j = 0; j < Bp1; ++j) {
-                const double f = from_fixed60(sums[j][1][v], sums[j][0][v]);
-                rho[j] = T.recip ? div_by(f, vb, T.rvol) : f / vb;
-            }
-            const double phi = rho[0] * V;
-            const bool huge = phi > M.vf_limit;
-            if (vx < size[0] && vy < size[1] && vz < size[2]) {
-                int s = B;
-#pragma unroll
-                for (int j = 0; j < B; ++j) {
-                    acc[j] += rho[j + 1] * rho[j + 1];
-#pragma unroll
-                    for (int k = j + 1; k < B; ++k) acc[s++] += rho[j + 1] * rho[k + 1];
-                }
-                acc[s] += huge ? E_HUGE_FIELD * phi : gphi * (phi * phi);
-                acc[s + 1] += huge ? 0.0 : T.vbV * (phi * phi);
-            }
-            if (GRAD) {
-                double d[Bp1];
-                d[0] = V * (huge ? E_HUGE_FIELD : dphi * phi);
-#pragma unroll
-                for (int j = 0; j < B; ++j) {
-                    double g = pref2[j] * rho[j + 1];
-#pragma unroll
-                    for (int k = 0; k < B; ++k) g += XX[j * B + k] * rho[k + 1];
-                    d[j + 1] = g;
-                }
-#pragma unroll
-                for (int j = 0; j < Bp1; ++j) sums[j][0][v] = (unsigned long long)__double_as_longlong(d[j]);
-            }
-        }
+        tile_voxels<B, GRAD, TILE_THREADS, TILE_SIDE>(M, T, c, X, sums, acc);
         __syncthreads();
         if (GRAD) {
             // trilinear chain rule at the beads of the tile's own cells
@@ -312,56 +431,143 @@ k_e_tile(EModel M, TileGeom T, const double *theta, const double *r, const int32
             const bool noted = no <= (uint32_t)TILE_OWN;
             for (uint32_t i = (uint32_t)t; i < (noted ? no : len); i += TILE_THREADS) {
                 const int32_t b = noted ? owned[i] : mine[i];
-                double x[3], w[3];
-                int ix[3];
-#pragma unroll
-                for (int j = 0; j < 3; ++j) x[j] = r[row3(b, j)];
-                tile_lower(M.G, T, x, ix, w);
-                int at[3][2];
-                bool own = true;
-                const int stride[3] = {1, TILE_SX, TILE_SX * TILE_SY};
-#pragma unroll
-                for (int j = 0; j < 3; ++j) {
-                    const int l = ix[j] - start[j];
-                    own = own && l >= 0 && l < size[j];
-                    at[j][0] = l * stride[j];
-                    at[j][1] = (T.nt[j] == 1 && l + 1 == size[j] ? 0 : l + 1) * stride[j];
-                }
-                if (!own) continue;
-                double st[B];
-#pragma unroll
-                for (int j = 0; j < B; ++j) st[j] = (double)M.states[(int64_t)j * M.N + b];
-                // along x first: A the interpolated value, D the difference, for each
-                // (y, z); then along y and z
-                const double ux = 1 - w[0], uy = 1 - w[1], uz = 1 - w[2];
-                double A[4], D[4];
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    double h[2];
-#pragma unroll
-                    for (int e = 0; e < 2; ++e) {
-                        const int v = at[0][e] + at[1][q & 1] + at[2][q >> 1];
-                        h[e] = __longlong_as_double((long long)sums[0][0][v]);
-#pragma unroll
-                        for (int j = 0; j < B; ++j)
-                            h[e] += st[j] * __longlong_as_double((long long)sums[j + 1][0][v]);
-                    }
-                    A[q] = w[0] * h[0] + ux * h[1];
-                    D[q] = h[1] - h[0];
-                }
-                double g[3];
-                g[0] = (w[2] * (w[1] * D[0] + uy * D[1]) + uz * (w[1] * D[2] + uy * D[3])) * T.rd[0];
-                g[1] = (w[2] * (A[1] - A[0]) + uz * (A[3] - A[2])) * T.rd[1];
-                g[2] = ((w[1] * A[2] + uy * A[3]) - (w[1] * A[0] + uy * A[1])) * T.rd[2];
-#pragma unroll
-                for (int j = 0; j < 3; ++j) g[j] = T.recip ? div_by(g[j], vb, T.rvol) : g[j] / vb;
-#pragma unroll
-                for (int j = 0; j < 3; ++j) grad[row3(b, j)] = g[j];
+                tile_gather<B, TILE_SIDE, false>(M, T, r, b, X, sums, grad);
             }
             __syncthreads();
         }
     }
     block_reduce_store<NT, TILE_THREADS>(acc, part);
+}
+
+// LDS of tile_parts.
+template <int B>
+struct PartLds {
+    TileSums<B, PART_SIDE> sums;
+    int32_t picked[PART_NOTES], npicked;    // beads near the part
+    int32_t owned[PART_NOTES], nowned;      // those in its cells
+    int32_t longs[LONG_GROUPS], nlong;      // long lists before each group of tiles, in all
+};
+
+// The tiles with long lists, each in 8 parts (halves per axis), one block per part: a
+// block picks its beads from the tile's list.  Adds the field's gradient to grad; writes
+// tile_voxels' sums to part, past the caches of this block's die.
+// A condensed chain fills few tiles, and one block per tile left most of the chip idle, the
+// others bound by their compute unit's LDS adds.  10^6 beads at 25 per voxel, B = 4, 128^3:
+// 744 -> 461 us an evaluation; 100,000 in 16^3 voxels of 64^3, B = 2: 237 -> 133 us.  What
+// bounds it: the adds still (a part lists 3.4 beads per own bead), and picking.
+template <int B, bool GRAD>
+__device__ __forceinline__ void tile_parts(const EModel &M, const TileGeom &T, const double *theta, const double *r,
+                                           const int32_t *cell, const int32_t *cnt, const ListPlace *base,
+                                           const int32_t *list, const LongTiles &L, double *grad, double *part,
+                                           PartLds<B> &S)
+{
+    constexpr int NT = B + B * (B - 1) / 2 + 2, SCAN = PART_SCAN;
+    const int t = threadIdx.x;
+    double acc[NT];
+#pragma unroll
+    for (int q = 0; q < NT; ++q) acc[q] = 0;
+    const VoxelCoef<B> c(M, T, theta);
+    const int groups = (T.ntiles + LONG_GROUP - 1) / LONG_GROUP;
+    if (t < WAVE) {
+        int sum = 0;
+        for (int g0 = 0; g0 < groups; g0 += WAVE) {
+            int all;
+            const int g = g0 + t, below = wave_excl_scan(g < groups ? L.count[g] : 0, all);
+            if (g < groups) S.longs[g] = sum + below;
+            sum += all;
+        }
+        if (t == 0) S.nlong = sum;
+    }
+    __syncthreads();
+    const int nlong = uni_i32(S.nlong);
+    for (int item = blockIdx.x; item < nlong * TILE_PARTS; item += gridDim.x) {
+        const int h = item / TILE_PARTS;
+        int lo = 0, hi = groups;
+        while (hi - lo > 1) {
+            const int mid = (lo + hi) >> 1;
+            if (uni_i32(S.longs[mid]) <= h) lo = mid;
+            else hi = mid;
+        }
+        const int tile = uni_i32(L.tile[LONG_GROUP * lo + (h - uni_i32(S.longs[lo]))]);
+        TileBox X = tile_box(T, tile);
+#pragma unroll
+        for (int j = 0; j < 3; ++j) tile_half((item >> j) & 1, X.start[j], X.size[j]);
+        if (X.size[0] == 0 || X.size[1] == 0 || X.size[2] == 0) continue;
+        const uint32_t len = (uint32_t)cnt[tile];
+        const int32_t *mine = list + base[tile];
+        for (int i = t; i < (int)(sizeof(S.sums) / 8); i += PART_THREADS) (&S.sums[0][0][0])[i] = 0;
+        if (t == 0) S.npicked = S.nowned = 0;
+        __syncthreads();
+        // picks beads from entry `from` of the list on, as many as S.picked[] surely holds;
+        // returns the entry after them.  near: those near the part, of which those in its
+        // cells are noted in S.owned[] while there is room; else those in its cells.
+        auto pick = [&](uint32_t from, bool near) {
+            static_assert(PART_NOTES >= 2 * SCAN * PART_THREADS, "two steps fit");
+            for (;;) {
+                int32_t bead[SCAN], at[SCAN];
+#pragma unroll
+                for (int q = 0; q < SCAN; ++q) {
+                    const uint32_t i = from + (uint32_t)(q * PART_THREADS + t);
+                    bead[q] = i < len ? mine[i] : -1;
+                }
+#pragma unroll
+                for (int q = 0; q < SCAN; ++q) at[q] = bead[q] >= 0 ? cell[bead[q]] : 0;
+#pragma unroll
+                for (int q = 0; q < SCAN; ++q) {
+                    int ix[3];
+                    cell_axes(T, at[q], ix);
+                    bool is = bead[q] >= 0, own = is;
+#pragma unroll
+                    for (int j = 0; j < 3; ++j) {
+                        is = is && tile_near(T.n[j], X.start[j], X.size[j], ix[j]);
+                        own = own && ix[j] >= X.start[j] && ix[j] < X.start[j] + X.size[j];
+                    }
+                    if (near ? is : own) S.picked[atomicAdd(&S.npicked, 1)] = bead[q];
+                    if (GRAD && near && own) {
+                        const int o = atomicAdd(&S.nowned, 1);
+                        if (o < PART_NOTES) S.owned[o] = bead[q];
+                    }
+                }
+                from += SCAN * PART_THREADS;
+                __syncthreads();
+                const int n = uni_i32(S.npicked);
+                // nobody adds to S.npicked before everybody has read it
+                __syncthreads();
+                if (from >= len || n > PART_NOTES - SCAN * PART_THREADS) return from;
+            }
+        };
+        for (uint32_t from = 0; from < len;) {
+            from = pick(from, true);
+            const uint32_t n = (uint32_t)uni_i32(S.npicked), per = (n + PART_THREADS - 1) / PART_THREADS;
+            for (uint32_t k = 0; k < per; ++k) {
+                const uint32_t i = (uint32_t)((t & 63) * (PART_THREADS / 64) + (t >> 6)) * per + k;
+                if (i < n) tile_add<B, PART_SIDE>(M, T, r, S.picked[i], X, S.sums, [](bool) {});
+            }
+            __syncthreads();
+            if (t == 0) S.npicked = 0;
+            __syncthreads();
+        }
+        tile_voxels<B, GRAD, PART_THREADS, PART_SIDE>(M, T, c, X, S.sums, acc);
+        __syncthreads();
+        if (!GRAD) continue;
+        const uint32_t no = (uint32_t)uni_i32(S.nowned);
+        if (no <= (uint32_t)PART_NOTES) {
+            for (uint32_t i = (uint32_t)t; i < no; i += PART_THREADS)
+                tile_gather<B, PART_SIDE, true>(M, T, r, S.owned[i], X, S.sums, grad);
+        } else {
+            for (uint32_t from = 0; from < len;) {
+                from = pick(from, false);
+                const uint32_t n = (uint32_t)uni_i32(S.npicked);
+                for (uint32_t i = (uint32_t)t; i < n; i += PART_THREADS)
+                    tile_gather<B, PART_SIDE, true>(M, T, r, S.picked[i], X, S.sums, grad);
+                __syncthreads();
+                if (t == 0) S.npicked = 0;
+                __syncthreads();
+            }
+        }
+        __syncthreads();
+    }
+    block_reduce_store<NT, PART_THREADS, true>(acc, part);
 }
 
 // ---- bead / bond terms -------------------------------------------------------
@@ -388,7 +594,7 @@ __device__ inline double E_pair_and_grad(const Bond &bd, const double *r0, const
 }
 
 // slots: [0] E_elastic, [1] E_bind, [2..2+B) D_j, [2+B..2+2B) sum s_j
-// grad: the field's gradient on entry (k_e_tile), the whole gradient on return.
+// grad: the field's gradient on entry (k_e_tile), with the bonds' on return.
 template <int B>
 __global__ void __launch_bounds__(EB) k_e_bead(EModel M, const double *theta, const double *r, double *grad,
                                                double *part)
@@ -454,18 +660,21 @@ __global__ void __launch_bounds__(EB) k_e_bead(EModel M, const double *theta, co
     block_reduce_store<NT>(acc, part);
 }
 
-// Sums of the block partials of ntv voxel terms and ntb bead terms, by one block of
-// FINAL_THREADS: wavefront w takes terms w, w + 16, ...; lane i adds partials i,
+// Sums of the block partials of ntv voxel terms and ntb bead terms, by one block of W
+// wavefronts: wavefront w takes terms w, w + W, ...; lane i adds partials i,
 // i + 64, ... in increasing order (loaded 16 at a time, so that one round trip
 // covers 16 of them), then a butterfly over the 64 lanes.  The order depends on
 // the sizes only, so the sums are the same on every run.
+// SHARED: partials that other blocks of the same launch wrote.
 constexpr int FINAL_THREADS = 1024;
+constexpr int FINAL_READ = 1024;    // partials of a term that one round trip covers
 
+template <int THREADS = FINAL_THREADS, bool SHARED = false>
 __device__ void final_sums(const double *vpart, int nbv, int ntv, const double *bpart, int nbb, int ntb,
                            double *sv, double *sb)
 {
     const int wv = threadIdx.x / 64, lane = threadIdx.x % 64;
-    for (int q = wv; q < ntv + ntb; q += FINAL_THREADS / 64) {
+    for (int q = wv; q < ntv + ntb; q += THREADS / 64) {
         const bool vox = q < ntv;
         const double *p = vox ? vpart : bpart;
         const int nbk = vox ? nbv : nbb, t = vox ? q : q - ntv;
@@ -475,7 +684,9 @@ __device__ void final_sums(const double *vpart, int nbv, int ntv, const double *
 #pragma unroll
             for (int j = 0; j < 16; ++j) {
                 const int i = i0 + 64 * j;
-                x[j] = i < nbk ? p[(int64_t)t * nbk + i] : 0.0;
+                const double *at = p + ((int64_t)t * nbk + i);
+                if (SHARED) x[j] = i < nbk ? __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0.0;
+                else x[j] = i < nbk ? *at : 0.0;
             }
 #pragma unroll
             for (int j = 0; j < 16; ++j)
@@ -487,16 +698,12 @@ __device__ void final_sums(const double *vpart, int nbv, int ntv, const double *
     __syncthreads();
 }
 
-// Final reduction over block partials (fixed order) and assembly, for B binders
-// (compile-time, so the coefficients and sums stay in registers).
+// The energies and dE/dtheta from the sums, for B binders (compile-time, so the
+// coefficients and sums stay in registers), by one thread.
 template <int B>
-__global__ void __launch_bounds__(FINAL_THREADS)
-k_e_final(EModel M, const double *theta, const double *vpart, int nbv, int ntv, const double *bpart, int nbb,
-          int ntb, double *E_out, double *gtheta)
+__device__ __forceinline__ void assemble(const EModel &M, const double *theta, const double *sv, const double *sb,
+                                         double *E_out, double *gtheta)
 {
-    __shared__ double sv[MAXT], sb[MAXT];
-    final_sums(vpart, nbv, ntv, bpart, nbb, ntb, sv, sb);
-    if (threadIdx.x != 0) return;
     const Coef c = coef_of<B>(M, theta);
     const double vb = M.G.vol_bin;
     double S[CHROMO_MAX_BINDERS * CHROMO_MAX_BINDERS];
@@ -545,6 +752,51 @@ k_e_final(EModel M, const double *theta, const double *vpart, int nbv, int ntv, 
 #pragma unroll
         for (int j = 0; j < B; ++j) gtheta[1 + B * (B + 1) / 2 + j] = -sb[2 + B + j];
     }
+}
+
+// Final reduction over block partials (fixed order) and assembly.
+template <int B>
+__global__ void __launch_bounds__(FINAL_THREADS)
+k_e_final(EModel M, const double *theta, const double *vpart, int nbv, int ntv, const double *bpart, int nbb,
+          int ntb, double *E_out, double *gtheta)
+{
+    __shared__ double sv[MAXT], sb[MAXT];
+    final_sums(vpart, nbv, ntv, bpart, nbb, ntb, sv, sb);
+    if (threadIdx.x == 0) assemble<B>(M, theta, sv, sb, E_out, gtheta);
+}
+
+// The same where lists may have to be split.  If they are, all blocks of the launch work on
+// those tiles first, and the last one done goes on; otherwise all but the first have
+// nothing to do.  (A launch of their own would cost every evaluation 4 us.  This costs 1.5
+// of 55 us at 100,000 beads, nothing measurable at 10^6.)
+template <int B, bool GRAD>
+__global__ void __launch_bounds__(PART_THREADS, 4)
+k_e_split(EModel M, TileGeom T, const double *theta, const double *r, const int32_t *cell, TileCounters C,
+          const ListPlace *base, const int32_t *list, LongTiles L, double *grad, double *lpart, const double *vpart,
+          int nbv, int ntv, const double *bpart, int nbb, int ntb, double *E_out, double *gtheta)
+{
+    __shared__ double sv[MAXT], sb[MAXT], sl[MAXT];
+    __shared__ PartLds<B> lds;
+    __shared__ int32_t ticket;
+    const bool split = uni_i32(*C.split) != 0;
+    if (split) {
+        tile_parts<B, GRAD>(M, T, theta, r, cell, C.cnt, base, list, L, grad, lpart, lds);
+        // this block's partials have arrived before its ticket is drawn
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (threadIdx.x == 0)
+            ticket = __hip_atomic_fetch_add(C.ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        if (ticket != (int)gridDim.x - 1) return;
+        final_sums<PART_THREADS, true>(lpart, (int)gridDim.x, ntv, nullptr, 0, 0, sl, nullptr);
+    } else if (blockIdx.x != 0) {
+        return;
+    }
+    final_sums<PART_THREADS>(vpart, nbv, ntv, bpart, nbb, ntb, sv, sb);
+    if (threadIdx.x != 0) return;
+    if (split)
+        for (int q = 0; q < ntv; ++q) sv[q] += sl[q];
+    assemble<B>(M, theta, sv, sb, E_out, gtheta);
 }
 
 // ---- the reference's compute_E (fields.pyx:1939-2286, polymers.pyx:1348-1381) ----
@@ -732,12 +984,33 @@ size_t energy_carve(const EModel &M, const PosView &P, double *rho, char *base, 
     return o;
 }
 
+// Where lists are split (tile_parts), the long ones: more than 1/512 of all entries (about
+// two per bead), so that one block would be at it when the others are done; and, where
+// there are tiles for every block, more than two and a half times the mean, so that a grid
+// that is full everywhere is not split.  They are where one list holds `huge` beads:
+// splitting costs 30 to 60 us beside the tile kernel's time for the lists below that
+// (20,000 beads in 9^3 voxels: 92 us with or without, 150 us split from 4,096 on).
+// Short chains' never are: looking for long lists costs 1.5 us of 49.
+void long_list(int64_t N, int64_t ntiles, LongTiles &L)
+{
+    constexpr int64_t NONE = 0x7fffffff;
+    int64_t most = LONG_LIST;
+    if (most < N / 256) most = N / 256;
+    if (ntiles >= PART_BLOCKS && most < 5 * N / ntiles) most = 5 * N / ntiles;
+    int64_t huge = 2 * most > HUGE_LIST ? 2 * most : HUGE_LIST;
+    if (N <= SPLIT_MIN) most = huge = NONE;
+    L.most = (int32_t)(most < NONE ? most : NONE);
+    L.huge = (int32_t)(huge < NONE ? huge : NONE);
+}
+
 // The same for the energy and its adjoint: the tiles' lists and the block partials.
 struct AdjointBufs {
-    int32_t *cnt = nullptr, *fill = nullptr, *cell = nullptr, *list = nullptr;
-    ListPlace *base = nullptr, *cursor = nullptr;
-    double *vpart = nullptr, *bpart = nullptr;
-    int gt = 0, gb = 0;
+    TileCounters C{};
+    int32_t *cell = nullptr, *list = nullptr;
+    ListPlace *base = nullptr;
+    LongTiles longs{};
+    double *vpart = nullptr, *bpart = nullptr, *lpart = nullptr;
+    int gt = 0, gb = 0, gl = 0;     // blocks of k_e_tile, k_e_bead, k_e_split (0: not used)
 };
 
 size_t adjoint_carve(const EModel &M, const TileGeom &T, char *base, AdjointBufs &Bf)
@@ -749,15 +1022,26 @@ size_t adjoint_carve(const EModel &M, const TileGeom &T, char *base, AdjointBufs
         return p;
     };
     Bf.gt = T.ntiles < TILE_BLOCKS ? T.ntiles : TILE_BLOCKS;
-    Bf.gb = grid_blocks(M.N);
-    Bf.cnt = (int32_t *)take(sizeof(int32_t) * T.ntiles);
-    Bf.fill = (int32_t *)take(sizeof(int32_t) * T.ntiles);
+    Bf.gb = grid_blocks(M.N) < FINAL_READ ? grid_blocks(M.N) : FINAL_READ;
+    Bf.C.n = T.ntiles;
+    Bf.C.cnt = (int32_t *)take(sizeof(int32_t) * T.ntiles);
+    Bf.C.fill = (int32_t *)take(sizeof(int32_t) * T.ntiles);
     Bf.base = (ListPlace *)take(sizeof(ListPlace) * T.ntiles);
-    Bf.cursor = (ListPlace *)take(sizeof(ListPlace));
+    Bf.C.cursor = (ListPlace *)take(sizeof(ListPlace));
     Bf.cell = (int32_t *)take(sizeof(int32_t) * M.N);
     Bf.list = (int32_t *)take(sizeof(int32_t) * M.N * tile_images(T));
     Bf.vpart = (double *)take(sizeof(double) * MAXT * Bf.gt);
     Bf.bpart = (double *)take(sizeof(double) * MAXT * Bf.gb);
+    const size_t groups = (size_t)((T.ntiles + LONG_GROUP - 1) / LONG_GROUP);
+    Bf.longs.tile = (int32_t *)take(sizeof(int32_t) * LONG_GROUP * groups);
+    Bf.longs.count = (int32_t *)take(sizeof(int32_t) * groups);
+    Bf.C.split = (int32_t *)take(sizeof(int32_t));
+    Bf.C.ticket = (int32_t *)take(sizeof(int32_t));
+    long_list(M.N, T.ntiles, Bf.longs);
+    // (all lists hold about two entries per bead)
+    const int64_t parts = TILE_PARTS * (2 * M.N / Bf.longs.most + 1);
+    Bf.gl = M.N <= SPLIT_MIN ? 0 : (parts < PART_BLOCKS ? (int)parts : PART_BLOCKS);
+    Bf.lpart = (double *)take(sizeof(double) * MAXT * Bf.gl);
     return o;
 }
 
@@ -775,15 +1059,22 @@ template <int B>
 void launch_adjoint(const EModel &M, const TileGeom &T, const double *r, const double *theta, double *E, double *grad,
                     double *gtheta, const AdjointBufs &Bf, hipStream_t st)
 {
-    if (grad)
-        hipLaunchKernelGGL((k_e_tile<B, true>), dim3(Bf.gt), dim3(TILE_THREADS), 0, st, M, T, theta, r, Bf.cnt, Bf.base,
-                           Bf.list, grad, Bf.vpart);
-    else
-        hipLaunchKernelGGL((k_e_tile<B, false>), dim3(Bf.gt), dim3(TILE_THREADS), 0, st, M, T, theta, r, Bf.cnt,
-                           Bf.base, Bf.list, grad, Bf.vpart);
-    hipLaunchKernelGGL(k_e_bead<B>, dim3(Bf.gb), dim3(EB), 0, st, M, theta, r, grad, Bf.bpart);
-    hipLaunchKernelGGL(k_e_final<B>, dim3(1), dim3(FINAL_THREADS), 0, st, M, theta, Bf.vpart, Bf.gt,
-                       B + B * (B - 1) / 2 + 2, Bf.bpart, Bf.gb, 2 + 2 * B, E, gtheta);
+    const auto go = [&](auto GRAD) {
+        constexpr bool G = decltype(GRAD)::value;
+        hipLaunchKernelGGL((k_e_tile<B, G>), dim3(Bf.gt), dim3(TILE_THREADS), 0, st, M, T, theta, r, Bf.C, Bf.base,
+                           Bf.list, Bf.longs, grad, Bf.vpart);
+        hipLaunchKernelGGL(k_e_bead<B>, dim3(Bf.gb), dim3(EB), 0, st, M, theta, r, grad, Bf.bpart);
+        constexpr int NV = B + B * (B - 1) / 2 + 2, NB = 2 + 2 * B;
+        if (Bf.gl == 0)
+            hipLaunchKernelGGL(k_e_final<B>, dim3(1), dim3(FINAL_THREADS), 0, st, M, theta, Bf.vpart, Bf.gt, NV, Bf.bpart,
+                               Bf.gb, NB, E, gtheta);
+        else
+            hipLaunchKernelGGL((k_e_split<B, G>), dim3(Bf.gl), dim3(PART_THREADS), 0, st, M, T, theta, r, Bf.cell, Bf.C,
+                               Bf.base, Bf.list, Bf.longs, grad, Bf.lpart, Bf.vpart, Bf.gt, NV, Bf.bpart, Bf.gb, NB, E,
+                               gtheta);
+    };
+    if (grad) go(std::true_type{});
+    else go(std::false_type{});
 }
 
 // E, dE/dr and dE/dtheta of M at (r, theta) with the buffers Bf.
@@ -794,12 +1085,13 @@ int energy_adjoint_run(const EModel &M, const TileGeom &T, const double *d_r, co
     const unsigned gb = (unsigned)((M.N + BIN_THREADS - 1) / BIN_THREADS), gt = (unsigned)((T.ntiles + 255) / 256);
     // cleared by a kernel rather than hipMemsetAsync: a caller may capture this
     // sequence in a HIP graph
-    hipLaunchKernelGGL(k_tile_clear, dim3(gt), dim3(256), 0, st, Bf.cnt, Bf.fill, Bf.cursor, T.ntiles);
-    hipLaunchKernelGGL(k_tile_bin<false>, dim3(gb), dim3(BIN_THREADS), 0, st, M.G, T, M.N, P, Bf.cell, Bf.cnt,
-                       (const ListPlace *)nullptr, (int32_t *)nullptr);
-    hipLaunchKernelGGL(k_tile_base, dim3(gt), dim3(256), 0, st, Bf.cnt, Bf.base, Bf.cursor, T.ntiles);
-    hipLaunchKernelGGL(k_tile_bin<true>, dim3(gb), dim3(BIN_THREADS), 0, st, M.G, T, M.N, P, Bf.cell, Bf.fill, Bf.base,
-                       Bf.list);
+    hipLaunchKernelGGL(k_tile_clear, dim3(gt), dim3(256), 0, st, Bf.C);
+    hipLaunchKernelGGL(k_tile_bin<false>, dim3(gb), dim3(BIN_THREADS), 0, st, M.G, T, M.N, P, Bf.cell, Bf.C.cnt,
+                       (const ListPlace *)nullptr, (int32_t *)nullptr, SplitBeads{});
+    static_assert(LONG_GROUP == 256, "the grid gt");
+    hipLaunchKernelGGL(k_tile_base, dim3(gt), dim3(LONG_GROUP), 0, st, Bf.C, Bf.base, Bf.longs);
+    hipLaunchKernelGGL(k_tile_bin<true>, dim3(gb), dim3(BIN_THREADS), 0, st, M.G, T, M.N, P, Bf.cell, Bf.C.fill, Bf.base,
+                       Bf.list, SplitBeads{Bf.C, Bf.longs, d_grad_r});
     switch (M.B) {
     case 1: launch_adjoint<1>(M, T, d_r, d_theta, d_E, d_grad_r, d_grad_theta, Bf, st); break;
     case 2: launch_adjoint<2>(M, T, d_r, d_theta, d_E, d_grad_r, d_grad_theta, Bf, st); break;

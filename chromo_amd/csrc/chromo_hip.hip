@@ -524,8 +524,8 @@ int density_jobs(const chromo_replica *h, int32_t n_reps, std::vector<ScatterJob
 }
 
 // Jobs run together while their scratch stays below this (a single larger one alone),
-// at most 65535 (grid rows) at a time: a run's scratch is bounded by its largest job or
-// this, not by the number of replicas.
+// at most DENSITY_GROUP_JOBS (grid rows, which may number 65535) at a time: a run's scratch
+// is bounded by its largest job or this, not by the number of replicas.
 constexpr size_t DENSITY_GROUP_BYTES = size_t(1) << 30;
 constexpr size_t DENSITY_GROUP_JOBS = 4096;
 

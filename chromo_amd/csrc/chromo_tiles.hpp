@@ -8,7 +8,8 @@
 // and their upper neighbours.  One block per tile then does what took four passes over
 // memory: it adds the beads' corner weights into LDS, turns each voxel's density into
 // its energy terms and dE/drho in place, and gathers dE/drho back at the beads of its
-// own cells.  Neither the densities nor dE/drho ever reach HBM.
+// own cells.  Neither the densities nor dE/drho ever reach HBM.  Where a condensed chain
+// crowds a few tiles, those are worked on in parts, a block per part.
 //
 // What bounds it: at 10^6 beads, B = 4, 128^3 voxels a third of the time is the adds (8
 // corners x species x 2 words per bead and tile, a third of them conflicting), a quarter
@@ -16,30 +17,37 @@
 // the barriers between; two blocks of eight wavefronts share a compute unit's LDS.
 // Tiles of 8 x 8 x 4 with four smaller blocks take the same time (less waiting, more
 // halo).  One evaluation there: 417 us as bucketed records, a gather of every record by
-// its eight voxels and passes for the voxel and bead terms; 280 us so.
+// its eight voxels and passes for the voxel and bead terms; 259 us so.
 #pragma once
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
 #include "chromo_device.hpp"
+#include "chromo_index.hpp"
 
 namespace chromo {
 namespace {
 
-// Tiles of at most 8 x 8 x 8 voxels.  Tile t of an axis of n voxels cut into nt tiles
-// starts at t n / nt: tiles of at least half the size when there are several, so a cell
-// touches at most one face per axis and the lists hold at most twice the beads per axis.
-// An axis that fits one tile is one tile that wraps onto itself.
-// The scatter needs no upper neighbours, and smaller tiles keep more wavefronts on a
-// compute unit.
+// The adjoint's tiles have at most 8 x 8 x 8 voxels (TILE_MAX).  Tile t of an axis of n
+// voxels cut into nt tiles starts at t n / nt: tiles of at least half the size when there
+// are several, so a cell touches at most one face per axis and the lists hold at most twice
+// the beads per axis.  An axis that fits one tile is one tile that wraps onto itself.
+// The scatter (FOLD_MAX and smaller) needs no upper neighbours, and smaller tiles keep more
+// wavefronts on a compute unit; a cell of its one-voxel tiles touches both faces, and only
+// the upper one counts.
 constexpr int TILE_MAX[3] = {8, 8, 8};
+static_assert((TILE_MAX[0] + 1) / 2 >= 2 && (TILE_MAX[1] + 1) / 2 >= 2 && (TILE_MAX[2] + 1) / 2 >= 2,
+              "a cell of a tile that also lists its upper neighbours lies on one face");
 constexpr int FOLD_MAX[3] = {4, 4, 4};
-constexpr int TILE_SX = 9, TILE_SY = 9, TILE_SZ = 9;    // a tile's voxels and their upper neighbours
-constexpr int TILE_VOX = TILE_SX * TILE_SY * TILE_SZ;
 constexpr int TILE_THREADS = 512;
 constexpr int TILE_OWN = 1024;              // beads of its own cells a tile notes down in LDS
 constexpr int TILE_BLOCKS = 1024;           // blocks of the tile kernel, at most
+constexpr int LONG_LIST = 2048, HUGE_LIST = 8192;       // beads of a list (long_list)
+constexpr int SPLIT_MIN = 4 * HUGE_LIST;    // beads of a chain whose lists are never split
+constexpr int TILE_PARTS = 8;               // of a tile with a long list
+constexpr int PART_THREADS = 512, PART_SCAN = 4, PART_NOTES = 4096;
+constexpr int PART_BLOCKS = 512;            // two per compute unit
 
 struct TileGeom {
     int32_t n[3], nt[3], ntiles;
@@ -92,9 +100,6 @@ inline int tile_images(const TileGeom &T)
     return k;
 }
 
-__device__ __forceinline__ int tile_start(int n, int nt, int t) { return (int)((int64_t)t * n / nt); }
-__device__ __forceinline__ int tile_of(int n, int nt, int c) { return (int)(((int64_t)(c + 1) * nt - 1) / n); }
-
 // grid_lower's cell and weights (chromo_density.hpp), bit for bit, with the exact
 // divisions from reciprocals where the grid allows.
 __device__ __forceinline__ void tile_lower(const GridGeom &G, const TileGeom &T, const double *x, int ix[3],
@@ -130,37 +135,41 @@ __device__ __forceinline__ void tile_lower(const GridGeom &G, const TileGeom &T,
     }
 }
 
-// The tiles of one axis that list a bead of cell c: its own and, when the cell lies on
-// a face, the neighbour behind that face (UPPER: behind either face, for tiles that
-// need their voxels' upper neighbours; else only behind the upper one, whose voxels the
-// bead's upper corners reach).  Returns how many.
-template <bool UPPER>
-__device__ __forceinline__ int axis_tiles(int n, int nt, int c, int t[2])
-{
-    t[0] = nt == 1 ? 0 : tile_of(n, nt, c);
-    t[1] = t[0];
-    if (nt == 1) return 1;
-    if (UPPER && c == tile_start(n, nt, t[0])) {
-        t[1] = t[0] == 0 ? nt - 1 : t[0] - 1;
-        return 2;
-    }
-    if (c + 1 == tile_start(n, nt, t[0] + 1)) {
-        t[1] = t[0] + 1 == nt ? 0 : t[0] + 1;
-        return 2;
-    }
-    return 1;
-}
-
 // Where a list begins in the array of all lists, which hold a bead up to eight times: 64
 // bits (268,435,456 beads in one-voxel tiles pass 2^31 entries).
 using ListPlace = unsigned long long;
 
-// Clears the lists' counters and the list cursor.
-__global__ void k_tile_clear(int32_t *cnt, int32_t *fill, ListPlace *cursor, int n)
+// What a count of the lists starts from: their lengths, the entries placed, the end of the
+// last list, whether long lists are split, and a ticket.
+struct TileCounters {
+    int32_t *cnt, *fill, *split, *ticket;
+    ListPlace *cursor;
+    int32_t n;
+};
+
+__global__ void k_tile_clear(TileCounters C)
 {
     const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-    if (i < n) cnt[i] = fill[i] = 0;
-    if (i == 0) *cursor = 0;
+    if (i < C.n) C.cnt[i] = C.fill[i] = 0;
+    if (i == 0) {
+        *C.cursor = 0;
+        *C.split = 0;
+        *C.ticket = 0;
+    }
+}
+
+// The long lists, of more than `most` beads, in tile order per block of k_tile_base: tiles
+// tile[LONG_GROUP g + k] for k < count[g].  They are split where one holds more than `huge`.
+constexpr int LONG_GROUP = 256, LONG_GROUPS = 2048;     // 2^22 voxels make 2^19 tiles at most
+struct LongTiles {
+    int32_t *tile, *count;
+    int32_t most, huge;
+};
+
+// Beads of a list from which on it is split; known once k_tile_base is done.
+__device__ __forceinline__ int32_t split_above(const TileCounters &C, const LongTiles &L)
+{
+    return uni_i32(*C.split) ? L.most : 0x7fffffff;
 }
 
 // Room for every list: a wavefront's lists in a row, the wavefronts in the order they
@@ -180,9 +189,25 @@ __device__ __forceinline__ void tile_bases(const int32_t *cnt, ListPlace *base, 
     if (i < n) base[i] = at + (ListPlace)(sum - k);
 }
 
-__global__ void k_tile_base(const int32_t *cnt, ListPlace *base, ListPlace *cursor, int n)
+__global__ void __launch_bounds__(LONG_GROUP)
+k_tile_base(TileCounters C, ListPlace *base, LongTiles L)
 {
-    tile_bases(cnt, base, cursor, n);
+    tile_bases(C.cnt, base, C.cursor, C.n);
+    __shared__ int32_t waves[LONG_GROUP / WAVE];
+    const int i = (int)(blockIdx.x * LONG_GROUP + threadIdx.x), w = (int)threadIdx.x / WAVE;
+    const int len = i < C.n ? C.cnt[i] : 0;
+    int mine;
+    int at = wave_excl_count(len > L.most, mine);
+    if (lane_id() == 0) waves[w] = mine;
+    if (len > L.huge) atomicOr(C.split, 1);
+    __syncthreads();
+    int all = 0;
+    for (int k = 0; k < LONG_GROUP / WAVE; ++k) {
+        at += k < w ? waves[k] : 0;
+        all += waves[k];
+    }
+    if (len > L.most) L.tile[(int)blockIdx.x * LONG_GROUP + at] = i;
+    if (threadIdx.x == 0) L.count[blockIdx.x] = all;
 }
 
 // PLACE false: each bead's cell into cell[], and the lists' lengths into num.  PLACE
@@ -191,17 +216,26 @@ __global__ void k_tile_base(const int32_t *cnt, ListPlace *base, ListPlace *curs
 // global atomic; a list that finds no room in the block's table takes its entries from
 // the global counter one by one.  STABLE: what a block places in a list through its
 // table is in bead order (a bit per bead and list in LDS, the rank the bits below).
-// Otherwise the order within a list is any.
+// Otherwise the order within a list is any.  UPPER: a bead whose own tile's list is split
+// gets a zero field gradient.
 constexpr int TILE_TABLE = 512, TILE_PROBES = 16, BIN_THREADS = 256;
+
+struct SplitBeads {
+    TileCounters C;
+    LongTiles L;
+    double *grad;           // N x 3, or nullptr
+};
 
 template <bool PLACE, bool UPPER, bool STABLE>
 __device__ __forceinline__ void tile_bin(const GridGeom &G, const TileGeom &T, int64_t N, const PosView &P,
-                                         int32_t *cell, int32_t *num, const ListPlace *base, int32_t *list)
+                                         int32_t *cell, int32_t *num, const ListPlace *base, int32_t *list,
+                                         const SplitBeads &X = SplitBeads{})
 {
     constexpr int W = BIN_THREADS / WAVE;
     __shared__ int32_t key[TILE_TABLE], cntl[TILE_TABLE], from[TILE_TABLE];
     __shared__ unsigned long long bits[STABLE && PLACE ? TILE_TABLE * W : 1];
     const int t = (int)threadIdx.x, wv = t / WAVE, lane = t % WAVE;
+    const int32_t most = PLACE && UPPER ? split_above(X.C, X.L) : 0;
     for (int i = t; i < TILE_TABLE; i += BIN_THREADS) {
         key[i] = -1;
         cntl[i] = 0;
@@ -258,6 +292,7 @@ __device__ __forceinline__ void tile_bin(const GridGeom &G, const TileGeom &T, i
             if (STABLE && PLACE)
                 for (int w = 0; w < W; ++w) n += __popcll(bits[i * W + w]);
             from[i] = atomicAdd(&num[key[i]], n);
+            if (PLACE && UPPER) cntl[i] = X.C.cnt[key[i]] > most;
         }
     if (!PLACE) return;
     __syncthreads();
@@ -274,23 +309,17 @@ __device__ __forceinline__ void tile_bin(const GridGeom &G, const TileGeom &T, i
         }
         list[at] = (int32_t)b;
     }
+    // entry 0 is the bead's own tile
+    if (UPPER && X.grad && tile[0] >= 0 && (slot[0] >= 0 ? cntl[slot[0]] != 0 : X.C.cnt[tile[0]] > most))
+        for (int j = 0; j < 3; ++j) X.grad[3 * b + j] = 0;
 }
 
 template <bool PLACE>
 __global__ void __launch_bounds__(BIN_THREADS) k_tile_bin(GridGeom G, TileGeom T, int64_t N, PosView P, int32_t *cell,
-                                                          int32_t *num, const ListPlace *base, int32_t *list)
+                                                          int32_t *num, const ListPlace *base, int32_t *list,
+                                                          SplitBeads X)
 {
-    tile_bin<PLACE, true, false>(G, T, N, P, cell, num, base, list);
-}
-
-// Place of a cell on one axis of a tile of `size` voxels from `start`: 0 .. size - 1
-// inside, -1 and size for the neighbours below and above.
-__device__ __forceinline__ int tile_local(int n, int start, int size, int c)
-{
-    int d = c - start;
-    if (d >= 0 && d < size) return d;
-    if (d < 0) d += n;
-    return d == size ? size : -1;
+    tile_bin<PLACE, true, false>(G, T, N, P, cell, num, base, list, X);
 }
 
 }  // namespace

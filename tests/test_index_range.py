@@ -28,10 +28,10 @@ def test_bead_rows(tmp_path):
 
 
 def test_kernels_index_beads_through_it():
-    """The tile kernel holds beads in 32 bits: no product of one with 3 outside row3."""
+    """The tiles' code holds beads in 32 bits: no product of one with 3 outside row3."""
     src = (ROOT / "chromo_amd" / "csrc" / "chromo_energy.hip").read_text()
-    tile = src[src.index("k_e_tile(EModel"):src.index("// ---- bead / bond terms")]
-    assert "3 * b" not in tile and tile.count("row3(b, j)") == 3
+    tile = src[src.index("// ---- field terms"):src.index("// ---- bead / bond terms")]
+    assert "int32_t b" in tile and "3 * b" not in tile and tile.count("row3(b, j)") >= 3
 
 
 def test_list_places_have_64_bits():
