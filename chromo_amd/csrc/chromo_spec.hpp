@@ -1322,6 +1322,8 @@ __device__ __forceinline__ void spec_run(const chromo_replica *R, const EvConst 
     }
     __syncthreads();
     if (gen) {
+        // after a wait that passed its bound there may be committed slots left to book
+        book_to<RING>(R, g, sctrl, sK, L, ctl->resolved);
         rng_store(R, g.rng, need_mt);
         if (lane == 0)
             for (int i = 0; i < g.nc; ++i) R->ctrl[i] = sctrl[i];
