@@ -17,13 +17,12 @@ from chromo_amd import workloads as W
 
 pytestmark = pytest.mark.gpu
 
-# Eight and four wavefronts per replica: an earlier source of those shapes faulted the
-# GPU (8) and hung and gave wrong voxel counts (4), with no cause found.  The current
-# source cannot build them: the speculative round's flags have one wavefront on each
-# side, and the per-wavefront LDS blocks are sized for two.  The entry point rejects
-# both; these cases stay as skips until a design for more wavefronts exists.
-W8_SKIP = "waves_per_replica = 8 is not built (two-wavefront round protocol); an earlier build faulted"
-W4_SKIP = "waves_per_replica = 4 is not built (two-wavefront round protocol); an earlier build hung"
+# waves_per_replica = 8 and 4: the entry point refuses both (2 asks for the speculative
+# kernel, which takes two or four wavefronts by itself).  Earlier sources of such shapes
+# faulted the GPU (8) and hung and gave wrong voxel counts (4), with no cause found;
+# nothing of that code is left.  These cases cover nothing today and stay as skips.
+W8_SKIP = "waves_per_replica = 8 is refused by the entry point; an earlier build of it faulted"
+W4_SKIP = "waves_per_replica = 4 is refused by the entry point; an earlier build of it hung"
 P4 = pytest.param(4, marks=pytest.mark.skip(reason=W4_SKIP))
 
 
@@ -54,8 +53,7 @@ def _dE_close(a, b):
 
 # ---------------------------------------------------------------- density ---
 
-# 96^3 voxels reach the gather that ranks voxels inside 1024-voxel blocks (grids of
-# at least 512 such blocks); the others use 256-voxel blocks
+# 96^3 voxels are folded in tiles of 4 x 4 x 4, the others in tiles of one voxel
 @pytest.mark.parametrize("N,nvox,seed", [(300, 7, 0), (2000, 16, 1), (5000, 12, 2), (64, 1, 3),
                                          (64, 2, 4), (1000, 5, 5), (200000, 96, 6)])
 def test_density_init_bitwise(oracle, N, nvox, seed):
@@ -330,9 +328,9 @@ def test_batched_equals_single(oracle):
 
 
 def test_density_init_many_beads_per_voxel(oracle):
-    """10^5 beads on a 4^3 grid (about 1,600 beads in every bucket): the buckets
-    are put in bead order by heapsort, and the scatter stays bitwise the
-    reference's bead-order loop."""
+    """10^5 beads on a 4^3 grid (one-voxel tiles with some 12,500 beads listed in each): lists
+    of more runs than the fold ranks in LDS are sorted in global memory, and the scatter
+    stays bitwise the reference's bead-order loop."""
     say("density_init 1e5 beads on 4^3")
     s = W.make_system(100000, 2, 4, seed=7)
     s.chain.states = np.random.RandomState(7).randint(0, 3, size=(100000, 2))

@@ -1,7 +1,8 @@
-"""The initial densities, bit for bit against the oracle's bead-order loop, on grids at
-the edges of the scatter's tiles (8 x 8 x 4 voxels): one-voxel axes (corners of a bead
-share a voxel), one tile that wraps onto itself, two tiles, ragged tiles; tiles whose
-bead lists pass what is sorted in LDS; every binder count; many replicas in one call."""
+"""The initial densities, bit for bit against the oracle's bead-order loop, on small and
+uneven grids, which the scatter folds in tiles of one voxel or 2 x 2 x 2 (the larger
+shapes: test_gpu_scatter_shapes.py): one-voxel axes (corners of a bead share a voxel),
+axes of two voxels, ragged tiles; lists of so many runs that they are sorted in global
+memory; every binder count; many replicas in one call."""
 import copy
 
 import numpy as np
