@@ -31,7 +31,7 @@
 // per-voxel fold lists (hash, position masks, numbering, dealing by length, list
 // building, divergent folds; moves above 32 beads one at a time): 512 replicas of
 // 2,000-20,000 beads at steady-state windows, 20 sweeps, two wavefronts each,
-// 50.4 -> 33.1 ms when it came in (30.2 ms now, with the slots of chromo_spec.hpp);
+// 50.4 -> 33.1 ms when it came in (30.2 to 30.9 ms now, with the slots of chromo_spec.hpp);
 // 16 replicas with one wavefront each, 10 sweeps, 25.1 -> 20.2 ms.
 #pragma once
 

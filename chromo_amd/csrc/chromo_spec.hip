@@ -63,8 +63,8 @@ hipError_t launch(const chromo_replica *d_reps, int n_reps, int64_t steps, hipSt
 
 // Four wavefronts per replica where every replica can have a compute unit of its own
 // (the block of three evaluators takes most of a unit's LDS), two otherwise.  128
-// replicas of 1,500-9,000 beads, B = 3, initial windows, 10 sweeps: 13.8 ms with one
-// wavefront each, 5.2 with four; one twisting chain, steady-state windows: 19.2 ms with
+// replicas of 1,500-9,000 beads, B = 3, the first 10 sweeps: 13.8 ms with one wavefront
+// each, 5.4 with four (6.3 for later ones, at wider windows); one twisting chain, steady-state windows: 19.2 ms with
 // one, 9.3 with four.
 template <bool TW>
 hipError_t launch_shape(const chromo_replica *d_reps, int n_reps, int64_t steps, hipStream_t st)

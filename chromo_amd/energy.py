@@ -154,6 +154,13 @@ class ChromoEnergy(torch.autograd.Function):
 
 
 def chromo_energy(r: torch.Tensor, theta: torch.Tensor, model: EnergyModel) -> torch.Tensor:
+    """E(r, theta), differentiable.
+
+    Where autograd would record the call (grad mode on and r or theta requires a
+    gradient), this evaluation takes dE/dr and dE/dtheta at once and keeps dE/dr (24 N
+    bytes) with the graph, also when theta alone needs one.  For E without its gradients
+    call it under ``torch.no_grad()``, or ``energy(model, r, theta, grad=False)``.
+    """
     return ChromoEnergy.apply(r, theta, model, torch.is_grad_enabled() and (r.requires_grad or theta.requires_grad))
 
 

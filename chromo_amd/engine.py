@@ -406,7 +406,8 @@ class DeviceReplicas:
     def run(self, num_steps: int, *, sync: bool = True, waves: Optional[int] = None) -> None:
         """mc_sim for every replica in one persistent launch, with ``waves``
         wavefronts per replica (default: ``self.waves``).  The result does not
-        depend on ``waves``."""
+        depend on ``waves``.  Beside a twisting chain every chain is launched with 1: the
+        others are faster in a DeviceReplicas of their own."""
         w = int(self.waves if waves is None else waves)
         if self.twist:
             w = 1       # the C entry takes twisting chains only so (their kernel is speculative all the same)
